@@ -36,6 +36,12 @@ FLAGS = [
     "-I" + CSRC,
 ]
 
+# The batched kernels keep a trajectory's whole state in registers.  Hoisted out
+# of their step loops, the constants of the step control and what follows from
+# each literal code took up to twice the state's registers and spilled it
+# (256 threads, one clause and one variable each: 161 registers, 80 without).
+FILE_FLAGS = {"asat_batch.hip": ["-mllvm", "-disable-machine-licm"]}
+
 
 def _run(cmd, verbose):
     if verbose:
@@ -50,7 +56,7 @@ def build(verbose=False):
     os.makedirs(OBJDIR, exist_ok=True)
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
     objs = [os.path.join(OBJDIR, os.path.splitext(s)[0] + ".o") for s in srcs]
-    jobs = [[HIPCC] + FLAGS + ["-c", "-o", o, os.path.join(CSRC, s)] for s, o in zip(srcs, objs)]
+    jobs = [[HIPCC] + FLAGS + FILE_FLAGS.get(s, []) + ["-c", "-o", o, os.path.join(CSRC, s)] for s, o in zip(srcs, objs)]
     with concurrent.futures.ThreadPoolExecutor(max(1, min(len(jobs), os.cpu_count() or 1))) as ex:
         for f in [ex.submit(_run, j, verbose) for j in jobs]:
             f.result()

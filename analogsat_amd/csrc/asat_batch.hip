@@ -15,11 +15,11 @@
 //   var phase:    each thread takes variables i = tid, tid+BS, ...; sums its
 //     contiguous run of contributions in slot order (the reference's
 //     accumulation order), writes k_J(s_i) and the next stage's spin input
-// For instances whose contributions do not fit in LDS, the clause-chunked
-// mode keeps no contribution array: per chunk of clauses the clause phase
-// leaves r_m in LDS, and each variable forms its terms of that chunk from
-// 8-byte var-major records (the clause, the sign, the other literals) and
-// adds them in the same order.
+// Instances that fit run in k_batch_reg, which keeps state and stage
+// derivatives in registers and contributions in LDS; instances whose
+// contributions do not fit in LDS run in k_batch_chunk, which takes the clauses
+// in chunks whose contributions do.  k_batch is the general form (contributions
+// in LDS or in global scratch).
 // Stage 6 forms x_new and |xerr/xscal|, a block FP64 max feeds the step
 // controller (thread 0, FP64, correctly rounded pow), which accepts (parity
 // flip) or rejects (retry with smaller h).  After each accepted step the
@@ -43,6 +43,7 @@
 #include <cstring>
 #include <memory>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 namespace asat {
@@ -61,17 +62,14 @@ struct Desc {                 // one instance / trajectory (device)
     long long code_off;       // into code[]
     long long row_off;        // into rowptr[]
     long long state_off;      // into xa[]/xb[] (N spins then M aux)
-    long long vcode_off;      // into vcode[] (clause-chunked mode; -1: not built)
+    long long rcode_off, rgroup_off, rvmap_off;   // register kernel's layout (-1: not built)
+    long long ccode_off, cgroup_off, crec_off, cstart_off;   // chunked kernel's layout (-1: not built)
     int n, m, k, nslots;      // nslots = number of contributions (non-padding slots)
     float knorm;
+    int ngroups, ncontrib;    // register kernel: groups of 64 ranks, contribution entries
+    int nchunks, chunk;       // chunked kernel: chunks, clauses per chunk
     int pad_;
 };
-
-// Clause-chunked mode: one 64-bit record per contribution, in var-major
-// order: bits 0..17 the clause, bit 18 the literal's sign, then the k - 1
-// other literals of the clause in clause order, 14 bits each (variable << 1
-// | negated; variable 0 = padding).
-constexpr int VC_OTHER_SHIFT = 19;
 
 struct TrajCtrl {             // persistent per-trajectory control (device)
     double t, h, hnext, hdid, errmax, sat_time;
@@ -99,17 +97,21 @@ struct Params {
     int chunk_steps;
     int check_every;         // take the violation count every this many accepted steps
     int sp_stride;           // floats reserved for the stage spins at the start of LDS
-    const unsigned long long* vcode;   // clause-chunked mode: var-major contribution records
-    int chunk_clauses;       // clause-chunked mode: clauses per chunk (LDS for their r_m)
+    const uint32_t* rcode;   // register kernel: literal codes, base and depth per group, rank -> variable
+    const int* rgroup;
+    const int* rvmap;
+    const uint2* ccode;      // chunked kernel: literal codes of a clause, (base, depth) per group of 64
+    const int2* cgroup;      // variables, its variables, their term indices (two per word), first
+    const uint16_t* cperm;   // group of each chunk
+    const uint32_t* crec;
+    const int* cstart;
+    int reg_lds;             // register kernel: LDS bytes of one trajectory
+    int chunk_terms;         // chunked kernel: term entries in LDS (the one after holds 0)
+    int fac_ranks;           // chunked kernel: factor pairs, then sums reserved in LDS
 };
 
 // ---------------------------------------------------------------------------
-// MODE 0: contributions in the workgroup's global scratch; 1: in LDS; 3:
-// clause-chunked, no contribution array: per chunk of clauses, the clause
-// phase leaves r_m = K_m knorm a_m in LDS and every variable walks on
-// through its contribution records of that chunk, forming each term
-// r_m * (product of the other factors) * (+-2) and adding it in the same
-// order as the other modes (LDS: spins, running sums, record cursors, r_m).
+// MODE 0: contributions in the workgroup's global scratch; 1: in LDS.
 template <int BS, int MODE>
 __global__ __launch_bounds__(BS) void k_batch(Params P)
 {
@@ -145,11 +147,6 @@ __global__ __launch_bounds__(BS) void k_batch(Params P)
         const uint32_t* code = P.code + d.code_off;
         const int* rowptr = P.rowptr + d.row_off;
         float* contrib = MODE == 1 ? (lds + P.sp_stride) : (scratch + 5 * P.scratch_stride);
-        float* vsum = lds + P.sp_stride;                          // MODE 3
-        int* vcur = (int*)(lds + 2 * P.sp_stride);                // MODE 3
-        float* rl = lds + 3 * P.sp_stride;                        // MODE 3
-        const unsigned long long* vcode = MODE == 3 ? P.vcode + d.vcode_off : nullptr;
-        const int chunk = MODE == 3 ? P.chunk_clauses : m;
         const float knorm = d.knorm;
         // scratch layout per k vector: spins at [0, n), aux at [n, n+m)
         double t = cp->t, h = cp->h, hnext = cp->hnext, hdid = cp->hdid, errmax_last = cp->errmax;
@@ -174,10 +171,8 @@ __global__ __launch_bounds__(BS) void k_batch(Params P)
                 double err_local = 0.0;
 #pragma unroll 1
                 for (int J = first_attempt ? 1 : 2; J <= 6; J++) {
-                  for (int c0 = 0; c0 < m; c0 += chunk) {
-                    const int c1 = min(m, c0 + chunk);
-                    // ---------------- clause phase (MODE 3: one chunk of clauses)
-                    for (int j = c0 + tid; j < c1; j += BS) {
+                    // ---------------- clause phase
+                    for (int j = tid; j < m; j += BS) {
                         const uint32_t* cj = code + (long long)j * k;
                         float f[KMAX];
                         uint32_t cc[KMAX];
@@ -230,81 +225,27 @@ __global__ __launch_bounds__(BS) void k_batch(Params P)
                         }
                         }
                         const float r = km * knorm * am;
-                        if constexpr (MODE == 3) {
-                            rl[j - c0] = r;
-                        } else {
 #pragma unroll
-                            for (int q = 0; q < KMAX; q++) {
-                                if (q < k && (cc[q] >> 19) != 0) {
-                                    float p = 1.0f;
-                                    bool first = true;
+                        for (int q = 0; q < KMAX; q++) {
+                            if (q < k && (cc[q] >> 19) != 0) {
+                                float p = 1.0f;
+                                bool first = true;
 #pragma unroll
-                                    for (int qq = 0; qq < KMAX; qq++) {
-                                        if (qq == q || qq >= k) continue;
-                                        p = first ? f[qq] : p * f[qq];
-                                        first = false;
-                                    }
-                                    float rr = r * p;
-                                    rr *= (cc[q] >> 18) & 1u ? -2.0f : 2.0f;
-                                    contrib[cc[q] & 0x3FFFFu] = rr;
+                                for (int qq = 0; qq < KMAX; qq++) {
+                                    if (qq == q || qq >= k) continue;
+                                    p = first ? f[qq] : p * f[qq];
+                                    first = false;
                                 }
+                                float rr = r * p;
+                                rr *= (cc[q] >> 18) & 1u ? -2.0f : 2.0f;
+                                contrib[cc[q] & 0x3FFFFu] = rr;
                             }
                         }
                     }
                     __syncthreads();
-                    if constexpr (MODE == 3) {
-                        // each variable's terms of this chunk, in record
-                        // (clause) order: the product of the other factors
-                        // as the clause phase forms it (KmiProd order)
-                        for (int i = tid; i < n; i += BS) {
-                            int e = c0 == 0 ? rowptr[i] : vcur[i];
-                            const int e1 = rowptr[i + 1];
-                            float sum = c0 == 0 ? 0.0f : vsum[i];
-                            bool more = e < e1;
-                            while (more) {
-                                // four records read ahead of the chunk-end test
-                                unsigned long long vb[4];
-#pragma unroll
-                                for (int u = 0; u < 4; u++) vb[u] = e + u < e1 ? vcode[e + u] : ~0ull;
-#pragma unroll
-                                for (int u = 0; u < 4; u++) {
-                                    if (!more) break;
-                                    const unsigned long long vc = vb[u];
-                                    const int j = (int)(vc & 0x3FFFFull);
-                                    if (e >= e1 || j >= c1) { more = false; break; }
-                                    float p = 1.0f;
-                                    bool first = true;
-                                    for (int t = 0; t < k - 1; t++) {
-                                        const unsigned o = (unsigned)(vc >> (VC_OTHER_SHIFT + 14 * t)) & 0x3FFFu;
-                                        const int v = (int)(o >> 1);
-                                        const float sv = v ? sp[v - 1] : -1.0f;
-                                        const float fo = (o & 1u) ? 1.0f + sv : 1.0f - sv;
-                                        p = first ? fo : p * fo;
-                                        first = false;
-                                    }
-                                    float rr = rl[j - c0] * p;
-                                    rr *= (vc >> 18) & 1ull ? -2.0f : 2.0f;
-                                    sum += rr;
-                                    e++;
-                                }
-                                more = more && e < e1;
-                            }
-                            vsum[i] = sum;
-                            vcur[i] = e;
-                        }
-                        __syncthreads();
-                    }
-                  }
                     // ---------------- var phase
                     for (int i = tid; i < n; i += BS) {
-                        float sum = 0.0f;
-                        if constexpr (MODE == 3) {
-                            sum = vsum[i];
-                        } else {
-                            const int e0 = rowptr[i], e1 = rowptr[i + 1];
-                            sum = sum_run(sum, contrib, e0, e1);
-                        }
-                        const float kj = sum;
+                        const float kj = sum_run(0.0f, contrib, rowptr[i], rowptr[i + 1]);
                         const float xi = x[i];
                         switch (J) {
                         case 1:
@@ -415,63 +356,197 @@ __global__ __launch_bounds__(BS) void k_batch(Params P)
 }
 
 // ---------------------------------------------------------------------------
-// Register-resident variant: thread tid owns clauses j = tid + u*BS (u < CPT)
-// and variables i = tid + v*BS (v < VPT) for the whole trajectory; their
-// state x and the stage derivatives k1..k5 live in registers, so a step
-// touches global memory only for the literal codes and row pointers (a few
-// hundred KB per trajectory, re-read every stage from L2).  The arithmetic
-// and its order are those of k_batch; x_new of the final stage goes to the
-// k2 registers, which the final combination does not read.
-template <int CPT, int VPT>
+// Register-resident variant: TT threads per trajectory, one workgroup of them,
+// or (TT = 64) a wave each in a workgroup of 256, which then needs no barriers.
+// Thread tid owns clauses j = tid + u*TT (u < CPT)
+// and the variables of rank tid + v*TT (v < VPT) for the whole trajectory;
+// their state x and the stage derivatives k1..k5 live in registers.  LDS holds
+// the stage factors and the contributions; a step touches global memory only
+// for the literal codes, and not even for those where they fit the registers
+// too.  The arithmetic and its order are those of k_batch; x_new of the final
+// stage goes to the k2 registers, which the final combination does not read.
+//
+// What bounds it is instruction issue and LDS, so the layout (reg_layout)
+// serves both:
+// - Variables are ranked by falling number of occurrences, so the 64 of one
+//   wave have nearly the same number, and a group of 64 keeps its
+//   contributions as rows of 64 (entry e of all 64 variables side by side):
+//   the sums read LDS without bank conflicts, without a bound per lane and
+//   with addresses that are constants past the group's base.  Missing entries
+//   hold -0.0, which changes no sum; every other entry is written again in
+//   every clause phase.
+// - The stage spins are kept as the two factors 1 - s and 1 + s, so a literal's
+//   factor is one LDS read at its code's low 16 bits.  Two ranks past the last
+//   variable are constants by the same rule: spin -1 (factor 2: a padding
+//   literal of a short clause) and spin 0 (factor 1: a literal beyond the
+//   instance's k, and the clauses that fill up the last wave).  Such literals
+//   store into an entry that nothing reads, so no slot needs a test.
+// - A code's low 16 bits are the byte address of its factor (8 rank + 4 if
+//   negated), its high 16 bits the index of its contribution.  Up to 2046
+//   variables bits 14 and 15 are zero and code >> 14 is that entry's byte
+//   address (WIDE = false); more variables shift twice.
+// - The violated-clause count of an accepted state is taken by the next step's
+//   first clause phase, whose factors already say s > 0 unless one is exactly 1.
+// Against the variable-major contribution runs before (a wave as slow as its
+// busiest variable, bank conflicts in the sums, 4 instructions to unpack a
+// slot), per 100 steps of 1024 trajectories with N = 2000, M = 8500: 26.0 ->
+// 14.7 ms; 1000 steps of 1000 with N = 50, M = 213: 10.8 -> 7.3 ms.
+constexpr int REG_WAVES = 4;     // TT = 64: trajectories (waves) per workgroup
+
+// a value every lane holds, moved to scalar registers
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ long long uni(long long v)
+{
+    return (long long)(((unsigned long long)(unsigned)uni((int)(v >> 32)) << 32) | (unsigned)uni((int)v));
+}
+__device__ __forceinline__ float uni(float v) { return __int_as_float(uni(__float_as_int(v))); }
+
+template <int TT>
+__device__ __forceinline__ int traj_tid()
+{
+    return TT == 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+}
+// LDS written before is seen by the trajectory's threads after.  One wave's
+// LDS accesses stay in order, so a wave alone only keeps the compiler to it.
+template <int TT>
+__device__ __forceinline__ void traj_sync()
+{
+    if constexpr (TT == 64) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+        __syncthreads();
+    }
+}
+// maximum and sum over the trajectory's threads, in every one of them; with
+// several waves two barriers each
+template <int TT>
+__device__ __forceinline__ double traj_max(double v, double* sh)
+{
+    v = wave_max_dpp(v);
+    if constexpr (TT == 64) return v;
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double r = sh[0];
+#pragma unroll
+    for (int i = 1; i < TT / 64; i++) r = fmax(r, sh[i]);
+    __syncthreads();
+    return r;
+}
+template <int TT>
+__device__ __forceinline__ int traj_sum(int v, int* sh)
+{
+    if constexpr (TT == 64) return wave_sum(v);
+    else return block_sum_all<TT>(v, sh);
+}
+
+template <int TT, int CPT, int VPT, int KK>
 struct RegState {
     float xa[CPT], a1[CPT], a2[CPT], a3[CPT], a4[CPT], a5[CPT];
     float xv[VPT], v1[VPT], v2[VPT], v3[VPT], v4[VPT], v5[VPT];
-    int e0[VPT], e1[VPT];
+    // registers of a thread at this workgroup size, less the state, the
+    // literal codes and about 36 for one clause's work
+    static constexpr int BUDGET = TT >= 1024 ? 128 : TT >= 768 ? 168 : 256;
+    static constexpr bool HOLD = CPT * (6 + KK) + VPT * 8 + 36 <= BUDGET;
+    uint32_t code[HOLD ? CPT : 1][KK];
 };
 
-// KK = 3 or 4: every instance of the launch has clauses of KK literal slots
-// (the code is compiled for that length); KK = 0: the length k is read at
-// run time (at most KMAX)
-template <int BS, int CPT, int VPT, int J, int KK>
-__device__ __forceinline__ void reg_stage(RegState<CPT, VPT>& R, const uint32_t* code, int n, int m, int k,
-                                          float knorm, float* sp, float* contrib, float hs, double h, double hnext,
-                                          double floor, double& err)
+template <bool WIDE>
+__device__ __forceinline__ float code_factor(const unsigned char* fac, uint32_t c)
 {
-    constexpr int KQ = KK ? KK : KMAX;
-    if constexpr (KK != 0) k = KK;
-    const int tid = threadIdx.x;
-    // ---------------- clause phase
-    // the next clause's codes are loaded while this one is processed
-    uint32_t nx[KQ];
+    return *(const float*)(fac + (c & (WIDE ? 0xFFFFu : 0x3FFFu)));
+}
+template <bool WIDE>
+__device__ __forceinline__ void code_store(unsigned char* con, uint32_t c, float v)
+{
+    if constexpr (WIDE) *(float*)(con + ((c >> 16) << 2)) = v;
+    else *(float*)(con + (c >> 14)) = v;
+}
+// v with its sign flipped for a negated literal (bit 2 of the code)
+__device__ __forceinline__ float code_sign(uint32_t c, float v)
+{
+    return __uint_as_float(((c << 29) & 0x80000000u) ^ __float_as_uint(v));
+}
+
+// the two factors of a spin, written by its variable's thread
+__device__ __forceinline__ void put_factors(unsigned char* fac, int rank, float sv)
+{
+    *(float2*)(fac + 8 * rank) = make_float2(1.0f - sv, 1.0f + sv);
+}
+
+// clauses [first, first + 64) of a wave: the codes are stored in whole groups
+// of 64 clauses, so a wave with any clause loads all of its lanes'
+template <int KK>
+__device__ __forceinline__ void load_code(const uint32_t* code, int j, uint32_t (&c)[KK])
+{
+    unsigned at = (unsigned)j * (4 * KK);
+    asm("" : "+v"(at));         // not kept in a register from stage to stage
+    const uint32_t* p = (const uint32_t*)((const char*)code + at);
 #pragma unroll
-    for (int q = 0; q < KQ; q++) nx[q] = (tid < m && (KK != 0 || q < k)) ? code[(long long)tid * k + q] : 0u;
+    for (int q = 0; q < KK; q++) c[q] = p[q];
+}
+
+// Clause phase of stage J.  COUNT (J = 1): viol receives the number of this
+// thread's clauses violated by the state whose factors are in LDS; pos has a
+// bit per rank, s > 0, for the factors that are exactly 1.
+template <int TT, int CPT, int VPT, int J, int KK, bool WIDE, bool COUNT>
+__device__ __forceinline__ void reg_clauses(RegState<TT, CPT, VPT, KK>& R, const uint32_t* code, int m, float knorm,
+                                            float knorm2, const unsigned char* fac, unsigned char* con, float hs,
+                                            double h, double hnext, double floor, double& err,
+                                            const unsigned long long* pos, int& viol)
+{
+    constexpr bool HOLD = RegState<TT, CPT, VPT, KK>::HOLD;
+    const int tid = traj_tid<TT>();
+    const int w0 = __builtin_amdgcn_readfirstlane(tid & ~63);
+    uint32_t nx[KK];
+    if constexpr (!HOLD) {
+        if (w0 < m) load_code<KK>(code, tid, nx);
+    }
 #pragma unroll
     for (int u = 0; u < CPT; u++) {
-        const int j = tid + u * BS;
-        uint32_t cur[KQ];
+        if (w0 + u * TT < m) {
+            uint32_t c[KK];
+            if constexpr (HOLD) {
 #pragma unroll
-        for (int q = 0; q < KQ; q++) cur[q] = nx[q];
-        if (u + 1 < CPT) {
-            const int jn = j + BS;
+                for (int q = 0; q < KK; q++) {
+                    // an opaque value: what follows from a code is formed
+                    // again in every stage, not kept in registers
+                    asm("" : "+v"(R.code[u][q]));
+                    c[q] = R.code[u][q];
+                }
+            } else {
+                // the next clause's codes are loaded while this one is processed
 #pragma unroll
-            for (int q = 0; q < KQ; q++) nx[q] = (jn < m && (KK != 0 || q < k)) ? code[(long long)jn * k + q] : 0u;
-        }
-        if (j < m) {
-            float f[KQ];
-            uint32_t cc[KQ];
+                for (int q = 0; q < KK; q++) c[q] = nx[q];
+                if (u + 1 < CPT && w0 + (u + 1) * TT < m) load_code<KK>(code, tid + (u + 1) * TT, nx);
+            }
+            float f[KK];
+#pragma unroll
+            for (int q = 0; q < KK; q++) f[q] = code_factor<WIDE>(fac, c[q]);
             float km = knorm;
 #pragma unroll
-            for (int q = 0; q < KQ; q++) {
-                f[q] = 1.0f;
-                cc[q] = 0;
-                if (KK != 0 || q < k) {
-                    uint32_t c = cur[q];
-                    cc[q] = c;
-                    int v = (int)(c >> 19);
-                    float s = v ? sp[v - 1] : -1.0f;
-                    f[q] = (c >> 18) & 1u ? 1.0f + s : 1.0f - s;
-                    km *= f[q];
+            for (int q = 0; q < KK; q++) km *= f[q];
+            if constexpr (COUNT) {
+                bool sat = false, unsat = true;
+#pragma unroll
+                for (int q = 0; q < KK; q++) {
+                    sat |= f[q] < 1.0f;
+                    unsat &= f[q] > 1.0f;
                 }
+                if (!sat && !unsat) {
+                    // a spin too small to move its factor, or NaN: its bit
+                    // decides (the constants' bits are 0: false)
+#pragma unroll
+                    for (int q = 0; q < KK; q++) {
+                        const uint32_t a = c[q] & (WIDE ? 0xFFFFu : 0x3FFFu);
+                        const int rank = (int)(a >> 3);
+                        const bool t = (pos[rank >> 6] >> (rank & 63)) & 1ull;
+                        const bool neg = (a >> 2) & 1u;
+                        sat |= neg ? !t : t;
+                    }
+                }
+                viol += (!sat && tid + u * TT < m) ? 1 : 0;
             }
             float am;
             if constexpr (J == 1) am = R.xa[u];
@@ -489,53 +564,86 @@ __device__ __forceinline__ void reg_stage(RegState<CPT, VPT>& R, const uint32_t*
                 R.a2[u] = xv;
                 err = fmax(err, e);
             }
-            const float r = km * knorm * am;
+            // the factor 2 of every term is in knorm2 = 2 knorm (a power of two)
+            const float r = km * knorm2 * am;
 #pragma unroll
-            for (int q = 0; q < KQ; q++) {
-                if ((KK != 0 || q < k) && (cc[q] >> 19) != 0) {
-                    float p = 1.0f;
-                    bool first = true;
+            for (int q = 0; q < KK; q++) {
+                float p = 1.0f;
+                bool first = true;
 #pragma unroll
-                    for (int qq = 0; qq < KQ; qq++) {
-                        if (qq == q || (KK == 0 && qq >= k)) continue;
-                        p = first ? f[qq] : p * f[qq];
-                        first = false;
-                    }
-                    float rr = r * p;
-                    rr *= (cc[q] >> 18) & 1u ? -2.0f : 2.0f;
-                    contrib[cc[q] & 0x3FFFFu] = rr;
+                for (int qq = 0; qq < KK; qq++) {
+                    if (qq == q) continue;
+                    p = first ? f[qq] : p * f[qq];
+                    first = false;
                 }
+                code_store<WIDE>(con, c[q], code_sign(c[q], r * p));
             }
         }
         // one clause at a time: keeps the live registers to the state plus
-        // one clause's temporaries
-        __builtin_amdgcn_sched_barrier(0);
+        // one clause's temporaries (a wave alone overlaps its few clauses)
+        if constexpr (TT > 64) __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
-    // ---------------- var phase
+}
+
+// left-to-right sum of a group's entries for this lane (depth is uniform)
+__device__ __forceinline__ float group_sum(const float* e, int depth)
+{
+    float sum = 0.0f;
+    int i = 0;
+    for (; i + 8 <= depth; i += 8, e += 8 * 64) {
+        float t[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) t[u] = e[64 * u];
+#pragma unroll
+        for (int u = 0; u < 8; u++) sum += t[u];
+    }
+    if (depth & 4) {
+        float t[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) t[u] = e[64 * u];
+#pragma unroll
+        for (int u = 0; u < 4; u++) sum += t[u];
+        e += 4 * 64;
+    }
+    if (depth & 2) {
+        const float t0 = e[0], t1 = e[64];
+        sum += t0;
+        sum += t1;
+        e += 2 * 64;
+    }
+    if (depth & 1) sum += e[0];
+    return sum;
+}
+
+// Var phase of stage J.  gb, gd: base entry and depth of the wave's groups
+// (depth -1: the wave has no such group).
+template <int TT, int CPT, int VPT, int J, int KK>
+__device__ __forceinline__ void reg_vars(RegState<TT, CPT, VPT, KK>& R, const int (&gb)[VPT], const int (&gd)[VPT],
+                                         unsigned char* fac, const unsigned char* con, float hs, double h,
+                                         double hnext, double floor, double& err)
+{
+    const int tid = traj_tid<TT>();
 #pragma unroll
     for (int v = 0; v < VPT; v++) {
-        const int i = tid + v * BS;
-        if (i < n) {
-            float sum = 0.0f;
-            sum = sum_run(sum, contrib, R.e0[v], R.e1[v]);
-            const float kj = sum;
+        if (gd[v] >= 0) {
+            const float kj = group_sum((const float*)con + gb[v] + (tid & 63), gd[v]);
             const float xi = R.xv[v];
+            const int rank = tid + v * TT;
             if constexpr (J == 1) {
                 R.v1[v] = kj;
-                sp[i] = stage_input<float, 2>(xi, kj, 0.f, 0.f, 0.f, 0.f, hs);
+                put_factors(fac, rank, stage_input<float, 2>(xi, kj, 0.f, 0.f, 0.f, 0.f, hs));
             } else if constexpr (J == 2) {
                 R.v2[v] = kj;
-                sp[i] = stage_input<float, 3>(xi, R.v1[v], kj, 0.f, 0.f, 0.f, hs);
+                put_factors(fac, rank, stage_input<float, 3>(xi, R.v1[v], kj, 0.f, 0.f, 0.f, hs));
             } else if constexpr (J == 3) {
                 R.v3[v] = kj;
-                sp[i] = stage_input<float, 4>(xi, R.v1[v], R.v2[v], kj, 0.f, 0.f, hs);
+                put_factors(fac, rank, stage_input<float, 4>(xi, R.v1[v], R.v2[v], kj, 0.f, 0.f, hs));
             } else if constexpr (J == 4) {
                 R.v4[v] = kj;
-                sp[i] = stage_input<float, 5>(xi, R.v1[v], R.v2[v], R.v3[v], kj, 0.f, hs);
+                put_factors(fac, rank, stage_input<float, 5>(xi, R.v1[v], R.v2[v], R.v3[v], kj, 0.f, hs));
             } else if constexpr (J == 5) {
                 R.v5[v] = kj;
-                sp[i] = stage_input<float, 6>(xi, R.v1[v], R.v2[v], R.v3[v], R.v4[v], kj, hs);
+                put_factors(fac, rank, stage_input<float, 6>(xi, R.v1[v], R.v2[v], R.v3[v], R.v4[v], kj, hs));
             } else {
                 float xn;
                 double e;
@@ -545,38 +653,58 @@ __device__ __forceinline__ void reg_stage(RegState<CPT, VPT>& R, const uint32_t*
             }
         }
     }
-    __syncthreads();
 }
 
-template <int BS, int CPT, int VPT, int KK>
-__global__ __launch_bounds__(BS) void k_batch_reg(Params P)
+// what else a trajectory keeps in LDS
+template <int TT, int VPT>
+struct alignas(16) RegShared {
+    unsigned long long pos[(TT / 64) * VPT];
+    double red[TT / 64];
+    int redi[TT / 64];
+    int traj;
+};
+
+template <int TT, int CPT, int VPT, int KK, bool WIDE>
+__global__ __launch_bounds__(TT == 64 ? 64 * REG_WAVES : TT) void k_batch_reg(Params P)
 {
-    extern __shared__ float lds[];          // [stage spins: sp_stride] then contributions
-    __shared__ double red[BS / 64];
-    __shared__ int redi[BS / 64];
-    __shared__ int s_traj;
-    float* sp = lds;
-    float* contrib = lds + P.sp_stride;
-    const int tid = threadIdx.x;
+    // per trajectory [factors: 2 per rank, TT * VPT ranks] [RegShared]
+    // [contributions]; no other LDS, so the factors start at address 0
+    extern __shared__ __attribute__((aligned(16))) unsigned char rlds[];
+    using Shared = RegShared<TT, VPT>;
+    const int tid = traj_tid<TT>();
+    const int sub = TT == 64 ? uni((int)(threadIdx.x >> 6)) : 0;
+    const int wave = TT == 64 ? 0 : uni(tid >> 6);
+    unsigned char* fac = rlds + (TT == 64 ? sub * P.reg_lds : 0);
+    Shared* sh = (Shared*)(fac + 8 * TT * VPT);
+    unsigned char* con = fac + 8 * TT * VPT + sizeof(Shared);
+    unsigned long long* pos = sh->pos;
 
     for (;;) {
-        if (tid == 0) s_traj = atomicAdd(P.queue, 1);
-        __syncthreads();
         // the trajectory id is the same in every lane: reading it as a
         // scalar lets the descriptor and the instance's base pointers live
         // in scalar registers, leaving the vector registers to the state
-        const int slot = __builtin_amdgcn_readfirstlane(s_traj);
-        __syncthreads();
+        int slot = 0;
+        if constexpr (TT == 64) {
+            if (tid == 0) slot = atomicAdd(P.queue, 1);
+        } else {
+            if (tid == 0) sh->traj = atomicAdd(P.queue, 1);
+            __syncthreads();
+            slot = sh->traj;
+            __syncthreads();
+        }
+        slot = __builtin_amdgcn_readfirstlane(slot);
         if (slot >= P.ntraj) break;
         const int tr = __builtin_amdgcn_readfirstlane(P.order[slot]);
         const Desc d = P.desc[tr];
         TrajCtrl* cp = P.ctrl + tr;
         if (cp->status != RUNNING) continue;    // uniform: every thread reads the same word
 
-        const int n = d.n, m = d.m, k = d.k;
-        const uint32_t* code = P.code + d.code_off;
-        const int* rowptr = P.rowptr + d.row_off;
-        const float knorm = d.knorm;
+        const int n = uni(d.n), m = uni(d.m);
+        const uint32_t* code = P.rcode + uni(d.rcode_off);
+        const int* group = P.rgroup + uni(d.rgroup_off);     // base and depth per 64 ranks
+        const int* vmap = P.rvmap + uni(d.rvmap_off);        // rank -> variable
+        const int ngroups = uni(d.ngroups);
+        const float knorm = uni(d.knorm), knorm2 = 2.0f * knorm;
         double t = cp->t, h = cp->h, hnext = cp->hnext, hdid = cp->hdid, errmax_last = cp->errmax;
         long long steps = cp->steps, attempts = cp->attempts, rhscount = cp->rhscount;
         int parity = cp->parity, min_viol = cp->min_viol, viol = cp->viol;
@@ -585,52 +713,95 @@ __global__ __launch_bounds__(BS) void k_batch_reg(Params P)
         double sat_time = cp->sat_time;
         int done_in_chunk = 0;
 
-        RegState<CPT, VPT> R;
+        RegState<TT, CPT, VPT, KK> R;
+        int gb[VPT], gd[VPT];
         {
             const float* x = (parity ? P.xb : P.xa) + d.state_off;
 #pragma unroll
             for (int u = 0; u < CPT; u++) {
-                const int j = tid + u * BS;
+                const int j = tid + u * TT;
                 R.xa[u] = j < m ? x[n + j] : 0.f;
                 R.a1[u] = R.a2[u] = R.a3[u] = R.a4[u] = R.a5[u] = 0.f;
+                if constexpr (RegState<TT, CPT, VPT, KK>::HOLD) {
+                    if (wave * 64 + u * TT < m) load_code<KK>(code, j, R.code[u]);
+                }
             }
 #pragma unroll
             for (int v = 0; v < VPT; v++) {
-                const int i = tid + v * BS;
-                R.xv[v] = i < n ? x[i] : 0.f;
-                R.e0[v] = i < n ? rowptr[i] : 0;
-                R.e1[v] = i < n ? rowptr[i + 1] : 0;
+                const int g = wave + v * (TT / 64), rank = tid + v * TT;
+                gb[v] = g < ngroups ? __builtin_amdgcn_readfirstlane(group[2 * g]) : 0;
+                gd[v] = g < ngroups ? __builtin_amdgcn_readfirstlane(group[2 * g + 1]) : -1;
+                // ranks n and n + 1 are the constants
+                R.xv[v] = rank < n ? x[vmap[rank]] : (rank == n ? -1.0f : 0.0f);
                 R.v1[v] = R.v2[v] = R.v3[v] = R.v4[v] = R.v5[v] = 0.f;
             }
         }
+        for (int i = tid; i < d.ncontrib; i += TT) ((float*)con)[i] = -0.0f;
+        bool count = false;       // the state is a newly accepted one whose violations are due
 
-        while (status == RUNNING && done_in_chunk < P.chunk_steps) {
-            // ---- stage 1 at x: spins into LDS
+        while (true) {
+            // ---- stage 1 at x: its factors, and where they do not tell, s > 0
 #pragma unroll
             for (int v = 0; v < VPT; v++) {
-                const int i = tid + v * BS;
-                if (i < n) sp[i] = R.xv[v];
+                const int rank = tid + v * TT;
+                if (gd[v] >= 0) {
+                    put_factors(fac, rank, R.xv[v]);
+                    // constants: positive literals that read as false
+                    const unsigned long long b = __ballot(rank < n && R.xv[v] > 0.0f);
+                    if ((tid & 63) == 0) pos[rank >> 6] = b;
+                }
             }
-            __syncthreads();
+            traj_sync<TT>();
+            const double h_at1 = h;
+            double err_local = 0.0;
+            int cnt = 0;
+            if (count) {
+                reg_clauses<TT, CPT, VPT, 1, KK, WIDE, true>(R, code, m, knorm, knorm2, fac, con, (float)h_at1, h_at1,
+                                                             hnext, P.floor, err_local, pos, cnt);
+                viol = traj_sum<TT>(cnt, sh->redi);
+                count = false;
+                if (viol < min_viol) min_viol = viol;
+                if (viol == 0) {
+                    status = SOLVED;
+                    sat_step = (int)steps;
+                    sat_time = t;
+                }
+                if (status == RUNNING && steps >= P.max_steps) status = BUDGET;
+                if (status == RUNNING && t >= P.max_time) status = MAXTIME;
+                if (status != RUNNING || done_in_chunk >= P.chunk_steps) break;
+            } else {
+                reg_clauses<TT, CPT, VPT, 1, KK, WIDE, false>(R, code, m, knorm, knorm2, fac, con, (float)h_at1, h_at1,
+                                                              hnext, P.floor, err_local, pos, cnt);
+                traj_sync<TT>();
+            }
+            reg_vars<TT, CPT, VPT, 1, KK>(R, gb, gd, fac, con, (float)h, h, hnext, P.floor, err_local);
+            traj_sync<TT>();
             bool accepted = false;
-            bool first_attempt = true;
-            while (!accepted) {
+            bool had_stage1 = true;
+            while (true) {
                 const float hs = (float)h;
-                const bool had_stage1 = first_attempt;
-                double err_local = 0.0;
-                if (first_attempt)
-                    reg_stage<BS, CPT, VPT, 1, KK>(R, code, n, m, k, knorm, sp, contrib, hs, h, hnext, P.floor, err_local);
-                first_attempt = false;
-                reg_stage<BS, CPT, VPT, 2, KK>(R, code, n, m, k, knorm, sp, contrib, hs, h, hnext, P.floor, err_local);
-                reg_stage<BS, CPT, VPT, 3, KK>(R, code, n, m, k, knorm, sp, contrib, hs, h, hnext, P.floor, err_local);
-                reg_stage<BS, CPT, VPT, 4, KK>(R, code, n, m, k, knorm, sp, contrib, hs, h, hnext, P.floor, err_local);
-                reg_stage<BS, CPT, VPT, 5, KK>(R, code, n, m, k, knorm, sp, contrib, hs, h, hnext, P.floor, err_local);
-                reg_stage<BS, CPT, VPT, 6, KK>(R, code, n, m, k, knorm, sp, contrib, hs, h, hnext, P.floor, err_local);
+                err_local = 0.0;
+#define ASAT_REG_STAGE(J)                                                                                             \
+    reg_clauses<TT, CPT, VPT, J, KK, WIDE, false>(R, code, m, knorm, knorm2, fac, con, hs, h, hnext, P.floor, err_local, \
+                                                  pos, cnt);                                                          \
+    traj_sync<TT>();                                                                                                  \
+    reg_vars<TT, CPT, VPT, J, KK>(R, gb, gd, fac, con, hs, h, hnext, P.floor, err_local);
+                ASAT_REG_STAGE(2)
+                traj_sync<TT>();
+                ASAT_REG_STAGE(3)
+                traj_sync<TT>();
+                ASAT_REG_STAGE(4)
+                traj_sync<TT>();
+                ASAT_REG_STAGE(5)
+                traj_sync<TT>();
+                ASAT_REG_STAGE(6)
+#undef ASAT_REG_STAGE
                 // ---------------- error norm + control (FP64), uniform in every thread
-                const double errmax = block_max_all<BS>(err_local, red) / P.eps;
+                const double errmax = traj_max<TT>(err_local, sh->red) / P.eps;
                 errmax_last = errmax;
                 attempts += 1;
                 rhscount += had_stage1 ? 6 : 5;
+                had_stage1 = false;
                 if (errmax <= 1.0) {
                     double hn = errmax > TabD::ERRCON ? TabD::SAFETY * h * pow_ctrl(errmax, 5) : 5.0 * h;
                     hdid = h;
@@ -639,26 +810,25 @@ __global__ __launch_bounds__(BS) void k_batch_reg(Params P)
                     hnext = hn;
                     h = hn;
                     accepted = true;
-                } else {
-                    double htemp = TabD::SAFETY * h * pow_ctrl(errmax, 4);
-                    double hn = h >= 0.0 ? fmax(htemp, TabD::HFACTOR * h) : fmin(htemp, TabD::HFACTOR * h);
-                    if (t + hn == t) {
-                        h = hn;
-                        status = UNDERFLOW_;
-                        break;
-                    }
-                    h = hn;
-                    // retry: stage-2 spin input from x, k1 and the reduced h
-                    const float hs2 = (float)h;
-#pragma unroll
-                    for (int v = 0; v < VPT; v++) {
-                        const int i = tid + v * BS;
-                        if (i < n) sp[i] = stage_input<float, 2>(R.xv[v], R.v1[v], 0.f, 0.f, 0.f, 0.f, hs2);
-                    }
-                    __syncthreads();
+                    break;
                 }
+                double htemp = TabD::SAFETY * h * pow_ctrl(errmax, 4);
+                double hn = h >= 0.0 ? fmax(htemp, TabD::HFACTOR * h) : fmin(htemp, TabD::HFACTOR * h);
+                h = hn;
+                if (t + hn == t) {
+                    status = UNDERFLOW_;
+                    break;
+                }
+                // retry: stage-2 spin input from x, k1 and the reduced h
+                const float hs2 = (float)h;
+#pragma unroll
+                for (int v = 0; v < VPT; v++)
+                    if (gd[v] >= 0)
+                        put_factors(fac, tid + v * TT,
+                                    stage_input<float, 2>(R.xv[v], R.v1[v], 0.f, 0.f, 0.f, 0.f, hs2));
+                traj_sync<TT>();
             }
-            if (status != RUNNING) break;
+            if (!accepted) break;
             // accept: x <- x_new (held in the k2 registers)
 #pragma unroll
             for (int u = 0; u < CPT; u++) R.xa[u] = R.a2[u];
@@ -666,54 +836,344 @@ __global__ __launch_bounds__(BS) void k_batch_reg(Params P)
             for (int v = 0; v < VPT; v++) R.xv[v] = R.v2[v];
             parity ^= 1;
             done_in_chunk += 1;
-            // ---------------- violated-clause count on the accepted state
-            if (steps % P.check_every == 0 || steps >= P.max_steps) {
-#pragma unroll
-                for (int v = 0; v < VPT; v++) {
-                    const int i = tid + v * BS;
-                    if (i < n) sp[i] = R.xv[v];
-                }
-                __syncthreads();
-                int cnt = 0;
-#pragma unroll
-                for (int u = 0; u < CPT; u++) {
-                    const int j = tid + u * BS;
-                    if (j >= m) continue;
-                    const uint32_t* cj = code + (long long)j * k;
-                    int sat = 0;
-                    for (int q = 0; q < k && !sat; q++) {
-                        uint32_t c = cj[q];
-                        int v = (int)(c >> 19);
-                        if (!v) continue;
-                        int tv = sp[v - 1] > 0.0f;
-                        sat = (c >> 18) & 1u ? !tv : tv;
-                    }
-                    cnt += !sat;
-                }
-                viol = block_sum_all<BS>(cnt, redi);
-                if (viol < min_viol) min_viol = viol;
-                if (viol == 0) {
-                    status = SOLVED;
-                    sat_step = (int)steps;
-                    sat_time = t;
-                }
+            count = steps % P.check_every == 0 || steps >= P.max_steps;
+            if (!count) {
+                if (t >= P.max_time) status = MAXTIME;
+                if (status != RUNNING || done_in_chunk >= P.chunk_steps) break;
             }
-            if (status == RUNNING && steps >= P.max_steps) status = BUDGET;
-            if (status == RUNNING && t >= P.max_time) status = MAXTIME;
-            __syncthreads();
         }
         // the state after the last accepted step goes to the parity buffer it names
         {
             float* x = (parity ? P.xb : P.xa) + d.state_off;
 #pragma unroll
             for (int u = 0; u < CPT; u++) {
-                const int j = tid + u * BS;
+                const int j = tid + u * TT;
                 if (j < m) x[n + j] = R.xa[u];
             }
 #pragma unroll
             for (int v = 0; v < VPT; v++) {
-                const int i = tid + v * BS;
-                if (i < n) x[i] = R.xv[v];
+                const int rank = tid + v * TT;
+                if (rank < n) x[vmap[rank]] = R.xv[v];
+            }
+        }
+        if (tid == 0) {
+            cp->t = t; cp->h = h; cp->hnext = hnext; cp->hdid = hdid; cp->errmax = errmax_last;
+            cp->steps = steps; cp->attempts = attempts; cp->rhscount = rhscount;
+            cp->parity = parity; cp->status = status; cp->min_viol = min_viol; cp->viol = viol;
+            cp->sat_step = sat_step; cp->sat_time = sat_time;
+        }
+        traj_sync<TT>();
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Clause-chunked variant, for instances whose contributions do not fit in LDS.
+// Clauses are taken in chunks whose KK terms per clause do.  Per chunk:
+//   clause phase: each thread's clauses leave their terms in LDS, term q of
+//     clause jl at q * chunk + jl (lanes side by side: no bank conflicts)
+//   var phase: the chunk's variables, 64 at a time and ranked by their number of
+//     occurrences in it, add the terms that their index list names to the
+//     variable's running sum in LDS
+// Chunks follow the clause order, so every variable's terms are added in the
+// reference's order.  After the last chunk each variable's stage combination
+// (state and derivatives of both kinds in global scratch) puts the next
+// stage's factors 1 - s and 1 + s into LDS.
+//
+// It is bound by memory: per slot and stage a 2-byte code and a 2-byte term
+// index, per clause the stage's derivatives (27 floats an attempt), about 60 %
+// less than 4-byte codes and 8-byte records, from which each variable formed
+// its terms itself (three LDS reads per slot and uncoalesced records).
+// 512 ragged instances (N in [50, 5000], 3- and 4-SAT) for 20 steps, their
+// smallest quarter in registers: 89 -> 19 ms; the largest quarter (M up to
+// 60 000) 21.9 -> 4.8 us per trajectory and attempt, on 128 of 256 CUs.
+template <int KK, int J, bool COUNT>
+__device__ __forceinline__ void chunk_clauses(const uint2* code, const float* x, float* const (&kb)[5], float* xn,
+                                              int c0, int cn, int cs, int n, float knorm, float knorm2,
+                                              const float* fac, float* term, float hs, double h, double hnext,
+                                              double floor, double& err, int& viol)
+{
+    constexpr int U = 2;                     // clauses whose loads are in flight together
+    const int BS = (int)blockDim.x;
+    for (int jb = (int)threadIdx.x; jb < cn; jb += U * BS) {
+        uint2 c[U];
+        float xa[U], a1[U], a2[U], a3[U], a4[U], a5[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int jl = jb + u * BS;
+            xa[u] = a1[u] = a2[u] = a3[u] = a4[u] = a5[u] = 0.f;
+            c[u] = make_uint2(0u, 0u);
+            if (jl < cn) {
+                c[u] = code[c0 + jl];
+                const int ai = n + c0 + jl;
+                xa[u] = x[ai];
+                if constexpr (J > 1) a1[u] = kb[0][ai];
+                if constexpr (J > 2) a2[u] = kb[1][ai];
+                if constexpr (J > 3) a3[u] = kb[2][ai];
+                if constexpr (J > 4) a4[u] = kb[3][ai];
+                if constexpr (J > 5) a5[u] = kb[4][ai];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int jl = jb + u * BS;
+            if (jl >= cn) break;
+            const uint32_t w[4] = {c[u].x & 0xFFFFu, c[u].x >> 16, c[u].y & 0xFFFFu, c[u].y >> 16};
+            float f[KK];
+            float km = knorm;
+#pragma unroll
+            for (int q = 0; q < KK; q++) {
+                f[q] = fac[w[q]];
+                km *= f[q];
+            }
+            if constexpr (COUNT) {
+                bool sat = false, unsat = true;
+#pragma unroll
+                for (int q = 0; q < KK; q++) {
+                    sat |= f[q] < 1.0f;
+                    unsat &= f[q] > 1.0f;
+                }
+                if (!sat && !unsat) {
+                    // a spin too small to move its factor, or NaN; the
+                    // constants (variables n and n + 1) are false
+#pragma unroll
+                    for (int q = 0; q < KK; q++) {
+                        const int v = (int)(w[q] >> 1);
+                        if (v >= n) continue;
+                        const bool t = x[v] > 0.0f;
+                        sat |= (w[q] & 1u) ? !t : t;
+                    }
+                }
+                viol += sat ? 0 : 1;
+            }
+            float am;
+            if constexpr (J == 1) am = xa[u];
+            else am = stage_input<float, J>(xa[u], a1[u], a2[u], a3[u], a4[u], a5[u], hs);
+            const float kj = am * km * km;
+            const int ai = n + c0 + jl;
+            if constexpr (J < 6) {
+                kb[J - 1][ai] = kj;
+            } else {
+                float xv;
+                double e;
+                final_combination<float>(xa[u], a1[u], a3[u], a4[u], a5[u], kj, hs, h, hnext, floor, xv, e);
+                xn[ai] = xv;
+                err = fmax(err, e);
+            }
+            const float r = km * knorm2 * am;
+#pragma unroll
+            for (int q = 0; q < KK; q++) {
+                float p = 1.0f;
+                bool first = true;
+#pragma unroll
+                for (int qq = 0; qq < KK; qq++) {
+                    if (qq == q) continue;
+                    p = first ? f[qq] : p * f[qq];
+                    first = false;
+                }
+                term[q * cs + jl] = __uint_as_float((w[q] << 31) ^ __float_as_uint(r * p));
+            }
+        }
+    }
+}
+
+// the chunk's variables: groups [g0, g1) of 64, a wave each
+__device__ __forceinline__ void chunk_vars(const int2* group, const uint16_t* perm, const uint32_t* rec, int g0,
+                                           int g1, const float* term, float* sums)
+{
+    const int lane = (int)(threadIdx.x & 63);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), nw = (int)(blockDim.x >> 6);
+    for (int g = g0 + wave; g < g1; g += nw) {
+        const int2 gd = group[g];            // first word, words per lane (two entries each)
+        const int v = perm[g * 64 + lane];
+        const uint32_t* r = rec + gd.x + lane;
+        float sum = sums[v];
+        int i = 0;
+        for (; i + 4 <= gd.y; i += 4) {
+            uint32_t w[4];
+            float t[8];
+#pragma unroll
+            for (int u = 0; u < 4; u++) w[u] = r[64 * (i + u)];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                t[2 * u] = term[w[u] & 0xFFFFu];
+                t[2 * u + 1] = term[w[u] >> 16];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) sum += t[u];
+        }
+        for (; i < gd.y; i++) {
+            const uint32_t w = r[64 * i];
+            const float t0 = term[w & 0xFFFFu], t1 = term[w >> 16];
+            sum += t0;
+            sum += t1;
+        }
+        sums[v] = sum;
+    }
+}
+
+template <int BS>
+__global__ __launch_bounds__(BS) void k_batch_chunk(Params P)
+{
+    // [factors: fac_ranks pairs] [running sums: fac_ranks] [terms, then 0]
+    extern __shared__ __attribute__((aligned(16))) float clds[];
+    __shared__ double red[BS / 64];
+    __shared__ int redi[BS / 64];
+    __shared__ int s_traj;
+    float* fac = clds;
+    float* sums = clds + 2 * P.fac_ranks;
+    float* term = clds + 3 * P.fac_ranks;
+    float* scratch = P.scratch + (long long)blockIdx.x * P.scratch_per_wg;
+    float* const kb[5] = {scratch, scratch + P.scratch_stride, scratch + 2 * P.scratch_stride,
+                          scratch + 3 * P.scratch_stride, scratch + 4 * P.scratch_stride};
+    const int tid = threadIdx.x;
+
+    for (;;) {
+        if (tid == 0) s_traj = atomicAdd(P.queue, 1);
+        __syncthreads();
+        const int slot = __builtin_amdgcn_readfirstlane(s_traj);
+        __syncthreads();
+        if (slot >= P.ntraj) break;
+        const int tr = __builtin_amdgcn_readfirstlane(P.order[slot]);
+        const Desc d = P.desc[tr];
+        TrajCtrl* cp = P.ctrl + tr;
+        if (cp->status != RUNNING) continue;    // uniform: every thread reads the same word
+
+        const int n = uni(d.n), m = uni(d.m), cs = uni(d.chunk), nc = uni(d.nchunks);
+        const uint2* code = P.ccode + uni(d.ccode_off);
+        const int2* group = P.cgroup + uni(d.cgroup_off);
+        const uint16_t* perm = P.cperm + uni(d.cgroup_off) * 64;
+        const uint32_t* rec = P.crec + uni(d.crec_off);
+        const int* cstart = P.cstart + uni(d.cstart_off);
+        const float knorm = uni(d.knorm), knorm2 = 2.0f * knorm;
+        const int klen = uni(d.k);
+        double t = cp->t, h = cp->h, hnext = cp->hnext, hdid = cp->hdid, errmax_last = cp->errmax;
+        long long steps = cp->steps, attempts = cp->attempts, rhscount = cp->rhscount;
+        int parity = cp->parity, min_viol = cp->min_viol, viol = cp->viol;
+        int status = RUNNING;
+        int sat_step = cp->sat_step;
+        double sat_time = cp->sat_time;
+        int done_in_chunk = 0;
+        bool count = false;       // the state is a newly accepted one whose violations are due
+        float* x = nullptr;
+        float* xn = nullptr;
+
+        auto put = [&](int i, float sv) { *(float2*)(fac + 2 * i) = make_float2(1.0f - sv, 1.0f + sv); };
+        if (tid == 0) {
+            put(n, -1.0f);        // a padding literal of a short clause: factor 2
+            put(n + 1, 0.0f);     // a literal beyond k: factor 1
+            term[P.chunk_terms] = 0.0f;   // entries that fill up a list
+        }
+        // one stage: every chunk's clauses and variables, then the variables'
+        // stage combination; with COUNT the violated clauses first
+        auto stage = [&](auto jc, auto cc, float hs, double& err, int& cnt) {
+            constexpr int J = decltype(jc)::value;
+            constexpr bool COUNT = decltype(cc)::value;
+            for (int i = tid; i <= n; i += BS) sums[i] = 0.0f;
+            for (int c = 0; c < nc; c++) {
+                const int c0 = c * cs, cn = min(cs, m - c0);
+                if (klen <= 3)
+                    chunk_clauses<3, J, COUNT>(code, x, kb, xn, c0, cn, cs, n, knorm, knorm2, fac, term, hs, h, hnext,
+                                               P.floor, err, cnt);
+                else
+                    chunk_clauses<4, J, COUNT>(code, x, kb, xn, c0, cn, cs, n, knorm, knorm2, fac, term, hs, h, hnext,
+                                               P.floor, err, cnt);
+                __syncthreads();
+                chunk_vars(group, perm, rec, cstart[c], cstart[c + 1], term, sums);
+                __syncthreads();
+            }
+            for (int i = tid; i < n; i += BS) {
+                const float kj = sums[i], xi = x[i];
+                if constexpr (J < 6) kb[J - 1][i] = kj;
+                if constexpr (J == 1) put(i, stage_input<float, 2>(xi, kj, 0.f, 0.f, 0.f, 0.f, hs));
+                else if constexpr (J == 2) put(i, stage_input<float, 3>(xi, kb[0][i], kj, 0.f, 0.f, 0.f, hs));
+                else if constexpr (J == 3) put(i, stage_input<float, 4>(xi, kb[0][i], kb[1][i], kj, 0.f, 0.f, hs));
+                else if constexpr (J == 4)
+                    put(i, stage_input<float, 5>(xi, kb[0][i], kb[1][i], kb[2][i], kj, 0.f, hs));
+                else if constexpr (J == 5)
+                    put(i, stage_input<float, 6>(xi, kb[0][i], kb[1][i], kb[2][i], kb[3][i], kj, hs));
+                else {
+                    float xv;
+                    double e;
+                    final_combination<float>(xi, kb[0][i], kb[2][i], kb[3][i], kb[4][i], kj, hs, h, hnext, P.floor, xv,
+                                             e);
+                    xn[i] = xv;
+                    err = fmax(err, e);
+                }
+            }
+            __syncthreads();
+        };
+        using std::integral_constant;
+        using NoCount = integral_constant<bool, false>;
+
+        while (true) {
+            x = (parity ? P.xb : P.xa) + d.state_off;
+            xn = (parity ? P.xa : P.xb) + d.state_off;
+            // ---- stage 1 at x
+            for (int i = tid; i < n; i += BS) put(i, x[i]);
+            __syncthreads();
+            double err_local = 0.0;
+            int cnt = 0;
+            if (count) {
+                stage(integral_constant<int, 1>{}, integral_constant<bool, true>{}, (float)h, err_local, cnt);
+                viol = block_sum_all<BS>(cnt, redi);
+                count = false;
+                if (viol < min_viol) min_viol = viol;
+                if (viol == 0) {
+                    status = SOLVED;
+                    sat_step = (int)steps;
+                    sat_time = t;
+                }
+                if (status == RUNNING && steps >= P.max_steps) status = BUDGET;
+                if (status == RUNNING && t >= P.max_time) status = MAXTIME;
+                if (status != RUNNING || done_in_chunk >= P.chunk_steps) break;
+            } else {
+                stage(integral_constant<int, 1>{}, NoCount{}, (float)h, err_local, cnt);
+            }
+            bool accepted = false;
+            bool had_stage1 = true;
+            while (true) {
+                const float hs = (float)h;
+                err_local = 0.0;
+                stage(integral_constant<int, 2>{}, NoCount{}, hs, err_local, cnt);
+                stage(integral_constant<int, 3>{}, NoCount{}, hs, err_local, cnt);
+                stage(integral_constant<int, 4>{}, NoCount{}, hs, err_local, cnt);
+                stage(integral_constant<int, 5>{}, NoCount{}, hs, err_local, cnt);
+                stage(integral_constant<int, 6>{}, NoCount{}, hs, err_local, cnt);
+                const double errmax = traj_max<BS>(err_local, red) / P.eps;
+                errmax_last = errmax;
+                attempts += 1;
+                rhscount += had_stage1 ? 6 : 5;
+                had_stage1 = false;
+                if (errmax <= 1.0) {
+                    double hn = errmax > TabD::ERRCON ? TabD::SAFETY * h * pow_ctrl(errmax, 5) : 5.0 * h;
+                    hdid = h;
+                    t += h;
+                    steps += 1;
+                    hnext = hn;
+                    h = hn;
+                    accepted = true;
+                    break;
+                }
+                double htemp = TabD::SAFETY * h * pow_ctrl(errmax, 4);
+                double hn = h >= 0.0 ? fmax(htemp, TabD::HFACTOR * h) : fmin(htemp, TabD::HFACTOR * h);
+                h = hn;
+                if (t + hn == t) {
+                    status = UNDERFLOW_;
+                    break;
+                }
+                // retry: stage-2 spin input from x, k1 and the reduced h
+                const float hs2 = (float)h;
+                for (int i = tid; i < n; i += BS)
+                    put(i, stage_input<float, 2>(x[i], kb[0][i], 0.f, 0.f, 0.f, 0.f, hs2));
+                __syncthreads();
+            }
+            if (!accepted) break;
+            parity ^= 1;
+            done_in_chunk += 1;
+            count = steps % P.check_every == 0 || steps >= P.max_steps;
+            if (!count) {
+                if (t >= P.max_time) status = MAXTIME;
+                if (status != RUNNING || done_in_chunk >= P.chunk_steps) break;
             }
         }
         if (tid == 0) {
@@ -743,27 +1203,138 @@ struct Instance {
     std::vector<float> pub0;      // n+m
 };
 
-// contribution records of the clause-chunked mode (see VC_OTHER_SHIFT), in
-// var-major (contribution) order
-static void build_vcode(const Instance& I, unsigned long long* out)
+// Layout of the register kernel for one instance: variables ranked by falling
+// number of occurrences, contributions in groups of 64 ranks with the entries of
+// one index side by side, codes padded to whole groups of 64 clauses and to kk
+// literals (see k_batch_reg).
+struct RegLayout {
+    std::vector<int> rank;      // variable -> rank
+    std::vector<int> vmap;      // rank -> variable
+    std::vector<int> group;     // base and depth per group of 64 ranks (two constant ranks at the end)
+    int ngroups = 0, ncontrib = 0;
+};
+
+static void reg_layout(const Instance& I, RegLayout& L)
 {
-    const int k = I.k;
-    for (int j = 0; j < I.m; j++) {
-        const uint32_t* cj = I.code.data() + (size_t)j * k;
-        for (int q = 0; q < k; q++) {
-            const uint32_t c = cj[q];
-            if ((c >> 19) == 0) continue;
-            unsigned long long vc = (unsigned long long)j | ((unsigned long long)((c >> 18) & 1u) << 18);
-            int t = 0;
-            for (int qq = 0; qq < k; qq++) {
-                if (qq == q) continue;
-                const uint32_t o = ((cj[qq] >> 19) << 1) | ((cj[qq] >> 18) & 1u);
-                vc |= (unsigned long long)o << (VC_OTHER_SHIFT + 14 * t);
-                t++;
-            }
-            out[c & 0x3FFFFu] = vc;
-        }
+    const int n = I.n;
+    int top = 0;
+    for (int i = 0; i < n; i++) top = std::max(top, I.rowptr[i + 1] - I.rowptr[i]);
+    std::vector<int> at((size_t)top + 2, 0);
+    for (int i = 0; i < n; i++) at[(size_t)(top - (I.rowptr[i + 1] - I.rowptr[i])) + 1]++;
+    for (int g = 0; g <= top; g++) at[(size_t)g + 1] += at[(size_t)g];
+    L.rank.resize((size_t)n);
+    L.vmap.resize((size_t)n);
+    for (int i = 0; i < n; i++) {
+        const int r = at[(size_t)(top - (I.rowptr[i + 1] - I.rowptr[i]))]++;
+        L.rank[i] = r;
+        L.vmap[r] = i;
     }
+    L.ngroups = ceil_div(n + 2, 64);
+    L.group.resize((size_t)2 * L.ngroups);
+    int base = 0;
+    for (int g = 0; g < L.ngroups; g++) {
+        const int v = 64 * g < n ? L.vmap[64 * g] : -1;      // the group's first rank occurs most
+        const int depth = v >= 0 ? I.rowptr[v + 1] - I.rowptr[v] : 0;
+        L.group[2 * g] = base;
+        L.group[2 * g + 1] = depth;
+        base += 64 * depth;
+    }
+    L.ncontrib = base;
+}
+
+// the codes, rcode_len(I, kk) words; entry L.ncontrib is the one nothing reads
+static long long rcode_len(const Instance& I, int kk) { return round_up_ll(I.m, 64) * kk; }
+static void reg_codes(const Instance& I, const RegLayout& L, int kk, uint32_t* out)
+{
+    const uint32_t none = (uint32_t)L.ncontrib << 16;
+    const uint32_t pad = none | (8u * (uint32_t)I.n), absent = none | (8u * (uint32_t)(I.n + 1));
+    for (int j = 0; j < I.m; j++)
+        for (int q = 0; q < kk; q++) {
+            uint32_t& o = out[(size_t)j * kk + q];
+            if (q >= I.k) { o = absent; continue; }
+            const uint32_t c = I.code[(size_t)j * I.k + q];
+            const int v = (int)(c >> 19) - 1;
+            if (v < 0) { o = pad; continue; }
+            const int r = L.rank[v], e = (int)(c & 0x3FFFFu) - I.rowptr[v];
+            const uint32_t at = (uint32_t)(L.group[2 * (r / 64)] + 64 * e + r % 64);
+            o = (at << 16) | (8u * (uint32_t)r) | (((c >> 18) & 1u) << 2);
+        }
+    for (long long s = (long long)I.m * kk; s < rcode_len(I, kk); s++) out[s] = absent;
+}
+
+// Layout of the chunked kernel for one instance (see k_batch_chunk): chunks of
+// cs clauses; per chunk its variables with any occurrence, ranked by their number
+// and 64 to a group, each with the indices of its terms in clause order, two
+// per word; missing entries and lanes name entry `zero` and variable n.
+struct ChunkLayout {
+    int nchunks = 0, cs = 0;
+    std::vector<uint2> code;
+    std::vector<int2> group;
+    std::vector<uint16_t> perm;
+    std::vector<uint32_t> rec;
+    std::vector<int> start;
+};
+
+static void chunk_layout(const Instance& I, int max_cs, int zero, ChunkLayout& L)
+{
+    const int n = I.n, m = I.m, k = I.k;
+    L.nchunks = ceil_div(m, max_cs);
+    L.cs = std::min(max_cs, (int)round_up_ll(ceil_div(m, L.nchunks), 64));
+    L.nchunks = ceil_div(m, L.cs);
+    L.code.resize((size_t)m);
+    std::vector<int> cnt((size_t)n), slot((size_t)n);
+    std::vector<int> vars, at;
+    for (int c = 0; c < L.nchunks; c++) {
+        const int c0 = c * L.cs, c1 = std::min(m, c0 + L.cs);
+        std::fill(cnt.begin(), cnt.end(), 0);
+        for (int j = c0; j < c1; j++) {
+            uint32_t w[4];
+            for (int q = 0; q < 4; q++) {
+                w[q] = 2u * (uint32_t)(n + 1);
+                if (q >= k) continue;
+                const uint32_t code = I.code[(size_t)j * k + q];
+                const int v = (int)(code >> 19) - 1;
+                w[q] = v < 0 ? 2u * (uint32_t)n : 2u * (uint32_t)v + ((code >> 18) & 1u);
+                if (v >= 0) cnt[v]++;
+            }
+            L.code[j] = make_uint2(w[0] | (w[1] << 16), w[2] | (w[3] << 16));
+        }
+        // variables by falling count, stable
+        int top = 0;
+        for (int v = 0; v < n; v++) top = std::max(top, cnt[v]);
+        at.assign((size_t)top + 2, 0);
+        int used = 0;
+        for (int v = 0; v < n; v++)
+            if (cnt[v]) { at[(size_t)(top - cnt[v]) + 1]++; used++; }
+        for (int g = 0; g <= top; g++) at[(size_t)g + 1] += at[(size_t)g];
+        vars.resize((size_t)used);
+        for (int v = 0; v < n; v++)
+            if (cnt[v]) {
+                const int r = at[(size_t)(top - cnt[v])]++;
+                vars[r] = v;
+                slot[v] = r;
+            }
+        const int g0 = (int)L.group.size(), ng = ceil_div(used, 64);
+        L.start.push_back(g0);
+        for (int g = 0; g < ng; g++) {
+            const int words = (cnt[vars[(size_t)64 * g]] + 1) / 2;
+            L.group.push_back(make_int2((int)L.rec.size(), words));
+            for (int l = 0; l < 64; l++)
+                L.perm.push_back((uint16_t)(64 * g + l < used ? vars[(size_t)(64 * g + l)] : n));
+            L.rec.resize(L.rec.size() + (size_t)64 * words, (uint32_t)zero | ((uint32_t)zero << 16));
+        }
+        std::fill(cnt.begin(), cnt.end(), 0);
+        for (int j = c0; j < c1; j++)
+            for (int q = 0; q < k; q++) {
+                const int v = (int)(I.code[(size_t)j * k + q] >> 19) - 1;
+                if (v < 0) continue;
+                const int r = slot[v], e = cnt[v]++;
+                uint32_t& w = L.rec[(size_t)L.group[(size_t)g0 + r / 64].x + (size_t)64 * (e / 2) + r % 64];
+                const uint32_t idx = (uint32_t)(q * L.cs + (j - c0));
+                w = (e & 1) ? (w & 0xFFFFu) | (idx << 16) : (w & 0xFFFF0000u) | idx;
+            }
+    }
+    L.start.push_back((int)L.group.size());
 }
 
 struct Bucket {
@@ -772,16 +1343,17 @@ struct Bucket {
     int lds = -1;                  // contributions in LDS (1) or global scratch (0); 2: register-
                                    // resident kernel (contributions in LDS); 3: clause-chunked
                                    // (no contribution array); -1 = auto
-    int chunk = 0;                 // clause-chunked mode: clauses per chunk
-    bool vcode = false;            // clause-chunked records built for this bucket's instances
-    int cpt = 0, vpt = 0;          // register kernel: clauses / variables per thread
-    int kk = 0;                    // register kernel: 3 when every instance has 3-literal clauses, else 0
+    bool chunked = false;          // the clause-chunked layout is built for this bucket's instances
+    int chunk_terms = 0;           // clause-chunked mode: term entries in LDS
+    const struct RegVariant* reg = nullptr;   // register kernel: its variant
+    int kk = 0;                    // register kernel: literals per clause (3 or 4)
+    int ncontrib = 0;              // register kernel: contribution entries of the largest instance
     int grid = 0;
     int maxn = 0, maxm = 0, maxl = 0;
     int sp_stride = 0;
     long long scratch_stride = 0, scratch_per_wg = 0;
     size_t lds_bytes = 0;
-    bool lds_fits = false;
+    bool lds_fits = false;         // contributions of k_batch fit in LDS
     int* d_order = nullptr;
     int* d_queue = nullptr;
     float* d_scratch = nullptr;
@@ -810,7 +1382,13 @@ struct Batch {
     // device
     Desc* d_desc = nullptr;
     uint32_t* d_code = nullptr;
-    unsigned long long* d_vcode = nullptr;
+    uint32_t* d_rcode = nullptr;
+    int *d_rgroup = nullptr, *d_rvmap = nullptr;
+    uint2* d_ccode = nullptr;
+    int2* d_cgroup = nullptr;
+    uint16_t* d_cperm = nullptr;
+    uint32_t* d_crec = nullptr;
+    int* d_cstart = nullptr;
     int* d_rowptr = nullptr;
     float* d_xa = nullptr;
     float* d_xb = nullptr;
@@ -829,9 +1407,13 @@ struct Batch {
     void free_dev()
     {
         (void)hipFree(d_desc); (void)hipFree(d_code); (void)hipFree(d_rowptr); (void)hipFree(d_xa);
-        (void)hipFree(d_xb); (void)hipFree(d_ctrl); (void)hipFree(d_vcode);
+        (void)hipFree(d_xb); (void)hipFree(d_ctrl);
+        for (void* q : {(void*)d_rcode, (void*)d_rgroup, (void*)d_rvmap, (void*)d_ccode, (void*)d_cgroup,
+                        (void*)d_cperm, (void*)d_crec, (void*)d_cstart})
+            (void)hipFree(q);
+        d_rcode = d_crec = nullptr; d_rgroup = d_rvmap = d_cstart = nullptr;
+        d_ccode = nullptr; d_cgroup = nullptr; d_cperm = nullptr;
         d_desc = nullptr; d_code = nullptr; d_rowptr = nullptr; d_xa = d_xb = nullptr; d_ctrl = nullptr;
-        d_vcode = nullptr;
         for (auto& b : buckets) b.free_dev();
     }
     ~Batch()
@@ -901,55 +1483,78 @@ static size_t bucket_lds(const Bucket& b, bool lds)
     return sizeof(float) * ((size_t)b.sp_stride + (lds ? (size_t)round_up_ll(b.maxl, 4) : 0));
 }
 
-// clause-chunked mode: spins, running sums and record cursors per variable,
-// then r_m of one chunk of clauses
-static size_t chunk_lds(const Bucket& b, int chunk)
+// register-resident variants: threads per trajectory, clauses and variables
+// per thread, more than 2046 variables (two shifts per contribution address).
+// The smallest that an instance fits comes first; 1024 x (12, 3) and 512 x (24, 6)
+// reach as far as the LDS does with 3-literal clauses.
+struct RegVariant {
+    int tt, cpt, vpt;
+    bool wide;
+    int block() const { return tt == 64 ? 64 * REG_WAVES : tt; }
+    int waves() const { return tt == 64 ? REG_WAVES : 1; }
+};
+#define ASAT_REG_VARIANTS(X)                                                                             \
+    X(64, 4, 1, false) X(64, 8, 2, false) X(256, 1, 1, false) X(256, 4, 2, false) X(512, 8, 4, false)    \
+    X(768, 12, 3, true) X(1024, 9, 2, false) X(512, 17, 4, false) X(1024, 12, 3, true) X(512, 24, 6, true)
+static const RegVariant REG_VARIANTS[] = {
+#define ASAT_REG_ROW(T, C, V, W) {T, C, V, W},
+    ASAT_REG_VARIANTS(ASAT_REG_ROW)
+#undef ASAT_REG_ROW
+};
+
+// LDS of one trajectory: factors of every rank, contributions, the entry
+// nothing reads
+static size_t reg_lds(const RegVariant& r, const Bucket& b)
 {
-    return sizeof(float) * (3 * (size_t)b.sp_stride + (size_t)round_up_ll(chunk, 4));
+    const size_t waves = (size_t)r.tt / 64;      // RegShared, rounded up
+    const size_t shared = ((size_t)8 * waves * r.vpt + 12 * waves + 4 + 15) / 16 * 16;
+    return 8 * (size_t)r.tt * r.vpt + shared + sizeof(float) * (size_t)round_up_ll(b.ncontrib + 1, 4);
+}
+constexpr size_t LDS_STATIC = 1024;      // the kernels' static shared arrays
+
+static bool reg_fits(const RegVariant& r, const Bucket& b, size_t lds_limit)
+{
+    return b.maxm <= r.tt * r.cpt && b.maxn + 2 <= r.tt * r.vpt && (r.wide || b.maxn <= 2046) &&
+           b.ncontrib + 1 <= 65535 && reg_lds(r, b) * r.waves() <= lds_limit;
 }
 
-// largest chunk (a multiple of 256 clauses, at most the bucket's largest m)
-// with which `wgs` workgroups fit in the LDS of one CU; 0 if none does
-static int chunk_for(const Batch& B, const Bucket& b, int wgs);
-
-// register-resident variants (workgroup size, clauses and variables per
-// thread); a bucket uses the first one its largest instance fits
-struct RegVariant {
-    int bs, cpt, vpt;
-};
-static const RegVariant REG_VARIANTS[] = {{256, 1, 1}, {256, 4, 2}, {512, 8, 4}, {768, 12, 3}, {1024, 9, 2}, {512, 17, 4}};
-
-// first variant the bucket's largest instance fits (of workgroup size bs, or any)
-static const RegVariant* reg_variant(const Bucket& b, int bs = 0)
+// first variant the bucket's instances fit (of workgroup size bs, or any)
+static const RegVariant* reg_variant(const Bucket& b, size_t lds_limit, int bs = 0)
 {
     for (const RegVariant& r : REG_VARIANTS)
-        if ((!bs || r.bs == bs) && b.maxm <= r.bs * r.cpt && b.maxn <= r.bs * r.vpt) return &r;
+        if ((!bs || r.block() == bs) && reg_fits(r, b, lds_limit)) return &r;
     return nullptr;
 }
 
-#define ASAT_REG_VARIANTS(X) X(256, 1, 1) X(256, 4, 2) X(512, 8, 4) X(768, 12, 3) X(1024, 9, 2) X(512, 17, 4)
-
-static const void* reg_kernel(int bs, int cpt, int vpt, int kk)
+static const void* reg_kernel(const RegVariant& r, int kk)
 {
-#define ASAT_REG_PTR(B, C, V)                                                          \
-    if (bs == B && cpt == C && vpt == V)                                               \
-        return kk == 3 ? (const void*)k_batch_reg<B, C, V, 3> : (const void*)k_batch_reg<B, C, V, 0>;
+#define ASAT_REG_PTR(T, C, V, W)                                                              \
+    if (r.tt == T && r.cpt == C)                                                              \
+        return kk == 3 ? (const void*)k_batch_reg<T, C, V, 3, W> : (const void*)k_batch_reg<T, C, V, 4, W>;
     ASAT_REG_VARIANTS(ASAT_REG_PTR)
 #undef ASAT_REG_PTR
-    return nullptr;
+    throw Error(ASAT_ERR_HIP, "no register-resident kernel for this tiling");
 }
 
-static void launch_reg(hipStream_t st, const Params& P, int grid, int bs, int cpt, int vpt, int kk, size_t shmem)
+static void launch_ptr(const void* f, hipStream_t st, const Params& P, int grid, int bs, size_t shmem)
 {
-#define ASAT_REG_LAUNCH(B, C, V)                                                               \
-    if (bs == B && cpt == C && vpt == V) {                                                     \
-        if (kk == 3) hipLaunchKernelGGL((k_batch_reg<B, C, V, 3>), dim3(grid), dim3(B), shmem, st, P); \
-        else hipLaunchKernelGGL((k_batch_reg<B, C, V, 0>), dim3(grid), dim3(B), shmem, st, P); \
-        return;                                                                                \
-    }
-    ASAT_REG_VARIANTS(ASAT_REG_LAUNCH)
-#undef ASAT_REG_LAUNCH
-    throw Error(ASAT_ERR_HIP, "no register-resident kernel for this tiling");
+    Params arg = P;
+    void* args[] = {&arg};
+    HIP_CHECK(hipLaunchKernel(f, dim3(grid), dim3(bs), args, shmem, st));
+}
+
+// chunked mode: LDS entries before the terms (factor pairs and sums), and the
+// clauses per chunk that an instance may take
+static int chunk_ranks(const Bucket& b) { return (int)round_up_ll((long long)b.maxn + 2, 4); }
+static int chunk_terms_for(const Bucket& b, size_t lds_limit)
+{
+    const long long t = (long long)(lds_limit - LDS_STATIC) / (long long)sizeof(float) - 3LL * chunk_ranks(b) - 1;
+    return (int)std::min<long long>(t, 65535);
+}
+static int chunk_max(const Instance& I, int terms, int force)
+{
+    const int cs = terms / (I.k <= 3 ? 3 : 4) / 64 * 64;
+    return force > 0 ? std::min(cs, std::max(force, 1)) : cs;
 }
 
 template <int MODE>
@@ -967,19 +1572,19 @@ static const void* kernel_of(int bs)
                                                                    : (const void*)k_batch<1024, MODE>;
 }
 
-static void set_lds_attr(int bs, int mode, size_t bytes)
+static const void* chunk_kernel(int bs)
 {
-    const void* f = mode == 1 ? kernel_of<1>(bs) : mode == 3 ? kernel_of<3>(bs) : kernel_of<0>(bs);
-    HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    return bs == 256 ? (const void*)k_batch_chunk<256> : bs == 512 ? (const void*)k_batch_chunk<512>
+                                                                   : (const void*)k_batch_chunk<1024>;
 }
 
 static void dispatch(hipStream_t st, const Params& P, const Bucket& b)
 {
     const int grid = b.grid, bs = b.block;
     const size_t shmem = b.lds_bytes;
-    if (b.lds == 2) launch_reg(st, P, grid, bs, b.cpt, b.vpt, b.kk, shmem);
+    if (b.lds == 2) launch_ptr(reg_kernel(*b.reg, b.kk), st, P, grid, bs, shmem);
     else if (b.lds == 1) launch_mode<1>(st, P, grid, bs, shmem);
-    else if (b.lds == 3) launch_mode<3>(st, P, grid, bs, shmem);
+    else if (b.lds == 3) launch_ptr(chunk_kernel(bs), st, P, grid, bs, shmem);
     else launch_mode<0>(st, P, grid, bs, shmem);
 }
 
@@ -992,8 +1597,11 @@ static Params params_of(const Batch& B, const Bucket& b)
     P.queue = b.d_queue; P.eps = B.eps; P.floor = B.floor; P.max_time = B.max_time; P.max_steps = B.max_steps;
     P.chunk_steps = B.chunk_steps; P.check_every = std::max(1, B.check_every);
     P.sp_stride = b.sp_stride;
-    P.vcode = B.d_vcode;
-    P.chunk_clauses = b.lds == 3 ? b.chunk : 0;
+    P.rcode = B.d_rcode; P.rgroup = B.d_rgroup; P.rvmap = B.d_rvmap;
+    P.ccode = B.d_ccode; P.cgroup = B.d_cgroup; P.cperm = B.d_cperm; P.crec = B.d_crec; P.cstart = B.d_cstart;
+    P.reg_lds = b.reg ? (int)reg_lds(*b.reg, b) : 0;
+    P.chunk_terms = b.chunk_terms;
+    P.fac_ranks = chunk_ranks(b);
     return P;
 }
 
@@ -1005,41 +1613,31 @@ static int per_cu(const Batch& B, int bs, size_t lds_bytes)
     return std::max(1, std::min(by_lds, by_threads));
 }
 
-static int chunk_for(const Batch& B, const Bucket& b, int wgs)
-{
-    // 1 KB left for the kernel's static shared arrays (block reductions)
-    const long long avail = (long long)(B.lds_limit / wgs) - (long long)chunk_lds(b, 0) - 1024;
-    long long c = std::min<long long>(avail / (long long)sizeof(float), round_up_ll(b.maxm, 256));
-    c = c / 256 * 256;
-    return c >= 256 ? (int)c : 0;
-}
-
 // mode: 0 contributions in global scratch, 1 in LDS, 2 register-resident
-// kernel (contributions in LDS; bs comes from its variant).  grid_cap > 0
-// limits the resident workgroups (global-scratch mode: the scattered
-// contribution writes of fewer workgroups stay in the Infinity Cache).
-static void configure_bucket(Batch& B, Bucket& b, int bs, int mode, int grid_cap = 0, int chunk = 0)
+// kernel (bs names the workgroup size of its variant, or rv the variant), 3
+// clause-chunked.  grid_cap > 0 limits the resident workgroups (global-scratch
+// mode: the scattered contribution writes of fewer workgroups stay in the
+// Infinity Cache).
+static void configure_bucket(Batch& B, Bucket& b, int bs, int mode, int grid_cap = 0, const RegVariant* rv = nullptr)
 {
-    const bool lds = mode == 1 || mode == 2;
+    b.reg = nullptr;
     if (mode == 2) {
-        const RegVariant* r = reg_variant(b, bs);
-        if (!r) r = reg_variant(b);
-        require(r != nullptr, ASAT_ERR_INVALID_ARGUMENT, "instances too large for the register-resident kernel");
-        bs = r->bs;
-        b.cpt = r->cpt;
-        b.vpt = r->vpt;
+        if (!rv) rv = reg_variant(b, B.lds_limit, bs);
+        if (!rv) rv = reg_variant(b, B.lds_limit);
+        require(rv != nullptr, ASAT_ERR_INVALID_ARGUMENT, "instances too large for the register-resident kernel");
+        b.reg = rv;
+        bs = rv->block();
     }
-    if (mode == 3) {
-        require(b.vcode, ASAT_ERR_INVALID_ARGUMENT, "clause-chunked records were not built for this bucket");
-        if (chunk <= 0) chunk = chunk_for(B, b, 1);
-        if (B.force_chunk > 0) chunk = std::min(chunk, B.force_chunk);
-        require(chunk > 0, ASAT_ERR_UNSUPPORTED, "instances too large for the clause-chunked kernel");
-    }
+    if (mode == 3)
+        require(b.chunked, ASAT_ERR_INVALID_ARGUMENT, "the clause-chunked layout was not built for this bucket");
     b.block = bs;
     b.lds = mode;
-    b.chunk = mode == 3 ? chunk : 0;
-    b.lds_bytes = mode == 3 ? chunk_lds(b, chunk) : bucket_lds(b, lds);
-    b.grid = std::max(1, std::min((int)b.ids.size(), B.cus * per_cu(B, bs, mode == 0 ? 0 : b.lds_bytes)));
+    const int per_wg = mode == 2 ? b.reg->waves() : 1;      // trajectories of a workgroup
+    b.lds_bytes = mode == 2   ? reg_lds(*b.reg, b) * per_wg
+                  : mode == 3 ? sizeof(float) * (3 * (size_t)chunk_ranks(b) + (size_t)b.chunk_terms + 1)
+                              : bucket_lds(b, mode == 1);
+    b.grid = std::max(1, std::min(ceil_div((long long)b.ids.size(), per_wg),
+                                  B.cus * per_cu(B, bs, mode == 0 ? 0 : b.lds_bytes)));
     if (grid_cap > 0) b.grid = std::min(b.grid, grid_cap);
     b.scratch_stride = round_up_ll((long long)b.maxn + b.maxm, 64);
     b.scratch_per_wg = mode == 2 ? 0 : 5 * b.scratch_stride + (mode == 0 ? round_up_ll(b.maxl, 64) : 0);
@@ -1048,11 +1646,11 @@ static void configure_bucket(Batch& B, Bucket& b, int bs, int mode, int grid_cap
     const size_t sbytes = sizeof(float) * std::max<size_t>((size_t)b.scratch_per_wg * b.grid, 1);
     HIP_CHECK(hipMalloc((void**)&b.d_scratch, sbytes));
     HIP_CHECK(hipMemset(b.d_scratch, 0, sbytes));
-    if (mode == 2)
-        HIP_CHECK(hipFuncSetAttribute(reg_kernel(bs, b.cpt, b.vpt, b.kk), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)b.lds_bytes));
-    else
-        set_lds_attr(bs, mode, b.lds_bytes);
+    const void* f = mode == 2   ? reg_kernel(*b.reg, b.kk)
+                    : mode == 3 ? chunk_kernel(bs)
+                    : mode == 1 ? kernel_of<1>(bs)
+                                : kernel_of<0>(bs);
+    HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b.lds_bytes));
 }
 
 static void reset_state(Batch& B)
@@ -1065,41 +1663,40 @@ static void reset_state(Batch& B)
     B.solved_wall_ms.assign(T, -1.0);
 }
 
-// Autotuner: for each bucket, time one short chunk (2 accepted steps of every
-// trajectory in the bucket) for each workgroup size and contribution placement
-// that fits (for global scratch also with the resident workgroups capped so
-// that their contribution scratch totals 64, 128 or 256 MB), keep the
-// fastest per trajectory-attempt, then restore the start.
+// Autotuner: for each bucket, time one short chunk (2 to 32 accepted steps of
+// every trajectory in the bucket, more for small instances, whose launch would
+// hide the difference) of each configuration that fits, keep the fastest per
+// trajectory-attempt, then restore the start.  Register variants exclude
+// the others, and the clause-chunked kernel excludes global scratch (never the
+// faster ones where both fit: N = 2000, 0.30 us per attempt in registers, 1.0 in
+// LDS, 3.2 in global scratch), unless asat_batch_set_tiling asks for one.
 static void autotune(Batch& B)
 {
     const int saved_chunk = B.chunk_steps;
-    B.chunk_steps = 2;
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
     for (auto& b : B.buckets) {
-        struct Cand { int bs, mode, cap, chunk; };
+        B.chunk_steps = std::min(32, std::max(2, 60000 / std::max(b.maxl, 1)));
+        struct Cand { int bs, mode, cap; const RegVariant* rv; };
         std::vector<Cand> cand;
-        for (int bs : {256, 512, 768, 1024}) {
-            const RegVariant* rv = reg_variant(b, bs);
-            if (rv && b.lds_fits && (B.force_lds == -1 || B.force_lds == 2) && (!B.force_block || B.force_block == bs))
-                cand.push_back({bs, 2, 0, 0});
-        }
+        if (B.force_lds == -1 || B.force_lds == 2)
+            for (const RegVariant& r : REG_VARIANTS)
+                if ((!B.force_block || r.block() == B.force_block) && reg_fits(r, b, B.lds_limit))
+                    cand.push_back({r.block(), 2, 0, &r});
+        const bool reg_only = !cand.empty() && B.force_lds == -1;
         const long long contrib_bytes = 4 * round_up_ll(b.maxl, 64);
         for (int bs : {256, 512, 1024}) {
+            if (reg_only) break;
             if (B.force_block && bs != B.force_block) continue;
-            if (b.lds_fits && (B.force_lds == -1 || B.force_lds == 1)) cand.push_back({bs, 1, 0, 0});
-            if (b.vcode && (B.force_lds == -1 || B.force_lds == 3))
-                for (int wgs : {1, 2}) {
-                    const int ch = chunk_for(B, b, wgs);
-                    if (ch > 0) cand.push_back({bs, 3, 0, ch});
-                }
-            if (B.force_lds == -1 || B.force_lds == 0) {
-                cand.push_back({bs, 0, 0, 0});
+            if (b.lds_fits && (B.force_lds == -1 || B.force_lds == 1)) cand.push_back({bs, 1, 0, nullptr});
+            if (b.chunked && (B.force_lds == -1 || B.force_lds == 3)) cand.push_back({bs, 3, 0, nullptr});
+            if (B.force_lds == 0 || (B.force_lds == -1 && !b.chunked && !b.lds_fits)) {
+                cand.push_back({bs, 0, 0, nullptr});
                 const int full = std::max(1, std::min((int)b.ids.size(), B.cus * per_cu(B, bs, 0)));
                 for (long long mb : {256LL, 128LL, 64LL}) {
                     const int cap = (int)std::max<long long>(8, (mb << 20) / std::max<long long>(contrib_bytes, 1));
-                    if (cap < full) cand.push_back({bs, 0, cap, 0});
+                    if (cap < full) cand.push_back({bs, 0, cap, nullptr});
                 }
             }
         }
@@ -1108,7 +1705,7 @@ static void autotune(Batch& B)
         Cand pick = cand.front();
         if (cand.size() > 1) {
             for (auto& c : cand) {
-                configure_bucket(B, b, c.bs, c.mode, c.cap, c.chunk);
+                configure_bucket(B, b, c.bs, c.mode, c.cap, c.rv);
                 reset_state(B);
                 Params P = params_of(B, b);
                 hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, B.stream, b.d_queue);
@@ -1127,13 +1724,20 @@ static void autotune(Batch& B)
                 if (us < best) { best = us; pick = c; }
             }
         }
-        configure_bucket(B, b, pick.bs, pick.mode, pick.cap, pick.chunk);
+        configure_bucket(B, b, pick.bs, pick.mode, pick.cap, pick.rv);
         b.tuned_us = best < 1e300 ? best : -1.0;
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     B.chunk_steps = saved_chunk;
     reset_state(B);
+}
+
+template <typename V>
+static void upload_vec(V*& d, const std::vector<V>& h)
+{
+    HIP_CHECK(hipMalloc((void**)&d, sizeof(V) * h.size()));
+    HIP_CHECK(hipMemcpy(d, h.data(), sizeof(V) * h.size(), hipMemcpyHostToDevice));
 }
 
 static void prepare(Batch& B, bool tune)
@@ -1163,7 +1767,8 @@ static void prepare(Batch& B, bool tune)
         desc[i].state_off = state_total;
         B.state_off[i] = state_total;
         desc[i].n = I.n; desc[i].m = I.m; desc[i].k = I.k; desc[i].nslots = I.nslots;
-        desc[i].vcode_off = -1;
+        desc[i].rcode_off = desc[i].rgroup_off = desc[i].rvmap_off = -1;
+        desc[i].ccode_off = desc[i].cgroup_off = desc[i].crec_off = desc[i].cstart_off = -1;
         desc[i].knorm = (float)std::pow(2.0, -I.k);
         code_total += (long long)I.code.size();
         row_total += (long long)I.rowptr.size();
@@ -1191,37 +1796,89 @@ static void prepare(Batch& B, bool tune)
         Bucket& b = B.buckets[q];
         int lo = (int)((long long)T * q / nb), hi = (int)((long long)T * (q + 1) / nb);
         b.ids.assign(order.begin() + lo, order.begin() + hi);
-        bool allk3 = true;
         for (int id : b.ids) {
             b.maxn = std::max(b.maxn, B.inst[id].n);
             b.maxm = std::max(b.maxm, B.inst[id].m);
             b.maxl = std::max(b.maxl, B.inst[id].nslots);
-            allk3 = allk3 && B.inst[id].k == 3;
+            b.kk = std::max(b.kk, B.inst[id].k <= 3 ? 3 : 4);
         }
-        b.kk = allk3 ? 3 : 0;
         b.sp_stride = (int)round_up_ll((long long)b.maxn + 1, 4);
         b.lds_fits = bucket_lds(b, true) <= B.lds_limit;
         HIP_CHECK(hipMalloc((void**)&b.d_order, sizeof(int) * b.ids.size()));
         HIP_CHECK(hipMalloc((void**)&b.d_queue, sizeof(int)));
         HIP_CHECK(hipMemcpy(b.d_order, b.ids.data(), sizeof(int) * b.ids.size(), hipMemcpyHostToDevice));
     }
-    // clause-chunked records for the buckets whose contributions do not fit in LDS
-    long long vc_total = 0;
-    for (auto& b : B.buckets) {
-        b.vcode = (!b.lds_fits || B.force_lds == 3) && chunk_for(B, b, 1) > 0;
-        if (!b.vcode) continue;
-        for (int id : b.ids) {
-            desc[id].vcode_off = vc_total;
-            vc_total += B.inst[id].nslots;
+    // the register kernel's layout for the buckets that fit one of its
+    // variants, the clause-chunked layout for the others
+    {
+        std::vector<RegLayout> reg((size_t)T);
+        long long rcode = 0, rgroup = 0, rvmap = 0;
+        for (auto& b : B.buckets) {
+            bool may = false;
+            for (const RegVariant& r : REG_VARIANTS) may = may || reg_fits(r, b, B.lds_limit);
+            if (!may || (B.force_lds != -1 && B.force_lds != 2)) { b.ncontrib = 1 << 30; continue; }
+            for (int id : b.ids) {
+                reg_layout(B.inst[id], reg[(size_t)id]);
+                b.ncontrib = std::max(b.ncontrib, reg[(size_t)id].ncontrib);
+            }
+            if (!reg_variant(b, B.lds_limit)) continue;
+            for (int id : b.ids) {
+                const RegLayout& L = reg[(size_t)id];
+                desc[id].rcode_off = rcode; desc[id].rgroup_off = rgroup; desc[id].rvmap_off = rvmap;
+                desc[id].ngroups = L.ngroups; desc[id].ncontrib = L.ncontrib;
+                rcode += rcode_len(B.inst[id], b.kk);
+                rgroup += (long long)L.group.size();
+                rvmap += (long long)L.vmap.size();
+            }
+        }
+        if (rcode > 0) {
+            std::vector<uint32_t> hc((size_t)rcode);
+            std::vector<int> hg((size_t)rgroup), hv((size_t)rvmap);
+            for (auto& b : B.buckets)
+                for (int id : b.ids) {
+                    if (desc[id].rcode_off < 0) continue;
+                    const RegLayout& L = reg[(size_t)id];
+                    reg_codes(B.inst[id], L, b.kk, hc.data() + desc[id].rcode_off);
+                    std::copy(L.group.begin(), L.group.end(), hg.begin() + desc[id].rgroup_off);
+                    std::copy(L.vmap.begin(), L.vmap.end(), hv.begin() + desc[id].rvmap_off);
+                }
+            upload_vec(B.d_rcode, hc);
+            upload_vec(B.d_rgroup, hg);
+            upload_vec(B.d_rvmap, hv);
         }
     }
-    if (vc_total > 0) {
-        std::vector<unsigned long long> vc((size_t)vc_total);
-        for (int i = 0; i < T; i++)
-            if (desc[i].vcode_off >= 0) build_vcode(B.inst[i], vc.data() + desc[i].vcode_off);
-        HIP_CHECK(hipMalloc((void**)&B.d_vcode, sizeof(unsigned long long) * (size_t)vc_total));
-        HIP_CHECK(hipMemcpy(B.d_vcode, vc.data(), sizeof(unsigned long long) * (size_t)vc_total,
-                            hipMemcpyHostToDevice));
+    {
+        std::vector<uint2> hcode;
+        std::vector<int2> hgroup;
+        std::vector<uint16_t> hperm;
+        std::vector<uint32_t> hrec;
+        std::vector<int> hstart;
+        for (auto& b : B.buckets) {
+            const bool want = B.force_lds == 3 || (B.force_lds == -1 && !reg_variant(b, B.lds_limit));
+            b.chunk_terms = chunk_terms_for(b, B.lds_limit);
+            b.chunked = want && b.chunk_terms >= 4 * 64;
+            if (!b.chunked) continue;
+            for (int id : b.ids) {
+                ChunkLayout L;
+                chunk_layout(B.inst[id], chunk_max(B.inst[id], b.chunk_terms, B.force_chunk), b.chunk_terms, L);
+                Desc& d = desc[id];
+                d.ccode_off = (long long)hcode.size(); d.cgroup_off = (long long)hgroup.size();
+                d.crec_off = (long long)hrec.size(); d.cstart_off = (long long)hstart.size();
+                d.nchunks = L.nchunks; d.chunk = L.cs;
+                hcode.insert(hcode.end(), L.code.begin(), L.code.end());
+                hgroup.insert(hgroup.end(), L.group.begin(), L.group.end());
+                hperm.insert(hperm.end(), L.perm.begin(), L.perm.end());
+                hrec.insert(hrec.end(), L.rec.begin(), L.rec.end());
+                hstart.insert(hstart.end(), L.start.begin(), L.start.end());
+            }
+        }
+        if (!hcode.empty()) {
+            upload_vec(B.d_ccode, hcode);
+            upload_vec(B.d_cgroup, hgroup);
+            upload_vec(B.d_cperm, hperm);
+            upload_vec(B.d_crec, hrec);
+            upload_vec(B.d_cstart, hstart);
+        }
     }
     HIP_CHECK(hipMalloc((void**)&B.d_desc, sizeof(Desc) * T));
     HIP_CHECK(hipMalloc((void**)&B.d_code, sizeof(uint32_t) * std::max<long long>(code_total, 1)));
@@ -1242,13 +1899,14 @@ static void prepare(Batch& B, bool tune)
     }
     for (auto& b : B.buckets) {
         int bs = B.force_block ? B.force_block : 1024;
-        const RegVariant* rv = reg_variant(b);
-        const bool reg_ok = rv && b.lds_fits && (!B.force_block || B.force_block == rv->bs);
-        int mode = B.force_lds == -1 ? (reg_ok ? 2 : (b.lds_fits ? 1 : (b.vcode ? 3 : 0))) : B.force_lds;
-        require(mode == 0 || mode == 3 || b.lds_fits, ASAT_ERR_UNSUPPORTED, "instances too large for LDS contributions");
-        require(mode != 3 || b.vcode, ASAT_ERR_UNSUPPORTED, "instances too large for the clause-chunked kernel");
-        require(mode != 2 || reg_variant(b), ASAT_ERR_UNSUPPORTED,
-                "instances too large for the register-resident kernel");
+        const bool reg_any = B.force_lds != 0 && B.force_lds != 1 && reg_variant(b, B.lds_limit);
+        const bool reg_ok = reg_any && (!B.force_block || reg_variant(b, B.lds_limit, B.force_block));
+        int mode = B.force_lds == -1 ? (reg_ok ? 2 : (b.lds_fits ? 1 : (b.chunked ? 3 : 0))) : B.force_lds;
+        require(mode == 0 || mode == 2 || mode == 3 || b.lds_fits, ASAT_ERR_UNSUPPORTED,
+                "instances too large for LDS contributions");
+        require(mode != 3 || b.chunked, ASAT_ERR_UNSUPPORTED, "instances too large for the clause-chunked kernel");
+        require(mode != 2 || reg_any, ASAT_ERR_UNSUPPORTED, "instances too large for the register-resident kernel");
+        if (mode == 2 && !B.force_block) bs = 0;
         configure_bucket(B, b, bs, mode);
     }
     reset_state(B);

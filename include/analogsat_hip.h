@@ -321,9 +321,9 @@ typedef struct {
 
 typedef struct {
     int trajectories, max_n, max_m, max_slots;
-    int block;               /* workgroup size chosen (256 / 512 / 1024) */
+    int block;               /* workgroup size chosen (256 / 512 / 768 / 1024) */
     int lds;                 /* 1: contributions in LDS, 0: in global scratch, 2: register-resident kernel,
-                                3: clause-chunked kernel (no contribution array) */
+                                3: clause-chunked kernel (a chunk's contributions in LDS) */
     int grid;                /* resident workgroups */
     long long lds_bytes;
     double tuned_us_per_attempt;   /* autotuner's measurement, -1 if not tuned */
@@ -343,10 +343,9 @@ int asat_batch_set_xscal_floor(asat_batch_t* b, double floor);
 /* block: 0 autotune or 256/512/1024; lds_mode: -1 auto, 0 contributions in
    global scratch, 1 in LDS, 2 register-resident kernel (state and stage
    derivatives in registers, contributions in LDS; its workgroup size is
-   fixed by the instance size), 3 clause-chunked kernel (per chunk of
-   clauses, their r_m in LDS and each variable's terms of that chunk formed
-   from 8-byte var-major records; for instances whose contributions do not
-   fit in LDS); nbuckets: size buckets (trajectories split by work, one
+   fixed by the instance size), 3 clause-chunked kernel (a chunk of clauses at
+   a time, its contributions in LDS; for instances whose contributions do not
+   fit there together); nbuckets: size buckets (trajectories split by work, one
    launch each) */
 int asat_batch_set_tiling(asat_batch_t* b, int block, int lds_mode, int nbuckets);
 /* clause-chunked kernel: at most `clauses` clauses per chunk (0: as many as
