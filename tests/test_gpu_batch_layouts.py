@@ -72,3 +72,31 @@ def test_register_variant_mixed_lengths_one_bucket():
 def test_chunked_layouts(n, m, k, block, chunk):
     insts = [instance(n, m, k, 70 + i, short=0.3 if i == 1 else 0.0, tiny=i == 1) for i in range(2)]
     run(insts, 6, block, 3, chunk=chunk)
+
+
+def test_states_in_any_order_and_after_every_change():
+    """state(i) in order (packed windows) and out of order (single copies) agree
+    with each other and follow every run and reset; states of different parity
+    and sizes, a window that ends inside the batch."""
+    sizes = [(20 + 7 * (i % 5), 60 + 11 * (i % 7)) for i in range(30)] + [(8000, 34000)] * 30   # 1.3e6 floats
+    insts = [instance(n, m, 3, 90 + i) for i, (n, m) in enumerate(sizes)]
+    b = A.HipBatch()
+    for p, pub in insts:
+        b.add(A.SatProblem(p.literals, p.lengths), pub)
+    b.set_params(eps=1e-6, max_steps=30, chunk_steps=1)
+    b.set_tiling(block=256, lds_mode=-1, nbuckets=3)
+    b.prepare(autotune=False)
+    count = len(insts)
+    seen = []
+    for limit in (0, 1, 2):
+        if limit:
+            b.run(max_chunks=1, graph_chunks=1)
+        inorder = [b.state(i) for i in range(count)]
+        backward = [b.state(i) for i in reversed(range(count))][::-1]
+        for i in range(count):
+            assert np.array_equal(inorder[i], backward[i]), (limit, i)
+        seen.append(inorder)
+    assert all(np.array_equal(seen[0][i], insts[i][1]) for i in range(count))
+    assert any(not np.array_equal(seen[1][i], seen[2][i]) for i in range(count))
+    b.reset()
+    assert all(np.array_equal(b.state(i), insts[i][1]) for i in range(count))
