@@ -2005,6 +2005,7 @@ static void run(Batch& B, int max_chunks, int graph_chunks)
     struct Owned {
         hipStream_t st;
         hipEvent_t e0 = nullptr, e1 = nullptr;
+        hipEvent_t fork = nullptr, join[3] = {nullptr, nullptr, nullptr};
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
         bool capturing = false;
@@ -2018,6 +2019,9 @@ static void run(Batch& B, int max_chunks, int graph_chunks)
             if (graph) (void)hipGraphDestroy(graph);
             if (e0) (void)hipEventDestroy(e0);
             if (e1) (void)hipEventDestroy(e1);
+            if (fork) (void)hipEventDestroy(fork);
+            for (hipEvent_t e : join)
+                if (e) (void)hipEventDestroy(e);
         }
     } o{B.stream};
     HIP_CHECK(hipEventCreate(&o.e0));
@@ -2027,14 +2031,34 @@ static void run(Batch& B, int max_chunks, int graph_chunks)
         std::lock_guard<std::mutex> lock(B.win_lock);
         B.drop_window();
     }
-    // one graph = graph_chunks x (per bucket: reset its queue, persistent launch)
+    // one graph = graph_chunks x (per bucket: reset its queue, persistent
+    // launch).  Buckets are independent, so their launches go to up to four
+    // branches: a bucket with fewer trajectories than resident workgroups leaves
+    // CUs to the next one, and so does the end of every launch, when the last
+    // trajectories run alone (512 ragged instances, 128 per bucket on 256 CUs:
+    // 19.5 -> 13.5 ms for 20 steps)
+    const int nb = (int)B.buckets.size(), branches = std::min(nb, 4);
+    HIP_CHECK(hipEventCreateWithFlags(&o.fork, hipEventDisableTiming));
+    for (int q = 1; q < branches; q++) {
+        if (!B.side[q - 1]) HIP_CHECK(hipStreamCreateWithFlags(&B.side[q - 1], hipStreamNonBlocking));
+        HIP_CHECK(hipEventCreateWithFlags(&o.join[q - 1], hipEventDisableTiming));
+    }
     HIP_CHECK(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
     o.capturing = true;
-    for (int c = 0; c < graph_chunks; c++) {
-        for (auto& b : B.buckets) {
-            Params P = params_of(B, b);
-            hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, B.stream, b.d_queue);
-            dispatch(B.stream, P, b);
+    HIP_CHECK(hipEventRecord(o.fork, B.stream));
+    for (int q = 0; q < branches; q++) {
+        hipStream_t st = q ? B.side[q - 1] : B.stream;
+        if (q) HIP_CHECK(hipStreamWaitEvent(st, o.fork, 0));
+        for (int c = 0; c < graph_chunks; c++)
+            for (int i = q; i < nb; i += branches) {
+                Bucket& b = B.buckets[(size_t)i];
+                Params P = params_of(B, b);
+                hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, st, b.d_queue);
+                dispatch(st, P, b);
+            }
+        if (q) {
+            HIP_CHECK(hipEventRecord(o.join[q - 1], st));
+            HIP_CHECK(hipStreamWaitEvent(B.stream, o.join[q - 1], 0));
         }
     }
     o.capturing = false;
