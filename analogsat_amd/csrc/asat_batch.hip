@@ -391,7 +391,7 @@ __global__ __launch_bounds__(BS) void k_batch(Params P)
 // Against the variable-major contribution runs before (a wave as slow as its
 // busiest variable, bank conflicts in the sums, 4 instructions to unpack a
 // slot), per 100 steps of 1024 trajectories with N = 2000, M = 8500: 26.0 ->
-// 14.7 ms; 1000 steps of 1000 with N = 50, M = 213: 10.8 -> 7.3 ms.
+// 13.2 ms; 1000 steps of 1000 with N = 50, M = 213: 10.8 -> 7.3 ms.
 constexpr int REG_WAVES = 4;     // TT = 64: trajectories (waves) per workgroup
 
 // a value every lane holds, moved to scalar registers
@@ -420,21 +420,35 @@ __device__ __forceinline__ void traj_sync()
         __syncthreads();
     }
 }
-// maximum and sum over the trajectory's threads, in every one of them; with
-// several waves two barriers each
+// Error norm / eps over the trajectory's threads and the power of it that the
+// step control needs (errmax^-0.2 on acceptance above ERRCON, errmax^-0.25 on
+// rejection), in every thread; with several waves two barriers.  One wave
+// computes them: in all of 16 waves the 190 dependent FP64 operations of
+// pow_ctrl would take four times as long, a quarter of the SIMDs' issue each.
+struct Control { double errmax, power; };
+__device__ __forceinline__ Control control_of(double err, double eps)
+{
+    Control c;
+    c.errmax = err / eps;
+    c.power = c.errmax > TabD::ERRCON ? pow_ctrl(c.errmax, c.errmax <= 1.0 ? 5 : 4) : 0.0;
+    return c;
+}
 template <int TT>
-__device__ __forceinline__ double traj_max(double v, double* sh)
+__device__ __forceinline__ Control traj_control(double v, double eps, double* red, Control* out)
 {
     v = wave_max_dpp(v);
-    if constexpr (TT == 64) return v;
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    if constexpr (TT == 64) return control_of(v, eps);
+    const int lane = (int)(threadIdx.x & 63);
+    if (lane == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    double r = sh[0];
-#pragma unroll
-    for (int i = 1; i < TT / 64; i++) r = fmax(r, sh[i]);
+    if (threadIdx.x < 64) {
+        const Control c = control_of(wave_max_dpp(lane < TT / 64 ? red[lane] : 0.0), eps);
+        if (lane == 0) *out = c;
+    }
     __syncthreads();
-    return r;
+    return *out;
 }
+// sum over the trajectory's threads, in every one of them
 template <int TT>
 __device__ __forceinline__ int traj_sum(int v, int* sh)
 {
@@ -464,10 +478,11 @@ __device__ __forceinline__ void code_store(unsigned char* con, uint32_t c, float
     if constexpr (WIDE) *(float*)(con + ((c >> 16) << 2)) = v;
     else *(float*)(con + (c >> 14)) = v;
 }
-// v with its sign flipped for a negated literal (bit 2 of the code)
+// v with its sign flipped for a negated literal: c << 29 is bit 2 alone (a code's
+// bits 0 and 1 are 0), and adding the top bit flips it
 __device__ __forceinline__ float code_sign(uint32_t c, float v)
 {
-    return __uint_as_float(((c << 29) & 0x80000000u) ^ __float_as_uint(v));
+    return __uint_as_float((c << 29) + __float_as_uint(v));
 }
 
 // the two factors of a spin, written by its variable's thread
@@ -488,12 +503,12 @@ __device__ __forceinline__ void load_code(const uint32_t* code, int j, uint32_t 
     for (int q = 0; q < KK; q++) c[q] = p[q];
 }
 
-// Clause phase of stage J.  COUNT (J = 1): viol receives the number of this
+// Clause phase of stage J; kn2 = 4^-k.  COUNT (J = 1): viol receives the number of this
 // thread's clauses violated by the state whose factors are in LDS; pos has a
 // bit per rank, s > 0, for the factors that are exactly 1.
 template <int TT, int CPT, int VPT, int J, int KK, bool WIDE, bool COUNT>
-__device__ __forceinline__ void reg_clauses(RegState<TT, CPT, VPT, KK>& R, const uint32_t* code, int m, float knorm,
-                                            float knorm2, const unsigned char* fac, unsigned char* con, float hs,
+__device__ __forceinline__ void reg_clauses(RegState<TT, CPT, VPT, KK>& R, const uint32_t* code, int m, float kn2,
+                                            const unsigned char* fac, unsigned char* con, float hs,
                                             double h, double hnext, double floor, double& err,
                                             const unsigned long long* pos, int& viol)
 {
@@ -520,14 +535,18 @@ __device__ __forceinline__ void reg_clauses(RegState<TT, CPT, VPT, KK>& R, const
                 // the next clause's codes are loaded while this one is processed
 #pragma unroll
                 for (int q = 0; q < KK; q++) c[q] = nx[q];
-                if (u + 1 < CPT && w0 + (u + 1) * TT < m) load_code<KK>(code, tid + (u + 1) * TT, nx);
+                // (past the wave's last one: its first again, which keeps
+                // the loads free of branches)
+                if (u + 1 < CPT) load_code<KK>(code, tid + (w0 + (u + 1) * TT < m ? (u + 1) * TT : 0), nx);
             }
             float f[KK];
 #pragma unroll
             for (int q = 0; q < KK; q++) f[q] = code_factor<WIDE>(fac, c[q]);
-            float km = knorm;
+            // products of the factors of K_m left to right, without 2^-k: the
+            // powers of two are exact wherever they are multiplied in
+            float km = f[0];
 #pragma unroll
-            for (int q = 0; q < KK; q++) km *= f[q];
+            for (int q = 1; q < KK; q++) km *= f[q];
             if constexpr (COUNT) {
                 bool sat = false, unsat = true;
 #pragma unroll
@@ -552,7 +571,8 @@ __device__ __forceinline__ void reg_clauses(RegState<TT, CPT, VPT, KK>& R, const
             float am;
             if constexpr (J == 1) am = R.xa[u];
             else am = stage_input<float, J>(R.xa[u], R.a1[u], R.a2[u], R.a3[u], R.a4[u], R.a5[u], hs);
-            const float kj = am * km * km;
+            const float am_km = am * km;
+            const float kj = am_km * km * kn2;
             if constexpr (J == 1) R.a1[u] = kj;
             else if constexpr (J == 2) R.a2[u] = kj;
             else if constexpr (J == 3) R.a3[u] = kj;
@@ -565,8 +585,8 @@ __device__ __forceinline__ void reg_clauses(RegState<TT, CPT, VPT, KK>& R, const
                 R.a2[u] = xv;
                 err = fmax(err, e);
             }
-            // the factor 2 of every term is in knorm2 = 2 knorm (a power of two)
-            const float r = km * knorm2 * am;
+            // K_m 2^-k a_m and the factor 2 of every term
+            const float r = am_km * (2.0f * kn2);
 #pragma unroll
             for (int q = 0; q < KK; q++) {
                 float p = 1.0f;
@@ -661,6 +681,7 @@ template <int TT, int VPT>
 struct alignas(16) RegShared {
     unsigned long long pos[(TT / 64) * VPT];
     double red[TT / 64];
+    Control control;
     int redi[TT / 64];
     int traj;
 };
@@ -705,7 +726,7 @@ __global__ __launch_bounds__(TT == 64 ? 64 * REG_WAVES : TT) void k_batch_reg(Pa
         const int* group = P.rgroup + uni(d.rgroup_off);     // base and depth per 64 ranks
         const int* vmap = P.rvmap + uni(d.rvmap_off);        // rank -> variable
         const int ngroups = uni(d.ngroups);
-        const float knorm = uni(d.knorm), knorm2 = 2.0f * knorm;
+        const float kn2 = uni(d.knorm * d.knorm);       // 4^-k
         double t = cp->t, h = cp->h, hnext = cp->hnext, hdid = cp->hdid, errmax_last = cp->errmax;
         long long steps = cp->steps, attempts = cp->attempts, rhscount = cp->rhscount;
         int parity = cp->parity, min_viol = cp->min_viol, viol = cp->viol;
@@ -757,7 +778,7 @@ __global__ __launch_bounds__(TT == 64 ? 64 * REG_WAVES : TT) void k_batch_reg(Pa
             double err_local = 0.0;
             int cnt = 0;
             if (count) {
-                reg_clauses<TT, CPT, VPT, 1, KK, WIDE, true>(R, code, m, knorm, knorm2, fac, con, (float)h_at1, h_at1,
+                reg_clauses<TT, CPT, VPT, 1, KK, WIDE, true>(R, code, m, kn2, fac, con, (float)h_at1, h_at1,
                                                              hnext, P.floor, err_local, pos, cnt);
                 viol = traj_sum<TT>(cnt, sh->redi);
                 count = false;
@@ -771,7 +792,7 @@ __global__ __launch_bounds__(TT == 64 ? 64 * REG_WAVES : TT) void k_batch_reg(Pa
                 if (status == RUNNING && t >= P.max_time) status = MAXTIME;
                 if (status != RUNNING || done_in_chunk >= P.chunk_steps) break;
             } else {
-                reg_clauses<TT, CPT, VPT, 1, KK, WIDE, false>(R, code, m, knorm, knorm2, fac, con, (float)h_at1, h_at1,
+                reg_clauses<TT, CPT, VPT, 1, KK, WIDE, false>(R, code, m, kn2, fac, con, (float)h_at1, h_at1,
                                                               hnext, P.floor, err_local, pos, cnt);
                 traj_sync<TT>();
             }
@@ -783,7 +804,7 @@ __global__ __launch_bounds__(TT == 64 ? 64 * REG_WAVES : TT) void k_batch_reg(Pa
                 const float hs = (float)h;
                 err_local = 0.0;
 #define ASAT_REG_STAGE(J)                                                                                             \
-    reg_clauses<TT, CPT, VPT, J, KK, WIDE, false>(R, code, m, knorm, knorm2, fac, con, hs, h, hnext, P.floor, err_local, \
+    reg_clauses<TT, CPT, VPT, J, KK, WIDE, false>(R, code, m, kn2, fac, con, hs, h, hnext, P.floor, err_local, \
                                                   pos, cnt);                                                          \
     traj_sync<TT>();                                                                                                  \
     reg_vars<TT, CPT, VPT, J, KK>(R, gb, gd, fac, con, hs, h, hnext, P.floor, err_local);
@@ -798,13 +819,14 @@ __global__ __launch_bounds__(TT == 64 ? 64 * REG_WAVES : TT) void k_batch_reg(Pa
                 ASAT_REG_STAGE(6)
 #undef ASAT_REG_STAGE
                 // ---------------- error norm + control (FP64), uniform in every thread
-                const double errmax = traj_max<TT>(err_local, sh->red) / P.eps;
+                const Control ctl = traj_control<TT>(err_local, P.eps, sh->red, &sh->control);
+                const double errmax = ctl.errmax;
                 errmax_last = errmax;
                 attempts += 1;
                 rhscount += had_stage1 ? 6 : 5;
                 had_stage1 = false;
                 if (errmax <= 1.0) {
-                    double hn = errmax > TabD::ERRCON ? TabD::SAFETY * h * pow_ctrl(errmax, 5) : 5.0 * h;
+                    double hn = errmax > TabD::ERRCON ? TabD::SAFETY * h * ctl.power : 5.0 * h;
                     hdid = h;
                     t += h;
                     steps += 1;
@@ -813,7 +835,7 @@ __global__ __launch_bounds__(TT == 64 ? 64 * REG_WAVES : TT) void k_batch_reg(Pa
                     accepted = true;
                     break;
                 }
-                double htemp = TabD::SAFETY * h * pow_ctrl(errmax, 4);
+                double htemp = TabD::SAFETY * h * ctl.power;
                 double hn = h >= 0.0 ? fmax(htemp, TabD::HFACTOR * h) : fmin(htemp, TabD::HFACTOR * h);
                 h = hn;
                 if (t + hn == t) {
@@ -1019,6 +1041,7 @@ __global__ __launch_bounds__(BS) void k_batch_chunk(Params P)
     extern __shared__ __attribute__((aligned(16))) float clds[];
     __shared__ double red[BS / 64];
     __shared__ int redi[BS / 64];
+    __shared__ Control s_control;
     __shared__ int s_traj;
     float* fac = clds;
     float* sums = clds + 2 * P.fac_ranks;
@@ -1140,13 +1163,14 @@ __global__ __launch_bounds__(BS) void k_batch_chunk(Params P)
                 stage(integral_constant<int, 4>{}, NoCount{}, hs, err_local, cnt);
                 stage(integral_constant<int, 5>{}, NoCount{}, hs, err_local, cnt);
                 stage(integral_constant<int, 6>{}, NoCount{}, hs, err_local, cnt);
-                const double errmax = traj_max<BS>(err_local, red) / P.eps;
+                const Control ctl = traj_control<BS>(err_local, P.eps, red, &s_control);
+                const double errmax = ctl.errmax;
                 errmax_last = errmax;
                 attempts += 1;
                 rhscount += had_stage1 ? 6 : 5;
                 had_stage1 = false;
                 if (errmax <= 1.0) {
-                    double hn = errmax > TabD::ERRCON ? TabD::SAFETY * h * pow_ctrl(errmax, 5) : 5.0 * h;
+                    double hn = errmax > TabD::ERRCON ? TabD::SAFETY * h * ctl.power : 5.0 * h;
                     hdid = h;
                     t += h;
                     steps += 1;
@@ -1155,7 +1179,7 @@ __global__ __launch_bounds__(BS) void k_batch_chunk(Params P)
                     accepted = true;
                     break;
                 }
-                double htemp = TabD::SAFETY * h * pow_ctrl(errmax, 4);
+                double htemp = TabD::SAFETY * h * ctl.power;
                 double hn = h >= 0.0 ? fmax(htemp, TabD::HFACTOR * h) : fmin(htemp, TabD::HFACTOR * h);
                 h = hn;
                 if (t + hn == t) {
@@ -1533,7 +1557,7 @@ static const RegVariant REG_VARIANTS[] = {
 static size_t reg_lds(const RegVariant& r, const Bucket& b)
 {
     const size_t waves = (size_t)r.tt / 64;      // RegShared, rounded up
-    const size_t shared = ((size_t)8 * waves * r.vpt + 12 * waves + 4 + 15) / 16 * 16;
+    const size_t shared = ((size_t)8 * waves * r.vpt + 12 * waves + 20 + 15) / 16 * 16;
     return 8 * (size_t)r.tt * r.vpt + shared + sizeof(float) * (size_t)round_up_ll(b.ncontrib + 1, 4);
 }
 constexpr size_t LDS_STATIC = 1024;      // the kernels' static shared arrays
