@@ -637,8 +637,9 @@ class HipRungeKutta:
         _check(lib().asat_rk_reset(self._h))
 
     def SetOneWorkgroup(self, enable):
-        """Allow (True, the default) or forbid the one-workgroup persistent
-        path for problems that fit in one workgroup's LDS."""
+        """Allow (True, the default) or forbid the persistent paths: one
+        workgroup for problems that fit in its LDS, 8 to 128 for larger ones
+        (False: the multi-kernel path)."""
         _check(lib().asat_rk_set_one_workgroup(self._h, 1 if enable else 0))
 
     def UsesOneWorkgroup(self):

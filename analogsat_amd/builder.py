@@ -19,7 +19,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libanalogsat_hip.so")
 OBJDIR = os.path.join(HERE, "_build")
 
-SOURCES = ["asat_plain.hip", "asat_batch.hip", "asat_adjoint.hip", "asat_noalloc.hip", "asat_problem.cpp"]
+SOURCES = ["asat_plain.hip", "asat_batch.hip", "asat_adjoint.hip", "asat_grid.hip", "asat_noalloc.hip", "asat_problem.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("ASAT_OFFLOAD_ARCH", "gfx950")
@@ -36,11 +36,12 @@ FLAGS = [
     "-I" + CSRC,
 ]
 
-# The batched kernels keep a trajectory's whole state in registers.  Hoisted out
-# of their step loops, the constants of the step control and what follows from
-# each literal code took up to twice the state's registers and spilled it
-# (256 threads, one clause and one variable each: 161 registers, 80 without).
-FILE_FLAGS = {"asat_batch.hip": ["-mllvm", "-disable-machine-licm"]}
+# Kernels that keep a trajectory's state in registers for a whole run: hoisted
+# out of the step loops, the constants of the step control and what follows from
+# each literal code took up to twice the state's registers and spilled it (batch,
+# 256 threads, one clause and one variable each: 161 registers, 80 without).
+NO_HOIST = ["-mllvm", "-disable-machine-licm"]
+FILE_FLAGS = {"asat_batch.hip": NO_HOIST, "asat_grid.hip": NO_HOIST}
 
 
 def _run(cmd, verbose):

@@ -52,6 +52,7 @@
 // Step(count) fills the slot spins of x, enqueues attempts without host
 // round trips and reads the control block back once per round of attempts.
 #include "asat_common.h"
+#include "asat_grid.h"
 #include "asat_small.h"
 
 #include <algorithm>
@@ -1707,6 +1708,12 @@ struct Sys {
     int nlist = 0;
     int runlen = 0;                // uniform run length of the lists (0: ragged)
     long long small_lds = 0;
+    // few-workgroup persistent path (asat_grid.h); grid_wgs = 0 when the problem
+    // does not use it
+    uint32_t* d_gcode = nullptr;
+    int *d_gcpos = nullptr, *d_gwg = nullptr, *d_ggroup = nullptr, *d_gvmap = nullptr;
+    int grid_wgs = 0, grid_cpt = 0, grid_groups = 0;
+    long long grid_lds = 0;
     int vg = 0, ngroups = 0, vg_blocks = 0;
     int family = ASAT_FAMILY_CTDS;
     double q = 1.1;              // tanh family parameter (CpuSatTanh.cpp:39)
@@ -1737,6 +1744,8 @@ struct Sys {
         dfree(d_pvar); dfree(d_pc0); dfree(d_pcontrib); dfree(d_pw16); dfree(d_pv0);
         split = false;
         dfree(d_vptr); dfree(d_spos_small); dfree(d_public);
+        dfree(d_gcode); dfree(d_gcpos); dfree(d_gwg); dfree(d_ggroup); dfree(d_gvmap);
+        grid_wgs = 0;
         perm.clear();
         nlist = 0;
         runlen = 0;
@@ -1827,6 +1836,138 @@ static void build_small_lists(Sys* s, const HostProblem& P)
     s->nlist = (int)nl;
     s->runlen = runlen;
     s->small_lds = bytes;
+}
+
+// Layout of the few-workgroup path (asat_grid.h).  Variables are ranked by
+// falling number of occurrences and dealt out in groups of 64, so workgroups
+// get the same work and a group's rows of terms are nearly full.  The workgroup
+// count is the smallest of 8, 16, .. whose largest clause list is two per
+// thread; from 64 on, as many per thread as the registers hold come before more
+// workgroups.  us per attempt with 8 / 16 / 32 / 64 / 128 workgroups:
+//   N =  2000, M =  8500, FP32   22.5 / 20.6 / 22.6 / 28.1 / 33.4
+//   N =  5000, M = 21250, FP32   36.5 / 31.8 / 30.9 / 32.9 / 39.1
+//   N = 12000, M = 51120, FP64      - /    - /    - / 59.9 / 69.5
+// The path ends where the spins of all variables no longer fit in LDS or the
+// clauses in registers; up to there it is faster than 13 kernels per attempt
+// (N = 24000, M = 102000, FP32: 67 against 79 us).
+constexpr int GRID_CPT_F64 = 4, GRID_CPT_F32 = 8;
+constexpr long long GRID_LDS = 158 * 1024;     // beside the kernel's 0.3 KB of static LDS
+static void build_grid(Sys* s, const HostProblem& P)
+{
+    const int n = P.n, m = P.m, K = P.k;
+    const int ng = ceil_div(n, 64), nranks = 64 * ng;
+    if (nranks + 2 > 32766 || (long long)s->esize * nranks > GRID_LDS) return;
+    const int cpt_max = s->esize == 8 ? GRID_CPT_F64 : GRID_CPT_F32;
+    if (m > (long long)GRID_MAX * GRID_BT * cpt_max) return;
+    std::vector<int> deg((size_t)n + 1, 0);
+    for (long long q = 0; q < (long long)m * K; q++) {
+        const int l = P.lit[(size_t)q];
+        if (l) deg[(size_t)std::abs(l)]++;
+    }
+    int top = 0;
+    for (int v = 1; v <= n; v++) top = std::max(top, deg[(size_t)v]);
+    std::vector<int> vmap((size_t)nranks, 0), rank((size_t)n + 1, 0), at((size_t)top + 2, 0);
+    for (int v = 1; v <= n; v++) at[(size_t)(top - deg[(size_t)v]) + 1]++;
+    for (int d = 0; d <= top; d++) at[(size_t)d + 1] += at[(size_t)d];
+    for (int v = 1; v <= n; v++) {
+        const int r = at[(size_t)(top - deg[(size_t)v])]++;
+        rank[(size_t)v] = r;
+        vmap[(size_t)r] = v;
+    }
+    // the workgroups of a clause, the first literal's first (it writes the clause)
+    auto owners = [&](int j, int g, int (&w)[4]) {
+        int ns = 0;
+        for (int q = 0; q < K; q++) {
+            const int l = P.lit[(size_t)j * K + q];
+            if (!l) continue;
+            const int x = (rank[(size_t)std::abs(l)] / 64) % g;
+            bool dup = false;
+            for (int i = 0; i < ns; i++) dup = dup || w[i] == x;
+            if (!dup) w[ns++] = x;
+        }
+        return ns;
+    };
+    std::vector<int> nwrite((size_t)GRID_MAX), nother((size_t)GRID_MAX);
+    int G = 0, most = 0, w4[4];
+    for (int g = 8; g <= GRID_MAX; g *= 2) {
+        if (ceil_div(ng, g) > GRID_WAVES) continue;
+        // a random instance's clauses are spread over nearly K workgroups each:
+        // skip counts that cannot hold them
+        if (g < GRID_MAX && (long long)m * (K - 1) > (long long)g * GRID_BT * cpt_max) continue;
+        std::fill(nwrite.begin(), nwrite.end(), 0);
+        std::fill(nother.begin(), nother.end(), 0);
+        for (int j = 0; j < m; j++) {
+            const int ns = owners(j, g, w4);
+            for (int i = 0; i < ns; i++) (i ? nother : nwrite)[(size_t)w4[i]]++;
+        }
+        most = 0;
+        for (int w = 0; w < g; w++) most = std::max(most, nwrite[(size_t)w] + nother[(size_t)w]);
+        G = g;
+        if (most <= 2 * GRID_BT || (g >= 64 && most <= cpt_max * GRID_BT)) break;
+    }
+    const int cpt = ceil_div(most, GRID_BT);
+    if (G == 0 || cpt > cpt_max) return;
+    // rows of terms: base of each group inside its workgroup
+    std::vector<int> group((size_t)2 * ng), ncon((size_t)G, 0);
+    for (int g = 0; g < ng; g++) {
+        const int depth = deg[(size_t)vmap[(size_t)64 * g]];
+        group[(size_t)2 * g] = ncon[(size_t)(g % G)];
+        group[(size_t)2 * g + 1] = depth;
+        ncon[(size_t)(g % G)] += 64 * depth;
+    }
+    const int most_con = *std::max_element(ncon.begin(), ncon.end());
+    const long long lds = (long long)s->esize * (nranks + 2 + most_con + 1);
+    if (most_con > 65535 || lds > GRID_LDS) return;
+    // entry of every slot: the variable's clauses in input order, literals in
+    // clause order (the reference's accumulation order)
+    std::vector<int> visit((size_t)m), fill((size_t)n + 1, 0), entry((size_t)m * K, 0);
+    for (int p = 0; p < m; p++) visit[(size_t)(P.perm.empty() ? p : P.perm[(size_t)p])] = p;
+    for (int c = 0; c < m; c++)
+        for (int q = 0; q < K; q++) {
+            const size_t sl = (size_t)visit[(size_t)c] * K + q;
+            if (P.lit[sl]) entry[sl] = fill[(size_t)std::abs(P.lit[sl])]++;
+        }
+    std::vector<int> wg((size_t)4 * G), fw((size_t)G), fo((size_t)G);
+    int total = 0;
+    for (int w = 0; w < G; w++) {
+        const int nw = nwrite[(size_t)w], nc = nw + nother[(size_t)w];
+        wg[(size_t)4 * w] = total;
+        wg[(size_t)4 * w + 1] = nc;
+        wg[(size_t)4 * w + 2] = nw;
+        wg[(size_t)4 * w + 3] = ncon[(size_t)w];
+        fw[(size_t)w] = total;
+        fo[(size_t)w] = total + nw;
+        total += nc;
+    }
+    std::vector<uint32_t> code((size_t)total * K);
+    std::vector<int> cpos((size_t)total);
+    for (int j = 0; j < m; j++) {
+        const int ns = owners(j, G, w4);
+        for (int i = 0; i < ns; i++) {
+            const int w = w4[i], to = (i ? fo : fw)[(size_t)w]++;
+            cpos[(size_t)to] = j;
+            for (int q = 0; q < K; q++) {
+                const size_t sl = (size_t)j * K + q;
+                const int l = P.lit[sl];
+                uint32_t where = (uint32_t)ncon[(size_t)w], rk = (uint32_t)nranks;
+                if (l) {
+                    rk = (uint32_t)rank[(size_t)std::abs(l)];
+                    const int g = (int)rk / 64;
+                    if (g % G == w) where = (uint32_t)(group[(size_t)2 * g] + 64 * entry[sl] + (int)(rk % 64));
+                }
+                code[(size_t)to * K + q] = (where << 16) | (rk << 1) | (l < 0 ? 1u : 0u);
+            }
+        }
+    }
+    upload(s->d_gcode, code);
+    upload(s->d_gcpos, cpos);
+    upload(s->d_gwg, wg);
+    upload(s->d_ggroup, group);
+    upload(s->d_gvmap, vmap);
+    s->grid_wgs = G;
+    s->grid_cpt = cpt <= 1 ? 1 : cpt <= 2 ? 2 : cpt <= 4 ? 4 : 8;
+    s->grid_groups = ng;
+    s->grid_lds = lds;
 }
 
 static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclauses)
@@ -1931,6 +2072,7 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
     else upload(s->d_csr_pos, P.csr_pos);
     upload(s->d_gstart, P.gstart);
     build_small_lists(s, P);
+    if (tiled && s->small_lds == 0) build_grid(s, P);
     if (!P.perm.empty()) upload(s->d_perm, P.perm);
     s->perm = std::move(P.perm);
     const size_t ncontrib = (size_t)P.gstart[P.ngroups] + REGION_ALIGN;
@@ -2201,6 +2343,9 @@ struct RK {
     int small_mode = 1;              // 1: one-workgroup path where the problem fits, 0: never
     SmallSolve* d_solve = nullptr;   // device SatSolver loop state (one-workgroup path)
     SmallSolve* h_solve = nullptr;   // pinned mirror
+    void* d_grid = nullptr;          // exchange buffers of the few-workgroup path
+    size_t grid_bytes = 0;
+    int* h_giveup = nullptr;         // pinned: its give-up flag
     void* pair[2] = {nullptr, nullptr};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = -1.f;
@@ -2225,7 +2370,9 @@ struct RK {
     {
         drop_graph();
         for (auto& p : k) dfree(p);
-        dfree(tmp); dfree(partial); dfree(d_ctrl); dfree(d_solve);
+        dfree(tmp); dfree(partial); dfree(d_ctrl); dfree(d_solve); dfree(d_grid);
+        grid_bytes = 0;
+        if (h_giveup) { (void)hipHostFree(h_giveup); h_giveup = nullptr; }
         if (h_ctrl) { (void)hipHostFree(h_ctrl); h_ctrl = nullptr; }
         if (h_solve) { (void)hipHostFree(h_solve); h_solve = nullptr; }
     }
@@ -2264,6 +2411,7 @@ static void rk_reset(RK* r)
 }
 
 static bool small_path(const RK* r);
+static bool grid_path(const RK* r);
 
 static void rk_configure(RK* r, Sys* s)
 {
@@ -2277,9 +2425,9 @@ static void rk_configure(RK* r, Sys* s)
         r->drop_graph();
         r->sys = s;
         r->gen = s->gen;
-        // the one-workgroup path keeps everything in LDS and reads none of
-        // these buffers (small instances: a caller solving start after start)
-        if (!small_path(r)) {
+        // the persistent paths keep everything on the CUs and read none of
+        // these buffers (a caller solving start after start)
+        if (!small_path(r) && !grid_path(r)) {
             const size_t bytes = (size_t)s->esize * s->alloc;
             for (auto& p : r->k) HIP_CHECK(hipMemsetAsync(p, 0, bytes, s->stream));
             HIP_CHECK(hipMemsetAsync(r->tmp, 0, (size_t)s->esize * (s->n + 1), s->stream));
@@ -2509,8 +2657,59 @@ static SmallArgs small_args(const RK* r, void* x)
     return a;
 }
 
-// Launches the persistent kernel until it reports done: each launch runs at
-// most SMALL_ATTEMPT_CAP attempts and leaves its state in the control block
+// ---------------------------------------------------------------------------
+// few-workgroup path (asat_grid.h), for the problems SetProblem laid it out for;
+// the same conditions as the one-workgroup path, CTDS family only
+// ---------------------------------------------------------------------------
+static bool grid_path(const RK* r)
+{
+    const Sys* s = r->sys;
+    return r->small_mode && s->grid_wgs > 0 && s->family == ASAT_FAMILY_CTDS && !(s->b > 0.0) && r->timer_kind < 0;
+}
+
+// the kernel's arguments; a holds what small_args gives plus the loop's limits
+static GridArgs grid_args(RK* r, const SmallArgs& a)
+{
+    const Sys* s = r->sys;
+    const size_t pub = (size_t)s->esize * 2 * 64 * s->grid_groups;
+    const size_t need = 64 + 2 * GRID_MAX * (sizeof(double) + sizeof(int)) + pub;
+    if (r->grid_bytes < need) {
+        dfree(r->d_grid);
+        r->grid_bytes = 0;
+        HIP_CHECK(hipMalloc(&r->d_grid, need));
+        r->grid_bytes = need;
+    }
+    if (!r->h_giveup) HIP_CHECK(hipHostMalloc((void**)&r->h_giveup, sizeof(int), hipHostMallocDefault));
+    GridArgs g;
+    memset(&g, 0, sizeof(g));
+    g.code = s->d_gcode; g.cpos = s->d_gcpos; g.wg = s->d_gwg; g.group = s->d_ggroup; g.vmap = s->d_gvmap;
+    g.x = a.x; g.ctrl = a.ctrl; g.solve = a.solve;
+    char* p = (char*)r->d_grid;
+    g.barrier = (unsigned*)p;
+    g.err = (double*)(p + 64);
+    g.count = (int*)(p + 64 + 2 * GRID_MAX * sizeof(double));
+    g.pub = p + 64 + 2 * GRID_MAX * (sizeof(double) + sizeof(int));
+    g.target = a.target; g.max_steps = a.max_steps; g.max_time = a.max_time;
+    g.time_float = a.time_float; g.batch = a.batch;
+    g.ngroups = s->grid_groups; g.aoff = s->aoff; g.k = s->k;
+    g.knorm = a.knorm;
+    return g;
+}
+
+static void grid_launch(RK* r, GridArgs& g)
+{
+    Sys* s = r->sys;
+    const void* f = grid_kernel(s->prec, s->k, s->grid_cpt);
+    require(f != nullptr, ASAT_ERR_HIP, "no few-workgroup kernel for this layout");
+    HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)s->grid_lds));
+    HIP_CHECK(hipMemsetAsync(g.barrier, 0, 2 * sizeof(unsigned), s->stream));
+    void* args[] = {&g};
+    HIP_CHECK(hipLaunchCooperativeKernel(f, dim3(s->grid_wgs), dim3(GRID_BT), args, (unsigned)s->grid_lds, s->stream));
+    HIP_CHECK(hipMemcpyAsync(r->h_giveup, g.barrier + 1, sizeof(int), hipMemcpyDeviceToHost, s->stream));
+}
+
+// Launches the persistent kernel of either path until it reports done: each
+// launch runs at most SMALL_ATTEMPT_CAP (GRID_ATTEMPT_CAP) attempts and leaves its state in the control block
 // (and the solver block), so the next launch resumes where it stopped.
 template <typename T>
 static void small_run(RK* r, const SmallArgs& a)
@@ -2519,11 +2718,16 @@ static void small_run(RK* r, const SmallArgs& a)
     hipStream_t st = s->stream;
     HIP_CHECK(hipEventRecord(r->ev0, st));
     long long last = r->h_ctrl->attempts;
+    const bool grid = grid_path(r);
+    GridArgs g;
+    if (grid) g = grid_args(r, a);
     for (;;) {
-        small_launch<T>(s, a, st);
+        if (grid) grid_launch(r, g);
+        else small_launch<T>(s, a, st);
         HIP_CHECK(hipMemcpyAsync(r->h_ctrl, r->d_ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, st));
         if (a.solve) HIP_CHECK(hipMemcpyAsync(r->h_solve, r->d_solve, sizeof(SmallSolve), hipMemcpyDeviceToHost, st));
         HIP_CHECK(hipStreamSynchronize(st));
+        require(!grid || *r->h_giveup == 0, ASAT_ERR_HIP, "the workgroups of the integrator did not all run");
         if (r->h_ctrl->underflow) break;
         if (a.solve ? r->h_solve->result >= 0 : r->h_ctrl->steps >= a.target) break;
         require(r->h_ctrl->attempts > last, ASAT_ERR_HIP, "integrator made no progress");
@@ -2549,7 +2753,7 @@ static int rk_step(RK* r, State* olds, State* news, int count)
     require(count >= 0, ASAT_ERR_INVALID_ARGUMENT, "negative step count");
     if (r->h_ctrl->underflow) return ASAT_UNDERFLOW;
     if (count == 0) return ASAT_OK;
-    if (small_path(r)) {
+    if (small_path(r) || grid_path(r)) {
         // the state stays in olds; news is not touched
         SmallArgs a = small_args(r, olds->d);
         a.target = r->h_ctrl->steps + count;
@@ -2578,7 +2782,7 @@ static void rk_solve(RK* r, State* olds, State* news, int batch, long long max_s
     require(max_steps >= 1, ASAT_ERR_INVALID_ARGUMENT, "Max iterations must be positive");
     require(max_time > 0.0, ASAT_ERR_INVALID_ARGUMENT, "Max time must be positive");
     memset(out, 0, sizeof(*out));
-    if (small_path(r) && !r->h_ctrl->underflow) {
+    if ((small_path(r) || grid_path(r)) && !r->h_ctrl->underflow) {
         SmallSolve init;
         memset(&init, 0, sizeof(init));
         init.result = -1;

@@ -204,9 +204,12 @@ int asat_rk_step(asat_rk_t* rk, asat_state_t* old_state, asat_state_t* new_state
    workgroup's LDS (about 150 KB: 7 state vectors, the spin stage input, the
    slot contributions, literals and term positions) and that use no bias term run
    Step and asat_rk_solve in one persistent single-workgroup kernel, with the
-   same arithmetic as the multi-kernel path (bit-identical results).
+   same arithmetic as the multi-kernel path (bit-identical results); larger
+   3- and 4-literal CTDS problems, up to about N = 20 000 in FP64 and 32 000 in
+   FP32, run in one of 8 to 128 workgroups.
    enable = 0 forces the multi-kernel path (13 launches per attempt);
-   asat_rk_uses_one_workgroup reports which path the configured problem takes. */
+   asat_rk_uses_one_workgroup reports whether the configured problem takes the
+   single-workgroup kernel. */
 int asat_rk_set_one_workgroup(asat_rk_t* rk, int enable);
 int asat_rk_uses_one_workgroup(const asat_rk_t* rk, int* uses);
 /* SatSolver::DoSolve's loop without a callback (AnalogSAT/solver/SatSolver.h:313-331):

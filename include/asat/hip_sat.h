@@ -250,8 +250,8 @@ public:
     void SetEpsilon(TFloat eps) { HipSafe(asat_rk_set_eps(h, (double)eps)); }
     // constant term of the error scale (reference: TINY = 1e-20, the default)
     void SetErrorFloor(double floor) { HipSafe(asat_rk_set_xscal_floor(h, floor)); }
-    // allow (default) or forbid the one-workgroup persistent path for
-    // problems whose integrator fits in one workgroup's LDS
+    // allow (default) or forbid the persistent paths: one workgroup for problems
+    // whose integrator fits in its LDS, 8 to 128 for larger ones
     void SetOneWorkgroup(bool enable) { HipSafe(asat_rk_set_one_workgroup(h, enable ? 1 : 0)); }
 
 private:
