@@ -29,6 +29,14 @@
 // Clauses of 3 or 4 literals, CTDS family, no bias term; the solver loop of
 // SatSolver runs on the device as in asat_small.h.
 //
+// One workgroup alone (SOLO, up to 1024 variables) keeps the same layout and
+// exchanges through LDS.  It is bound by the latency of its phases, and holding
+// the state in registers and reading a variable's terms as rows without bank
+// conflicts leaves fewer of them than asat_small.h, which has every vector in
+// LDS (us per attempt, FP64: N = 200, M = 852 7.0 against 10.7, N = 240 7.3
+// against 12.0).  With 256 threads, up to 512 clauses, it was no faster (N = 50:
+// 4.7-5.1 against 4.6), so those keep asat_small.h.
+//
 // The launch is cooperative, so all workgroups are resident; a wait that lasts
 // GRID_POLLS polls gives up and the host reports an error.
 // Bound by the latency of its six exchanges: N = 2000, M = 8500 takes 20.6 us an
@@ -69,8 +77,9 @@ struct GridArgs {
     double knorm;
 };
 
-// the kernel for a precision, clause length and clauses per thread (null: none)
-const void* grid_kernel(int precision, int k, int cpt);
+// the kernel for a precision, clause length and clauses per thread (null: none);
+// solo: the one-workgroup form
+const void* grid_kernel(int precision, int k, int cpt, bool solo);
 
 template <typename T>
 __device__ __forceinline__ T agent_load(const T* p)
@@ -182,7 +191,9 @@ __device__ __forceinline__ void grid_clauses(GridRegs<T, KT, CPT>& R, const T* s
     }
 }
 
-// left-to-right sum of this lane's entries in `depth` rows of 64
+// left-to-right sum of this lane's entries in `depth` rows of 64.  Eight loads in
+// flight: 32 at once spilled, 128 registers being what 1024 threads have
+// (N = 400 alone, FP64: 13.6 against 9.3 us an attempt).
 template <typename T>
 __device__ __forceinline__ T grid_sum(const T* e, int depth)
 {
@@ -204,7 +215,7 @@ __device__ __forceinline__ T grid_sum(const T* e, int depth)
     return sum;
 }
 
-template <typename T, int KT, int CPT>
+template <typename T, int KT, int CPT, bool SOLO>
 __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
 {
     // [spins by rank, then the padding rank] [terms, then one that nothing reads]
@@ -212,13 +223,13 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
     __shared__ GridShared sh;
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int w = (int)blockIdx.x, G = (int)gridDim.x;
+    const int w = SOLO ? 0 : (int)blockIdx.x, G = SOLO ? GRID_WAVES : (int)gridDim.x;
     const int nranks = 64 * a.ngroups;
     T* s = (T*)grid_lds;
     T* con = s + nranks + 2;
     const int c0 = a.wg[4 * w], nclause = a.wg[4 * w + 1], nwrite = a.wg[4 * w + 2], ncon = a.wg[4 * w + 3];
-    // wave v owns group w + v * G
-    const int grp = w + wave * G;
+    // wave v owns group w + v * G (alone: group v)
+    const int grp = SOLO ? wave : w + wave * G;
     const bool own = grp < a.ngroups;
     const int rank = grp * 64 + lane;
     const int var = own ? a.vmap[rank] : 0;
@@ -256,12 +267,45 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
     __syncthreads();
 
     unsigned phase = 0;
+    double ctl_errmax = 0.0, ctl_power = 0.0;     // what an exchange brought
+    int ctl_count = 0;
     // Publish this thread's spin (waves that own a group), wait for every
     // workgroup, then take everyone's spins into LDS.  ERR: with the
     // workgroups' error maxima, from which wave 0 forms errmax and its power;
     // CNT: with their violation counts.  False when the wait was given up.
     auto exchange = [&](T val, auto errc, double e, auto cntc, int cnt) -> bool {
         constexpr bool ERR = decltype(errc)::value, CNT = decltype(cntc)::value;
+        if constexpr (SOLO) {
+            if (own) s[rank] = val;
+            if constexpr (ERR) {
+                e = wave_max_dpp(e);
+                if (lane == 0) sh.red[wave] = e;
+            }
+            if constexpr (CNT) {
+                cnt = wave_sum(cnt);
+                if (lane == 0) sh.redi[wave] = cnt;
+            }
+            __syncthreads();
+            if constexpr (ERR) {
+                double m = sh.red[0];
+#pragma unroll
+                for (int i = 1; i < GRID_WAVES; i++) m = fmax(m, sh.red[i]);
+                if (wave == 0) {
+                    m /= eps;
+                    const double pw = m > TabD::ERRCON ? pow_ctrl(m, m <= 1.0 ? 5 : 4) : 0.0;
+                    if (lane == 0) { sh.errmax = m; sh.power = pw; }
+                }
+                __syncthreads();
+                ctl_errmax = sh.errmax;
+                ctl_power = sh.power;
+            }
+            if constexpr (CNT) {
+                ctl_count = sh.redi[0];
+#pragma unroll
+                for (int i = 1; i < GRID_WAVES; i++) ctl_count += sh.redi[i];
+            }
+            return true;
+        }
         const int half = (int)(phase & 1u);
         T* pub = (T*)a.pub + (long long)half * nranks;
         if (own) agent_store(pub + rank, val);
@@ -323,6 +367,8 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
             }
         }
         __syncthreads();
+        if constexpr (ERR) { ctl_errmax = sh.errmax; ctl_power = sh.power; }
+        if constexpr (CNT) ctl_count = sh.count;
         return true;
     };
     using Yes = std::integral_constant<bool, true>;
@@ -349,7 +395,7 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
         }
         if (check) {
             ss.check = 0;
-            ss.last_viol = sh.count;
+            ss.last_viol = ctl_count;
             if (ss.last_viol == 0) {
                 ss.result = SMALL_SAT;
                 break;
@@ -395,12 +441,12 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
             }
             if (!(alive = exchange(xn, Yes{}, err, No{}, 0))) break;
             launched++;
-            errmax = sh.errmax;
+            errmax = ctl_errmax;
             attempts += 1;
             rhscount += first ? 6 : 5;
             first = false;
             if (errmax <= 1.0) {
-                const double hn = errmax > TabD::ERRCON ? TabD::SAFETY * h * sh.power : 5.0 * h;
+                const double hn = errmax > TabD::ERRCON ? TabD::SAFETY * h * ctl_power : 5.0 * h;
                 hdid = h;
                 time += h;
                 if (hlog && steps < hlog_len && w == 0 && tid == 0) hlog[steps] = h;
@@ -413,7 +459,7 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
                 accepted = true;
                 break;
             }
-            const double htemp = TabD::SAFETY * h * sh.power;
+            const double htemp = TabD::SAFETY * h * ctl_power;
             const double hn = h >= 0.0 ? fmax(htemp, TabD::HFACTOR * h) : fmin(htemp, TabD::HFACTOR * h);
             h = hn;
             if (time + hn == time) {

@@ -4,22 +4,30 @@
 
 namespace asat {
 
-template <typename T, int KT>
+template <typename T, int KT, bool SOLO>
 static const void* grid_kernel_of(int cpt)
 {
-    if (cpt == 1) return (const void*)k_grid<T, KT, 1>;
-    if (cpt == 2) return (const void*)k_grid<T, KT, 2>;
-    if (cpt == 4) return (const void*)k_grid<T, KT, 4>;
-    if constexpr (sizeof(T) == 4) {
-        if (cpt == 8) return (const void*)k_grid<T, KT, 8>;
+    if (cpt == 1) return (const void*)k_grid<T, KT, 1, SOLO>;
+    if (cpt == 2) return (const void*)k_grid<T, KT, 2, SOLO>;
+    if constexpr (!SOLO || sizeof(T) == 4) {
+        if (cpt == 4) return (const void*)k_grid<T, KT, 4, SOLO>;
+    }
+    if constexpr (!SOLO && sizeof(T) == 4) {
+        if (cpt == 8) return (const void*)k_grid<T, KT, 8, SOLO>;
     }
     return nullptr;
 }
 
-const void* grid_kernel(int precision, int k, int cpt)
+template <typename T, bool SOLO>
+static const void* grid_kernel_k(int k, int cpt)
 {
-    if (precision == ASAT_F64) return k == 3 ? grid_kernel_of<double, 3>(cpt) : grid_kernel_of<double, 4>(cpt);
-    return k == 3 ? grid_kernel_of<float, 3>(cpt) : grid_kernel_of<float, 4>(cpt);
+    return k == 3 ? grid_kernel_of<T, 3, SOLO>(cpt) : grid_kernel_of<T, 4, SOLO>(cpt);
+}
+
+const void* grid_kernel(int precision, int k, int cpt, bool solo)
+{
+    if (precision == ASAT_F64) return solo ? grid_kernel_k<double, true>(k, cpt) : grid_kernel_k<double, false>(k, cpt);
+    return solo ? grid_kernel_k<float, true>(k, cpt) : grid_kernel_k<float, false>(k, cpt);
 }
 
 }  // namespace asat

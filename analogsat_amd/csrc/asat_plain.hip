@@ -1889,11 +1889,15 @@ static void build_grid(Sys* s, const HostProblem& P)
     };
     std::vector<int> nwrite((size_t)GRID_MAX), nother((size_t)GRID_MAX);
     int G = 0, most = 0, w4[4];
-    for (int g = 8; g <= GRID_MAX; g *= 2) {
+    // one workgroup alone while its threads hold the clauses (us per attempt
+    // against 8 workgroups: N = 480, FP64 10.5 / 16.4, N = 960, FP32 13.2 / 16.6,
+    // 4-SAT N = 200, FP64 14.1 / 21.1)
+    const int solo_max = (s->esize == 8 ? 2 : 4) * GRID_BT;
+    for (int g = n <= 64 * GRID_WAVES && m <= solo_max ? 1 : 8; g <= GRID_MAX; g = g == 1 ? 8 : 2 * g) {
         if (ceil_div(ng, g) > GRID_WAVES) continue;
         // a random instance's clauses are spread over nearly K workgroups each:
         // skip counts that cannot hold them
-        if (g < GRID_MAX && (long long)m * (K - 1) > (long long)g * GRID_BT * cpt_max) continue;
+        if (g > 1 && g < GRID_MAX && (long long)m * (K - 1) > (long long)g * GRID_BT * cpt_max) continue;
         std::fill(nwrite.begin(), nwrite.end(), 0);
         std::fill(nother.begin(), nother.end(), 0);
         for (int j = 0; j < m; j++) {
@@ -1903,7 +1907,7 @@ static void build_grid(Sys* s, const HostProblem& P)
         most = 0;
         for (int w = 0; w < g; w++) most = std::max(most, nwrite[(size_t)w] + nother[(size_t)w]);
         G = g;
-        if (most <= 2 * GRID_BT || (g >= 64 && most <= cpt_max * GRID_BT)) break;
+        if (g == 1 || most <= 2 * GRID_BT || (g >= 64 && most <= cpt_max * GRID_BT)) break;
     }
     const int cpt = ceil_div(most, GRID_BT);
     if (G == 0 || cpt > cpt_max) return;
@@ -2072,7 +2076,8 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
     else upload(s->d_csr_pos, P.csr_pos);
     upload(s->d_gstart, P.gstart);
     build_small_lists(s, P);
-    if (tiled && s->small_lds == 0) build_grid(s, P);
+    // up to 512 clauses and variables asat_small.h is the faster one
+    if (tiled && (s->small_lds == 0 || std::max(P.m, P.n) > 512)) build_grid(s, P);
     if (!P.perm.empty()) upload(s->d_perm, P.perm);
     s->perm = std::move(P.perm);
     const size_t ncontrib = (size_t)P.gstart[P.ngroups] + REGION_ALIGN;
@@ -2699,11 +2704,16 @@ static GridArgs grid_args(RK* r, const SmallArgs& a)
 static void grid_launch(RK* r, GridArgs& g)
 {
     Sys* s = r->sys;
-    const void* f = grid_kernel(s->prec, s->k, s->grid_cpt);
+    const bool solo = s->grid_wgs == 1;
+    const void* f = grid_kernel(s->prec, s->k, s->grid_cpt, solo);
     require(f != nullptr, ASAT_ERR_HIP, "no few-workgroup kernel for this layout");
     HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)s->grid_lds));
-    HIP_CHECK(hipMemsetAsync(g.barrier, 0, 2 * sizeof(unsigned), s->stream));
     void* args[] = {&g};
+    if (solo) {
+        HIP_CHECK(hipLaunchKernel(f, dim3(1), dim3(GRID_BT), args, (size_t)s->grid_lds, s->stream));
+        return;
+    }
+    HIP_CHECK(hipMemsetAsync(g.barrier, 0, 2 * sizeof(unsigned), s->stream));
     HIP_CHECK(hipLaunchCooperativeKernel(f, dim3(s->grid_wgs), dim3(GRID_BT), args, (unsigned)s->grid_lds, s->stream));
     HIP_CHECK(hipMemcpyAsync(r->h_giveup, g.barrier + 1, sizeof(int), hipMemcpyDeviceToHost, s->stream));
 }
@@ -2727,7 +2737,7 @@ static void small_run(RK* r, const SmallArgs& a)
         HIP_CHECK(hipMemcpyAsync(r->h_ctrl, r->d_ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, st));
         if (a.solve) HIP_CHECK(hipMemcpyAsync(r->h_solve, r->d_solve, sizeof(SmallSolve), hipMemcpyDeviceToHost, st));
         HIP_CHECK(hipStreamSynchronize(st));
-        require(!grid || *r->h_giveup == 0, ASAT_ERR_HIP, "the workgroups of the integrator did not all run");
+        require(!grid || s->grid_wgs == 1 || *r->h_giveup == 0, ASAT_ERR_HIP, "the workgroups of the integrator did not all run");
         if (r->h_ctrl->underflow) break;
         if (a.solve ? r->h_solve->result >= 0 : r->h_ctrl->steps >= a.target) break;
         require(r->h_ctrl->attempts > last, ASAT_ERR_HIP, "integrator made no progress");

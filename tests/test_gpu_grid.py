@@ -108,3 +108,30 @@ def test_solve_ends_like_the_host_loop(m, batch, max_steps, max_time):
     assert np.array_equal(ends[0][5], ends[1][5])
     if m == 2000:
         assert ends[0][0] == A.SatResult.SAT_SOLUTION_FOUND
+
+
+@pytest.mark.parametrize("prec,n,m,k,short", [
+    ("f64", 120, 513, 3, 0.0), ("f64", 64, 600, 4, 0.3), ("f64", 65, 1024, 3, 0.2), ("f64", 500, 2048, 3, 0.0),
+    ("f32", 1024, 4096, 3, 0.1), ("f32", 513, 300, 3, 0.0), ("f32", 400, 3972, 4, 0.2)])
+def test_one_workgroup_with_state_in_registers(prec, n, m, k, short):
+    """One workgroup of 1024 threads: from 513 clauses or variables on, up to what
+    its threads hold."""
+    p = make(n, m, k, 12, short)
+    pub = start(p, prec)
+    out = []
+    for persistent in (True, False):
+        sat = A.HipSat(prec)
+        sat.SetProblem(A.SatProblem(p.literals, p.lengths))
+        rk = A.HipRungeKutta()
+        rk.SetEpsilon(1e-6)
+        rk.Configure(sat)
+        rk.SetOneWorkgroup(persistent)
+        old, new = sat.MakeState(), sat.MakeState()
+        old.CopyFrom(pub)
+        assert rk.Step(old, new, 23)
+        r = rk.SolveBatches(old, new, 3, 31, 1e300)
+        st = rk.stats()
+        out.append((r.result, r.steps, r.last_violations, st.time, st.hdid, st.hnext, st.attempts, st.rhscount,
+                    old.CopyTo()))
+    assert out[0][:-1] == out[1][:-1]
+    assert np.array_equal(out[0][-1], out[1][-1])
