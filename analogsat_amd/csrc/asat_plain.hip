@@ -523,6 +523,10 @@ struct StageArgs {
     const unsigned* runs;  // big tiles: per tile, run table in place of spos
     int run_stride;        // words per tile of the run tables
     const int* csr_ptr;
+    const int* litq;       // generic pass, K <= 10: literals and contribution positions by literal (mq apart)
+    const int* posq;
+    int mq;
+    double* th;            // its tanh table, 2 per variable from 0 (null: not used)
     const int* csr_pos;    // per-variable contribution positions (gather var pass)
     const uint16_t* csr_loc;   // the same relative to the region start (LDS var pass)
     const long long* gstart;   // region starts, ngroups+1
@@ -1036,6 +1040,138 @@ __global__ __launch_bounds__(BLK) void k_clause_gen(StageArgs<T> a)
     }
 }
 
+// ---- clause pass, K <= 10 other than the tiled 3 and 4 ---------------------
+// KT: the compile-time bound of K (2, 6, 8 or 10), so that a clause's factors
+// and their left-to-right products stay in registers: k_clause_gen keeps them
+// in LDS, 64 KB per workgroup in FP64, with 2 K^2 LDS reads per clause and two
+// waves per SIMD.  Literals and positions lie by literal, so every load is one
+// run per wave.  The product without factor q is the running product of the
+// factors before it times those after it: the same multiplications in the same
+// order, K (K - 1) / 2 of them.  One clause; results as k_clause_gen's.
+// TAB (tanh family, with the wide var pass: few variables in many clauses, as in
+// Ramsey encodings): a slot's tanh(q f) depends on its literal alone, so the var
+// pass leaves tanh of both factors of every variable in a.th, and the 2.85e6 tanh
+// of a stage of R(5,5) at N = 30 become 870.
+// Bound by the gathers of the spins and the scattered stores of the terms.
+// R(5,5) at N = 30 (tanh, FP64, K = 10, M = 285 012): 50 -> 16 us a pass, 21 with
+// the table rebuilt by every workgroup; N = 60 013, M = 231 000, clauses of 2 to 6
+// literals, FP32: 15 -> 12 us.
+template <typename T, int KT, int J, bool TAB>
+__device__ __forceinline__ void clause_k(const StageArgs<T>& a, int m, const T* sp, const T* x, T* xnew,
+                                          T hs, double h, double hnext, double floor, double& err,
+                                         double& asum)
+{
+    const int K = a.k;
+    int l[KT], at[KT];
+    T sv[KT], f[KT], pre[KT + 1];
+#pragma unroll
+    for (int q = 0; q < KT; q++) {
+        l[q] = q < K ? a.litq[(size_t)q * a.mq + m] : 0;
+        at[q] = q < K ? a.posq[(size_t)q * a.mq + m] : 0;
+    }
+    const size_t ai = (size_t)a.aoff + m;
+    T k1 = 0, k2 = 0, k3 = 0, k4 = 0, k5 = 0;
+    const T xa = x[ai];
+    if constexpr (J > 1) k1 = a.k1[ai];
+    if constexpr (J > 2) k2 = a.k2[ai];
+    if constexpr (J > 3) k3 = a.k3[ai];
+    if constexpr (J > 4) k4 = a.k4[ai];
+    if constexpr (J > 5) k5 = a.k5[ai];
+#pragma unroll
+    for (int q = 0; q < KT; q++) sv[q] = (q < K && l[q] != 0) ? sp[l[q] < 0 ? -l[q] : l[q]] : (T)-1.0;
+    T km = a.knorm;
+    pre[0] = (T)1.0;
+#pragma unroll
+    for (int q = 0; q < KT; q++) {
+        // past K: factor 1, which changes no product
+        f[q] = q < K ? (l[q] < 0 ? (T)1.0 + sv[q] : (T)1.0 - sv[q]) : (T)1.0;
+        km *= f[q];
+        pre[q + 1] = q == 0 ? f[0] : pre[q] * f[q];
+    }
+    T am;
+    if constexpr (J == 1) am = xa;
+    else am = stage_input<T, J>(xa, k1, k2, k3, k4, k5, hs);
+    const T kj = am * km * km;
+    asum = (double)am;
+    if constexpr (J == 1) a.k1[ai] = kj;
+    else if constexpr (J == 2) a.k2[ai] = kj;
+    else if constexpr (J == 3) a.k3[ai] = kj;
+    else if constexpr (J == 4) a.k4[ai] = kj;
+    else if constexpr (J == 5) a.k5[ai] = kj;
+    else {
+        T xn;
+        final_combination<T>(xa, k1, k3, k4, k5, kj, hs, h, hnext, floor, xn, err);
+        xnew[ai] = xn;
+    }
+    const T r = TAB ? a.knorm * am : km * a.knorm * am;
+#pragma unroll
+    for (int q = 0; q < KT; q++) {
+        if (q < K && l[q] != 0) {      // a clause's padding literals are its last ones
+            T p = q == 0 ? (T)1.0 : pre[q];
+#pragma unroll
+            for (int qq = q + 1; qq < KT; qq++) p = (q == 0 && qq == 1) ? f[1] : p * f[qq];
+            T rr;
+            if constexpr (TAB) {
+                const T ap = p < (T)0 ? -p : p;
+                const double t = a.th[2 * (l[q] < 0 ? -l[q] : l[q]) + (l[q] < 0 ? 1 : 0)];
+                if constexpr (sizeof(T) == 4) rr = (T)((double)(r * ap) * t);
+                else rr = r * ap * t;
+                rr = l[q] < 0 ? -rr : rr;
+            } else {
+                rr = r * p;
+                rr *= l[q] < 0 ? (T)-2.0 : (T)2.0;
+            }
+            a.contrib[at[q]] = rr;
+        }
+    }
+}
+
+template <typename T, int KT, int J, bool TAB>
+__global__ __launch_bounds__(BLK) void k_clause_k(StageArgs<T> a)
+{
+    __shared__ double sh[BLK / 64];
+    const Ctrl* c = a.ctrl;
+    int parity = 0;
+    double h = 0.0, hnext = 0.0, floor = TabD::TINY;
+    if (c) {
+        if (!c->active) return;
+        if (J == 1 && !c->step_start) return;
+        parity = c->parity; h = c->h; hnext = c->hnext; floor = c->floor;
+    }
+    const T* x = parity ? a.xb : a.xa;
+    T* xnew = parity ? a.xa : a.xb;
+    const int m = clause_of_thread(a.clause_per_xcd);
+    double err = 0.0, asum = 0.0;
+    if (m < a.m)
+        clause_k<T, KT, J, TAB>(a, m, (J == 1) ? x : a.tmp, x, xnew, (T)h, h, hnext, floor, err, asum);
+    if (a.bias) {
+        const double bs = block_sum_all<BLK>(asum, sh);
+        if (threadIdx.x == 0) a.apart[blockIdx.x] = bs;
+    }
+    if constexpr (J == 6) {
+        const double bm = block_max<BLK>(err, sh);
+        if (threadIdx.x == 0) a.partial[blockIdx.x] = bm;
+    }
+}
+
+// tanh(q f) of both factors f = 1 -+ s of a spin, as tanh_term forms it for
+// clauses of 3 to 10 literals: half 0 or 1 of the variable's entry
+template <typename T>
+__device__ __forceinline__ double tanh_half(T sv, T q, int half)
+{
+    const T f = half ? (T)1.0 + sv : (T)1.0 - sv;
+    return tanh((double)(q * f));
+}
+
+// the table of a state's spins, before the first stage; the wide var pass then
+// keeps it (entry 0, the padding literal's, is never read)
+template <typename T>
+__global__ __launch_bounds__(BLK) void k_tanh_fill(const T* x, int n, T q, double* th)
+{
+    const int i = (int)(blockIdx.x * BLK + threadIdx.x);
+    if (i < 2 * (n + 1)) th[i] = tanh_half<T>(x[i >> 1], q, i & 1);
+}
+
 // ---- var pass: deterministic per-variable sums + spin stage combination ---
 // The state values the stage combination of variable i reads (x and the
 // earlier stage derivatives it needs), loaded ahead of the sums.
@@ -1103,8 +1239,16 @@ __device__ __forceinline__ T var_stage(const StageArgs<T>& a, int i, bool fresh,
 template <typename T, int BLOCK>
 __device__ __forceinline__ T bias_prefactor(const StageArgs<T>& a, double* sh)
 {
+    // eight loads in flight; added in order
     double v = 0.0;
-    for (int i = threadIdx.x; i < a.nblk_clause; i += BLOCK) v += a.apart[i];
+    for (int i = threadIdx.x; i < a.nblk_clause; i += 8 * BLOCK) {
+        double t[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) t[u] = i + u * BLOCK < a.nblk_clause ? a.apart[i + u * BLOCK] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (i + u * BLOCK < a.nblk_clause) v += t[u];
+    }
     const double tot = block_sum_all<BLOCK>(v, sh);
     const T mean = (T)tot / (T)a.m;
     return mean * a.alpha * a.bb * (T)1.570796326794897;
@@ -1335,7 +1479,11 @@ __global__ __launch_bounds__(BLK) void k_var(StageArgs<T> a)
 // The variable's contributions pass through two LDS buffers of WIDE_STAGE
 // values: while thread 0 adds one buffer in slot order (so the sum is the
 // gather kernel's, and the reference's, exactly), waves 1..3 stage the next
-// chunk into the other.
+// chunk into the other.  The generic clause pass stores a variable's terms side
+// by side (wide_run); the tiled one leaves them where csr_pos says.  It is bound
+// by that chain of additions, so thread 0 reads the next values while it adds:
+// reading 16, waiting and adding them made it 51 us at R(5,5), N = 30, FP64 (6551
+// values a row), 43 now; the additions alone are 20, at 3.0 ns each.
 constexpr int WIDE_BLK = 256;
 constexpr int WIDE_STAGE = 2048;
 constexpr long long WIDE_MIN_ROW = 64;
@@ -1345,6 +1493,7 @@ __global__ __launch_bounds__(WIDE_BLK) void k_var_wide(StageArgs<T> a)
 {
     __shared__ double sh[WIDE_BLK / 64];
     __shared__ __attribute__((aligned(16))) T vals[2][WIDE_STAGE];
+    __shared__ T s_sine;
     const Ctrl* c = a.ctrl;
     int parity = 0;
     double h = 0.0, hnext = 0.0, floor = TabD::TINY;
@@ -1358,49 +1507,94 @@ __global__ __launch_bounds__(WIDE_BLK) void k_var_wide(StageArgs<T> a)
     const T* x = parity ? a.xb : a.xa;
     T* xnew = parity ? a.xa : a.xb;
     const int i = (int)blockIdx.x + 1;          // grid: one workgroup per variable 1..n
+    const int t = (int)threadIdx.x;
     double err = 0.0;
-    const T pref = (a.bias && fresh) ? bias_prefactor<T, WIDE_BLK>(a, sh) : (T)0;
-    T sum = (T)0;
+    // the stage combination's inputs, ahead of the sum
+    VarIn<T> in = var_load<T, J>(a, i, x, fresh);
+    T sum = (T)0, pref = (T)0;
     if (fresh) {
         const int e0 = a.csr_ptr[i], e1 = a.csr_ptr[i + 1];
-        const int t = (int)threadIdx.x;
-        {   // chunk 0, every thread
-            const int r1 = std::min(e1, e0 + WIDE_STAGE);
-            for (int e = e0 + t; e < r1; e += WIDE_BLK) vals[0][e - e0] = a.contrib[a.csr_pos[e]];
+        auto at = [&](int e) { return a.contrib[a.csr_pos ? a.csr_pos[e] : e]; };
+        // chunk 0 through registers, so that the bias term's sums overlap its loads
+        constexpr int U0 = WIDE_STAGE / WIDE_BLK;
+        T first[U0];
+#pragma unroll
+        for (int u = 0; u < U0; u++) {
+            const int e = e0 + t + u * WIDE_BLK;
+            first[u] = e < e1 ? at(e) : (T)-0.0;
         }
+        if (a.bias) {
+            if (t == 64) s_sine = bias_sine<T>(J == 1 ? x[i] : a.tmp[i]);
+            pref = bias_prefactor<T, WIDE_BLK>(a, sh);
+        }
+#pragma unroll
+        for (int u = 0; u < U0; u++) vals[0][t + u * WIDE_BLK] = first[u];
         __syncthreads();
         for (int r0 = e0, ch = 0; r0 < e1; r0 += WIDE_STAGE, ch++) {
             const int r1 = std::min(e1, r0 + WIDE_STAGE);
             if (t >= 64) {
-                // stage chunk ch + 1 into the buffer added in round ch - 1
+                // stage chunk ch + 1 into the buffer added in round ch - 1,
+                // every load of a thread in flight together
+                constexpr int NT = WIDE_BLK - 64, U = (WIDE_STAGE + NT - 1) / NT;
                 const int n1 = std::min(e1, r1 + WIDE_STAGE);
                 T* dst = vals[(ch + 1) & 1];
-                for (int e = r1 + (t - 64); e < n1; e += WIDE_BLK - 64) dst[e - r1] = a.contrib[a.csr_pos[e]];
+                T g[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int e = r1 + (t - 64) + u * NT;
+                    g[u] = e < n1 ? at(e) : (T)-0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int o = (t - 64) + u * NT;
+                    if (o < WIDE_STAGE) dst[o] = g[u];
+                }
             } else if (t == 0) {
-                // 16-byte LDS reads, eight ahead; the additions stay in slot order
-                constexpr int V = 16 / (int)sizeof(T);
+                // 16-byte LDS reads, one batch of eight ahead of the additions,
+                // which stay in slot order
+                constexpr int V = 16 / (int)sizeof(T), B = 8 * V;
                 typedef T vT __attribute__((ext_vector_type(V)));
                 const T* v = vals[ch & 1];
-                const int len = r1 - r0;
-                int e = 0;
-                for (; e + 8 * V <= len; e += 8 * V) {
-                    vT q[8];
+                // whole batches: past the row's end the buffer holds -0.0,
+                // which changes no sum
+                const int full = (r1 - r0 + 2 * B - 1) / (2 * B) * (2 * B);
+                auto get = [&](vT (&q)[8], int e) {
 #pragma unroll
                     for (int u = 0; u < 8; u++) q[u] = *(const vT*)(v + e + u * V);
+                };
+                auto add = [&](const vT (&q)[8]) {
 #pragma unroll
                     for (int u = 0; u < 8; u++)
 #pragma unroll
                         for (int w = 0; w < V; w++) sum += q[u][w];
+                };
+                vT qa[8], qb[8];
+                get(qa, 0);
+                for (int e = 0; e < full; e += 2 * B) {
+                    get(qb, e + B);
+                    __builtin_amdgcn_sched_barrier(0);
+                    add(qa);
+                    // past the last batch: the first again, unused
+                    get(qa, e + 2 * B < full ? e + 2 * B : 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    add(qb);
                 }
-                for (; e < len; e++) sum += v[e];
             }
             __syncthreads();
         }
     }
-    if (threadIdx.x == 0) {
-        T kj = sum;
-        if (a.bias && fresh) kj += pref * bias_sine<T>(J == 1 ? x[i] : a.tmp[i]);
-        var_stage<T, J>(a, i, fresh, kj, var_load<T, J>(a, i, x, fresh), xnew, hs, h, hnext, floor, err);
+    if (t < 64) {
+        T out = (T)0;
+        if (t == 0) {
+            T kj = sum;
+            if (a.bias && fresh) kj += pref * s_sine;
+            out = var_stage<T, J>(a, i, fresh, kj, in, xnew, hs, h, hnext, floor, err);
+        }
+        if (a.th) {
+            // the next stage's entries of the tanh table, a lane each
+            out = __shfl(out, 0, 64);
+            if (t < 2) a.th[2 * i + t] = tanh_half<T>(out, a.q, t);
+        }
     }
     if constexpr (J == 6) {
         double bm = block_max<WIDE_BLK>(err, sh);
@@ -1683,6 +1877,10 @@ struct Sys {
     hipStream_t stream = nullptr;
     int* d_lit = nullptr;
     int* d_pos = nullptr;        // generic-K clause pass only
+    int *d_litq = nullptr, *d_posq = nullptr;   // the same by literal, K <= 10
+    int mq = 0;
+    double* d_th = nullptr;      // tanh table (generic pass with the wide var pass)
+    bool wide_run = false;       // wide var pass: a variable's contributions lie side by side
     int* d_spos = nullptr;       // tiled clause pass (K = 3, 4)
     uint16_t* d_srank = nullptr;
     unsigned* d_runs = nullptr;  // big tiles: run tables in place of d_spos
@@ -1737,7 +1935,8 @@ struct Sys {
 
     void free_problem()
     {
-        dfree(d_lit); dfree(d_pos); dfree(d_spos); dfree(d_srank); dfree(d_csr_ptr); dfree(d_csr_pos);
+        dfree(d_lit); dfree(d_pos); dfree(d_litq); dfree(d_posq); dfree(d_th); dfree(d_spos);
+        dfree(d_srank); dfree(d_csr_ptr); dfree(d_csr_pos);
         dfree(d_runs);
         run_stride = 0;
         dfree(d_csr_loc); dfree(d_gstart); dfree(d_perm); dfree(d_contrib); dfree(d_apart);
@@ -2034,6 +2233,13 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
     // the gather kernel would add a block's rows one after another, so each
     // variable gets a workgroup of its own
     s->wide_var = !lds_var && s->nslots >= WIDE_MIN_ROW * (long long)P.n;
+    // the generic clause pass can store anywhere: a variable's terms side by side
+    s->wide_run = s->wide_var && !tiled;
+    if (s->wide_run) {
+        std::vector<int> fill(P.csr_ptr.begin(), P.csr_ptr.end() - 1);
+        for (size_t sl = 0; sl < P.lit.size(); sl++)
+            if (P.lit[sl]) P.pos[sl] = fill[(size_t)std::abs(P.lit[sl])]++;
+    }
     s->var_region_cap = lds_var ? (int)P.max_region : 0;
     s->var_lds = lds_var ? var_lds_bytes(P.max_region, s->esize) : 0;
     // two FP32 var workgroups per CU (LDS for both; the FP64 kernel's
@@ -2065,15 +2271,34 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
             HIP_CHECK(hipMemset(s->d_pcontrib, 0, (size_t)s->esize * np));
         }
     } else {
-        P.pos.resize(mpad * P.k, -1);
-        upload(s->d_pos, P.pos);
+        s->mq = 0;
+        if (P.k <= 10) {
+            // literals and positions by literal (k_clause_k)
+            s->mq = (int)round_up((long long)P.m, BLK);
+            std::vector<int> lq((size_t)s->mq * P.k, 0), pq((size_t)s->mq * P.k, 0);
+            for (int j = 0; j < P.m; j++)
+                for (int q = 0; q < P.k; q++) {
+                    lq[(size_t)q * s->mq + j] = P.lit[(size_t)j * P.k + q];
+                    pq[(size_t)q * s->mq + j] = P.pos[(size_t)j * P.k + q];
+                }
+            upload(s->d_litq, lq);
+            upload(s->d_posq, pq);
+            if (s->wide_var && (s->esize == 8 || P.k >= 3))
+                HIP_CHECK(hipMalloc((void**)&s->d_th, sizeof(double) * 2 * ((size_t)P.n + 1)));
+        }
+        // k_clause_gen's positions: more than 10 literals, or the tanh family
+        // without its table
+        if (!s->d_th) {
+            P.pos.resize(mpad * P.k, -1);
+            upload(s->d_pos, P.pos);
+        }
     }
     upload(s->d_csr_ptr, P.csr_ptr);
     if (lds_var) {
         P.csr_loc.resize(P.csr_loc.size() + 8, 0);   // rounded-up 16-byte loads of the last range
         upload(s->d_csr_loc, P.csr_loc);
     }
-    else upload(s->d_csr_pos, P.csr_pos);
+    else if (!s->wide_run) upload(s->d_csr_pos, P.csr_pos);
     upload(s->d_gstart, P.gstart);
     build_small_lists(s, P);
     // up to 512 clauses and variables asat_small.h is the faster one
@@ -2179,6 +2404,8 @@ static StageArgs<T> stage_args(Sys* s, T* xa, T* xb, T* const* kk, T* tmp, doubl
     memset(&a, 0, sizeof(a));   // padding too: the arguments are compared bytewise (captured attempts)
     a.lit = s->d_lit; a.pos = s->d_pos; a.spos = s->d_spos; a.srank = s->d_srank;
     a.runs = s->d_runs; a.run_stride = s->run_stride;
+    a.litq = s->d_litq; a.posq = s->d_posq; a.mq = s->mq;
+    a.th = s->family == ASAT_FAMILY_TANH ? s->d_th : nullptr;
     a.csr_ptr = s->d_csr_ptr; a.csr_pos = s->d_csr_pos; a.csr_loc = s->d_csr_loc; a.gstart = s->d_gstart;
     a.pvar = s->d_pvar; a.pw16 = s->d_pw16; a.pv0 = s->d_pv0; a.pc0 = s->d_pc0; a.pcontrib = (T*)s->d_pcontrib; a.split = s->split ? 1 : 0;
     a.contrib = (T*)s->d_contrib;
@@ -2207,9 +2434,24 @@ static StageArgs<T> stage_args(Sys* s, T* xa, T* xb, T* const* kk, T* tmp, doubl
 }
 
 
+// k_clause_k and its tanh-table form by the clause length
+template <typename T, int J, int KT>
+static void launch_clause_k(const StageArgs<T>& a, hipStream_t st)
+{
+    if (a.th) hipLaunchKernelGGL((k_clause_k<T, KT, J, true>), dim3(a.nblk_clause), dim3(BLK), 0, st, a);
+    else hipLaunchKernelGGL((k_clause_k<T, KT, J, false>), dim3(a.nblk_clause), dim3(BLK), 0, st, a);
+}
+
 template <typename T, int J>
 static void launch_clause(const StageArgs<T>& a, const Sys* s, hipStream_t st)
 {
+    if (!s->tiled && a.litq && (a.family != ASAT_FAMILY_TANH || a.th)) {
+        if (a.k <= 2) launch_clause_k<T, J, 2>(a, st);
+        else if (a.k <= 6) launch_clause_k<T, J, 6>(a, st);
+        else if (a.k <= 8) launch_clause_k<T, J, 8>(a, st);
+        else launch_clause_k<T, J, 10>(a, st);
+        return;
+    }
     dim3 g(a.nblk_clause), b(BLK);
     const bool tiled = s->tiled;
     const bool ss = a.slot_spins != 0;
@@ -2302,6 +2544,7 @@ static void sys_rhs(Sys* s, State* dxdt, const State* x)
     StageArgs<T> a = stage_args<T>(s, (T*)x->d, nullptr, kk, nullptr, nullptr, nullptr);
     // dxdt.SetZero(): padding and the constant slot read as 0
     HIP_CHECK(hipMemsetAsync(dxdt->d, 0, (size_t)s->esize * s->alloc, s->stream));
+    fill_tanh<T>(a, (const T*)x->d, s->stream);
     launch_clause<T, 1>(a, s, s->stream);
     launch_var<T, 1>(a, s, s->stream);
     HIP_CHECK(hipGetLastError());
@@ -2477,11 +2720,20 @@ static void rk_configure(RK* r, Sys* s)
 // rejected attempt's J = 1 clause pass is skipped, and its J = 1 var pass
 // (which reuses k1 and reads no contributions) writes stage 2's spins.
 template <typename T>
+static void fill_tanh(const StageArgs<T>& a, const T* x, hipStream_t st)
+{
+    if (!a.th) return;
+    hipLaunchKernelGGL(k_tanh_fill<T>, dim3(ceil_div(2LL * (a.n + 1), BLK)), dim3(BLK), 0, st, x, a.n, a.q, a.th);
+    HIP_CHECK(hipGetLastError());
+}
+
+template <typename T>
 static StageArgs<T> rk_stage_args(RK* r, int parity)
 {
     Sys* s = r->sys;
     T* kk[5] = {(T*)r->k[0], (T*)r->k[1], (T*)r->k[2], (T*)r->k[3], (T*)r->k[4]};
     StageArgs<T> a = stage_args<T>(s, (T*)r->pair[0], (T*)r->pair[1], kk, (T*)r->tmp, r->partial, r->d_ctrl);
+    fill_tanh<T>(a, (const T*)r->pair[parity], s->stream);
     if (s->tiled && s->lds_var) {
         a.slot_spins = 1;
         hipLaunchKernelGGL(k_slot_fill<T>, dim3(ceil_div(s->n, BLK)), dim3(BLK), 0, s->stream,
