@@ -1982,7 +1982,9 @@ static void upload(V*& d, const std::vector<V>& h)
 // Variable groups for the LDS var pass: about 2048 (float) / 1024 (double)
 // variables per group, a multiple of 256 groups once there are more than
 // 256 (one workgroup per CU per round), at least 256 groups while groups
-// keep 256+ variables; halved until the largest region fits in LDS.  When no
+// keep 128+ variables (4-SAT, N = 20 011, M = 196 107: 143 us per attempt with
+// FP64 and 115 with FP32, against 152 and 120 with 256+; sizes with 256 groups
+// either way are the same); halved until the largest region fits in LDS.  When no
 // size fits (a variable with more occurrences than the LDS holds), the gather
 // var pass runs with ~400 KB regions.
 // LDS of the region var pass: the region and its variables' uint16 offsets
@@ -1996,7 +1998,7 @@ static bool choose_layout(HostProblem& P, int esize)
 {
     const long long cap = (VAR_LDS_BYTES - 48) / (esize + 2);
     const long long target = esize == 4 ? 2048 : 1024;
-    long long G = std::max(ceil_div((long long)P.n, target), std::min(256, ceil_div((long long)P.n, 256)));
+    long long G = std::max(ceil_div((long long)P.n, target), std::min(256, ceil_div((long long)P.n, 128)));
     if (G > 256) G = round_up(G, 256);
     int vg = ceil_div((long long)P.n, G);
     // direct primary slots wherever the tiled pass meets the LDS var pass
@@ -2747,7 +2749,9 @@ static StageArgs<T> rk_stage_args(RK* r, int parity)
 // Launch-bound problems (few literal slots) replay a captured graph of
 // GRAPH_ATTEMPTS attempts instead of launching 13 kernels per attempt, as
 // long as a round still needs that many; the rest are launched one by one.
-constexpr long long GRAPH_MAX_SLOTS = 1LL << 20;
+// Larger ones gain nothing (N = 20 011, M = 196 107: 143 and 144 us per attempt)
+// and would pay the capture in their first Step (0.3 ms).
+constexpr long long GRAPH_MAX_SLOTS = 1LL << 18;
 constexpr int GRAPH_ATTEMPTS = 8;
 
 template <typename T>
