@@ -19,11 +19,18 @@
 //   u_a    = w_a K^2 + sum_q w_q 2 c_q K K_q
 //   u_s[p] = w_a (-2 a c_p K K_p) + w_p (-2 a K_p^2) + sum_{q!=p} w_q (-4 a c_q c_p K K_qp)
 // Per-variable sums run over each variable's slots in slot order
-// (deterministic).  FP32 terms are written at their var-major positions (a
-// variable's terms are one contiguous run; 510 KB per trajectory at
-// N = 1e4, M = 42 500, L2-resident); FP64 terms stay in clause order and are gathered through the
-// var-major slot list (scattered FP64 writes cost more than the gathers).
-// Internal layout of every vector: [0 | s_1..s_N | a_1..a_M], stride D.
+// (deterministic); terms are written at their var-major positions, so a
+// variable's terms are one run.
+// Internal layout: vectors [0 | s_1..s_N | a_1..a_M] of D elements, the values of
+// tp trajectories side by side for every element (tiles of tp: element i of
+// trajectory tr at ((tr / tp) D + i) tp + tr % tp; slot terms likewise).  A wave
+// then takes 64 / tp clauses or variables of tp trajectories: the literals and
+// positions they share are read once, and a gather or scatter touches 64 / tp
+// places of tp values each.  One trajectory per wave touched 64 of them, which
+// kept the texture addressers busy while little memory moved.  64 trajectories of
+// N = 1e4, M = 42 500, 64 steps, forward and backward: 134 to 55 ms; in a stage of
+// the backward the product with its mu 99 to 37-47 us (about 5 TB/s), the sums 44
+// to 13; a forward clause pass 43-51 to 14-21 us.
 #include "asat_common.h"
 
 #include <algorithm>
@@ -42,42 +49,140 @@ constexpr int BLK = 256;
 struct Dev {
     const int* lit;       // m*k (zero padded)
     const int* csr_ptr;   // n+2, var-major over slots
-    const int* csr_slot;  // slot indices, ascending per variable
     const int* slot_pos;  // each slot's position in that var-major order, -1: padding
     int n, m, k;
-    long long D;          // vector stride (>= n+m+1)
+    long long D;          // elements of a vector (>= n+m+1)
     long long L;          // m*k
-    int ntraj;            // trajectories (grids are padded to a multiple of 8)
+    int ntraj;            // trajectories
+    int sh;               // log2 tp
+    int sx;               // log2 of the XCDs that share a tile
 };
 
-// Trajectory-batched grids are (blocks per trajectory, ntraj rounded up to
-// 8).  Workgroups are dealt to the 8 XCDs round-robin by linear id; the id is
-// remapped so that every block of trajectory tr runs on XCD tr % 8, and each
-// XCD keeps its own trajectories' gather targets (spins, contributions) in
-// its L2.  Blocks of the padding trajectories (tr >= ntraj) return at once.
+// log2 of the trajectories per tile, for L slots.  Eight trajectories' FP64 terms
+// beyond an XCD's 4 MB L2 (L > 2^16): up to 16 (N = 1e4, M = 42 500, 32 steps
+// forward and backward, ms with 1, 4, 8 and 16 per tile: 64 trajectories 59.2, 37.0,
+// 29.0, 26.8; 16: 18.6, 13.6, 11.7, 11.3).  Else a tile for every XCD first, which
+// keeps each trajectory's gathers in one L2, then up to 8 (N = 1000, M = 4200: 64
+// trajectories 9.1, 7.2, 6.5, 7.7; 8: 5.7, 6.3, 6.4).  At most an eighth of the
+// vectors is padding.
+static inline int tile_shift(int ntraj, long long L)
+{
+    int best = 0;
+    for (int sh = 1; sh <= (L > 65536 ? 4 : 3); sh++) {
+        if (L <= 65536 && (4 << sh) >= ntraj) break;
+        if (((long long)ceil_div(ntraj, 1 << sh) << sh) * 8 <= 9LL * ntraj) best = sh;
+    }
+    return best;
+}
+
+// Grids are (blocks per tile, tiles rounded up to 8).  Workgroups are dealt to
+// the 8 XCDs round-robin by linear id; the id is remapped so that every block of
+// tile t runs on XCD t % 8, and each XCD keeps its own trajectories' gather
+// targets (spins, terms) in its L2.  Fewer than 8 tiles (rounded up to 1, 2 or
+// 4): 8, 4 or 2 XCDs take turns at the blocks of one tile.
+static inline int tile_xcds(int tiles)
+{
+    int sx = 3;
+    while (sx > 0 && (8 >> sx) < tiles) sx--;
+    return sx;
+}
+
 struct TB {
-    long long x, tr;
+    long long x;          // block of the tile
+    int e;                // this thread's element
+    int tr;               // and trajectory
+    bool live;            // a trajectory of the batch
+    long long v, l;       // places of element 0 of its vectors and of its slot terms
+    int tp;               // stride between a trajectory's elements
+    __device__ __forceinline__ long long at(long long i) const { return v + i * tp; }
+    __device__ __forceinline__ long long slot(long long i) const { return l + i * tp; }
 };
-static inline int ntraj8(int ntraj) { return (ntraj + 7) / 8 * 8; }
 
-__device__ __forceinline__ TB traj_block()
+__device__ __forceinline__ TB traj_block(const Dev& d)
 {
     const long long per = 8LL * gridDim.x;
-    const long long L = (long long)blockIdx.y * gridDim.x + blockIdx.x;
-    const long long r = L % per;
-    return {r >> 3, (L / per) * 8 + (r & 7)};
+    const long long id = (long long)blockIdx.y * gridDim.x + blockIdx.x;
+    const long long r = id % per;
+    const int xcd = (int)(r & 7);
+    const int tile = (int)(id / per) * 8 + (xcd >> d.sx);
+    TB t;
+    t.x = ((r >> 3) << d.sx) + (xcd & ((1 << d.sx) - 1));
+    t.tp = 1 << d.sh;
+    const long long g = t.x * BLK + (int)threadIdx.x;
+    const int lane = (int)g & (t.tp - 1);
+    t.e = (int)(g >> d.sh);
+    t.tr = tile * t.tp + lane;
+    t.live = t.tr < d.ntraj;
+    t.v = (long long)tile * d.D * t.tp + lane;
+    t.l = (long long)tile * d.L * t.tp + lane;
+    return t;
+}
+
+// maximum over the block's elements for each trajectory of its tile, in the
+// threads of the block's first element (threadIdx.x < tp)
+__device__ __forceinline__ double tile_max(double v, int tp, double (*sh)[64])
+{
+    for (int o = tp; o < 64; o <<= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    const int lane = (int)threadIdx.x & 63;
+    if (lane < tp) sh[threadIdx.x >> 6][lane] = v;
+    __syncthreads();
+    if ((int)threadIdx.x < tp) {
+        v = sh[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < BLK / 64; w++) v = fmax(v, sh[w][threadIdx.x]);
+    }
+    return v;
+}
+
+// public rows [s | a] of every trajectory into the internal layout, and back
+template <typename T>
+__global__ __launch_bounds__(BLK) void k_import(Dev d, const T* pub, T slot0, T* x)
+{
+    const TB tb = traj_block(d);
+    if (!tb.live || tb.e > d.n + d.m) return;
+    x[tb.at(tb.e)] = tb.e == 0 ? slot0 : pub[(long long)tb.tr * (d.n + d.m) + tb.e - 1];
+}
+template <typename T>
+__global__ __launch_bounds__(BLK) void k_export(Dev d, const T* x, T* pub)
+{
+    const TB tb = traj_block(d);
+    if (!tb.live || tb.e >= d.n + d.m) return;
+    pub[(long long)tb.tr * (d.n + d.m) + tb.e] = x[tb.at(tb.e + 1)];
+}
+
+// spin factor of literal l: sp points at element 0 of the trajectory's spins
+template <typename T>
+__device__ __forceinline__ T tile_factor(int l, const T* sp, int tp)
+{
+    const T sv = l != 0 ? sp[(long long)(l < 0 ? -l : l) * tp] : (T)-1.0;
+    return l < 0 ? (T)1.0 + sv : (T)1.0 - sv;
+}
+
+// left-to-right sum of a variable's run of terms [e0, e1), four loads in flight
+template <typename T>
+__device__ __forceinline__ T tile_sum(const T* c, int e0, int e1, int tp)
+{
+    T s = (T)0;
+    int e = e0;
+    for (; e + 4 <= e1; e += 4) {
+        const T a = c[(long long)e * tp], b = c[(long long)(e + 1) * tp], x = c[(long long)(e + 2) * tp],
+                y = c[(long long)(e + 3) * tp];
+        s += a;
+        s += b;
+        s += x;
+        s += y;
+    }
+    for (; e < e1; e++) s += c[(long long)e * tp];
+    return s;
 }
 
 // ---- recompute (forward arithmetic; T = float, or double for the FP64 replay)
 template <typename T, int K>
 __global__ __launch_bounds__(BLK) void k_rhs_clause(Dev d, const T* Y, T* out, T* contrib)
 {
-    const TB tb = traj_block();
-    const int m = tb.x * BLK + threadIdx.x;
-    const long long tr = tb.tr;
-    if (tr >= d.ntraj) return;
-    if (m >= d.m) return;
-    const T* y = Y + tr * d.D;
+    const TB tb = traj_block(d);
+    const int m = tb.e;
+    if (!tb.live || m >= d.m) return;
     int l[K];
     T f[K];
 #pragma unroll
@@ -85,45 +190,29 @@ __global__ __launch_bounds__(BLK) void k_rhs_clause(Dev d, const T* Y, T* out, T
     T km = (T)(1.0 / (1 << K));
 #pragma unroll
     for (int q = 0; q < K; q++) {
-        f[q] = spin_factor<T>(l[q], y);
+        f[q] = tile_factor<T>(l[q], Y + tb.v, tb.tp);
         km *= f[q];
     }
-    const long long ai = d.n + 1 + m;
-    const T am = y[ai];
-    out[tr * d.D + ai] = am * km * km;
+    const long long ai = tb.at(d.n + 1 + m);
+    const T am = Y[ai];
+    out[ai] = am * km * km;
     const T r = km * (T)(1.0 / (1 << K)) * am;
     T o[K];
 #pragma unroll
     for (int q = 0; q < K; q++) o[q] = (T)0;
     write_contribs<T, K, 0>(l, f, r, o);
-    if constexpr (sizeof(T) == 4) {
-        T* c = contrib + tr * d.L;
 #pragma unroll
-        for (int q = 0; q < K; q++)
-            if (l[q] != 0) c[d.slot_pos[(size_t)m * K + q]] = o[q];
-    } else {
-        T* c = contrib + tr * d.L + (long long)m * K;
-#pragma unroll
-        for (int q = 0; q < K; q++)
-            if (l[q] != 0) c[q] = o[q];
-    }
+    for (int q = 0; q < K; q++)
+        if (l[q] != 0) contrib[tb.slot(d.slot_pos[(size_t)m * K + q])] = o[q];
 }
 
 template <typename T>
 __global__ __launch_bounds__(BLK) void k_rhs_var(Dev d, const T* contrib, T* out)
 {
-    const TB tb = traj_block();
-    const int i = tb.x * BLK + threadIdx.x + 1;
-    const long long tr = tb.tr;
-    if (tr >= d.ntraj) return;
-    if (i > d.n) return;
-    const T* c = contrib + tr * d.L;
-    T sum = (T)0;
-    if constexpr (sizeof(T) == 4)
-        sum = sum_run(sum, c, d.csr_ptr[i], d.csr_ptr[i + 1]);
-    else
-        sum = sum_run_idx(sum, c, d.csr_slot, d.csr_ptr[i], d.csr_ptr[i + 1]);
-    out[tr * d.D + i] = sum;
+    const TB tb = traj_block(d);
+    const int i = tb.e + 1;
+    if (!tb.live || i > d.n) return;
+    out[tb.at(i)] = tile_sum<T>(contrib + tb.l, d.csr_ptr[i], d.csr_ptr[i + 1], tb.tp);
 }
 
 // stage input J of every element (spins and aux) for every trajectory
@@ -131,13 +220,11 @@ template <typename T, int J>
 __global__ __launch_bounds__(BLK) void k_stage(Dev d, const T* X, const T* k1, const T* k2, const T* k3, const T* k4,
                                                 const T* k5, const double* h, T* Y)
 {
-    const TB tb = traj_block();
-    const long long i = (long long)tb.x * BLK + threadIdx.x + 1;
-    const long long tr = tb.tr;
-    if (tr >= d.ntraj) return;
-    if (i > (long long)d.n + d.m) return;
-    const long long o = tr * d.D + i;
-    const T hs = (T)h[tr];
+    const TB tb = traj_block(d);
+    const long long i = tb.e + 1;
+    if (!tb.live || i > (long long)d.n + d.m) return;
+    const long long o = tb.at(i);
+    const T hs = (T)h[tb.tr];
     Y[o] = stage_input<T, J>(X[o], k1[o], J > 2 ? k2[o] : (T)0, J > 3 ? k3[o] : (T)0, J > 4 ? k4[o] : (T)0,
                              J > 5 ? k5[o] : (T)0, hs);
 }
@@ -146,18 +233,16 @@ template <typename T>
 __global__ __launch_bounds__(BLK) void k_final(Dev d, const T* X, const T* k1, const T* k3, const T* k4, const T* k6,
                                                const double* h, T* Xn)
 {
-    const TB tb = traj_block();
-    const long long i = (long long)tb.x * BLK + threadIdx.x;
-    const long long tr = tb.tr;
-    if (tr >= d.ntraj) return;
-    if (i > (long long)d.n + d.m) return;
-    const long long o = tr * d.D + i;
+    const TB tb = traj_block(d);
+    const long long i = tb.e;
+    if (!tb.live || i > (long long)d.n + d.m) return;
+    const long long o = tb.at(i);
     if (i == 0) {
         Xn[o] = (T)-1.0;
         return;
     }
     using B = Tab<T>;
-    const T hs = (T)h[tr];
+    const T hs = (T)h[tb.tr];
     Xn[o] = X[o] + hs * (B::c1 * k1[o] + B::c3 * k3[o] + B::c4 * k4[o] + B::c6 * k6[o]);
 }
 
@@ -172,39 +257,68 @@ __device__ __forceinline__ double prod_skip(const double (&fd)[K], int s1, int s
     return p;
 }
 
-// u_a directly, per-slot spin contributions into contrib64
-template <int K>
-__global__ __launch_bounds__(BLK) void k_vjp_clause(Dev d, const float* Y, const double* w, double* u,
-                                                    double* contrib)
+// mu_l = h * (Cw_l lam + sum_{j>l} B_jl nu_j) of one element (j ascending); nu_j
+// is vs elements past nu_{j-1}
+template <int LL>
+__device__ __forceinline__ double mu_of(const double* lam, const double* nu, long long o, long long vs, double hh)
 {
-    const TB tb = traj_block();
-    const int m = tb.x * BLK + threadIdx.x;
-    const long long tr = tb.tr;
-    if (tr >= d.ntraj) return;
-    if (m >= d.m) return;
-    const float* y = Y + tr * d.D;
-    const double* wt = w + tr * d.D;
+    using B = Tab<float>;
+    constexpr double Bj[7][6] = {
+        {0}, {0},
+        {(double)B::b21},
+        {(double)B::b31, (double)B::b32},
+        {(double)B::b41, (double)B::b42, (double)B::b43},
+        {(double)B::b51, (double)B::b52, (double)B::b53, (double)B::b54},
+        {(double)B::b61, (double)B::b62, (double)B::b63, (double)B::b64, (double)B::b65}};
+    constexpr double Cw[7] = {0, (double)B::c1, 0, (double)B::c3, (double)B::c4, 0, (double)B::c6};
+    double acc = Cw[LL] * lam[o];
+#pragma unroll
+    for (int j = LL + 1; j <= 6; j++) acc += Bj[j][LL - 1] * nu[(long long)(j - 1) * vs + o];
+    return hh * acc;
+}
+
+// mu_l of the spins, which the clause pass gathers
+template <int LL>
+__global__ __launch_bounds__(BLK) void k_mu(Dev d, const double* lam, const double* nu, long long vs, const double* hh,
+                                            double* mu)
+{
+    const TB tb = traj_block(d);
+    if (!tb.live || tb.e > d.n) return;
+    const long long o = tb.at(tb.e);
+    mu[o] = tb.e == 0 ? 0.0 : mu_of<LL>(lam, nu, o, vs, hh[tb.tr]);
+}
+
+// One clause's product: u_a = nu_l of its aux element, per-slot spin terms at
+// their var-major positions.  Its own aux element's mu_l is formed here from lam
+// and the later stages' nu (read in any case once per stage; a mu vector of them
+// all would be written and read again).
+template <int K, int LL>
+__global__ __launch_bounds__(BLK) void k_vjp_clause(Dev d, const float* Y, const double* mu, const double* lam,
+                                                    double* nu, long long vs, const double* hh, double* contrib)
+{
+    const TB tb = traj_block(d);
+    const int m = tb.e;
+    if (!tb.live || m >= d.m) return;
     const double kn = 1.0 / (1 << K);
     int v[K];
     double fd[K], cs[K], wv[K];
+    const long long ai = tb.at(d.n + 1 + m);
+    const double a = (double)Y[ai];
+    const double wa = mu_of<LL>(lam, nu, ai, vs, hh[tb.tr]);
 #pragma unroll
     for (int q = 0; q < K; q++) {
         const int l = d.lit[(size_t)m * K + q];
         v[q] = l < 0 ? -l : l;
         cs[q] = l < 0 ? -1.0 : 1.0;
-        fd[q] = (double)spin_factor<float>(l, y);
-        wv[q] = v[q] ? wt[v[q]] : 0.0;
+        fd[q] = (double)tile_factor<float>(l, Y + tb.v, tb.tp);
+        wv[q] = v[q] ? mu[tb.at(v[q])] : 0.0;
     }
     const double Kc = prod_skip<K>(fd, -1, -1, kn);
-    const long long ai = d.n + 1 + m;
-    const double a = (double)y[ai];
-    const double wa = wt[ai];
     double ua = wa * Kc * Kc;
 #pragma unroll
     for (int q = 0; q < K; q++)
         if (v[q]) ua += wv[q] * (2.0 * cs[q] * Kc * prod_skip<K>(fd, q, -1, kn));
-    u[tr * d.D + ai] = ua;
-    double* c = contrib + tr * d.L + (long long)m * K;
+    nu[(long long)(LL - 1) * vs + ai] = ua;
 #pragma unroll
     for (int p = 0; p < K; p++) {
         if (!v[p]) continue;
@@ -215,23 +329,17 @@ __global__ __launch_bounds__(BLK) void k_vjp_clause(Dev d, const float* Y, const
             if (q == p || !v[q]) continue;
             t += wv[q] * (-4.0 * a * cs[q] * cs[p] * Kc * prod_skip<K>(fd, q, p, kn));
         }
-        c[p] = t;
+        contrib[tb.slot(d.slot_pos[(size_t)m * K + p])] = t;
     }
 }
 
-// grad V: aux K^2, spin contributions -2 a c K K_p; per-block partial sums of V
+// grad V: aux K^2, spin contributions -2 a c K K_p; vc: each clause's share of V
 template <typename TX, int K>
-__global__ __launch_bounds__(BLK) void k_gradv_clause(Dev d, const TX* X, double* g, double* contrib,
-                                                      double* vpart, int nblk)
+__global__ __launch_bounds__(BLK) void k_gradv_clause(Dev d, const TX* X, double* g, double* contrib, double* vc)
 {
-    const TB tb = traj_block();
-    __shared__ double sh[BLK / 64];
-    const int m = tb.x * BLK + threadIdx.x;
-    const long long tr = tb.tr;
-    if (tr >= d.ntraj) return;
-    double vloc = 0.0;
-    if (m < d.m) {
-        const TX* x = X + tr * d.D;
+    const TB tb = traj_block(d);
+    const int m = tb.e;
+    if (tb.live && m < d.m) {
         const double kn = 1.0 / (1 << K);
         int v[K];
         double fd[K], cs[K];
@@ -240,20 +348,28 @@ __global__ __launch_bounds__(BLK) void k_gradv_clause(Dev d, const TX* X, double
             const int l = d.lit[(size_t)m * K + q];
             v[q] = l < 0 ? -l : l;
             cs[q] = l < 0 ? -1.0 : 1.0;
-            fd[q] = (double)spin_factor<TX>(l, x);
+            fd[q] = (double)tile_factor<TX>(l, X + tb.v, tb.tp);
         }
         const double Kc = prod_skip<K>(fd, -1, -1, kn);
-        const long long ai = d.n + 1 + m;
-        const double a = (double)x[ai];
-        vloc = a * Kc * Kc;
-        g[tr * d.D + ai] = Kc * Kc;
-        double* c = contrib + tr * d.L + (long long)m * K;
+        const long long ai = tb.at(d.n + 1 + m);
+        const double a = (double)X[ai];
+        vc[ai] = a * Kc * Kc;
+        g[ai] = Kc * Kc;
 #pragma unroll
         for (int p = 0; p < K; p++)
-            if (v[p]) c[p] = -2.0 * a * cs[p] * Kc * prod_skip<K>(fd, p, -1, kn);
+            if (v[p])
+                contrib[tb.slot(d.slot_pos[(size_t)m * K + p])] =
+                    -2.0 * a * cs[p] * Kc * prod_skip<K>(fd, p, -1, kn);
     }
-    // deterministic block sum (fixed tree), summed in block order on the host side
-    double s = vloc;
+}
+
+// V: deterministic sums (fixed tree) of blocks of 256 clauses, the same for every
+// number of trajectories; the blocks are added in order afterwards
+__global__ __launch_bounds__(BLK) void k_v_blocks(Dev d, const double* vc, double* vpart)
+{
+    __shared__ double sh[BLK / 64];
+    const int m = (int)(blockIdx.x * BLK + threadIdx.x), tr = blockIdx.y, tp = 1 << d.sh;
+    double s = m < d.m ? vc[((long long)(tr >> d.sh) * d.D + d.n + 1 + m) * tp + (tr & (tp - 1))] : 0.0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
@@ -261,69 +377,35 @@ __global__ __launch_bounds__(BLK) void k_gradv_clause(Dev d, const TX* X, double
     if (threadIdx.x == 0) {
         double t = 0.0;
         for (int i = 0; i < BLK / 64; i++) t += sh[i];
-        vpart[tr * nblk + tb.x] = t;
+        vpart[(long long)tr * gridDim.x + blockIdx.x] = t;
     }
 }
 
 __global__ void k_sum_parts(const double* vpart, int nblk, double* V)
 {
     const int tr = blockIdx.x;
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int b = 0; b < nblk; b++) t += vpart[(long long)tr * nblk + b];
-        V[tr] = t;
+    // a wave per trajectory; the blocks' sums are added in block order
+    __shared__ double sh[256];
+    double t = 0.0;
+    for (int b0 = 0; b0 < nblk; b0 += 256) {
+        for (int i = (int)threadIdx.x; i < 256 && b0 + i < nblk; i += 64) sh[i] = vpart[(long long)tr * nblk + b0 + i];
+        __syncthreads();
+        if (threadIdx.x == 0)
+            for (int i = 0; i < 256 && b0 + i < nblk; i++) t += sh[i];
+        __syncthreads();
     }
+    if (threadIdx.x == 0) V[tr] = t;
 }
 
-// mu = h * (Cw_l lam + sum_{j>l} B_jl nu_j)   (j descending order of terms as written)
-__global__ __launch_bounds__(BLK) void k_mu(Dev d, int l, const double* lam, const double* nu, const double* hh,
-                                            double* mu)
+__global__ __launch_bounds__(BLK) void k_lam(Dev d, double* lam, const double* nu, long long vs)
 {
-    const TB tb = traj_block();
-    const double Bj[7][6] = {
-        {0}, {0},
-        {(double)Tab<float>::b21},
-        {(double)Tab<float>::b31, (double)Tab<float>::b32},
-        {(double)Tab<float>::b41, (double)Tab<float>::b42, (double)Tab<float>::b43},
-        {(double)Tab<float>::b51, (double)Tab<float>::b52, (double)Tab<float>::b53, (double)Tab<float>::b54},
-        {(double)Tab<float>::b61, (double)Tab<float>::b62, (double)Tab<float>::b63, (double)Tab<float>::b64,
-         (double)Tab<float>::b65}};
-    const double Cw[7] = {0, (double)Tab<float>::c1, 0, (double)Tab<float>::c3, (double)Tab<float>::c4, 0,
-                          (double)Tab<float>::c6};
-    const long long i = (long long)tb.x * BLK + threadIdx.x;
-    const long long tr = tb.tr;
-    if (tr >= d.ntraj) return;
-    if (i > (long long)d.n + d.m) return;
-    const long long o = tr * d.D + i;
-    if (i == 0) {
-        mu[o] = 0.0;
-        return;
-    }
-    const long long vs = (long long)d.ntraj * d.D;   // stride between nu_j vectors
-    double acc = Cw[l] * lam[o];
-    for (int j = l + 1; j <= 6; j++) acc += Bj[j][l - 1] * nu[(long long)(j - 1) * vs + o];
-    mu[o] = hh[tr] * acc;
-}
-
-__global__ __launch_bounds__(BLK) void k_lam(Dev d, double* lam, const double* nu)
-{
-    const TB tb = traj_block();
-    const long long i = (long long)tb.x * BLK + threadIdx.x + 1;
-    const long long tr = tb.tr;
-    if (tr >= d.ntraj) return;
-    if (i > (long long)d.n + d.m) return;
-    const long long o = tr * d.D + i;
-    const long long vs = (long long)d.ntraj * d.D;
+    const TB tb = traj_block(d);
+    const long long i = tb.e + 1;
+    if (!tb.live || i > (long long)d.n + d.m) return;
+    const long long o = tb.at(i);
     lam[o] = lam[o] + nu[o] + nu[vs + o] + nu[2 * vs + o] + nu[3 * vs + o] + nu[4 * vs + o] + nu[5 * vs + o];
 }
 
-__global__ void k_zero_slot0(double* v, long long D, int ntraj)
-{
-    const int tr = blockIdx.x * blockDim.x + threadIdx.x;
-    if (tr < ntraj) v[(long long)tr * D] = 0.0;
-}
-
-// plain-solver layout (spins 1..N, aux at aoff) -> internal layout (aux at N+1)
 // ---- lockstep adaptive forward (FP32 state, FP64 control) -------------------
 // Every trajectory runs CpuRungeKutta's Step/rkqs (AnalogSAT/cpu_sat/
 // CpuRungeKutta.cpp:65-100,217-267) with its own h; all trajectories take
@@ -379,20 +461,18 @@ __global__ __launch_bounds__(BLK) void k_ctl_batch(TCtl* ctl, const double* part
     hcur[tr] = c.h;
 }
 
-// accepted trajectories: x <- x_new, and the checkpoint when one is due
+// accepted trajectories: x <- x_new, and the checkpoint when one is due (V
+// elements per checkpoint)
 __global__ __launch_bounds__(BLK) void k_accept(Dev d, const TCtl* ctl, const float* Xn, float* X, float* ckpt,
-                                                long long ntraj)
+                                                long long V)
 {
-    const TB tb = traj_block();
-    const long long i = (long long)tb.x * BLK + threadIdx.x;
-    const long long tr = tb.tr;
-    if (tr >= d.ntraj) return;
-    if (i > (long long)d.n + d.m || !ctl[tr].accept) return;
-    const long long o = tr * d.D + i;
+    const TB tb = traj_block(d);
+    if (!tb.live || tb.e > d.n + d.m || !ctl[tb.tr].accept) return;
+    const long long o = tb.at(tb.e);
     const float v = Xn[o];
     X[o] = v;
-    const int c = ctl[tr].ckpt;
-    if (c >= 0) ckpt[((long long)c * ntraj + tr) * d.D + i] = v;
+    const int c = ctl[tb.tr].ckpt;
+    if (c >= 0) ckpt[(long long)c * V + o] = v;
 }
 
 __global__ void k_ctl_init(TCtl* ctl, double* hcur, int ntraj)
@@ -427,9 +507,9 @@ struct FArgs {
     float* Xn;            // null: no x_new (frozen step whose successor is not needed)
     float* k[6];          // k1..k6 (k6 is not stored)
     float* S;             // adaptive: spin input of the next stage
-    float* Y;             // frozen: [6][ntraj][D] stage inputs
-    float* c;             // [ntraj][L] slot terms, var-major
-    long long V;          // ntraj * D
+    float* Y;             // frozen: six stage inputs, V elements each
+    float* c;             // slot terms, var-major
+    long long V;          // elements of a vector of all trajectories
     const double* hcol;   // frozen: step size of every trajectory
     const TCtl* ctl;      // adaptive: control blocks
     double* parts;
@@ -439,88 +519,82 @@ struct FArgs {
 template <int K, int J, bool FZ>
 __global__ __launch_bounds__(BLK) void k_fclause(FArgs a)
 {
-    __shared__ double sh[BLK / 64];
-    const TB tb = traj_block();
-    const long long tr = tb.tr;
-    if (tr >= a.d.ntraj) return;
-    if (!FZ && !a.ctl[tr].active) return;
-    const int m = tb.x * BLK + threadIdx.x;
-    const double h = FZ ? a.hcol[tr] : a.ctl[tr].h;
-    const double hnext = FZ ? h : a.ctl[tr].hnext;
-    const float hs = (float)h;
-    const long long row = tr * a.d.D;
-    const float* x = a.X + row;
-    const float* sp = J == 1 ? x : (FZ ? a.Y + (J - 1) * a.V : a.S) + row;
+    __shared__ double sh[BLK / 64][64];
+    const TB tb = traj_block(a.d);
+    const int m = tb.e;
+    const bool run = tb.live && (FZ || a.ctl[tb.tr].active);
     double err = 0.0;
-    if (m < a.d.m) {
-        int l[K];
+    if (run && m < a.d.m) {
+        const double h = FZ ? a.hcol[tb.tr] : a.ctl[tb.tr].h;
+        const double hnext = FZ ? h : a.ctl[tb.tr].hnext;
+        const float hs = (float)h;
+        const float* x = a.X;
+        const float* sp = (J == 1 ? x : (FZ ? a.Y + (J - 1) * a.V : a.S)) + tb.v;
+        int l[K], pos[K];
         float f[K];
 #pragma unroll
-        for (int q = 0; q < K; q++) l[q] = a.d.lit[(size_t)m * K + q];
+        for (int q = 0; q < K; q++) {
+            l[q] = a.d.lit[(size_t)m * K + q];
+            pos[q] = a.d.slot_pos[(size_t)m * K + q];
+        }
         float km = (float)(1.0 / (1 << K));
 #pragma unroll
         for (int q = 0; q < K; q++) {
-            f[q] = spin_factor<float>(l[q], sp);
+            f[q] = tile_factor<float>(l[q], sp, tb.tp);
             km *= f[q];
         }
-        const long long ai = a.d.n + 1 + m;
+        const long long ai = tb.at(a.d.n + 1 + m);
+        const float xa = x[ai];
         float am, k1 = 0.f, k3 = 0.f, k4 = 0.f, k5 = 0.f;
         if constexpr (J == 1) {
-            am = x[ai];
+            am = xa;
         } else {
-            k1 = a.k[0][row + ai];
-            const float k2 = J > 2 ? a.k[1][row + ai] : 0.f;
-            k3 = J > 3 ? a.k[2][row + ai] : 0.f;
-            k4 = J > 4 ? a.k[3][row + ai] : 0.f;
-            k5 = J > 5 ? a.k[4][row + ai] : 0.f;
-            am = stage_input<float, J>(x[ai], k1, k2, k3, k4, k5, hs);
+            k1 = a.k[0][ai];
+            const float k2 = J > 2 ? a.k[1][ai] : 0.f;
+            k3 = J > 3 ? a.k[2][ai] : 0.f;
+            k4 = J > 4 ? a.k[3][ai] : 0.f;
+            k5 = J > 5 ? a.k[4][ai] : 0.f;
+            am = stage_input<float, J>(xa, k1, k2, k3, k4, k5, hs);
         }
-        if constexpr (FZ) a.Y[(J - 1) * a.V + row + ai] = am;
+        if constexpr (FZ) a.Y[(J - 1) * a.V + ai] = am;
         const float kj = am * km * km;
         if constexpr (J < 6) {
-            a.k[J - 1][row + ai] = kj;
+            a.k[J - 1][ai] = kj;
         } else if (a.Xn) {
             float xn;
-            final_combination<float>(x[ai], k1, k3, k4, k5, kj, hs, h, hnext, TabD::TINY, xn, err);
-            a.Xn[row + ai] = xn;
-            if (m == 0) a.Xn[row] = -1.0f;
+            final_combination<float>(xa, k1, k3, k4, k5, kj, hs, h, hnext, TabD::TINY, xn, err);
+            a.Xn[ai] = xn;
+            if (m == 0) a.Xn[tb.v] = -1.0f;
         }
         const float r = km * (float)(1.0 / (1 << K)) * am;
         float o[K];
 #pragma unroll
         for (int q = 0; q < K; q++) o[q] = 0.f;
         write_contribs<float, K, 0>(l, f, r, o);
-        float* cr = a.c + tr * a.d.L;
 #pragma unroll
         for (int q = 0; q < K; q++)
-            if (l[q] != 0) cr[a.d.slot_pos[(size_t)m * K + q]] = o[q];
+            if (l[q] != 0) a.c[tb.slot(pos[q])] = o[q];
     }
     if constexpr (J == 6 && !FZ) {
-        const double bm = block_max<BLK>(err, sh);
-        if (threadIdx.x == 0) a.parts[tr * (a.nblk_c + a.nblk_v) + tb.x] = bm;
+        const double bm = tile_max(err, tb.tp, sh);
+        if ((int)threadIdx.x < tb.tp && run && tb.x < a.nblk_c) a.parts[(long long)tb.tr * (a.nblk_c + a.nblk_v) + tb.x] = bm;
     }
 }
 
 template <int J, bool FZ>
 __global__ __launch_bounds__(BLK) void k_fvar(FArgs a)
 {
-    __shared__ double sh[BLK / 64];
-    const TB tb = traj_block();
-    const long long tr = tb.tr;
-    if (tr >= a.d.ntraj) return;
-    if (!FZ && !a.ctl[tr].active) return;
-    const int i = tb.x * BLK + threadIdx.x + 1;
-    const double h = FZ ? a.hcol[tr] : a.ctl[tr].h;
-    const double hnext = FZ ? h : a.ctl[tr].hnext;
-    const float hs = (float)h;
-    const long long row = tr * a.d.D;
+    __shared__ double sh[BLK / 64][64];
+    const TB tb = traj_block(a.d);
+    const int i = tb.e + 1;
+    const bool run = tb.live && (FZ || a.ctl[tb.tr].active);
     double err = 0.0;
-    if (i <= a.d.n) {
-        const float* cr = a.c + tr * a.d.L;
-        float sum = 0.f;
-        sum = sum_run(sum, cr, a.d.csr_ptr[i], a.d.csr_ptr[i + 1]);
-        const float kj = sum;
-        const long long o = row + i;
+    if (run && i <= a.d.n) {
+        const double h = FZ ? a.hcol[tb.tr] : a.ctl[tb.tr].h;
+        const double hnext = FZ ? h : a.ctl[tb.tr].hnext;
+        const float hs = (float)h;
+        const long long o = tb.at(i);
+        const float kj = tile_sum<float>(a.c + tb.l, a.d.csr_ptr[i], a.d.csr_ptr[i + 1], tb.tp);
         const float xi = a.X[o];
         // stage J+1's spin input goes to S, or to Y_{J+1} in a frozen step
         float* nxt = FZ ? a.Y + J * a.V : a.S;
@@ -548,8 +622,9 @@ __global__ __launch_bounds__(BLK) void k_fvar(FArgs a)
         }
     }
     if constexpr (J == 6 && !FZ) {
-        const double bm = block_max<BLK>(err, sh);
-        if (threadIdx.x == 0) a.parts[tr * (a.nblk_c + a.nblk_v) + a.nblk_c + tb.x] = bm;
+        const double bm = tile_max(err, tb.tp, sh);
+        if ((int)threadIdx.x < tb.tp && run && tb.x < a.nblk_v)
+            a.parts[(long long)tb.tr * (a.nblk_c + a.nblk_v) + a.nblk_c + tb.x] = bm;
     }
 }
 
@@ -563,18 +638,18 @@ struct Adj {
     bool have_problem = false, have_forward = false;
     std::vector<int> lits_in, lens_in;
     hipStream_t stream = nullptr;
-    int *d_lit = nullptr, *d_csr_ptr = nullptr, *d_csr_slot = nullptr, *d_slot_pos = nullptr;
-    // per batch
-    float* ckpt = nullptr;       // [ncheck][ntraj][D]
-    float* seg = nullptr;        // [C+1][ntraj][D]
-    float* Y = nullptr;          // [6][ntraj][D]
-    float* Yseg = nullptr;       // [C][6][ntraj][D] stage inputs of a segment's steps (backward)
-    float* kk = nullptr;         // [6][ntraj][D]
-    float* c32 = nullptr;        // [ntraj][L]
-    double* c64 = nullptr;       // [ntraj][L]
-    double* lam = nullptr;       // [ntraj][D]
-    double* mu = nullptr;        // [ntraj][D]
-    double* nu = nullptr;        // [6][ntraj][D]
+    int *d_lit = nullptr, *d_csr_ptr = nullptr, *d_slot_pos = nullptr;
+    // per batch; "vectors" and "terms": of all trajectories, in tiles
+    float* ckpt = nullptr;       // ncheck vectors
+    float* seg = nullptr;        // C + 1 vectors
+    float* Y = nullptr;          // 6 vectors
+    float* Yseg = nullptr;       // 6 C vectors, stage inputs of a segment's steps (backward)
+    float* kk = nullptr;         // 6 vectors
+    float* c32 = nullptr;        // terms
+    double* c64 = nullptr;       // terms
+    double* lam = nullptr;       // vector
+    double* mu = nullptr;        // vector (the spins' part; also the stage of imports and exports)
+    double* nu = nullptr;        // 6 vectors
     double* hlog = nullptr;      // [ntraj][T]
     double* hcol = nullptr;      // [T][ntraj] step sizes by step
     double* hcolr = nullptr;     // [T][ntraj] FP32-rounded step sizes (adjoint)
@@ -586,6 +661,7 @@ struct Adj {
     double* hstep = nullptr;     // [ntraj] current attempt's step size
     double* eparts = nullptr;    // [ntraj][nblk] error-norm block maxima
     int ncheck = 0;
+    int buf_T = -1, buf_C = -1;   // step and checkpoint counts the buffers were made for
     double fwd_ms = 0, bwd_ms = 0;
     long long fwd_attempts = 0;   // forward: attempts summed over the trajectories
     long long fwd_lockstep = 0;   // forward: lockstep attempts launched
@@ -603,10 +679,21 @@ struct Adj {
     ~Adj()
     {
         free_batch();
-        (void)hipFree(d_lit); (void)hipFree(d_csr_ptr); (void)hipFree(d_csr_slot); (void)hipFree(d_slot_pos);
+        (void)hipFree(d_lit); (void)hipFree(d_csr_ptr); (void)hipFree(d_slot_pos);
         if (stream) (void)hipStreamDestroy(stream);
     }
-    Dev dev() const { return Dev{d_lit, d_csr_ptr, d_csr_slot, d_slot_pos, n, m, k, D, L, ntraj}; }
+    int sh() const { return tile_shift(ntraj, L); }
+    int tiles() const { return ceil_div(ntraj, 1 << sh()); }
+    Dev dev() const { return Dev{d_lit, d_csr_ptr, d_slot_pos, n, m, k, D, L, ntraj, sh(), tile_xcds(tiles())}; }
+    // elements of a vector of all trajectories, and of its slot terms (whole tiles)
+    size_t vec() const { return (size_t)tiles() * D << sh(); }
+    size_t terms() const { return (size_t)tiles() * L << sh(); }
+    // one thread per element and trajectory
+    int blocks(long long elems) const { return ceil_div(elems << sh(), BLK); }
+    dim3 grid(long long elems) const
+    {
+        return dim3(ceil_div(blocks(elems), 1 << tile_xcds(tiles())), (tiles() + 7) / 8 * 8);
+    }
 };
 
 static void set_problem(Adj& A, const int* lits, const int* lens, int nclauses)
@@ -640,24 +727,19 @@ static void set_problem(Adj& A, const int* lits, const int* lens, int nclauses)
     // var-major position of every slot: variables in order, each variable's
     // slots ascending (the reference's accumulation order)
     std::vector<int> spos(std::max<size_t>(C.size(), 1), -1);
-    std::vector<int> slot(std::max(ptr[n + 1], 1));
     std::vector<int> fill(ptr.begin(), ptr.end() - 1);
     for (size_t s = 0; s < C.size(); s++)
-        if (C[s]) {
-            spos[s] = fill[std::abs(C[s])]++;
-            slot[(size_t)spos[s]] = (int)s;
-        }
+        if (C[s]) spos[s] = fill[std::abs(C[s])]++;
     if (!A.stream) HIP_CHECK(hipStreamCreateWithFlags(&A.stream, hipStreamNonBlocking));
     HIP_CHECK(hipStreamSynchronize(A.stream));
     A.free_batch();
-    (void)hipFree(A.d_lit); (void)hipFree(A.d_csr_ptr); (void)hipFree(A.d_csr_slot); (void)hipFree(A.d_slot_pos);
+    (void)hipFree(A.d_lit); (void)hipFree(A.d_csr_ptr); (void)hipFree(A.d_slot_pos);
+    A.d_lit = A.d_csr_ptr = A.d_slot_pos = nullptr;
     HIP_CHECK(hipMalloc((void**)&A.d_lit, sizeof(int) * C.size()));
     HIP_CHECK(hipMalloc((void**)&A.d_csr_ptr, sizeof(int) * ptr.size()));
-    HIP_CHECK(hipMalloc((void**)&A.d_csr_slot, sizeof(int) * slot.size()));
     HIP_CHECK(hipMalloc((void**)&A.d_slot_pos, sizeof(int) * spos.size()));
     HIP_CHECK(hipMemcpy(A.d_lit, C.data(), sizeof(int) * C.size(), hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(A.d_csr_ptr, ptr.data(), sizeof(int) * ptr.size(), hipMemcpyHostToDevice));
-    HIP_CHECK(hipMemcpy(A.d_csr_slot, slot.data(), sizeof(int) * slot.size(), hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(A.d_slot_pos, spos.data(), sizeof(int) * spos.size(), hipMemcpyHostToDevice));
     A.n = n; A.m = m; A.k = k;
     A.D = (long long)((n + m + 1 + 63) / 64) * 64;
@@ -668,35 +750,67 @@ static void set_problem(Adj& A, const int* lits, const int* lens, int nclauses)
     A.have_forward = false;
 }
 
+// buffers for ntraj trajectories, kept while the problem, the number of
+// trajectories and the step and checkpoint counts stay the same (3.3 GB at
+// N = 1e4, M = 42 500, 64 trajectories, checkpoints every 32)
 static void alloc_batch(Adj& A, int ntraj)
 {
+    A.have_forward = false;
+    const int nc = (A.T + A.C - 1) / A.C + 1;
+    if (A.ckpt && A.ntraj == ntraj && A.buf_T == A.T && A.buf_C == A.C) return;
+    HIP_CHECK(hipStreamSynchronize(A.stream));
     A.free_batch();
     A.ntraj = ntraj;
-    A.ncheck = (A.T + A.C - 1) / A.C + 1;
-    const size_t V = (size_t)ntraj * A.D;
-    HIP_CHECK(hipMalloc((void**)&A.ckpt, sizeof(float) * V * A.ncheck));
+    A.ncheck = nc;
+    A.buf_T = A.T;
+    A.buf_C = A.C;
+    const size_t V = A.vec();
     HIP_CHECK(hipMalloc((void**)&A.seg, sizeof(float) * V * (A.C + 1)));
     HIP_CHECK(hipMalloc((void**)&A.Y, sizeof(float) * V * 6));
     HIP_CHECK(hipMalloc((void**)&A.Yseg, sizeof(float) * V * 6 * A.C));
     HIP_CHECK(hipMalloc((void**)&A.kk, sizeof(float) * V * 6));
-    HIP_CHECK(hipMalloc((void**)&A.c32, sizeof(float) * (size_t)ntraj * A.L));
-    HIP_CHECK(hipMalloc((void**)&A.c64, sizeof(double) * (size_t)ntraj * A.L));
+    HIP_CHECK(hipMalloc((void**)&A.c32, sizeof(float) * A.terms()));
+    HIP_CHECK(hipMalloc((void**)&A.c64, sizeof(double) * A.terms()));
     HIP_CHECK(hipMalloc((void**)&A.lam, sizeof(double) * V));
     HIP_CHECK(hipMalloc((void**)&A.mu, sizeof(double) * V));
     HIP_CHECK(hipMalloc((void**)&A.nu, sizeof(double) * V * 6));
     HIP_CHECK(hipMalloc((void**)&A.hlog, sizeof(double) * (size_t)ntraj * std::max(A.T, 1)));
     HIP_CHECK(hipMalloc((void**)&A.hcol, sizeof(double) * (size_t)ntraj * std::max(A.T, 1)));
     HIP_CHECK(hipMalloc((void**)&A.hcolr, sizeof(double) * (size_t)ntraj * std::max(A.T, 1)));
-    const int nblk = ceil_div(A.m, BLK);
-    HIP_CHECK(hipMalloc((void**)&A.vpart, sizeof(double) * (size_t)ntraj * nblk));
+    const int nblk = A.blocks(A.m), nblkv = A.blocks(A.n);
+    HIP_CHECK(hipMalloc((void**)&A.vpart, sizeof(double) * (size_t)ntraj * ceil_div(A.m, BLK)));
     HIP_CHECK(hipMalloc((void**)&A.dV, sizeof(double) * ntraj));
     HIP_CHECK(hipMalloc((void**)&A.ctl, sizeof(TCtl) * ntraj));
     HIP_CHECK(hipMalloc((void**)&A.hstep, sizeof(double) * ntraj));
-    HIP_CHECK(hipMalloc((void**)&A.eparts, sizeof(double) * (size_t)ntraj * (ceil_div(A.m, BLK) + ceil_div(A.n, BLK))));
+    HIP_CHECK(hipMalloc((void**)&A.eparts, sizeof(double) * (size_t)ntraj * (nblk + nblkv)));
     HIP_CHECK(hipMemset(A.seg, 0, sizeof(float) * V * (A.C + 1)));
     HIP_CHECK(hipMemset(A.Y, 0, sizeof(float) * V * 6));
     HIP_CHECK(hipMemset(A.kk, 0, sizeof(float) * V * 6));
+    HIP_CHECK(hipMemset(A.lam, 0, sizeof(double) * V));
+    // the last one: its presence says that all are there
+    HIP_CHECK(hipMalloc((void**)&A.ckpt, sizeof(float) * V * A.ncheck));
     HIP_CHECK(hipMemset(A.ckpt, 0, sizeof(float) * V * A.ncheck));
+}
+
+// start states, public rows on the host, into x; stage: ntraj (n + m) values on
+// the device for the copy in between
+template <typename T>
+static void import_rows(Adj& A, const T* pub, T* stage, T* x)
+{
+    HIP_CHECK(hipMemcpyAsync(stage, pub, sizeof(T) * (size_t)A.ntraj * (A.n + A.m), hipMemcpyHostToDevice, A.stream));
+    hipLaunchKernelGGL(k_import<T>, A.grid((long long)A.n + A.m + 1), dim3(BLK), 0, A.stream, A.dev(), (const T*)stage,
+                       (T)-1.0, x);
+    HIP_CHECK(hipGetLastError());
+}
+
+// and a vector back to public rows on the host
+template <typename T>
+static void export_rows(Adj& A, const T* x, T* stage, T* pub)
+{
+    hipLaunchKernelGGL(k_export<T>, A.grid((long long)A.n + A.m), dim3(BLK), 0, A.stream, A.dev(), x, stage);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipMemcpyAsync(pub, stage, sizeof(T) * (size_t)A.ntraj * (A.n + A.m), hipMemcpyDeviceToHost, A.stream));
+    HIP_CHECK(hipStreamSynchronize(A.stream));
 }
 
 // f = RHS(Y) for all trajectories (FP32, forward arithmetic)
@@ -704,7 +818,7 @@ template <typename T>
 static void rhs_all(Adj& A, const T* Yv, T* out, T* contrib)
 {
     const Dev d = A.dev();
-    dim3 gc(ceil_div(A.m, BLK), ntraj8(A.ntraj)), gv(ceil_div(A.n, BLK), ntraj8(A.ntraj));
+    const dim3 gc = A.grid(A.m), gv = A.grid(A.n);
     if (A.k == 3) hipLaunchKernelGGL((k_rhs_clause<T, 3>), gc, dim3(BLK), 0, A.stream, d, Yv, out, contrib);
     else hipLaunchKernelGGL((k_rhs_clause<T, 4>), gc, dim3(BLK), 0, A.stream, d, Yv, out, contrib);
     hipLaunchKernelGGL(k_rhs_var<T>, gv, dim3(BLK), 0, A.stream, d, (const T*)contrib, out);
@@ -716,11 +830,11 @@ template <typename T>
 static void frozen_step(Adj& A, const T* X, T* Xn, T* Y, T* kk, T* contrib)
 {
     const Dev d = A.dev();
-    const size_t V = (size_t)A.ntraj * A.D;
+    const size_t V = A.vec();
     T* Yl[6];
     T* kl[6];
     for (int i = 0; i < 6; i++) { Yl[i] = Y + i * V; kl[i] = kk + i * V; }
-    dim3 ge(ceil_div((long long)A.n + A.m, BLK), ntraj8(A.ntraj));
+    const dim3 ge = A.grid((long long)A.n + A.m);
     HIP_CHECK(hipMemcpyAsync(Yl[0], X, sizeof(T) * V, hipMemcpyDeviceToDevice, A.stream));
     rhs_all<T>(A, Yl[0], kl[0], contrib);
     hipLaunchKernelGGL((k_stage<T, 2>), ge, dim3(BLK), 0, A.stream, d, X, kl[0], kl[1], kl[2], kl[3], kl[4], A.hcur, Yl[1]);
@@ -734,7 +848,7 @@ static void frozen_step(Adj& A, const T* X, T* Xn, T* Y, T* kk, T* contrib)
     hipLaunchKernelGGL((k_stage<T, 6>), ge, dim3(BLK), 0, A.stream, d, X, kl[0], kl[1], kl[2], kl[3], kl[4], A.hcur, Yl[5]);
     rhs_all<T>(A, Yl[5], kl[5], contrib);
     if (Xn) {
-        dim3 gf(ceil_div((long long)A.n + A.m + 1, BLK), ntraj8(A.ntraj));
+        const dim3 gf = A.grid((long long)A.n + A.m + 1);
         hipLaunchKernelGGL(k_final<T>, gf, dim3(BLK), 0, A.stream, d, X, kl[0], kl[2], kl[3], kl[5], A.hcur, Xn);
     }
 }
@@ -746,14 +860,13 @@ static void energy(Adj& A, const TX* X, bool want_grad)
 {
     const Dev d = A.dev();
     const int nblk = ceil_div(A.m, BLK);
-    dim3 gc(nblk, ntraj8(A.ntraj)), gv(ceil_div(A.n, BLK), ntraj8(A.ntraj));
+    double* vc = A.nu;   // free outside a backward step
+    const dim3 gc = A.grid(A.m), gv = A.grid(A.n);
     double* g = A.lam;
-    if (A.k == 3) hipLaunchKernelGGL((k_gradv_clause<TX, 3>), gc, dim3(BLK), 0, A.stream, d, X, g, A.c64, A.vpart, nblk);
-    else hipLaunchKernelGGL((k_gradv_clause<TX, 4>), gc, dim3(BLK), 0, A.stream, d, X, g, A.c64, A.vpart, nblk);
-    if (want_grad) {
-        hipLaunchKernelGGL(k_rhs_var<double>, gv, dim3(BLK), 0, A.stream, d, (const double*)A.c64, g);
-        hipLaunchKernelGGL(k_zero_slot0, dim3(ceil_div(A.ntraj, 64)), dim3(64), 0, A.stream, g, A.D, A.ntraj);
-    }
+    if (A.k == 3) hipLaunchKernelGGL((k_gradv_clause<TX, 3>), gc, dim3(BLK), 0, A.stream, d, X, g, A.c64, vc);
+    else hipLaunchKernelGGL((k_gradv_clause<TX, 4>), gc, dim3(BLK), 0, A.stream, d, X, g, A.c64, vc);
+    if (want_grad) hipLaunchKernelGGL(k_rhs_var<double>, gv, dim3(BLK), 0, A.stream, d, (const double*)A.c64, g);
+    hipLaunchKernelGGL(k_v_blocks, dim3(nblk, A.ntraj), dim3(BLK), 0, A.stream, d, (const double*)vc, A.vpart);
     hipLaunchKernelGGL(k_sum_parts, dim3(A.ntraj), dim3(64), 0, A.stream, (const double*)A.vpart, nblk, A.dV);
 }
 
@@ -761,7 +874,7 @@ static void energy(Adj& A, const TX* X, bool want_grad)
 template <int K, bool FZ>
 static void fused_stages(Adj& A, const FArgs& fa)
 {
-    const dim3 gc(fa.nblk_c, ntraj8(A.ntraj)), gv(fa.nblk_v, ntraj8(A.ntraj));
+    const dim3 gc = A.grid(A.m), gv = A.grid(A.n);
     hipLaunchKernelGGL((k_fclause<K, 1, FZ>), gc, dim3(BLK), 0, A.stream, fa);
     hipLaunchKernelGGL((k_fvar<1, FZ>), gv, dim3(BLK), 0, A.stream, fa);
     hipLaunchKernelGGL((k_fclause<K, 2, FZ>), gc, dim3(BLK), 0, A.stream, fa);
@@ -783,12 +896,12 @@ static FArgs fused_args(Adj& A, const float* X, float* Xn)
     fa.d = A.dev();
     fa.X = X;
     fa.Xn = Xn;
-    const size_t V = (size_t)A.ntraj * A.D;
+    const size_t V = A.vec();
     for (int i = 0; i < 6; i++) fa.k[i] = A.kk + i * V;
     fa.V = (long long)V;
     fa.c = A.c32;
-    fa.nblk_c = ceil_div(A.m, BLK);
-    fa.nblk_v = ceil_div(A.n, BLK);
+    fa.nblk_c = A.blocks(A.m);
+    fa.nblk_v = A.blocks(A.n);
     return fa;
 }
 
@@ -806,18 +919,18 @@ static void frozen_step_fused(Adj& A, const float* X, float* Xn, float* Y)
 
 // Adaptive forward of every trajectory in lockstep: T accepted steps each,
 // step sizes logged in hlog, checkpoints c = 0..ceil(T/C) (x at step c*C,
-// the last one x_T).  X0 holds the start states in the internal layout.
-static void forward_lockstep(Adj& A, const std::vector<float>& X0)
+// the last one x_T).
+static void forward_lockstep(Adj& A, const float* pub0)
 {
     const Dev d = A.dev();
-    const size_t V = (size_t)A.ntraj * A.D;
+    const size_t V = A.vec();
     float* X = A.seg;          // seg has C + 1 >= 2 slots
     float* Xn = A.seg + V;
-    HIP_CHECK(hipMemcpyAsync(X, X0.data(), sizeof(float) * V, hipMemcpyHostToDevice, A.stream));
+    import_rows<float>(A, pub0, (float*)A.mu, X);
     HIP_CHECK(hipMemcpyAsync(A.ckpt, X, sizeof(float) * V, hipMemcpyDeviceToDevice, A.stream));
     hipLaunchKernelGGL(k_ctl_init, dim3(ceil_div(A.ntraj, 64)), dim3(64), 0, A.stream, A.ctl, A.hstep, A.ntraj);
     A.hcur = A.hstep;
-    const dim3 ge(ceil_div((long long)A.n + A.m + 1, BLK), ntraj8(A.ntraj));
+    const dim3 ge = A.grid((long long)A.n + A.m + 1);
     FArgs fa = fused_args(A, X, Xn);
     fa.S = A.Y;
     fa.ctl = A.ctl;
@@ -833,7 +946,7 @@ static void forward_lockstep(Adj& A, const std::vector<float>& X0)
             hipLaunchKernelGGL(k_ctl_batch, dim3(A.ntraj), dim3(BLK), 0, A.stream, A.ctl, (const double*)A.eparts,
                                nblk, A.eps, A.T, A.C, A.hlog, A.hstep);
             hipLaunchKernelGGL(k_accept, ge, dim3(BLK), 0, A.stream, d, (const TCtl*)A.ctl, (const float*)Xn, X,
-                               A.ckpt, (long long)A.ntraj);
+                               A.ckpt, (long long)V);
         }
         HIP_CHECK(hipGetLastError());
         HIP_CHECK(hipMemcpyAsync(hc.data(), A.ctl, sizeof(TCtl) * hc.size(), hipMemcpyDeviceToHost, A.stream));
@@ -876,6 +989,25 @@ static void load_h(Adj& A, int s)
 {
     A.hcur = A.hcol + (size_t)s * A.ntraj;
     A.hcurr = A.hcolr + (size_t)s * A.ntraj;
+}
+
+// nu_l of one step for every trajectory: mu_l of the spins, the clauses' products,
+// the variables' sums.  Ys: the step's six stage inputs.
+template <int LL>
+static void vjp_stage(Adj& A, const Dev& d, const float* Ys)
+{
+    const size_t V = A.vec();
+    double* nul = A.nu + (size_t)(LL - 1) * V;
+    const float* Yl = Ys + (size_t)(LL - 1) * V;
+    hipLaunchKernelGGL(k_mu<LL>, A.grid((long long)A.n + 1), dim3(BLK), 0, A.stream, d, (const double*)A.lam,
+                       (const double*)A.nu, (long long)V, A.hcurr, A.mu);
+    if (A.k == 3)
+        hipLaunchKernelGGL((k_vjp_clause<3, LL>), A.grid(A.m), dim3(BLK), 0, A.stream, d, Yl, (const double*)A.mu,
+                           (const double*)A.lam, A.nu, (long long)V, A.hcurr, A.c64);
+    else
+        hipLaunchKernelGGL((k_vjp_clause<4, LL>), A.grid(A.m), dim3(BLK), 0, A.stream, d, Yl, (const double*)A.mu,
+                           (const double*)A.lam, A.nu, (long long)V, A.hcurr, A.c64);
+    hipLaunchKernelGGL(k_rhs_var<double>, A.grid(A.n), dim3(BLK), 0, A.stream, d, (const double*)A.c64, nul);
 }
 
 }  // namespace adj
@@ -949,13 +1081,8 @@ int asat_adj_forward(asat_adj_t* a, int ntraj, const float* pub0, double* V_out)
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
     HIP_CHECK(hipEventRecord(e0, A.stream));
-    const size_t V = (size_t)A.ntraj * A.D;
-    std::vector<float> x0(V, 0.f);
-    for (int t = 0; t < ntraj; t++) {
-        x0[(size_t)t * A.D] = -1.0f;
-        std::copy(pub0 + (size_t)t * (A.n + A.m), pub0 + (size_t)(t + 1) * (A.n + A.m), x0.begin() + (size_t)t * A.D + 1);
-    }
-    forward_lockstep(A, x0);
+    const size_t V = A.vec();
+    forward_lockstep(A, pub0);
     make_columns(A);
     // V(T) from the last checkpoint (= x_T)
     const int last = (A.T + A.C - 1) / A.C;
@@ -988,15 +1115,10 @@ int asat_adj_replay(asat_adj_t* a, int ntraj, const float* pub0, const double* h
     Adj& A = a->a;
     require(A.have_problem && A.T > 0, ASAT_ERR_NOT_CONFIGURED, "adjoint problem/parameters not set");
     alloc_batch(A, ntraj);
-    const size_t V = (size_t)ntraj * A.D;
+    const size_t V = A.vec();
     HIP_CHECK(hipMemcpy(A.hlog, h, sizeof(double) * (size_t)ntraj * A.T, hipMemcpyHostToDevice));
     make_columns(A);
-    std::vector<float> x0(V, 0.f);
-    for (int t = 0; t < ntraj; t++) {
-        x0[(size_t)t * A.D] = -1.0f;
-        std::copy(pub0 + (size_t)t * (A.n + A.m), pub0 + (size_t)(t + 1) * (A.n + A.m), x0.begin() + (size_t)t * A.D + 1);
-    }
-    HIP_CHECK(hipMemcpy(A.seg, x0.data(), sizeof(float) * V, hipMemcpyHostToDevice));
+    import_rows<float>(A, pub0, (float*)A.mu, A.seg);
     float* cur = A.seg;
     float* nxt = A.seg + V;
     for (int s = 0; s < A.T; s++) {
@@ -1007,13 +1129,7 @@ int asat_adj_replay(asat_adj_t* a, int ntraj, const float* pub0, const double* h
     energy(A, cur, false);
     HIP_CHECK(hipStreamSynchronize(A.stream));
     if (V_out) HIP_CHECK(hipMemcpy(V_out, A.dV, sizeof(double) * ntraj, hipMemcpyDeviceToHost));
-    if (xT_out) {
-        std::vector<float> xt(V);
-        HIP_CHECK(hipMemcpy(xt.data(), cur, sizeof(float) * V, hipMemcpyDeviceToHost));
-        for (int t = 0; t < ntraj; t++)
-            std::copy(xt.begin() + (size_t)t * A.D + 1, xt.begin() + (size_t)t * A.D + 1 + A.n + A.m,
-                      xT_out + (size_t)t * (A.n + A.m));
-    }
+    if (xT_out) export_rows<float>(A, cur, (float*)A.mu, xT_out);
     A.have_forward = false;
     AAPI_END
 }
@@ -1025,20 +1141,15 @@ int asat_adj_replay_f64(asat_adj_t* a, int ntraj, const double* pub0, const doub
     Adj& A = a->a;
     require(A.have_problem && A.T > 0, ASAT_ERR_NOT_CONFIGURED, "adjoint problem/parameters not set");
     alloc_batch(A, ntraj);
-    const size_t V = (size_t)ntraj * A.D;
+    const size_t V = A.vec();
     HIP_CHECK(hipMemcpy(A.hlog, h, sizeof(double) * (size_t)ntraj * A.T, hipMemcpyHostToDevice));
     make_columns(A);
-    std::vector<double> x0(V, 0.0);
-    for (int t = 0; t < ntraj; t++) {
-        x0[(size_t)t * A.D] = -1.0;
-        std::copy(pub0 + (size_t)t * (A.n + A.m), pub0 + (size_t)(t + 1) * (A.n + A.m), x0.begin() + (size_t)t * A.D + 1);
-    }
     // FP64 state: the current and next state, six stage inputs, six stage derivatives
     double* buf = nullptr;
     HIP_CHECK(hipMalloc((void**)&buf, sizeof(double) * V * 14));
     double* cur = buf;
     double* nxt = buf + V;
-    HIP_CHECK(hipMemcpy(cur, x0.data(), sizeof(double) * V, hipMemcpyHostToDevice));
+    import_rows<double>(A, pub0, A.mu, cur);
     for (int s = 0; s < A.T; s++) {
         load_h(A, s);
         frozen_step<double>(A, cur, nxt, buf + 2 * V, buf + 8 * V, A.c64);
@@ -1059,7 +1170,7 @@ int asat_adj_backward(asat_adj_t* a, double* grad_out)
     Adj& A = a->a;
     require(A.have_forward, ASAT_ERR_NOT_CONFIGURED, "asat_adj_forward must run first");
     const Dev d = A.dev();
-    const size_t V = (size_t)A.ntraj * A.D;
+    const size_t V = A.vec();
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
@@ -1067,8 +1178,7 @@ int asat_adj_backward(asat_adj_t* a, double* grad_out)
     const int nseg = (A.T + A.C - 1) / A.C;
     // lam = grad V(x_T)
     energy(A, A.ckpt + (size_t)nseg * V, true);
-    dim3 ge(ceil_div((long long)A.n + A.m + 1, BLK), ntraj8(A.ntraj)), ge1(ceil_div((long long)A.n + A.m, BLK), ntraj8(A.ntraj));
-    dim3 gc(ceil_div(A.m, BLK), ntraj8(A.ntraj)), gv(ceil_div(A.n, BLK), ntraj8(A.ntraj));
+    const dim3 ge = A.grid((long long)A.n + A.m), gv = A.grid(A.n);
     for (int sg = nseg - 1; sg >= 0; sg--) {
         const int s0 = sg * A.C, s1 = std::min(A.T, s0 + A.C);
         // recompute the segment's states from its checkpoint
@@ -1081,16 +1191,10 @@ int asat_adj_backward(asat_adj_t* a, double* grad_out)
         }
         for (int s = s1 - 1; s >= s0; s--) {
             load_h(A, s);
-            for (int l = 6; l >= 1; l--) {
-                hipLaunchKernelGGL(k_mu, ge, dim3(BLK), 0, A.stream, d, l, (const double*)A.lam,
-                                   (const double*)A.nu, A.hcurr, A.mu);
-                double* nul = A.nu + (size_t)(l - 1) * V;
-                const float* Yl = A.Yseg + ((size_t)(s - s0) * 6 + (l - 1)) * V;
-                if (A.k == 3) hipLaunchKernelGGL(k_vjp_clause<3>, gc, dim3(BLK), 0, A.stream, d, Yl, (const double*)A.mu, nul, A.c64);
-                else hipLaunchKernelGGL(k_vjp_clause<4>, gc, dim3(BLK), 0, A.stream, d, Yl, (const double*)A.mu, nul, A.c64);
-                hipLaunchKernelGGL(k_rhs_var<double>, gv, dim3(BLK), 0, A.stream, d, (const double*)A.c64, nul);
-            }
-            hipLaunchKernelGGL(k_lam, ge1, dim3(BLK), 0, A.stream, d, A.lam, (const double*)A.nu);
+            const float* Ys = A.Yseg + (size_t)(s - s0) * 6 * V;
+            vjp_stage<6>(A, d, Ys); vjp_stage<5>(A, d, Ys); vjp_stage<4>(A, d, Ys);
+            vjp_stage<3>(A, d, Ys); vjp_stage<2>(A, d, Ys); vjp_stage<1>(A, d, Ys);
+            hipLaunchKernelGGL(k_lam, ge, dim3(BLK), 0, A.stream, d, A.lam, (const double*)A.nu, (long long)V);
         }
     }
     HIP_CHECK(hipGetLastError());
@@ -1101,11 +1205,7 @@ int asat_adj_backward(asat_adj_t* a, double* grad_out)
     A.bwd_ms = ms;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    std::vector<double> lam(V);
-    HIP_CHECK(hipMemcpy(lam.data(), A.lam, sizeof(double) * V, hipMemcpyDeviceToHost));
-    for (int t = 0; t < A.ntraj; t++)
-        std::copy(lam.begin() + (size_t)t * A.D + 1, lam.begin() + (size_t)t * A.D + 1 + A.n + A.m,
-                  grad_out + (size_t)t * (A.n + A.m));
+    export_rows<double>(A, A.lam, A.mu, grad_out);
     AAPI_END
 }
 
