@@ -24,8 +24,9 @@
 //                     to the tile's first (pv0), the primary literal's position
 //                     and sign, in place of pvar and the primary slots' ranks
 //   csr_ptr[0..N+1]   var-major CSR row pointers
-//   csr_loc[e]        uint16 offset of each of a variable's contributions in
-//                     its group's region, in slot order
+//   rloc, ploc        uint16 per region entry, and per clause for its direct
+//                     primary term: its place in the group's var-major slot
+//                     list (variables in order, each one's slots in slot order)
 //   state buffer      [ -1, s_1..s_N, pad | a_1..a_M, pad ], aux at aoff
 //   k1..k5            same layout as the state (stage derivatives)
 //   tmp               spin part of the next stage's input (aux stage inputs are
@@ -84,6 +85,7 @@ constexpr int TC_MAX = TC_BIG;
 constexpr unsigned PW_VMASK = 0x1FFFu;    // big tiles' primary words: relative variable bits,
 constexpr int PW_QSHIFT = 13;             // then the primary literal's position, then its sign
 constexpr int TILE_BT = 1024;             // threads per tile workgroup (a clause each)
+constexpr int VAR_SUM = 8;              // terms of a variable in flight in the var pass
 constexpr int VBLK = 1024;                // var-pass workgroup (one variable group)
 constexpr int VAR_LDS_BYTES = 147456;     // LDS holding one group's contribution region
 constexpr int VAR_LDS_CU = 163840 - 1024; // LDS two var workgroups may share on one CU
@@ -103,7 +105,7 @@ struct HostProblem {
     std::vector<int> pos;          // m*k: the slot's contribution position, -1 for padding
     std::vector<int> csr_ptr;      // n+2
     std::vector<int> csr_pos;      // contribution positions of each variable, in slot order
-    std::vector<uint16_t> csr_loc; // the same relative to the variable's region start
+    std::vector<uint16_t> csr_loc; // the same relative to the variable's region start (primary terms past its end)
     // tiled clause pass: per tile of TC clauses, its slots sorted by position
     std::vector<int> spos;         // ntiles*TC*k positions (-1 past the tile's last slot)
     // big tiles: per tile, a run table in place of spos.
@@ -301,104 +303,6 @@ static void build_layout(HostProblem& P, int vg, int pv)
     }
 }
 
-// Big tiles: a tile's slots of one group may hold the run's positions in any
-// order (ranks follow positions, and the var pass adds each variable's terms
-// in the order of its offset list, whatever the positions).  The var pass
-// reads the k-th list entry of each of a wave's variables with one LDS
-// instruction, and writes the slot spins back the same way; entries of such
-// a read that share an LDS bank serialise.  Greedy, run by run: each slot
-// takes the free position whose bank its (wave, k) bucket has used least,
-// counting the group's primary entries (fixed, behind the region) first.
-// Banks are counted modulo 32 (a wave's access served as two 32-lane
-// halves); modulo 64 measured the same within noise.  N = 1e6: the six var
-// passes 172.6 -> 169.8 us per attempt, 2331 -> 2342 attempts/s.
-constexpr int LDS_BANKS = 32;
-static void spread_run_banks(HostProblem& P, int pv)
-{
-    const int K = P.k, vg = P.vg, n = P.n, m = P.m;
-    const size_t per = (size_t)P.tc * K;
-    const size_t L = P.lit.size();
-    std::vector<int> row((size_t)m);
-    for (int j = 0; j < m; j++) row[P.perm.empty() ? j : P.perm[j]] = j;
-    // each slot's index in its variable's list (the reference's order)
-    std::vector<int> kidx(L, 0);
-    {
-        std::vector<int> fill((size_t)n + 1, 0);
-        for (int mo = 0; mo < m; mo++)
-            for (int q = 0; q < K; q++) {
-                const size_t sl = (size_t)row[mo] * K + q;
-                const int l = P.lit[sl];
-                if (l) kidx[sl] = fill[(size_t)std::abs(l)]++;
-            }
-    }
-    int kmax = 1;
-    for (int v = 1; v <= n; v++) kmax = std::max(kmax, P.csr_ptr[(size_t)v + 1] - P.csr_ptr[v]);
-    // a variable's wave in its group's var workgroup (VBLK threads, a
-    // variable each, the group's later variables in further passes)
-    const int waves_pass = VBLK / 64;
-    const int nw = ceil_div(vg, VBLK) * waves_pass;
-    auto wave_of = [&](int v) {
-        const int lv = (v - 1) % vg;
-        return (lv / VBLK) * waves_pass + (lv % VBLK) / 64;
-    };
-    // the groups' non-primary slots, in slot order
-    std::vector<long long> gofs((size_t)P.ngroups + 1, 0);
-    for (size_t sl = 0; sl < L; sl++)
-        if (P.lit[sl] && P.pos[sl] >= 0) gofs[(size_t)(std::abs(P.lit[sl]) - 1) / vg + 1]++;
-    for (int g = 0; g < P.ngroups; g++) gofs[(size_t)g + 1] += gofs[g];
-    std::vector<int> gsl((size_t)gofs[P.ngroups]);
-    {
-        std::vector<long long> f(gofs.begin(), gofs.end() - 1);
-        for (size_t sl = 0; sl < L; sl++)
-            if (P.lit[sl] && P.pos[sl] >= 0) gsl[(size_t)f[(size_t)(std::abs(P.lit[sl]) - 1) / vg]++] = (int)sl;
-    }
-    std::vector<uint16_t> used((size_t)nw * kmax * LDS_BANKS);
-    std::vector<int> cand;
-    for (int g = 0; g < P.ngroups; g++) {
-        std::fill(used.begin(), used.end(), (uint16_t)0);
-        const long long rlen = P.gstart[(size_t)g + 1] - P.gstart[g];
-        const int pb = P.pc0[g] / pv * pv;
-        for (int j = P.pc0[g]; j < P.pc0[(size_t)g + 1]; j++) {
-            const size_t sl = (size_t)j * K + P.pq[(size_t)j];
-            const long long off = rlen + j - pb;
-            used[((size_t)wave_of(P.pvar[(size_t)j]) * kmax + kidx[sl]) * LDS_BANKS + (size_t)(off % LDS_BANKS)]++;
-        }
-        for (long long a = gofs[g]; a < gofs[(size_t)g + 1];) {
-            // one run: the group's slots of one tile, positions p0 .. p0+c-1
-            const size_t t = (size_t)gsl[(size_t)a] / per;
-            long long b = a;
-            int p0 = INT_MAX;
-            while (b < gofs[(size_t)g + 1] && (size_t)gsl[(size_t)b] / per == t) p0 = std::min(p0, P.pos[(size_t)gsl[(size_t)b++]]);
-            const int c = (int)(b - a);
-            cand.assign((size_t)c, 1);
-            for (long long e = a; e < b; e++) {
-                const size_t sl = (size_t)gsl[(size_t)e];
-                const int v = std::abs(P.lit[sl]);
-                uint16_t* u = &used[((size_t)wave_of(v) * kmax + kidx[sl]) * LDS_BANKS];
-                int best = -1;
-                for (int i = 0; i < c; i++) {
-                    if (!cand[(size_t)i]) continue;
-                    const long long off = p0 + i - P.gstart[g];
-                    if (best < 0 || u[off % LDS_BANKS] < u[(p0 + best - P.gstart[g]) % LDS_BANKS]) best = i;
-                }
-                cand[(size_t)best] = 0;
-                P.pos[sl] = p0 + best;
-                u[(p0 + best - P.gstart[g]) % LDS_BANKS]++;
-            }
-            a = b;
-        }
-    }
-    // the offset lists follow the new positions
-    for (size_t sl = 0; sl < L; sl++) {
-        const int l = P.lit[sl];
-        if (!l || P.pos[sl] < 0) continue;
-        const int v = std::abs(l);
-        const size_t e = (size_t)P.csr_ptr[v] + kidx[sl];
-        P.csr_pos[e] = P.pos[sl];
-        if (!P.csr_loc.empty()) P.csr_loc[e] = (uint16_t)(P.pos[sl] - P.gstart[(size_t)(v - 1) / vg]);
-    }
-}
-
 // Per tile of TC clauses: the tile's slots in ascending position order.
 // Positions inside a region follow slot order, so this is a stable counting
 // sort of the tile's slots by variable group; the clause pass then writes
@@ -528,7 +432,8 @@ struct StageArgs {
     int mq;
     double* th;            // its tanh table, 2 per variable from 0 (null: not used)
     const int* csr_pos;    // per-variable contribution positions (gather var pass)
-    const uint16_t* csr_loc;   // the same relative to the region start (LDS var pass)
+    const uint16_t* rloc;      // LDS var pass: list place of each region entry
+    const uint16_t* ploc;      // and of each clause's direct primary term
     const long long* gstart;   // region starts, ngroups+1
     const int* pvar;       // direct primary slots: primary variable of each clause (processing order)
     const uint16_t* pw16;  // big tiles: primary word of each clause (in place of pvar)
@@ -550,7 +455,6 @@ struct StageArgs {
     int n, m, k, aoff;
     int nblk_clause;   // clause-pass grid (its J = 6 error partials come first)
     int vg;            // variables per group
-    int var_region_cap;   // LDS var pass: elements reserved for a region
     int var_stagger;      // LDS var pass: CUs whose second workgroup starts late (0: none)
     int vg_blocks;     // gather var pass: blocks per variable group
     int ngroups;
@@ -1262,15 +1166,21 @@ __device__ __forceinline__ T bias_sine(T s)
 }
 
 // LDS var pass: one workgroup per variable group.  The group's whole
-// contribution region and its variables' 16-bit region offsets (one
-// contiguous CSR range) are read into LDS with coalesced 16-byte loads, all
-// issued before the first LDS write; then each thread adds its variables'
-// runs from LDS in slot order (the reference's accumulation order).  With
-// slot spins on, each thread then writes its variables' output spins (stage
-// J+1's input, or x_new) over their own region entries, and the workgroup
-// streams the region back to contrib as the next clause pass's slot spins.
-// Each region entry belongs to one slot of one variable, so the entries a
-// thread reads and overwrites are its own.
+// contribution region is read with coalesced 16-byte loads, together with each
+// entry's place in the group's var-major slot list, and scattered to those places
+// in LDS: every variable's terms then lie side by side, and one thread adds them
+// left to right (slot order, the reference's accumulation order) without looking
+// up where they are.  With slot spins on, the thread then writes its variable's
+// output spin (stage J+1's input, or x_new) over its own terms, and the workgroup
+// gathers the region back and streams it to contrib as the next clause pass's
+// slot spins.  The two permutations are spread over all 1024 threads; a variable
+// that looked up its own terms instead did so with the few waves that a group of
+// 128 to 1000 variables has, each entry behind a branch: 6 of the pass's 9 us in a
+// workgroup for 4-SAT, N = 20 011, M = 196 107, FP64, against 3 now (us per
+// attempt: 147 to 121; 3-SAT, N = 163 840, FP64: 185 to 174; N = 1e6, FP32: 448 to
+// 430; N = 60 013, clauses of 3 to 6, FP32: 111 to 102).  The positions that a tile's
+// slots take within its run are free, but spreading them over the LDS banks
+// (0.2 %) is not worth the work.
 // FP32: two 1024-thread workgroups per CU (LDS holds two regions) need 8
 // waves per SIMD, which caps the scalar registers: at J = 6 the compiler
 // otherwise takes 90 of them, only one workgroup fits, and the pass took 44
@@ -1280,11 +1190,12 @@ __global__ __launch_bounds__(VBLK) __attribute__((amdgpu_waves_per_eu(sizeof(T) 
 void k_var_region(StageArgs<T> a)
 {
     constexpr int V = 16 / (int)sizeof(T);
-    constexpr int R = 4;              // 16-byte loads in flight per thread and round
+    constexpr int R = sizeof(T) == 4 ? 4 : 6;   // 16-byte loads in flight per thread and round
     typedef T vT __attribute__((ext_vector_type(V)));
-    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+    typedef unsigned short vL __attribute__((ext_vector_type(V)));
     __shared__ double sh[VBLK / 64];
-    // dynamic LDS: the region (largest region x sizeof(T)), then the offsets
+    // dynamic LDS: the group's slot list, a place for entries of no slot, and
+    // room for the last variable's rounded-up reads
     extern __shared__ __attribute__((aligned(16))) unsigned char var_lds[];
     const Ctrl* c = a.ctrl;
     int parity = 0;
@@ -1308,112 +1219,134 @@ void k_var_region(StageArgs<T> a)
     if (g >= a.var_stagger && g < 2 * a.var_stagger) __builtin_amdgcn_s_sleep(127);
     const int i0 = g * a.vg + 1, i1 = (int)std::min<long long>((long long)(g + 1) * a.vg, a.n);
     T* reg = (T*)var_lds;
-    const uint16_t* loc = (const uint16_t*)(var_lds + (size_t)a.var_region_cap * sizeof(T));
     T* s_next = a.slot_spins ? a.contrib : nullptr;
     const long long r0 = a.gstart[g];
     const int nreg = (int)(a.gstart[g + 1] - r0) / V;
-    const int rlen = nreg * V;
+    const int ebase = a.csr_ptr[i0], nlist = a.csr_ptr[i1 + 1] - ebase;
     // each thread's state values, loaded before the region (groups of at most
-    // 2 * VBLK variables; larger groups load them in the loop)
-    constexpr int VP = 2;
+    // VP * VBLK variables; larger groups load them in the loop)
+    constexpr int VP = J == 6 && sizeof(T) == 4 ? 1 : 2;   // (2 would spill)
     const bool pre = i1 - i0 + 1 <= VP * VBLK;
     VarIn<T> vin[VP];
+    int row[VP][2];
     if (pre) {
 #pragma unroll
         for (int u = 0; u < VP; u++) {
             const int i = i0 + (int)threadIdx.x + u * VBLK;
-            if (i <= i1) vin[u] = var_load<T, J>(a, i, x, fresh);
+            if (i <= i1) {
+                row[u][0] = a.csr_ptr[i] - ebase;
+                row[u][1] = a.csr_ptr[i + 1] - ebase;
+                vin[u] = var_load<T, J>(a, i, x, fresh);
+            }
         }
     }
-    int ebase = 0;
+    // the places of this thread's first RP region units, for the way back: FP64
+    // keeps them; FP32, with half the registers, would spill, and reads them
+    // again (from L2) before it adds
+    constexpr bool KEEP = sizeof(T) == 8;
+    constexpr int RP = KEEP ? R : 3;
+    vL place[RP];
+    const vL* const places = (const vL*)(a.rloc + r0);
     if (fresh || s_next) {
-        // region sizes are multiples of REGION_ALIGN and the offsets of a group
-        // number at most its region size; the host sized the LDS for both and
-        // padded csr_loc by 8 entries for the rounded-up 16-byte loads.  A
-        // retry's J = 1 pass needs only the offsets (for the slot spins).
-        const int nv = fresh ? nreg : 0;
-        const int e_first = a.csr_ptr[i0], e_end = a.csr_ptr[i1 + 1];
-        ebase = e_first & ~7;
-        const int nc = (e_end - ebase + 7) >> 3;
+        // region sizes are multiples of REGION_ALIGN.  A retry's J = 1 pass
+        // needs only the places (for the slot spins).
         const vT* src = (const vT*)(a.contrib + r0);
-        // direct primary slots: the group's primary terms follow the region
-        // in LDS, read from the 16-byte unit holding its first clause
+        // direct primary slots: the group's primary terms, read from the
+        // 16-byte unit holding its first clause; the first and the last unit
+        // may hold other groups' terms
         const vT* psrc = src;
-        int npv = 0;
+        const vL* plsrc = places;
+        int npv = 0, pb = 0, p0 = 0, p1 = 0;
         if (a.split && fresh) {
-            const int pb = a.pc0[g] / V * V;
+            p0 = a.pc0[g];
+            p1 = a.pc0[g + 1];
+            pb = p0 / V * V;
             psrc = (const vT*)(a.pcontrib + pb);
-            npv = (a.pc0[g + 1] - pb + V - 1) / V;
+            plsrc = (const vL*)(a.ploc + pb);
+            npv = (p1 - pb + V - 1) / V;
         }
-        const int nt = nv + npv;
-        const v4u* csrc = (const v4u*)(a.csr_loc + ebase);
-        vT* dst = (vT*)reg;
-        v4u* cdst = (v4u*)loc;
-        const int nmax = nt > nc ? nt : nc;
-        for (int base = 0; base < nmax; base += R * VBLK) {
+        const int nt = nreg + npv;
+        for (int base = 0; base < nt; base += R * VBLK) {
             vT rb[R];
-            v4u cb[R];
+            vL lb[R];
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 const int v = base + r * VBLK + (int)threadIdx.x;
-                if (v < nt) rb[r] = ld_g(v < nv ? src + v : psrc + (v - nv));
-                if (v < nc) cb[r] = ld_g(csrc + v);
+                if (v < nt) {
+                    if (fresh) rb[r] = ld_g(v < nreg ? src + v : psrc + (v - nreg));
+                    lb[r] = ld_g(v < nreg ? places + v : plsrc + (v - nreg));
+                }
             }
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 const int v = base + r * VBLK + (int)threadIdx.x;
-                if (v < nt) dst[v] = rb[r];
-                if (v < nc) cdst[v] = cb[r];
+                if (KEEP && base == 0 && r < RP) place[r] = lb[r];
+                if (v < nt && fresh)
+#pragma unroll
+                    for (int q = 0; q < V; q++) {
+                        const int j = pb + (v - nreg) * V + q;
+                        const bool own = v < nreg || (j >= p0 && j < p1);
+                        reg[own ? (int)lb[r][q] : nlist] = rb[r][q];
+                    }
             }
         }
         __syncthreads();
+        if (!KEEP && s_next) {
+#pragma unroll
+            for (int r = 0; r < RP; r++)
+                if (r * VBLK + (int)threadIdx.x < nreg) place[r] = ld_g(places + r * VBLK + (int)threadIdx.x);
+        }
     }
     double err = 0.0;
     const T pref = (a.bias && fresh) ? bias_prefactor<T, VBLK>(a, sh) : (T)0;
     int u = 0;
     for (int i = i0 + (int)threadIdx.x; i <= i1; i += VBLK, u++) {
         T kj = (T)0;
-        const int e0 = a.csr_ptr[i] - ebase, e1 = a.csr_ptr[i + 1] - ebase;
+        int e0, e1;
+        VarIn<T> in;
+        if (pre) {
+            e0 = u == 0 ? row[0][0] : row[VP - 1][0];
+            e1 = u == 0 ? row[0][1] : row[VP - 1][1];
+            in = u == 0 ? vin[0] : vin[VP - 1];
+        } else {
+            e0 = a.csr_ptr[i] - ebase;
+            e1 = a.csr_ptr[i + 1] - ebase;
+            in = var_load<T, J>(a, i, x, fresh);
+        }
         if (fresh) {
-            // four entries in flight per round (offsets, then values), added
-            // left to right; lanes past their row read element 0 and skip it
+            // VAR_SUM entries in flight, added left to right; past the row's end
+            // a -0, which changes no sum
             T sum = (T)0;
-            for (int e = e0; e < e1; e += 4) {
-                int o[4];
-                T v[4];
+            for (int e = e0; e < e1; e += VAR_SUM) {
+                T v[VAR_SUM];
 #pragma unroll
-                for (int q = 0; q < 4; q++) o[q] = e + q < e1 ? loc[e + q] : 0;
+                for (int q = 0; q < VAR_SUM; q++) v[q] = reg[e + q];
 #pragma unroll
-                for (int q = 0; q < 4; q++) v[q] = reg[o[q]];
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (e + q < e1) sum += v[q];
+                for (int q = 0; q < VAR_SUM; q++) sum += e + q < e1 ? v[q] : (T)-0.0;
             }
             kj = sum;
             if (a.bias) kj += pref * bias_sine<T>(J == 1 ? x[i] : a.tmp[i]);
         }
-        VarIn<T> in;
-        if (pre) in = u == 0 ? vin[0] : vin[1];
-        else in = var_load<T, J>(a, i, x, fresh);
         const T out = var_stage<T, J>(a, i, fresh, kj, in, xnew, hs, h, hnext, floor, err);
-        if (s_next)   // region entries only (direct primary entries lie past the region)
-            for (int e = e0; e < e1; e += 4) {
-                int o[4];
-#pragma unroll
-                for (int q = 0; q < 4; q++) o[q] = e + q < e1 ? loc[e + q] : rlen;
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (o[q] < rlen) reg[o[q]] = out;
-            }
+        if (s_next)
+            for (int e = e0; e < e1; e++) reg[e] = out;
     }
     if (s_next) {
-        // the region's entries not owned by a variable (alignment padding)
-        // are written out too, with whatever the LDS holds; no slot reads them
+        // the region's entries of no slot (alignment padding) are written out
+        // too, with whatever the LDS holds; no slot reads them
         __syncthreads();
-        const vT* src = (const vT*)reg;
         vT* dst = (vT*)(s_next + r0);
-        // ordinary stores: the next clause pass reads these lines right away
-        for (int v = (int)threadIdx.x; v < nreg; v += VBLK) dst[v] = src[v];
+        auto give = [&](int v, vL l) {
+            vT o;
+#pragma unroll
+            for (int q = 0; q < V; q++) o[q] = reg[l[q]];
+            // ordinary stores: the next clause pass reads these lines right away
+            dst[v] = o;
+        };
+#pragma unroll
+        for (int r = 0; r < RP; r++)
+            if (r * VBLK + (int)threadIdx.x < nreg) give(r * VBLK + (int)threadIdx.x, place[r]);
+        for (int v = RP * VBLK + (int)threadIdx.x; v < nreg; v += VBLK) give(v, places[v]);
     }
     if constexpr (J == 6) {
         double bm = block_max<VBLK>(err, sh);
@@ -1737,19 +1670,20 @@ __global__ void k_uniform(T* out, int len, unsigned long long seed, unsigned lon
 // Slot spins of a state: each variable's spin at all of its contribution
 // positions (the layout the LDS var pass writes after each stage).
 template <typename T>
-__global__ __launch_bounds__(BLK) void k_slot_fill(const T* x, const int* csr_ptr, const uint16_t* csr_loc,
-                                                   const long long* gstart, int vg, int n, T* sl)
+__global__ __launch_bounds__(VBLK) void k_slot_fill(const T* x, const int* csr_ptr, const uint16_t* rloc,
+                                                    const long long* gstart, int vg, int n, T* sl)
 {
-    const int i = blockIdx.x * BLK + (int)threadIdx.x + 1;
-    if (i > n) return;
-    const T v = x[i];
-    const int g = (i - 1) / vg;
-    T* base = sl + gstart[g];
-    const long long rlen = gstart[g + 1] - gstart[g];   // direct primary entries lie past the region
-    for (int e = csr_ptr[i]; e < csr_ptr[i + 1]; e++) {
-        const int o = csr_loc[e];
-        if (o < rlen) base[o] = v;
+    extern __shared__ __attribute__((aligned(16))) unsigned char var_lds[];
+    T* reg = (T*)var_lds;
+    const int g = blockIdx.x;
+    const int i0 = g * vg + 1, i1 = (int)std::min<long long>((long long)(g + 1) * vg, n);
+    const int ebase = csr_ptr[i0];
+    for (int i = i0 + (int)threadIdx.x; i <= i1; i += VBLK) {
+        const T v = x[i];
+        for (int e = csr_ptr[i] - ebase; e < csr_ptr[i + 1] - ebase; e++) reg[e] = v;
     }
+    __syncthreads();
+    for (long long r = gstart[g] + threadIdx.x; r < gstart[g + 1]; r += VBLK) sl[r] = reg[rloc[r]];
 }
 
 template <typename T>
@@ -1887,7 +1821,8 @@ struct Sys {
     int run_stride = 0;
     int* d_csr_ptr = nullptr;
     int* d_csr_pos = nullptr;    // gather var pass only
-    uint16_t* d_csr_loc = nullptr;   // LDS var pass only
+    uint16_t* d_rloc = nullptr;      // LDS var pass only
+    uint16_t* d_ploc = nullptr;      // and only with direct primary slots
     long long* d_gstart = nullptr;
     int* d_pvar = nullptr;       // direct primary slots: primary variable per clause
     uint16_t* d_pw16 = nullptr;  // big tiles: primary word per clause (in place of d_pvar)
@@ -1919,9 +1854,8 @@ struct Sys {
     int tc = TC;                 // tiled pass: clauses per tile (TC or TC_BIG)
     bool lds_var = false;        // var pass: LDS region kernel or gather kernel
     bool wide_var = false;       // gather path with long rows: one workgroup per variable
-    int var_lds = 0;             // LDS region kernel: dynamic LDS bytes (region + offsets)
+    int var_lds = 0;             // LDS region kernel: dynamic LDS bytes (a group's slot list)
     int var_stagger = 0;         // LDS region kernel: CUs whose second workgroup starts late
-    int var_region_cap = 0;      // LDS region kernel: elements reserved for a region
     void* d_contrib = nullptr;
     double* d_apart = nullptr;   // bias term: per clause-block aux sums
     void* d_public = nullptr;    // a state in public order, on its way to or from the host
@@ -1939,7 +1873,7 @@ struct Sys {
         dfree(d_srank); dfree(d_csr_ptr); dfree(d_csr_pos);
         dfree(d_runs);
         run_stride = 0;
-        dfree(d_csr_loc); dfree(d_gstart); dfree(d_perm); dfree(d_contrib); dfree(d_apart);
+        dfree(d_rloc); dfree(d_ploc); dfree(d_gstart); dfree(d_perm); dfree(d_contrib); dfree(d_apart);
         dfree(d_pvar); dfree(d_pc0); dfree(d_pcontrib); dfree(d_pw16); dfree(d_pv0);
         split = false;
         dfree(d_vptr); dfree(d_spos_small); dfree(d_public);
@@ -1987,12 +1921,9 @@ static void upload(V*& d, const std::vector<V>& h)
 // either way are the same); halved until the largest region fits in LDS.  When no
 // size fits (a variable with more occurrences than the LDS holds), the gather
 // var pass runs with ~400 KB regions.
-// LDS of the region var pass: the region and its variables' uint16 offsets
-// (at most one per region element), plus room for the rounded 16-byte loads
-static int var_lds_bytes(long long max_region, int esize)
-{
-    return (int)(max_region * esize + round_up(max_region * 2 + 32, 16));
-}
+// LDS of the region var pass: the longest group's slot list, a place for entries
+// of no slot, and the rounded-up reads past the last variable's terms
+static int var_lds_bytes(int max_list, int esize) { return (int)round_up((max_list + 1 + VAR_SUM) * esize, 16); }
 
 static bool choose_layout(HostProblem& P, int esize)
 {
@@ -2213,7 +2144,6 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
             if (P.pvar[(size_t)j1] - P.pvar[(size_t)j0] > (int)PW_VMASK) P.tc = TC;
         }
     }
-    if (tiled && P.tc != TC) spread_run_banks(P, 16 / s->esize);
     if (tiled) build_tile_order(P);
     HIP_CHECK(hipStreamSynchronize(s->stream));
     s->free_problem();
@@ -2242,8 +2172,10 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
         for (size_t sl = 0; sl < P.lit.size(); sl++)
             if (P.lit[sl]) P.pos[sl] = fill[(size_t)std::abs(P.lit[sl])]++;
     }
-    s->var_region_cap = lds_var ? (int)P.max_region : 0;
-    s->var_lds = lds_var ? var_lds_bytes(P.max_region, s->esize) : 0;
+    int max_list = 0;
+    for (int i = 1; i <= P.n; i += P.vg)
+        max_list = std::max(max_list, P.csr_ptr[std::min(P.n + 1, i + P.vg)] - P.csr_ptr[i]);
+    s->var_lds = lds_var ? var_lds_bytes(max_list, s->esize) : 0;
     // two FP32 var workgroups per CU (LDS for both; the FP64 kernel's
     // registers allow one) and more groups than CUs: stagger the pairs
     s->var_stagger = 0;
@@ -2297,8 +2229,22 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
     }
     upload(s->d_csr_ptr, P.csr_ptr);
     if (lds_var) {
-        P.csr_loc.resize(P.csr_loc.size() + 8, 0);   // rounded-up 16-byte loads of the last range
-        upload(s->d_csr_loc, P.csr_loc);
+        // the inverse of the variables' lists; entries of no slot go past the list
+        std::vector<uint16_t> rloc((size_t)P.gstart[P.ngroups]), ploc(P.split ? mpad + 16 : 0, 0);
+        for (int g = 0; g < P.ngroups; g++) {
+            const int i0 = g * P.vg + 1, i1 = std::min(P.n, (g + 1) * P.vg);
+            const int e0 = P.csr_ptr[i0], e1 = P.csr_ptr[i1 + 1];
+            const long long r0 = P.gstart[g], rlen = P.gstart[(size_t)g + 1] - r0;
+            std::fill(rloc.begin() + r0, rloc.begin() + r0 + rlen, (uint16_t)(e1 - e0));
+            const int v16 = 16 / s->esize;
+            for (int e = e0; e < e1; e++) {
+                const long long o = P.csr_loc[(size_t)e];
+                if (o < rlen) rloc[(size_t)(r0 + o)] = (uint16_t)(e - e0);
+                else ploc[(size_t)(P.pc0[g] / v16 * v16 + o - rlen)] = (uint16_t)(e - e0);
+            }
+        }
+        upload(s->d_rloc, rloc);
+        if (P.split) upload(s->d_ploc, ploc);
     }
     else if (!s->wide_run) upload(s->d_csr_pos, P.csr_pos);
     upload(s->d_gstart, P.gstart);
@@ -2408,7 +2354,7 @@ static StageArgs<T> stage_args(Sys* s, T* xa, T* xb, T* const* kk, T* tmp, doubl
     a.runs = s->d_runs; a.run_stride = s->run_stride;
     a.litq = s->d_litq; a.posq = s->d_posq; a.mq = s->mq;
     a.th = s->family == ASAT_FAMILY_TANH ? s->d_th : nullptr;
-    a.csr_ptr = s->d_csr_ptr; a.csr_pos = s->d_csr_pos; a.csr_loc = s->d_csr_loc; a.gstart = s->d_gstart;
+    a.csr_ptr = s->d_csr_ptr; a.csr_pos = s->d_csr_pos; a.rloc = s->d_rloc; a.ploc = s->d_ploc; a.gstart = s->d_gstart;
     a.pvar = s->d_pvar; a.pw16 = s->d_pw16; a.pv0 = s->d_pv0; a.pc0 = s->d_pc0; a.pcontrib = (T*)s->d_pcontrib; a.split = s->split ? 1 : 0;
     a.contrib = (T*)s->d_contrib;
     a.xa = xa; a.xb = xb;
@@ -2421,7 +2367,6 @@ static StageArgs<T> stage_args(Sys* s, T* xa, T* xb, T* const* kk, T* tmp, doubl
     a.clause_per_xcd = ceil_div(s->tiled ? a.ntiles : ceil_div(s->m, BLK), 8);
     a.nblk_clause = clause_grid(s);
     a.vg = s->vg;
-    a.var_region_cap = s->var_region_cap;
     a.var_stagger = s->var_stagger;
     a.vg_blocks = s->vg_blocks;
     a.ngroups = s->ngroups;
@@ -2495,6 +2440,9 @@ static void var_lds_attrs()
 {
     var_lds_attr<T, 1>(); var_lds_attr<T, 2>(); var_lds_attr<T, 3>();
     var_lds_attr<T, 4>(); var_lds_attr<T, 5>(); var_lds_attr<T, 6>();
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_slot_fill<T>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, VAR_LDS_BYTES);
+    HIP_CHECK(attr);
 }
 
 template <typename T, int J>
@@ -2738,8 +2686,8 @@ static StageArgs<T> rk_stage_args(RK* r, int parity)
     fill_tanh<T>(a, (const T*)r->pair[parity], s->stream);
     if (s->tiled && s->lds_var) {
         a.slot_spins = 1;
-        hipLaunchKernelGGL(k_slot_fill<T>, dim3(ceil_div(s->n, BLK)), dim3(BLK), 0, s->stream,
-                           (const T*)r->pair[parity], s->d_csr_ptr, s->d_csr_loc, s->d_gstart, s->vg, s->n,
+        hipLaunchKernelGGL(k_slot_fill<T>, dim3(s->ngroups), dim3(VBLK), (size_t)s->var_lds, s->stream,
+                           (const T*)r->pair[parity], s->d_csr_ptr, s->d_rloc, s->d_gstart, s->vg, s->n,
                            (T*)s->d_contrib);
         HIP_CHECK(hipGetLastError());
     }
