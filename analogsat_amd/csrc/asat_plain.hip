@@ -4,7 +4,7 @@
 //
 // Data layout in HBM (T = double for ASAT_F64, float for ASAT_F32):
 //   lit[m*K + q]      int32 signed literal (+v / -v, 0 = padding), clause-major,
-//                     padded to whole tiles of TC clauses
+//                     padded to whole tiles of at most TC clauses
 //   contrib[p]        per-slot contribution 2 c a K K_mi of the current stage.
 //                     Variables are split into groups (at most about 2048 float
 //                     / 1024 double variables, halved until the largest region
@@ -78,7 +78,7 @@ static inline long long round_up(long long a, long long b) { return (a + b - 1) 
 // ===========================================================================
 // problem (host)
 // ===========================================================================
-constexpr int TC = 2048;                  // clauses per tile of the tiled clause pass (one workgroup)
+constexpr int TC = 2048;                  // clauses per tile of the tiled clause pass (one workgroup), at most
 constexpr int TC_BIG = 4608;              // FP32 3-literal systems with direct primary slots: the most
                                           // clauses a tile may have (its size is chosen per problem)
 constexpr int TC_MAX = TC_BIG;
@@ -318,7 +318,7 @@ static void build_tile_order(HostProblem& P)
     // run tables (big tiles): a tile's positions in one region are
     // consecutive (tiles are ranges of slots, region positions follow slot
     // order), so the sorted list is one run per group
-    const bool rt = P.split && TCt != TC;
+    const bool rt = P.split && TCt > TC;
     require(!rt || (long long)(P.ngroups + 1) * 4 <= (long long)nper, ASAT_ERR_UNSUPPORTED,
             "run tables larger than the positions they replace");
     P.runs.clear();
@@ -330,7 +330,7 @@ static void build_tile_order(HostProblem& P)
         P.spos.assign((size_t)ntiles * nper, -1);
     }
     // big tiles store K - 1 ranks per clause (the primary one is in pw16)
-    const bool cp = P.split && TCt != TC;
+    const bool cp = P.split && TCt > TC;
     const int KR = cp ? NR : K;
     const size_t rper = (size_t)TCt * KR;
     P.srank.assign((size_t)ntiles * rper, 0xFFFF);
@@ -740,7 +740,7 @@ void k_clause_tile(StageArgs<T> a)
     double err = 0.0, asum = 0.0;
     const int tile = (b & 7) * a.clause_per_xcd + (b >> 3);
     if (tile < a.ntiles) {
-        const int TS = PL ? a.tile_clauses : TCt;
+        const int TS = a.tile_clauses;
         const long long c0 = (long long)tile * TS;
         int ps[NP];
         T psv[CPTG];
@@ -2144,6 +2144,17 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
             if (P.pvar[(size_t)j1] - P.pvar[(size_t)j0] > (int)PW_VMASK) P.tc = TC;
         }
     }
+    // Other problems of 16 tiles and more, but FP32 3-literal ones: tiles of 512 to
+    // 2048 clauses, sized so that they fill whole rounds of one workgroup per CU (us
+    // per attempt with 2048-clause tiles and these: FP64, 3-SAT, N = 20 011: 83 and
+    // 70, 40 000: 98 and 88, 163 840: 170 and 166, 400 000: 346 and 340; 4-SAT,
+    // N = 20 011: 121 and 109, 60 000: 200 and 187; FP32, 4-SAT, N = 20 011: 95 and
+    // 90; 100 000: 190 both; 3-SAT, N = 20 011: 59 both, so 2048 stays there).
+    if (tiled && P.tc == TC && P.m >= 16 * TC && (s->esize == 8 || P.k == 4)) {
+        const long long cus = ncu > 0 ? ncu : 1;
+        const long long rounds = ceil_div((long long)P.m, cus * TC);
+        P.tc = (int)std::max<long long>(512, round_up(ceil_div((long long)P.m, rounds * cus), 64));
+    }
     if (tiled) build_tile_order(P);
     HIP_CHECK(hipStreamSynchronize(s->stream));
     s->free_problem();
@@ -2406,7 +2417,7 @@ static void launch_clause(const StageArgs<T>& a, const Sys* s, hipStream_t st)
     require(!ss || ps, ASAT_ERR_INVALID_ARGUMENT, "slot spins without direct primary slots");
     const dim3 tb(TILE_BT);
     constexpr int TB = TC_BIG, TS = TC;
-    const bool big = s->tc != TC;
+    const bool big = s->tc > TC;
     require(!big || (sizeof(T) == 4 && ps && a.k == 3 && a.pw16 && a.pv0 && a.runs), ASAT_ERR_INVALID_ARGUMENT,
             "big clause tiles without their layout");
     if constexpr (sizeof(T) == 4) {
