@@ -40,8 +40,8 @@
 // The launch is cooperative, so all workgroups are resident; a wait that lasts
 // GRID_POLLS polls gives up and the host reports an error.
 // Bound by the latency of its six exchanges: N = 2000, M = 8500 takes 20.6 us an
-// attempt in FP32 and 24.3 in FP64 (multi-kernel path 74 and 84), N = 12000,
-// M = 51120 43 and 60 (77 and 88).
+// attempt in FP32 and 24.3 in FP64 (multi-kernel path 65 and 73), N = 12000,
+// M = 51120 43 and 58 (68 and 66).
 #pragma once
 
 #include <type_traits>

@@ -1981,7 +1981,7 @@ static void build_small_lists(Sys* s, const HostProblem& P)
 //   N = 12000, M = 51120, FP64      - /    - /    - / 59.9 / 69.5
 // The path ends where the spins of all variables no longer fit in LDS or the
 // clauses in registers; up to there it is faster than 13 kernels per attempt
-// (N = 24000, M = 102000, FP32: 67 against 79 us).
+// (N = 24000, M = 102000, FP32: 68 against 76 us; N = 14000, FP64: 63 against 67).
 constexpr int GRID_CPT_F64 = 4, GRID_CPT_F32 = 8;
 constexpr long long GRID_LDS = 158 * 1024;     // beside the kernel's 0.3 KB of static LDS
 static void build_grid(Sys* s, const HostProblem& P)

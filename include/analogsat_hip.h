@@ -121,7 +121,7 @@ int asat_sys_clause_order(const asat_sys_t* sys, int* order);
 
 /* No reference counterpart (the CUDA classes pick their kernels by class):
    which passes and launch shapes SetProblem chose for this problem. */
-#define ASAT_CLAUSE_TILED 0    /* tiles of 2048 clauses, K = 3 or 4 */
+#define ASAT_CLAUSE_TILED 0    /* tiles of clauses, K = 3 or 4 */
 #define ASAT_CLAUSE_GENERIC 1  /* thread per clause, any K <= 32 */
 #define ASAT_VAR_REGION 0      /* one workgroup per variable group, region in LDS */
 #define ASAT_VAR_GATHER 1      /* gather from global memory, many variables per workgroup */
