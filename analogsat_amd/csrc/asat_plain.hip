@@ -708,12 +708,16 @@ __device__ __forceinline__ void tile_group(const StageArgs<T>& a, long long c0, 
 // extra tile running alone cost about 5 us per pass).  Phase 1 takes their
 // clauses one at a time, which keeps them at 8 waves per SIMD without
 // spills; two at a time spilled at J = 6 and ran 1-4 us slower per pass.
+// FP64 3-literal tiles run 8 waves per SIMD too, two workgroups per CU (62-76
+// registers and one workgroup otherwise: N = 163 840, M = 696 320 169 us per
+// attempt, 157 now, 158.5 with spills instead of one clause at a time from
+// J = 4 on); 4-literal ones would spill and lose (109 and 111.5 us).
 template <typename T, int K, int J, int BT, int TCt, bool SS, bool PS>
-__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(TCt > TC ? 8 : 1)))
+__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(TCt > TC || (sizeof(T) == 8 && K == 3) ? 8 : 1)))
 void k_clause_tile(StageArgs<T> a)
 {
     constexpr int CPT = (TCt + BT - 1) / BT;
-    constexpr int G = TCt > TC ? 1 : (CPT < 2 ? CPT : 2);
+    constexpr int G = TCt > TC || (sizeof(T) == 8 && K == 3 && J >= 4) ? 1 : (CPT < 2 ? CPT : 2);
     constexpr int CPTG = (CPT + G - 1) / G * G;   // clause slots of the groups (past CPT: none of the tile)
     constexpr int NR = PS ? K - 1 : K;
     constexpr int NP = CPT * NR;
@@ -2147,7 +2151,8 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
     // Other problems of 16 tiles and more, but FP32 3-literal ones: tiles of 512 to
     // 2048 clauses, sized so that they fill whole rounds of one workgroup per CU (us
     // per attempt with 2048-clause tiles and these: FP64, 3-SAT, N = 20 011: 83 and
-    // 70, 40 000: 98 and 88, 163 840: 170 and 166, 400 000: 346 and 340; 4-SAT,
+    // 70, 40 000: 98 and 88, 163 840: 170 and 166, 400 000: 346 and 340 (157 and 322 since two of
+    // their workgroups fit on a CU); 4-SAT,
     // N = 20 011: 121 and 109, 60 000: 200 and 187; FP32, 4-SAT, N = 20 011: 95 and
     // 90; 100 000: 190 both; 3-SAT, N = 20 011: 59 both, so 2048 stays there).
     if (tiled && P.tc == TC && P.m >= 16 * TC && (s->esize == 8 || P.k == 4)) {
