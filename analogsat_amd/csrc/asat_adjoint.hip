@@ -760,6 +760,7 @@ static void set_problem(Adj& A, const int* lits, const int* lens, int nclauses)
         if (C[s]) spos[s] = fill[std::abs(C[s])]++;
     if (!A.stream) HIP_CHECK(hipStreamCreateWithFlags(&A.stream, hipStreamNonBlocking));
     HIP_CHECK(hipStreamSynchronize(A.stream));
+    A.have_problem = A.have_forward = false;
     A.free_batch();
     (void)hipFree(A.d_lit); (void)hipFree(A.d_csr_ptr); (void)hipFree(A.d_slot_pos);
     A.d_lit = A.d_csr_ptr = A.d_slot_pos = nullptr;

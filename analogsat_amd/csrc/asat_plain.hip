@@ -2151,10 +2151,10 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
     // Other problems of 16 tiles and more, but FP32 3-literal ones: tiles of 512 to
     // 2048 clauses, sized so that they fill whole rounds of one workgroup per CU (us
     // per attempt with 2048-clause tiles and these: FP64, 3-SAT, N = 20 011: 83 and
-    // 70, 40 000: 98 and 88, 163 840: 170 and 166, 400 000: 346 and 340 (157 and 322 since two of
-    // their workgroups fit on a CU); 4-SAT,
-    // N = 20 011: 121 and 109, 60 000: 200 and 187; FP32, 4-SAT, N = 20 011: 95 and
-    // 90; 100 000: 190 both; 3-SAT, N = 20 011: 59 both, so 2048 stays there).
+    // 70, 40 000: 98 and 88, 163 840: 170 and 166, 400 000: 346 and 340, the last
+    // two 157 and 322 since two of their workgroups fit on a CU; 4-SAT, N = 20 011:
+    // 121 and 109, 60 000: 200 and 187; FP32, 4-SAT, N = 20 011: 95 and 90,
+    // 100 000: 190 both; 3-SAT, N = 20 011: 59 both, so 2048 stays there).
     if (tiled && P.tc == TC && P.m >= 16 * TC && (s->esize == 8 || P.k == 4)) {
         const long long cus = ncu > 0 ? ncu : 1;
         const long long rounds = ceil_div((long long)P.m, cus * TC);
@@ -2456,9 +2456,6 @@ static void var_lds_attrs()
 {
     var_lds_attr<T, 1>(); var_lds_attr<T, 2>(); var_lds_attr<T, 3>();
     var_lds_attr<T, 4>(); var_lds_attr<T, 5>(); var_lds_attr<T, 6>();
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_slot_fill<T>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, VAR_LDS_BYTES);
-    HIP_CHECK(attr);
 }
 
 template <typename T, int J>
@@ -2702,6 +2699,9 @@ static StageArgs<T> rk_stage_args(RK* r, int parity)
     fill_tanh<T>(a, (const T*)r->pair[parity], s->stream);
     if (s->tiled && s->lds_var) {
         a.slot_spins = 1;
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_slot_fill<T>),
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, VAR_LDS_BYTES);
+        HIP_CHECK(attr);
         hipLaunchKernelGGL(k_slot_fill<T>, dim3(s->ngroups), dim3(VBLK), (size_t)s->var_lds, s->stream,
                            (const T*)r->pair[parity], s->d_csr_ptr, s->d_rloc, s->d_gstart, s->vg, s->n,
                            (T*)s->d_contrib);
