@@ -38,12 +38,14 @@
 #include "asat_common.h"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
 #include <memory>
 #include <mutex>
 #include <numeric>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -1434,12 +1436,23 @@ struct Batch {
     float* d_x0 = nullptr;          // start states
     long long state_total = 0;      // floats of a state buffer
     std::vector<long long> state_off;
-    // states on their way to the host, see get_state
+    // states on their way to the host, see get_state.  run() holds the lock over its
+    // capture and over each launch with what follows it up to the control
+    // blocks' copy, so a state read from another thread is the one of the latest
+    // finished launch; readers counts the threads that wait for it
     std::mutex win_lock;
+    std::atomic<int> readers{0};
     float *d_win = nullptr, *h_win = nullptr;
     int win_first = 0, win_last = 0;   // trajectories whose current states h_win holds
     int last_state = -1;               // trajectory of the latest get_state since the states changed
     void drop_window() { win_first = win_last = 0; last_state = -1; }
+    // the lock for a launch; waiting readers go first (a mutex alone would give it
+    // back to the thread that has just released it)
+    std::unique_lock<std::mutex> launch_lock()
+    {
+        while (readers.load() > 0) std::this_thread::yield();
+        return std::unique_lock<std::mutex>(win_lock);
+    }
     hipStream_t stream = nullptr;
     hipStream_t side[3] = {nullptr, nullptr, nullptr};   // further buckets' launches, see run
     int cus = 0;
@@ -1728,7 +1741,9 @@ static void get_state(Batch& B, int index, float* pub)
 {
     const Instance& I = B.inst[(size_t)index];
     const size_t len = (size_t)I.n + I.m;
+    B.readers++;
     std::lock_guard<std::mutex> lock(B.win_lock);
+    B.readers--;
     HIP_CHECK(hipStreamSynchronize(B.stream));
     const bool in_order = B.last_state >= 0 && index == B.last_state + 1;
     B.last_state = index;
@@ -2051,10 +2066,6 @@ static void run(Batch& B, int max_chunks, int graph_chunks)
     HIP_CHECK(hipEventCreate(&o.e0));
     HIP_CHECK(hipEventCreate(&o.e1));
     hipEvent_t e0 = o.e0, e1 = o.e1;
-    {
-        std::lock_guard<std::mutex> lock(B.win_lock);
-        B.drop_window();
-    }
     // one graph = graph_chunks x (per bucket: reset its queue, persistent
     // launch).  Buckets are independent, so their launches go to up to four
     // branches: a bucket with fewer trajectories than resident workgroups leaves
@@ -2067,6 +2078,7 @@ static void run(Batch& B, int max_chunks, int graph_chunks)
         if (!B.side[q - 1]) HIP_CHECK(hipStreamCreateWithFlags(&B.side[q - 1], hipStreamNonBlocking));
         HIP_CHECK(hipEventCreateWithFlags(&o.join[q - 1], hipEventDisableTiming));
     }
+    std::unique_lock<std::mutex> lock = B.launch_lock();   // no reader's work gets into the capture
     HIP_CHECK(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
     o.capturing = true;
     HIP_CHECK(hipEventRecord(o.fork, B.stream));
@@ -2087,6 +2099,7 @@ static void run(Batch& B, int max_chunks, int graph_chunks)
     }
     o.capturing = false;
     HIP_CHECK(hipStreamEndCapture(B.stream, &o.graph));
+    lock.unlock();
     HIP_CHECK(hipGraphInstantiate(&o.exec, o.graph, nullptr, nullptr, 0));
     hipGraphExec_t exec = o.exec;
     auto t0 = std::chrono::steady_clock::now();
@@ -2094,10 +2107,13 @@ static void run(Batch& B, int max_chunks, int graph_chunks)
     int launched = 0;
     std::vector<TrajCtrl>& hc = B.h_ctrl;
     while (launched < max_chunks) {
+        lock = B.launch_lock();
+        B.drop_window();
         HIP_CHECK(hipGraphLaunch(exec, B.stream));
         launched += graph_chunks;
         HIP_CHECK(hipMemcpyAsync(hc.data(), B.d_ctrl, sizeof(TrajCtrl) * T, hipMemcpyDeviceToHost, B.stream));
         HIP_CHECK(hipStreamSynchronize(B.stream));
+        lock.unlock();
         double now = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         int live = 0;
         for (int i = 0; i < T; i++) {
