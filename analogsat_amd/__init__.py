@@ -199,6 +199,7 @@ def lib():
                                     ctypes.POINTER(SolveResult), ctypes.POINTER(RkStats)], i),
             "asat_rk_set_one_workgroup": ([vp, i], i),
             "asat_rk_uses_one_workgroup": ([vp, ctypes.POINTER(i)], i),
+            "asat_rk_set_grid_limits": ([vp, i, ctypes.c_longlong, i], i),
             "asat_rk_solve": ([vp, vp, vp, i, ctypes.c_longlong, ctypes.c_double, i, ctypes.POINTER(SolveResult)], i),
             "asat_rk_reset": ([vp], i),
             "asat_rk_stats": ([vp, ctypes.POINTER(RkStats)], i),
@@ -641,6 +642,11 @@ class HipRungeKutta:
         workgroup for problems that fit in its LDS, 8 to 128 for larger ones
         (False: the multi-kernel path)."""
         _check(lib().asat_rk_set_one_workgroup(self._h, 1 if enable else 0))
+
+    def SetGridLimits(self, workgroups=0, attempts=0, launches=-1):
+        """Test hook: limits of the 8 to 128 workgroup kernel (most workgroups,
+        attempts per launch, launches before a wait is given up at once)."""
+        _check(lib().asat_rk_set_grid_limits(self._h, int(workgroups), int(attempts), int(launches)))
 
     def UsesOneWorkgroup(self):
         v = ctypes.c_int()

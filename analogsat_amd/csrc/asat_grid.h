@@ -37,8 +37,12 @@
 // against 12.0).  With 256 threads, up to 512 clauses, it was no faster (N = 50:
 // 4.7-5.1 against 4.6), so those keep asat_small.h.
 //
-// The launch is cooperative, so all workgroups are resident; a wait that lasts
-// GRID_POLLS polls gives up and the host reports an error.
+// The layout is used where the device holds all its workgroups at once, and the
+// launch is cooperative. Where they wait for each other all the same (another
+// process keeps part of the CUs busy), a wait that lasts GRID_POLLS polls gives
+// up: it marks the arrival word unless the last arrival came in between, so
+// every workgroup gives up at the same exchange, and none stores anything. The
+// launch then has had no effect and the host goes on by another path.
 // Bound by the latency of its six exchanges: N = 2000, M = 8500 takes 20.6 us an
 // attempt in FP32 and 24.3 in FP64 (multi-kernel path 65 and 73), N = 12000,
 // M = 51120 43 and 58 (68 and 66).
@@ -54,7 +58,8 @@ namespace asat {
 constexpr int GRID_BT = 1024;            // threads per workgroup
 constexpr int GRID_MAX = 128;            // workgroups
 constexpr int GRID_WAVES = GRID_BT / 64; // variable groups a workgroup can own
-constexpr int GRID_POLLS = 1 << 25;
+constexpr int GRID_POLLS = 1 << 21;      // a second or two
+constexpr unsigned GRID_GIVE_UP = 1u << 31;    // in the arrival word
 constexpr long long GRID_ATTEMPT_CAP = 4096;   // attempts per launch
 
 struct GridArgs {
@@ -69,7 +74,9 @@ struct GridArgs {
     void* pub;               // [2][64 * ngroups] published spins
     double* err;             // [2][GRID_MAX] error maxima
     int* count;              // [2][GRID_MAX] violated clauses
-    unsigned* barrier;       // arrivals, then the give-up flag; cleared before the launch
+    unsigned* barrier;       // arrivals, and GRID_GIVE_UP; cleared before the launch
+    int polls;               // of a wait before it is given up
+    long long attempt_cap;   // attempts per launch
     long long target, max_steps;
     double max_time;
     int time_float, batch;
@@ -338,10 +345,19 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
             __hip_atomic_fetch_add(a.barrier, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const unsigned want = phase * (unsigned)G;
             int polls = 0;
-            while (agent_load(a.barrier) < want) {
-                if (++polls > GRID_POLLS) {
+            for (;;) {
+                unsigned v = agent_load(a.barrier);
+                if (v & GRID_GIVE_UP) {
                     sh.give_up = 1;
-                    agent_store(a.barrier + 1, 1u);
+                    break;
+                }
+                if (v >= want) break;
+                // marked only while an arrival is missing: nobody has passed
+                // this exchange, and nobody will
+                if (++polls > a.polls &&
+                    __hip_atomic_compare_exchange_strong(a.barrier, &v, v | GRID_GIVE_UP, __ATOMIC_RELAXED,
+                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                    sh.give_up = 1;
                     break;
                 }
             }
@@ -379,7 +395,7 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
     bool alive = true;
     while (!done && alive) {
         // ---- a step: stage 1 at x
-        if (launched >= GRID_ATTEMPT_CAP) break;      // pause between steps
+        if (launched >= a.attempt_cap) break;         // pause between steps
         double err = 0.0;
         int cnt = 0;
         T hs = (T)h;
@@ -480,6 +496,7 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
             done = true;
         }
     }
+    if (!alive) return;
     // newest state: spins by their owners, each clause by the one that writes it
     if (var) x[var] = R.xv;
 #pragma unroll

@@ -1988,6 +1988,22 @@ static void build_small_lists(Sys* s, const HostProblem& P)
 // (N = 24000, M = 102000, FP32: 68 against 76 us; N = 14000, FP64: 63 against 67).
 constexpr int GRID_CPT_F64 = 4, GRID_CPT_F32 = 8;
 constexpr long long GRID_LDS = 158 * 1024;     // beside the kernel's 0.3 KB of static LDS
+
+// Workgroups of the kernel that the device holds at once; 0 where it cannot
+// launch cooperatively.  A whole MI355X has 256 CUs and holds the largest layout
+// twice, a partition of it may have fewer than the layout has workgroups.
+static int grid_resident(const void* f, size_t lds)
+{
+    int dev = 0, coop = 0, ncu = 0, per_cu = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    HIP_CHECK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+    HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    if (!f || !coop) return 0;
+    HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, GRID_BT, lds));
+    return per_cu * ncu;
+}
+
 static void build_grid(Sys* s, const HostProblem& P)
 {
     const int n = P.n, m = P.m, K = P.k;
@@ -2058,6 +2074,8 @@ static void build_grid(Sys* s, const HostProblem& P)
     const int most_con = *std::max_element(ncon.begin(), ncon.end());
     const long long lds = (long long)s->esize * (nranks + 2 + most_con + 1);
     if (most_con > 65535 || lds > GRID_LDS) return;
+    const int kcpt = cpt <= 1 ? 1 : cpt <= 2 ? 2 : cpt <= 4 ? 4 : 8;
+    if (G > 1 && grid_resident(grid_kernel(s->prec, K, kcpt, false), (size_t)lds) < G) return;
     // entry of every slot: the variable's clauses in input order, literals in
     // clause order (the reference's accumulation order)
     std::vector<int> visit((size_t)m), fill((size_t)n + 1, 0), entry((size_t)m * K, 0);
@@ -2105,7 +2123,7 @@ static void build_grid(Sys* s, const HostProblem& P)
     upload(s->d_ggroup, group);
     upload(s->d_gvmap, vmap);
     s->grid_wgs = G;
-    s->grid_cpt = cpt <= 1 ? 1 : cpt <= 2 ? 2 : cpt <= 4 ? 4 : 8;
+    s->grid_cpt = kcpt;
     s->grid_groups = ng;
     s->grid_lds = lds;
 }
@@ -2556,7 +2574,11 @@ struct RK {
     SmallSolve* h_solve = nullptr;   // pinned mirror
     void* d_grid = nullptr;          // exchange buffers of the few-workgroup path
     size_t grid_bytes = 0;
-    int* h_giveup = nullptr;         // pinned: its give-up flag
+    unsigned* h_arrived = nullptr;   // pinned: its arrival word after a launch
+    bool grid_off = false;           // its workgroups did not all run: not tried again for this problem
+    // test limits (asat_rk_set_grid_limits)
+    int grid_workgroups = 0, grid_launches = -1;
+    long long grid_attempts = 0;
     void* pair[2] = {nullptr, nullptr};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = -1.f;
@@ -2583,7 +2605,7 @@ struct RK {
         for (auto& p : k) dfree(p);
         dfree(tmp); dfree(partial); dfree(d_ctrl); dfree(d_solve); dfree(d_grid);
         grid_bytes = 0;
-        if (h_giveup) { (void)hipHostFree(h_giveup); h_giveup = nullptr; }
+        if (h_arrived) { (void)hipHostFree(h_arrived); h_arrived = nullptr; }
         if (h_ctrl) { (void)hipHostFree(h_ctrl); h_ctrl = nullptr; }
         if (h_solve) { (void)hipHostFree(h_solve); h_solve = nullptr; }
     }
@@ -2629,6 +2651,7 @@ static void rk_configure(RK* r, Sys* s)
     s->require_ready();
     HIP_CHECK(hipStreamSynchronize(s->stream));
     const int npartial = clause_grid(s) + var_grid(s);
+    if (r->sys != s || r->gen != s->gen) r->grid_off = false;
     if (r->configured && r->sys == s && r->alloc == s->alloc && r->prec == s->prec && r->npartial == npartial &&
         r->tmp_n == s->n) {
         // same sizes (SatSolver configures before every Solve): keep the
@@ -2889,7 +2912,8 @@ static SmallArgs small_args(const RK* r, void* x)
 static bool grid_path(const RK* r)
 {
     const Sys* s = r->sys;
-    return r->small_mode && s->grid_wgs > 0 && s->family == ASAT_FAMILY_CTDS && !(s->b > 0.0) && r->timer_kind < 0;
+    return r->small_mode && s->grid_wgs > 0 && !r->grid_off && s->family == ASAT_FAMILY_CTDS && !(s->b > 0.0) &&
+           r->timer_kind < 0 && !(r->grid_workgroups > 0 && s->grid_wgs > r->grid_workgroups);
 }
 
 // the kernel's arguments; a holds what small_args gives plus the loop's limits
@@ -2904,7 +2928,7 @@ static GridArgs grid_args(RK* r, const SmallArgs& a)
         HIP_CHECK(hipMalloc(&r->d_grid, need));
         r->grid_bytes = need;
     }
-    if (!r->h_giveup) HIP_CHECK(hipHostMalloc((void**)&r->h_giveup, sizeof(int), hipHostMallocDefault));
+    if (!r->h_arrived) HIP_CHECK(hipHostMalloc((void**)&r->h_arrived, sizeof(unsigned), hipHostMallocDefault));
     GridArgs g;
     memset(&g, 0, sizeof(g));
     g.code = s->d_gcode; g.cpos = s->d_gcpos; g.wg = s->d_gwg; g.group = s->d_ggroup; g.vmap = s->d_gvmap;
@@ -2918,6 +2942,8 @@ static GridArgs grid_args(RK* r, const SmallArgs& a)
     g.time_float = a.time_float; g.batch = a.batch;
     g.ngroups = s->grid_groups; g.aoff = s->aoff; g.k = s->k;
     g.knorm = a.knorm;
+    g.polls = GRID_POLLS;
+    g.attempt_cap = r->grid_attempts > 0 ? r->grid_attempts : GRID_ATTEMPT_CAP;
     return g;
 }
 
@@ -2933,31 +2959,41 @@ static void grid_launch(RK* r, GridArgs& g)
         HIP_CHECK(hipLaunchKernel(f, dim3(1), dim3(GRID_BT), args, (size_t)s->grid_lds, s->stream));
         return;
     }
-    HIP_CHECK(hipMemsetAsync(g.barrier, 0, 2 * sizeof(unsigned), s->stream));
+    HIP_CHECK(hipMemsetAsync(g.barrier, 0, sizeof(unsigned), s->stream));
     HIP_CHECK(hipLaunchCooperativeKernel(f, dim3(s->grid_wgs), dim3(GRID_BT), args, (unsigned)s->grid_lds, s->stream));
-    HIP_CHECK(hipMemcpyAsync(r->h_giveup, g.barrier + 1, sizeof(int), hipMemcpyDeviceToHost, s->stream));
+    HIP_CHECK(hipMemcpyAsync(r->h_arrived, g.barrier, sizeof(unsigned), hipMemcpyDeviceToHost, s->stream));
 }
 
 // Launches the persistent kernel of either path until it reports done: each
-// launch runs at most SMALL_ATTEMPT_CAP (GRID_ATTEMPT_CAP) attempts and leaves its state in the control block
-// (and the solver block), so the next launch resumes where it stopped.
+// launch runs at most SMALL_ATTEMPT_CAP (GRID_ATTEMPT_CAP) attempts and leaves its
+// state in the control block (and the solver block), so the next launch resumes
+// where it stopped.  False: the workgroups of a launch did not all run, which has
+// changed nothing, and no persistent kernel is left for the problem; the
+// control and solver blocks say how far the launches before it came.
 template <typename T>
-static void small_run(RK* r, const SmallArgs& a)
+static bool small_run(RK* r, const SmallArgs& a)
 {
     Sys* s = r->sys;
     hipStream_t st = s->stream;
     HIP_CHECK(hipEventRecord(r->ev0, st));
     long long last = r->h_ctrl->attempts;
-    const bool grid = grid_path(r);
+    bool grid = grid_path(r), left = true;
     GridArgs g;
     if (grid) g = grid_args(r, a);
-    for (;;) {
+    for (int launch = 0;; launch++) {
+        if (r->grid_launches >= 0 && launch >= r->grid_launches) g.polls = 0;
         if (grid) grid_launch(r, g);
         else small_launch<T>(s, a, st);
         HIP_CHECK(hipMemcpyAsync(r->h_ctrl, r->d_ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, st));
         if (a.solve) HIP_CHECK(hipMemcpyAsync(r->h_solve, r->d_solve, sizeof(SmallSolve), hipMemcpyDeviceToHost, st));
         HIP_CHECK(hipStreamSynchronize(st));
-        require(!grid || s->grid_wgs == 1 || *r->h_giveup == 0, ASAT_ERR_HIP, "the workgroups of the integrator did not all run");
+        if (grid && s->grid_wgs > 1 && (*r->h_arrived & GRID_GIVE_UP)) {
+            r->grid_off = true;
+            grid = false;
+            left = small_path(r);
+            if (left) continue;
+            break;
+        }
         if (r->h_ctrl->underflow) break;
         if (a.solve ? r->h_solve->result >= 0 : r->h_ctrl->steps >= a.target) break;
         require(r->h_ctrl->attempts > last, ASAT_ERR_HIP, "integrator made no progress");
@@ -2966,6 +3002,7 @@ static void small_run(RK* r, const SmallArgs& a)
     HIP_CHECK(hipEventRecord(r->ev1, st));
     HIP_CHECK(hipEventSynchronize(r->ev1));
     HIP_CHECK(hipEventElapsedTime(&r->last_ms, r->ev0, r->ev1));
+    return left;
 }
 
 static void rk_check_states(const RK* r, const State* olds, const State* news)
@@ -2987,9 +3024,9 @@ static int rk_step(RK* r, State* olds, State* news, int count)
         // the state stays in olds; news is not touched
         SmallArgs a = small_args(r, olds->d);
         a.target = r->h_ctrl->steps + count;
-        if (r->prec == ASAT_F64) small_run<double>(r, a);
-        else small_run<float>(r, a);
-        return r->h_ctrl->underflow ? ASAT_UNDERFLOW : ASAT_OK;
+        if (r->prec == ASAT_F64 ? small_run<double>(r, a) : small_run<float>(r, a))
+            return r->h_ctrl->underflow ? ASAT_UNDERFLOW : ASAT_OK;
+        count = (int)(a.target - r->h_ctrl->steps);
     }
     return r->prec == ASAT_F64 ? rk_step_impl<double>(r, olds, news, count)
                                : rk_step_impl<float>(r, olds, news, count);
@@ -3012,6 +3049,12 @@ static void rk_solve(RK* r, State* olds, State* news, int batch, long long max_s
     require(max_steps >= 1, ASAT_ERR_INVALID_ARGUMENT, "Max iterations must be positive");
     require(max_time > 0.0, ASAT_ERR_INVALID_ARGUMENT, "Max time must be positive");
     memset(out, 0, sizeof(*out));
+    // the host loop's state, which starts at the top of the loop or, where the
+    // persistent kernel gave up, where its last full launch stopped
+    long long steps = 0;
+    double time = 0.0;
+    int lastv = 0, result = -1, todo = 0;     // todo: steps left of the batch
+    bool due = false;                         // a batch has ended and its count is due
     if ((small_path(r) || grid_path(r)) && !r->h_ctrl->underflow) {
         SmallSolve init;
         memset(&init, 0, sizeof(init));
@@ -3024,31 +3067,41 @@ static void rk_solve(RK* r, State* olds, State* news, int batch, long long max_s
         a.max_steps = max_steps;
         a.max_time = max_time;
         a.time_float = time_float;
-        if (r->prec == ASAT_F64) small_run<double>(r, a);
-        else small_run<float>(r, a);
-        out->result = r->h_solve->result;
-        out->steps = r->h_solve->solver_steps;
-        out->last_violations = r->h_solve->last_viol;
-        out->on_device = 1;
-        return;
+        if (r->prec == ASAT_F64 ? small_run<double>(r, a) : small_run<float>(r, a)) {
+            out->result = r->h_solve->result;
+            out->steps = r->h_solve->solver_steps;
+            out->last_violations = r->h_solve->last_viol;
+            out->on_device = 1;
+            return;
+        }
+        steps = r->h_solve->solver_steps;
+        time = r->h_ctrl->time;
+        lastv = r->h_solve->last_viol;
+        todo = r->h_solve->bleft;
+        due = r->h_solve->check != 0;
     }
     auto tcmp = [&](double t) { return time_float ? (double)(float)t : t; };
-    long long steps = 0;
-    double time = 0.0;
-    int lastv = 0, result = -1;
-    while (tcmp(time) < max_time && steps < max_steps) {
-        const long long before = r->h_ctrl->steps;
-        if (rk_step(r, olds, news, batch) == ASAT_UNDERFLOW) {
+    for (;;) {
+        if (due) {
+            due = false;
+            lastv = r->prec == ASAT_F64 ? sys_violations<double>(r->sys, olds) : sys_violations<float>(r->sys, olds);
+            if (lastv == 0) {
+                result = SMALL_SAT;
+                break;
+            }
+        }
+        if (todo == 0) {
+            if (!(tcmp(time) < max_time && steps < max_steps)) break;
+            todo = batch;
+        }
+        if (rk_step(r, olds, news, todo) == ASAT_UNDERFLOW) {
             result = SMALL_UNDERFLOW;
             break;
         }
-        steps += r->h_ctrl->steps - before;
+        steps += batch;
         time = r->h_ctrl->time;
-        lastv = r->prec == ASAT_F64 ? sys_violations<double>(r->sys, olds) : sys_violations<float>(r->sys, olds);
-        if (lastv == 0) {
-            result = SMALL_SAT;
-            break;
-        }
+        todo = 0;
+        due = true;
     }
     if (result < 0) {
         if (tcmp(time) >= max_time) result = SMALL_MAXTIME;
@@ -3526,6 +3579,17 @@ int asat_rk_uses_one_workgroup(const asat_rk_t* rk, int* uses)
     CHECK_PTR(rk); CHECK_PTR(uses);
     rk->r.require_configured();
     *uses = small_path(&rk->r) ? 1 : 0;
+    API_END
+}
+
+int asat_rk_set_grid_limits(asat_rk_t* rk, int workgroups, long long attempts, int launches)
+{
+    API_BEGIN
+    CHECK_PTR(rk);
+    require(workgroups >= 0 && attempts >= 0, ASAT_ERR_INVALID_ARGUMENT, "limits must be >= 0");
+    rk->r.grid_workgroups = workgroups;
+    rk->r.grid_attempts = attempts;
+    rk->r.grid_launches = launches;
     API_END
 }
 

@@ -206,12 +206,21 @@ int asat_rk_step(asat_rk_t* rk, asat_state_t* old_state, asat_state_t* new_state
    Step and asat_rk_solve in one persistent single-workgroup kernel, with the
    same arithmetic as the multi-kernel path (bit-identical results); larger
    3- and 4-literal CTDS problems, up to about N = 20 000 in FP64 and 32 000 in
-   FP32, run in one of 8 to 128 workgroups.
+   FP32, run in one of 8 to 128 workgroups where the device holds that many at once.
    enable = 0 forces the multi-kernel path (13 launches per attempt);
    asat_rk_uses_one_workgroup reports whether the configured problem takes the
    single-workgroup kernel. */
 int asat_rk_set_one_workgroup(asat_rk_t* rk, int enable);
 int asat_rk_uses_one_workgroup(const asat_rk_t* rk, int* uses);
+/* Test hook, no reference counterpart: limits of the 8 to 128 workgroup kernel.
+   workgroups: a problem that needs more takes the multi-kernel path, as on a
+   device that does not hold them all at once (0: what the device says);
+   attempts: after so many a launch pauses between steps (0: the default);
+   launches: from this launch of a Step or solve on, a workgroup that has to wait
+   for another at all gives up, as after a long wait for one that does not run;
+   the problem then goes on by the multi-kernel path (negative: none does).
+   Results do not depend on any of them. */
+int asat_rk_set_grid_limits(asat_rk_t* rk, int workgroups, long long attempts, int launches);
 /* SatSolver::DoSolve's loop without a callback (AnalogSAT/solver/SatSolver.h:313-331):
    while (time < max_time && steps < max_steps) { Step(batch); count the
    violated clauses of old_state; stop on 0 }, ending with SAT_UNDERFLOW on
