@@ -199,6 +199,7 @@ def lib():
                                     ctypes.POINTER(SolveResult), ctypes.POINTER(RkStats)], i),
             "asat_rk_set_one_workgroup": ([vp, i], i),
             "asat_rk_uses_one_workgroup": ([vp, ctypes.POINTER(i)], i),
+            "asat_rk_workgroups": ([vp, ctypes.POINTER(i)], i),
             "asat_rk_set_grid_limits": ([vp, i, ctypes.c_longlong, i], i),
             "asat_rk_solve": ([vp, vp, vp, i, ctypes.c_longlong, ctypes.c_double, i, ctypes.POINTER(SolveResult)], i),
             "asat_rk_reset": ([vp], i),
@@ -647,6 +648,13 @@ class HipRungeKutta:
         """Test hook: limits of the 8 to 128 workgroup kernel (most workgroups,
         attempts per launch, launches before a wait is given up at once)."""
         _check(lib().asat_rk_set_grid_limits(self._h, int(workgroups), int(attempts), int(launches)))
+
+    def Workgroups(self):
+        """Workgroups of the persistent kernel that runs the configured problem
+        (0: the multi-kernel path)."""
+        v = ctypes.c_int()
+        _check(lib().asat_rk_workgroups(self._h, ctypes.byref(v)))
+        return v.value
 
     def UsesOneWorkgroup(self):
         v = ctypes.c_int()

@@ -2916,6 +2916,12 @@ static bool grid_path(const RK* r)
            r->timer_kind < 0 && !(r->grid_workgroups > 0 && s->grid_wgs > r->grid_workgroups);
 }
 
+// workgroups of the persistent kernel that runs the problem (0: the multi-kernel path)
+static int persistent_workgroups(const RK* r)
+{
+    return grid_path(r) ? r->sys->grid_wgs : small_path(r) ? 1 : 0;
+}
+
 // the kernel's arguments; a holds what small_args gives plus the loop's limits
 static GridArgs grid_args(RK* r, const SmallArgs& a)
 {
@@ -3578,7 +3584,16 @@ int asat_rk_uses_one_workgroup(const asat_rk_t* rk, int* uses)
     API_BEGIN
     CHECK_PTR(rk); CHECK_PTR(uses);
     rk->r.require_configured();
-    *uses = small_path(&rk->r) ? 1 : 0;
+    *uses = small_path(&rk->r) && persistent_workgroups(&rk->r) == 1 ? 1 : 0;
+    API_END
+}
+
+int asat_rk_workgroups(const asat_rk_t* rk, int* workgroups)
+{
+    API_BEGIN
+    CHECK_PTR(rk); CHECK_PTR(workgroups);
+    rk->r.require_configured();
+    *workgroups = persistent_workgroups(&rk->r);
     API_END
 }
 

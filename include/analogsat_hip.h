@@ -207,11 +207,14 @@ int asat_rk_step(asat_rk_t* rk, asat_state_t* old_state, asat_state_t* new_state
    same arithmetic as the multi-kernel path (bit-identical results); larger
    3- and 4-literal CTDS problems, up to about N = 20 000 in FP64 and 32 000 in
    FP32, run in one of 8 to 128 workgroups where the device holds that many at once.
-   enable = 0 forces the multi-kernel path (13 launches per attempt);
-   asat_rk_uses_one_workgroup reports whether the configured problem takes the
-   single-workgroup kernel. */
+   enable = 0 forces the multi-kernel path (13 launches per attempt).
+   asat_rk_workgroups reports in how many workgroups of a persistent kernel Step
+   and asat_rk_solve run the configured problem (0: the multi-kernel path);
+   asat_rk_uses_one_workgroup whether it fits the single-workgroup kernel and runs
+   in one workgroup. */
 int asat_rk_set_one_workgroup(asat_rk_t* rk, int enable);
 int asat_rk_uses_one_workgroup(const asat_rk_t* rk, int* uses);
+int asat_rk_workgroups(const asat_rk_t* rk, int* workgroups);
 /* Test hook, no reference counterpart: limits of the 8 to 128 workgroup kernel.
    workgroups: a problem that needs more takes the multi-kernel path, as on a
    device that does not hold them all at once (0: what the device says);

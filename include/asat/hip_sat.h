@@ -253,6 +253,8 @@ public:
     // allow (default) or forbid the persistent paths: one workgroup for problems
     // whose integrator fits in its LDS, 8 to 128 for larger ones
     void SetOneWorkgroup(bool enable) { HipSafe(asat_rk_set_one_workgroup(h, enable ? 1 : 0)); }
+    // workgroups of the persistent kernel that runs the configured problem (0: multi-kernel path)
+    int GetWorkgroups() const { int n = 0; HipSafe(asat_rk_workgroups(h, &n)); return n; }
 
 private:
     asat_rk_t* h = nullptr;

@@ -1,0 +1,45 @@
+"""Which integrator runs: the number of workgroups that the query reports, for sizes
+on both sides of each rule and for the settings that rule a path out."""
+import pytest
+
+import analogsat_amd as A
+
+pytestmark = pytest.mark.gpu
+
+
+def configured(prec, n, m, k=3, family="ctds"):
+    sat = A.HipSatTanh(prec) if family == "tanh" else A.HipSat(prec)
+    sat.SetProblem(A.fastsat(n, m, k, 2))
+    rk = A.HipRungeKutta()
+    rk.Configure(sat)
+    return sat, rk
+
+
+@pytest.mark.parametrize("prec,n,m,k,fewest,most,one", [
+    ("f64", 50, 213, 3, 1, 1, True), ("f64", 200, 852, 3, 1, 1, True),      # fits one workgroup's LDS
+    ("f64", 450, 1900, 3, 1, 1, False), ("f64", 200, 1990, 4, 1, 1, False),  # one workgroup, state in registers
+    ("f32", 1100, 1500, 3, 8, 128, False),                                  # fits that LDS, but runs in eight
+    ("f64", 650, 2800, 3, 8, 128, False), ("f32", 24000, 102000, 3, 8, 128, False),
+    ("f64", 30000, 127500, 3, 0, 0, False), ("f64", 20, 600, 5, 1, 1, True)])
+def test_workgroups(prec, n, m, k, fewest, most, one):
+    sat, rk = configured(prec, n, m, k)
+    print("[gpu-paths]", prec, n, m, k, rk.Workgroups(), flush=True)
+    assert fewest <= rk.Workgroups() <= most
+    assert rk.UsesOneWorkgroup() == one
+    rk.SetOneWorkgroup(False)
+    assert rk.Workgroups() == 0 and not rk.UsesOneWorkgroup()
+
+
+def test_settings_that_rule_a_path_out():
+    sat, rk = configured("f64", 2000, 8500)
+    assert rk.Workgroups() >= 8
+    rk.SetGridLimits(workgroups=7)
+    assert rk.Workgroups() == 0
+    rk.SetGridLimits()
+    assert rk.Workgroups() >= 8
+    sat.Set_B(2.0)
+    assert rk.Workgroups() == 0
+    sat.Set_B(0.0)
+    assert rk.Workgroups() >= 8
+    assert configured("f64", 2000, 8500, family="tanh")[1].Workgroups() == 0
+    assert configured("f64", 50, 213, family="tanh")[1].Workgroups() == 1
