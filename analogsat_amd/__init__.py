@@ -646,7 +646,7 @@ class HipRungeKutta:
 
     def SetGridLimits(self, workgroups=0, attempts=0, launches=-1):
         """Test hook: limits of the 8 to 128 workgroup kernel (most workgroups,
-        attempts per launch, launches before a wait is given up at once)."""
+        attempts per launch, the launch whose first workgroup gives up)."""
         _check(lib().asat_rk_set_grid_limits(self._h, int(workgroups), int(attempts), int(launches)))
 
     def Workgroups(self):

@@ -75,7 +75,7 @@ struct GridArgs {
     double* err;             // [2][GRID_MAX] error maxima
     int* count;              // [2][GRID_MAX] violated clauses
     unsigned* barrier;       // arrivals, and GRID_GIVE_UP; cleared before the launch
-    int polls;               // of a wait before it is given up
+    int polls;               // of a wait before it is given up (< 0: the first workgroup gives up instead of arriving)
     long long attempt_cap;   // attempts per launch
     long long target, max_steps;
     double max_time;
@@ -342,10 +342,15 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
                 agent_store(a.count + half * GRID_MAX + w, m);
             }
             if constexpr (ERR || CNT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __hip_atomic_fetch_add(a.barrier, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const unsigned want = phase * (unsigned)G;
             int polls = 0;
-            for (;;) {
+            if (a.polls < 0 && w == 0) {
+                __hip_atomic_fetch_or(a.barrier, GRID_GIVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                sh.give_up = 1;
+            } else {
+                __hip_atomic_fetch_add(a.barrier, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            while (!sh.give_up) {
                 unsigned v = agent_load(a.barrier);
                 if (v & GRID_GIVE_UP) {
                     sh.give_up = 1;
@@ -354,7 +359,7 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
                 if (v >= want) break;
                 // marked only while an arrival is missing: nobody has passed
                 // this exchange, and nobody will
-                if (++polls > a.polls &&
+                if (++polls > a.polls && a.polls >= 0 &&
                     __hip_atomic_compare_exchange_strong(a.barrier, &v, v | GRID_GIVE_UP, __ATOMIC_RELAXED,
                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                     sh.give_up = 1;

@@ -2987,7 +2987,7 @@ static bool small_run(RK* r, const SmallArgs& a)
     GridArgs g;
     if (grid) g = grid_args(r, a);
     for (int launch = 0;; launch++) {
-        if (r->grid_launches >= 0 && launch >= r->grid_launches) g.polls = 0;
+        if (r->grid_launches >= 0 && launch >= r->grid_launches) g.polls = -1;
         if (grid) grid_launch(r, g);
         else small_launch<T>(s, a, st);
         HIP_CHECK(hipMemcpyAsync(r->h_ctrl, r->d_ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, st));

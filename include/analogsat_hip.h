@@ -219,9 +219,9 @@ int asat_rk_workgroups(const asat_rk_t* rk, int* workgroups);
    workgroups: a problem that needs more takes the multi-kernel path, as on a
    device that does not hold them all at once (0: what the device says);
    attempts: after so many a launch pauses between steps (0: the default);
-   launches: from this launch of a Step or solve on, a workgroup that has to wait
-   for another at all gives up, as after a long wait for one that does not run;
-   the problem then goes on by the multi-kernel path (negative: none does).
+   launches: in this launch of a Step or solve the first workgroup gives up, as
+   after a long wait for one that does not run; the problem then goes on by the
+   multi-kernel path (negative: in none).
    Results do not depend on any of them. */
 int asat_rk_set_grid_limits(asat_rk_t* rk, int workgroups, long long attempts, int launches);
 /* SatSolver::DoSolve's loop without a callback (AnalogSAT/solver/SatSolver.h:313-331):
