@@ -57,6 +57,7 @@
 #include "asat_small.h"
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -104,8 +105,10 @@ struct HostProblem {
     std::vector<long long> gstart; // ngroups+1
     std::vector<int> pos;          // m*k: the slot's contribution position, -1 for padding
     std::vector<int> csr_ptr;      // n+2
-    std::vector<int> csr_pos;      // contribution positions of each variable, in slot order
-    std::vector<uint16_t> csr_loc; // the same relative to the variable's region start (primary terms past its end)
+    std::vector<int> csr_pos;      // gather var pass: contribution positions of each variable, in slot order
+    // LDS var pass: each region entry's place in its group's var-major slot list
+    // (entries of no slot: past the list), and each clause's direct primary term's
+    std::vector<uint16_t> rloc, ploc;
     // tiled clause pass: per tile of TC clauses, its slots sorted by position
     std::vector<int> spos;         // ntiles*TC*k positions (-1 past the tile's last slot)
     // big tiles: per tile, a run table in place of spos.
@@ -224,29 +227,38 @@ static void reorder_clauses(HostProblem& P)
 // var-major slot list (role of CudaSat3::InitProblem,
 // AnalogSAT/cuda_sat/CudaSat3.cu:266-307, without the pad-to-32).
 // pv > 0 (tiled pass with primary variables): direct primary slots.  The
-// regions then hold only the other slots, and a variable's list entry for a
-// primary slot points past its group's region: the LDS var pass loads the
-// group's primary terms (pcontrib from pc0[g] rounded down to a multiple of pv
-// elements, its 16-byte load unit) right behind the region.
-static void build_layout(HostProblem& P, int vg, int pv)
+// regions then hold only the other slots, and the LDS var pass reads the
+// group's primary terms from pcontrib (from pc0[g] rounded down to a multiple of
+// pv elements, its 16-byte load unit).
+// cap > 0: for the LDS var pass; false, with nothing but the regions' sizes made,
+// when the largest region with its primary terms exceeds cap entries.
+static bool build_layout(HostProblem& P, int vg, int pv, long long cap)
 {
-    const int n = P.n, K = P.k;
+    const int n = P.n, m = P.m, K = P.k;
     const bool split = pv > 0 && !P.pvar.empty();
     P.split = split;
     P.vg = vg;
     P.ngroups = (n + vg - 1) / vg;
-    auto is_prim = [&](size_t s) { return split && P.pq[s / K] == (unsigned char)(s % K); };
+    std::vector<int> grp((size_t)n + 1, 0);
+    for (int v = 1; v <= n; v++) grp[(size_t)v] = (v - 1) / vg;
+    // f(slot, clause, variable, the clause's primary slot?) over all literals
+    auto each = [&](auto f) {
+        for (int j = 0; j < m; j++) {
+            const int pq = split ? P.pq[(size_t)j] : -1;
+            for (int q = 0; q < K; q++) {
+                const size_t s = (size_t)j * K + q;
+                if (P.lit[s]) f(s, j, std::abs(P.lit[s]), q == pq);
+            }
+        }
+    };
     std::vector<long long> gcount((size_t)P.ngroups, 0);
-    for (size_t s = 0; s < P.lit.size(); s++) {
-        int l = P.lit[s];
-        if (l && !is_prim(s)) gcount[(size_t)(std::abs(l) - 1) / vg]++;
-    }
+    each([&](size_t, int, int v, bool prim) { gcount[(size_t)grp[(size_t)v]] += !prim; });
     P.pc0.clear();
     if (split) {
         // clauses are sorted by primary variable: group g's primaries are the
         // processing range [pc0[g], pc0[g+1])
-        P.pc0.assign((size_t)P.ngroups + 1, P.m);
-        for (int j = P.m - 1; j >= 0; j--) P.pc0[(size_t)(P.pvar[(size_t)j] - 1) / vg] = j;
+        P.pc0.assign((size_t)P.ngroups + 1, m);
+        for (int j = m - 1; j >= 0; j--) P.pc0[(size_t)grp[(size_t)P.pvar[(size_t)j]]] = j;
         for (int g = P.ngroups - 1; g >= 0; g--) P.pc0[g] = std::min(P.pc0[g], P.pc0[(size_t)g + 1]);
     }
     P.gstart.assign((size_t)P.ngroups + 1, 0);
@@ -258,49 +270,49 @@ static void build_layout(HostProblem& P, int vg, int pv)
         if (split) lds += round_up(P.pc0[(size_t)g + 1] - (P.pc0[g] / pv) * pv, pv);
         P.max_region = std::max(P.max_region, lds);
     }
+    if (cap > 0 && P.max_region > cap) return false;
     require(P.gstart[P.ngroups] < (1LL << 31), ASAT_ERR_UNSUPPORTED, "contribution array exceeds 2^31 entries");
     P.pos.assign(P.lit.size(), -1);
-    std::vector<long long> gfill(P.gstart.begin(), P.gstart.end() - 1);
-    for (size_t s = 0; s < P.lit.size(); s++) {
-        int l = P.lit[s];
-        if (l && !is_prim(s)) P.pos[s] = (int)gfill[(size_t)(std::abs(l) - 1) / vg]++;
-    }
-    // per-variable lists of contribution positions; slots visited in the
-    // original clause order, which is the reference's accumulation order
     P.csr_ptr.assign((size_t)n + 2, 0);
-    for (size_t s = 0; s < P.lit.size(); s++) {
-        int l = P.lit[s];
-        if (l) P.csr_ptr[(size_t)std::abs(l) + 1]++;
-    }
+    std::vector<long long> gfill(P.gstart.begin(), P.gstart.end() - 1);
+    each([&](size_t s, int, int v, bool prim) {
+        if (!prim) P.pos[s] = (int)gfill[(size_t)grp[(size_t)v]]++;
+        P.csr_ptr[(size_t)v + 1]++;
+    });
     for (int i = 0; i <= n; i++) P.csr_ptr[i + 1] += P.csr_ptr[i];
-    P.csr_pos.assign((size_t)P.csr_ptr[n + 1], 0);
-    std::vector<long long> cloc(split ? P.csr_pos.size() : 0);
+    // the variables' slot lists; slots visited in the original clause order,
+    // which is the reference's accumulation order
+    std::vector<int> row((size_t)m);
+    for (int j = 0; j < m; j++) row[P.perm.empty() ? j : P.perm[j]] = j;
+    P.csr_pos.clear();
+    P.rloc.clear();
+    P.ploc.clear();
     std::vector<int> fill(P.csr_ptr.begin(), P.csr_ptr.end() - 1);
-    std::vector<int> row((size_t)P.m);
-    for (int j = 0; j < P.m; j++) row[P.perm.empty() ? j : P.perm[j]] = j;
-    for (int mo = 0; mo < P.m; mo++)
-        for (int q = 0; q < K; q++) {
-            const size_t s = (size_t)row[mo] * K + q;
-            int l = P.lit[s];
-            if (!l) continue;
-            const int v = std::abs(l);
-            const int e = fill[v]++;
-            P.csr_pos[(size_t)e] = P.pos[s];
-            if (split) {
-                const size_t g = (size_t)(v - 1) / vg;
-                cloc[(size_t)e] = is_prim(s) ? (P.gstart[g + 1] - P.gstart[g]) + row[mo] - (P.pc0[g] / pv) * pv
-                                             : P.pos[s] - P.gstart[g];
-            }
+    if (cap > 0) {
+        // cursors relative to the group's list
+        P.rloc.resize((size_t)P.gstart[P.ngroups]);
+        if (split) P.ploc.resize((size_t)m);
+        for (int g = 0; g < P.ngroups; g++) {
+            const int i0 = g * vg + 1, i1 = std::min(n, (g + 1) * vg), e0 = P.csr_ptr[i0];
+            for (int v = i0; v <= i1; v++) fill[(size_t)v] -= e0;
+            std::fill(P.rloc.begin() + P.gstart[g], P.rloc.begin() + P.gstart[(size_t)g + 1],
+                      (uint16_t)(P.csr_ptr[i1 + 1] - e0));
         }
-    P.csr_loc.clear();
-    if (P.max_region <= 65536) {
-        P.csr_loc.resize(P.csr_pos.size());
-        for (int i = 1; i <= n; i++) {
-            const long long base = P.gstart[(size_t)(i - 1) / vg];
-            for (int e = P.csr_ptr[i]; e < P.csr_ptr[i + 1]; e++)
-                P.csr_loc[e] = (uint16_t)(split ? cloc[(size_t)e] : P.csr_pos[e] - base);
+    } else {
+        P.csr_pos.resize((size_t)P.csr_ptr[n + 1]);
+    }
+    for (int mo = 0; mo < m; mo++) {
+        const int j = row[(size_t)mo], pq = split ? P.pq[(size_t)j] : -1;
+        for (int q = 0; q < K; q++) {
+            const size_t s = (size_t)j * K + q;
+            if (!P.lit[s]) continue;
+            const int e = fill[(size_t)std::abs(P.lit[s])]++;
+            if (cap == 0) P.csr_pos[(size_t)e] = P.pos[s];
+            else if (q == pq) P.ploc[(size_t)j] = (uint16_t)e;
+            else P.rloc[(size_t)P.pos[s]] = (uint16_t)e;
         }
     }
+    return true;
 }
 
 // Per tile of TC clauses: the tile's slots in ascending position order.
@@ -1845,10 +1857,13 @@ struct Sys {
     int nlist = 0;
     int runlen = 0;                // uniform run length of the lists (0: ragged)
     long long small_lds = 0;
-    // few-workgroup persistent path (asat_grid.h); grid_wgs = 0 when the problem
-    // does not use it
-    uint32_t* d_gcode = nullptr;
-    int *d_gcpos = nullptr, *d_gwg = nullptr, *d_ggroup = nullptr, *d_gvmap = nullptr;
+    // few-workgroup persistent path (asat_grid.h), laid out when an integrator
+    // first asks for it; grid_wgs = 0 when the problem does not use it
+    std::mutex grid_lock;
+    std::atomic<bool> grid_due{false};   // the problem may use it and has not been laid out
+    int* d_grid = nullptr;               // one block: the arrays below
+    const uint32_t* d_gcode = nullptr;
+    const int *d_gcpos = nullptr, *d_gwg = nullptr, *d_ggroup = nullptr, *d_gvmap = nullptr;
     int grid_wgs = 0, grid_cpt = 0, grid_groups = 0;
     long long grid_lds = 0;
     int vg = 0, ngroups = 0, vg_blocks = 0;
@@ -1881,8 +1896,9 @@ struct Sys {
         dfree(d_pvar); dfree(d_pc0); dfree(d_pcontrib); dfree(d_pw16); dfree(d_pv0);
         split = false;
         dfree(d_vptr); dfree(d_spos_small); dfree(d_public);
-        dfree(d_gcode); dfree(d_gcpos); dfree(d_gwg); dfree(d_ggroup); dfree(d_gvmap);
+        dfree(d_grid);
         grid_wgs = 0;
+        grid_due = false;
         perm.clear();
         nlist = 0;
         runlen = 0;
@@ -1940,12 +1956,11 @@ static bool choose_layout(HostProblem& P, int esize)
     // (primary variables exist only for the tiled pass's clause order)
     const int pv = 16 / esize;
     for (;;) {
-        build_layout(P, vg, pv);
-        if (P.max_region <= cap && !P.csr_loc.empty()) return true;
+        if (build_layout(P, vg, pv, cap)) return true;
         if (vg <= 64) break;
         vg = (vg + 1) / 2;
     }
-    build_layout(P, esize == 4 ? 8192 : 4096, 0);
+    build_layout(P, esize == 4 ? 8192 : 4096, 0, 0);
     return false;
 }
 
@@ -1957,6 +1972,7 @@ static bool choose_layout(HostProblem& P, int esize)
 static void build_small_lists(Sys* s, const HostProblem& P)
 {
     const int n = P.n, m = P.m, K = P.k;
+    if (small_lds_bytes(n, m, K, s->alloc, 0, s->esize) > SMALL_LDS_MAX) return;    // without any list
     std::vector<int> vptr((size_t)n + 2), spos((size_t)m * K), visit;
     if (!P.perm.empty()) {
         visit.resize((size_t)m);
@@ -2004,18 +2020,15 @@ static int grid_resident(const void* f, size_t lds)
     return per_cu * ncu;
 }
 
-static void build_grid(Sys* s, const HostProblem& P)
+// lit: m K literals in processing order, as SetProblem left them
+static void build_grid(Sys* s, const std::vector<int>& lit)
 {
-    const int n = P.n, m = P.m, K = P.k;
+    const int n = s->n, m = s->m, K = s->k;
     const int ng = ceil_div(n, 64), nranks = 64 * ng;
-    if (nranks + 2 > 32766 || (long long)s->esize * nranks > GRID_LDS) return;
-    const int cpt_max = s->esize == 8 ? GRID_CPT_F64 : GRID_CPT_F32;
-    if (m > (long long)GRID_MAX * GRID_BT * cpt_max) return;
+    const size_t slots = (size_t)m * K;
     std::vector<int> deg((size_t)n + 1, 0);
-    for (long long q = 0; q < (long long)m * K; q++) {
-        const int l = P.lit[(size_t)q];
-        if (l) deg[(size_t)std::abs(l)]++;
-    }
+    for (size_t sl = 0; sl < slots; sl++)
+        if (lit[sl]) deg[(size_t)std::abs(lit[sl])]++;
     int top = 0;
     for (int v = 1; v <= n; v++) top = std::max(top, deg[(size_t)v]);
     std::vector<int> vmap((size_t)nranks, 0), rank((size_t)n + 1, 0), at((size_t)top + 2, 0);
@@ -2026,19 +2039,23 @@ static void build_grid(Sys* s, const HostProblem& P)
         rank[(size_t)v] = r;
         vmap[(size_t)r] = v;
     }
-    // the workgroups of a clause, the first literal's first (it writes the clause)
+    // the rank of every slot's variable, -1 for padding (a clause's last literals)
+    std::vector<int> srank(slots);
+    for (size_t sl = 0; sl < slots; sl++) srank[sl] = lit[sl] ? rank[(size_t)std::abs(lit[sl])] : -1;
+    // the workgroups of a clause, the first literal's first (it writes the clause);
+    // g: workgroups, a power of two
     auto owners = [&](int j, int g, int (&w)[4]) {
+        const int* r = srank.data() + (size_t)j * K;
         int ns = 0;
-        for (int q = 0; q < K; q++) {
-            const int l = P.lit[(size_t)j * K + q];
-            if (!l) continue;
-            const int x = (rank[(size_t)std::abs(l)] / 64) % g;
+        for (int q = 0; q < K && r[q] >= 0; q++) {
+            const int x = (r[q] >> 6) & (g - 1);
             bool dup = false;
-            for (int i = 0; i < ns; i++) dup = dup || w[i] == x;
+            for (int i = 0; i < ns; i++) dup |= w[i] == x;
             if (!dup) w[ns++] = x;
         }
         return ns;
     };
+    const int cpt_max = s->esize == 8 ? GRID_CPT_F64 : GRID_CPT_F32;
     std::vector<int> nwrite((size_t)GRID_MAX), nother((size_t)GRID_MAX);
     int G = 0, most = 0, w4[4];
     // one workgroup alone while its threads hold the clauses (us per attempt
@@ -2054,7 +2071,8 @@ static void build_grid(Sys* s, const HostProblem& P)
         std::fill(nother.begin(), nother.end(), 0);
         for (int j = 0; j < m; j++) {
             const int ns = owners(j, g, w4);
-            for (int i = 0; i < ns; i++) (i ? nother : nwrite)[(size_t)w4[i]]++;
+            nwrite[(size_t)w4[0]]++;
+            for (int i = 1; i < ns; i++) nother[(size_t)w4[i]]++;
         }
         most = 0;
         for (int w = 0; w < g; w++) most = std::max(most, nwrite[(size_t)w] + nother[(size_t)w]);
@@ -2076,17 +2094,21 @@ static void build_grid(Sys* s, const HostProblem& P)
     if (most_con > 65535 || lds > GRID_LDS) return;
     const int kcpt = cpt <= 1 ? 1 : cpt <= 2 ? 2 : cpt <= 4 ? 4 : 8;
     if (G > 1 && grid_resident(grid_kernel(s->prec, K, kcpt, false), (size_t)lds) < G) return;
-    // entry of every slot: the variable's clauses in input order, literals in
-    // clause order (the reference's accumulation order)
-    std::vector<int> visit((size_t)m), fill((size_t)n + 1, 0), entry((size_t)m * K, 0);
-    for (int p = 0; p < m; p++) visit[(size_t)(P.perm.empty() ? p : P.perm[(size_t)p])] = p;
+    // term entry of every slot in its variable's workgroup: the variable's clauses
+    // in input order, literals in clause order (the reference's accumulation order)
+    std::vector<int> visit((size_t)m), fill((size_t)nranks), entry(slots);
+    for (int p = 0; p < m; p++) visit[(size_t)(s->perm.empty() ? p : s->perm[(size_t)p])] = p;
+    for (int r = 0; r < nranks; r++) fill[(size_t)r] = group[(size_t)2 * (r / 64)] + r % 64;
     for (int c = 0; c < m; c++)
         for (int q = 0; q < K; q++) {
             const size_t sl = (size_t)visit[(size_t)c] * K + q;
-            if (P.lit[sl]) entry[sl] = fill[(size_t)std::abs(P.lit[sl])]++;
+            if (srank[sl] < 0) break;
+            entry[sl] = fill[(size_t)srank[sl]];
+            fill[(size_t)srank[sl]] += 64;
         }
-    std::vector<int> wg((size_t)4 * G), fw((size_t)G), fo((size_t)G);
     int total = 0;
+    std::vector<int> fw((size_t)G), fo((size_t)G);
+    std::vector<int> wg((size_t)4 * G);
     for (int w = 0; w < G; w++) {
         const int nw = nwrite[(size_t)w], nc = nw + nother[(size_t)w];
         wg[(size_t)4 * w] = total;
@@ -2097,35 +2119,64 @@ static void build_grid(Sys* s, const HostProblem& P)
         fo[(size_t)w] = total + nw;
         total += nc;
     }
-    std::vector<uint32_t> code((size_t)total * K);
-    std::vector<int> cpos((size_t)total);
+    // one block: codes, positions, workgroups, groups, rank -> variable
+    std::vector<int> blk;
+    const size_t ncode = (size_t)total * K;
+    blk.reserve(ncode + (size_t)total + wg.size() + group.size() + vmap.size());
+    blk.resize(ncode + (size_t)total);
     for (int j = 0; j < m; j++) {
         const int ns = owners(j, G, w4);
         for (int i = 0; i < ns; i++) {
             const int w = w4[i], to = (i ? fo : fw)[(size_t)w]++;
-            cpos[(size_t)to] = j;
+            blk[ncode + (size_t)to] = j;
             for (int q = 0; q < K; q++) {
                 const size_t sl = (size_t)j * K + q;
-                const int l = P.lit[sl];
+                const int r = srank[sl];
                 uint32_t where = (uint32_t)ncon[(size_t)w], rk = (uint32_t)nranks;
-                if (l) {
-                    rk = (uint32_t)rank[(size_t)std::abs(l)];
-                    const int g = (int)rk / 64;
-                    if (g % G == w) where = (uint32_t)(group[(size_t)2 * g] + 64 * entry[sl] + (int)(rk % 64));
+                if (r >= 0) {
+                    rk = (uint32_t)r;
+                    if (((r >> 6) & (G - 1)) == w) where = (uint32_t)entry[sl];
                 }
-                code[(size_t)to * K + q] = (where << 16) | (rk << 1) | (l < 0 ? 1u : 0u);
+                blk[(size_t)to * K + q] = (int)((where << 16) | (rk << 1) | (lit[sl] < 0 ? 1u : 0u));
             }
         }
     }
-    upload(s->d_gcode, code);
-    upload(s->d_gcpos, cpos);
-    upload(s->d_gwg, wg);
-    upload(s->d_ggroup, group);
-    upload(s->d_gvmap, vmap);
-    s->grid_wgs = G;
+    blk.insert(blk.end(), wg.begin(), wg.end());
+    blk.insert(blk.end(), group.begin(), group.end());
+    blk.insert(blk.end(), vmap.begin(), vmap.end());
+    upload(s->d_grid, blk);
+    s->d_gcode = (const uint32_t*)s->d_grid;
+    s->d_gcpos = s->d_grid + ncode;
+    s->d_gwg = s->d_gcpos + total;
+    s->d_ggroup = s->d_gwg + wg.size();
+    s->d_gvmap = s->d_ggroup + group.size();
     s->grid_cpt = kcpt;
     s->grid_groups = ng;
     s->grid_lds = lds;
+    s->grid_wgs = G;
+}
+
+// The layout, at the first integrator that can use it: a system that only serves
+// GetDerivatives, the tanh family or a bias term never pays for it (N = 2000,
+// M = 8500: 0.54 ms of SetProblem's 1.7).  Integrators of one system may ask from
+// several threads.  Without memory for it the problem goes without.
+static void ensure_grid(Sys* s)
+{
+    if (!s->grid_due) return;
+    std::lock_guard<std::mutex> lock(s->grid_lock);
+    if (!s->grid_due) return;
+    const int nranks = 64 * ceil_div(s->n, 64), cpt = s->esize == 8 ? GRID_CPT_F64 : GRID_CPT_F32;
+    if (nranks + 2 <= 32766 && (long long)s->esize * nranks <= GRID_LDS && s->m <= (long long)GRID_MAX * GRID_BT * cpt) {
+        std::vector<int> lit((size_t)s->m * s->k);
+        HIP_CHECK(hipMemcpy(lit.data(), s->d_lit, sizeof(int) * lit.size(), hipMemcpyDeviceToHost));
+        try {
+            build_grid(s, lit);
+        } catch (const Error&) {
+            (void)hipGetLastError();
+            dfree(s->d_grid);
+        }
+    }
+    s->grid_due = false;
 }
 
 static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclauses)
@@ -2263,28 +2314,15 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
     }
     upload(s->d_csr_ptr, P.csr_ptr);
     if (lds_var) {
-        // the inverse of the variables' lists; entries of no slot go past the list
-        std::vector<uint16_t> rloc((size_t)P.gstart[P.ngroups]), ploc(P.split ? mpad + 16 : 0, 0);
-        for (int g = 0; g < P.ngroups; g++) {
-            const int i0 = g * P.vg + 1, i1 = std::min(P.n, (g + 1) * P.vg);
-            const int e0 = P.csr_ptr[i0], e1 = P.csr_ptr[i1 + 1];
-            const long long r0 = P.gstart[g], rlen = P.gstart[(size_t)g + 1] - r0;
-            std::fill(rloc.begin() + r0, rloc.begin() + r0 + rlen, (uint16_t)(e1 - e0));
-            const int v16 = 16 / s->esize;
-            for (int e = e0; e < e1; e++) {
-                const long long o = P.csr_loc[(size_t)e];
-                if (o < rlen) rloc[(size_t)(r0 + o)] = (uint16_t)(e - e0);
-                else ploc[(size_t)(P.pc0[g] / v16 * v16 + o - rlen)] = (uint16_t)(e - e0);
-            }
+        upload(s->d_rloc, P.rloc);
+        if (P.split) {
+            P.ploc.resize(mpad + 16, 0);
+            upload(s->d_ploc, P.ploc);
         }
-        upload(s->d_rloc, rloc);
-        if (P.split) upload(s->d_ploc, ploc);
     }
     else if (!s->wide_run) upload(s->d_csr_pos, P.csr_pos);
     upload(s->d_gstart, P.gstart);
     build_small_lists(s, P);
-    // up to 512 clauses and variables asat_small.h is the faster one
-    if (tiled && (s->small_lds == 0 || std::max(P.m, P.n) > 512)) build_grid(s, P);
     if (!P.perm.empty()) upload(s->d_perm, P.perm);
     s->perm = std::move(P.perm);
     const size_t ncontrib = (size_t)P.gstart[P.ngroups] + REGION_ALIGN;
@@ -2292,6 +2330,8 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
     HIP_CHECK(hipMemset(s->d_contrib, 0, (size_t)s->esize * ncontrib));
     HIP_CHECK(hipMalloc((void**)&s->d_apart, sizeof(double) * clause_grid(s)));
     HIP_CHECK(hipMemset(s->d_apart, 0, sizeof(double) * clause_grid(s)));
+    // up to 512 clauses and variables asat_small.h is the faster one
+    s->grid_due = tiled && (s->small_lds == 0 || std::max(P.m, P.n) > 512);
     s->ready = true;
 }
 
@@ -2575,7 +2615,8 @@ struct RK {
     void* d_grid = nullptr;          // exchange buffers of the few-workgroup path
     size_t grid_bytes = 0;
     unsigned* h_arrived = nullptr;   // pinned: its arrival word after a launch
-    bool grid_off = false;           // its workgroups did not all run: not tried again for this problem
+    bool grid_off = false;           // its workgroups did not all run, or it had no memory: not tried again for
+                                     // this problem
     // test limits (asat_rk_set_grid_limits)
     int grid_workgroups = 0, grid_launches = -1;
     long long grid_attempts = 0;
@@ -2644,7 +2685,7 @@ static void rk_reset(RK* r)
 }
 
 static bool small_path(const RK* r);
-static bool grid_path(const RK* r);
+static bool grid_path(RK* r);
 
 static void rk_configure(RK* r, Sys* s)
 {
@@ -2667,6 +2708,7 @@ static void rk_configure(RK* r, Sys* s)
             HIP_CHECK(hipMemsetAsync(r->tmp, 0, (size_t)s->esize * (s->n + 1), s->stream));
             HIP_CHECK(hipMemsetAsync(r->partial, 0, sizeof(double) * r->npartial, s->stream));
         }
+        (void)grid_path(r);     // its layout, where the problem has one
         rk_reset(r);
         return;
     }
@@ -2696,6 +2738,7 @@ static void rk_configure(RK* r, Sys* s)
     if (!r->ev0) HIP_CHECK(hipEventCreate(&r->ev0));
     if (!r->ev1) HIP_CHECK(hipEventCreate(&r->ev1));
     r->configured = true;
+    (void)grid_path(r);
     rk_reset(r);
 }
 
@@ -2906,24 +2949,26 @@ static SmallArgs small_args(const RK* r, void* x)
 }
 
 // ---------------------------------------------------------------------------
-// few-workgroup path (asat_grid.h), for the problems SetProblem laid it out for;
+// few-workgroup path (asat_grid.h), for the problems it can be laid out for;
 // the same conditions as the one-workgroup path, CTDS family only
 // ---------------------------------------------------------------------------
-static bool grid_path(const RK* r)
+static bool grid_path(RK* r)
 {
-    const Sys* s = r->sys;
-    return r->small_mode && s->grid_wgs > 0 && !r->grid_off && s->family == ASAT_FAMILY_CTDS && !(s->b > 0.0) &&
-           r->timer_kind < 0 && !(r->grid_workgroups > 0 && s->grid_wgs > r->grid_workgroups);
+    Sys* s = r->sys;
+    if (!r->small_mode || r->grid_off || s->family != ASAT_FAMILY_CTDS || s->b > 0.0 || r->timer_kind >= 0) return false;
+    ensure_grid(s);
+    return s->grid_wgs > 0 && !(r->grid_workgroups > 0 && s->grid_wgs > r->grid_workgroups);
 }
 
 // workgroups of the persistent kernel that runs the problem (0: the multi-kernel path)
-static int persistent_workgroups(const RK* r)
+static int persistent_workgroups(RK* r)
 {
     return grid_path(r) ? r->sys->grid_wgs : small_path(r) ? 1 : 0;
 }
 
-// the kernel's arguments; a holds what small_args gives plus the loop's limits
-static GridArgs grid_args(RK* r, const SmallArgs& a)
+// the kernel's arguments; a holds what small_args gives plus the loop's limits.
+// False without memory for the exchange buffers.
+static bool grid_args(RK* r, const SmallArgs& a, GridArgs& g)
 {
     const Sys* s = r->sys;
     const size_t pub = (size_t)s->esize * 2 * 64 * s->grid_groups;
@@ -2931,11 +2976,14 @@ static GridArgs grid_args(RK* r, const SmallArgs& a)
     if (r->grid_bytes < need) {
         dfree(r->d_grid);
         r->grid_bytes = 0;
-        HIP_CHECK(hipMalloc(&r->d_grid, need));
+        if (hipMalloc(&r->d_grid, need) != hipSuccess) {
+            (void)hipGetLastError();
+            r->d_grid = nullptr;
+            return false;
+        }
         r->grid_bytes = need;
     }
     if (!r->h_arrived) HIP_CHECK(hipHostMalloc((void**)&r->h_arrived, sizeof(unsigned), hipHostMallocDefault));
-    GridArgs g;
     memset(&g, 0, sizeof(g));
     g.code = s->d_gcode; g.cpos = s->d_gcpos; g.wg = s->d_gwg; g.group = s->d_ggroup; g.vmap = s->d_gvmap;
     g.x = a.x; g.ctrl = a.ctrl; g.solve = a.solve;
@@ -2950,7 +2998,7 @@ static GridArgs grid_args(RK* r, const SmallArgs& a)
     g.knorm = a.knorm;
     g.polls = GRID_POLLS;
     g.attempt_cap = r->grid_attempts > 0 ? r->grid_attempts : GRID_ATTEMPT_CAP;
-    return g;
+    return true;
 }
 
 static void grid_launch(RK* r, GridArgs& g)
@@ -2981,11 +3029,15 @@ static bool small_run(RK* r, const SmallArgs& a)
 {
     Sys* s = r->sys;
     hipStream_t st = s->stream;
-    HIP_CHECK(hipEventRecord(r->ev0, st));
-    long long last = r->h_ctrl->attempts;
     bool grid = grid_path(r), left = true;
     GridArgs g;
-    if (grid) g = grid_args(r, a);
+    if (grid && !grid_args(r, a, g)) {
+        r->grid_off = true;
+        grid = false;
+        if (!small_path(r)) return false;
+    }
+    HIP_CHECK(hipEventRecord(r->ev0, st));
+    long long last = r->h_ctrl->attempts;
     for (int launch = 0;; launch++) {
         if (r->grid_launches >= 0 && launch >= r->grid_launches) g.polls = -1;
         if (grid) grid_launch(r, g);
@@ -3584,7 +3636,7 @@ int asat_rk_uses_one_workgroup(const asat_rk_t* rk, int* uses)
     API_BEGIN
     CHECK_PTR(rk); CHECK_PTR(uses);
     rk->r.require_configured();
-    *uses = small_path(&rk->r) && persistent_workgroups(&rk->r) == 1 ? 1 : 0;
+    *uses = small_path(&rk->r) && persistent_workgroups(const_cast<RK*>(&rk->r)) == 1 ? 1 : 0;
     API_END
 }
 
@@ -3593,7 +3645,7 @@ int asat_rk_workgroups(const asat_rk_t* rk, int* workgroups)
     API_BEGIN
     CHECK_PTR(rk); CHECK_PTR(workgroups);
     rk->r.require_configured();
-    *workgroups = persistent_workgroups(&rk->r);
+    *workgroups = persistent_workgroups(const_cast<RK*>(&rk->r));
     API_END
 }
 

@@ -1,5 +1,8 @@
 """Which integrator runs: the number of workgroups that the query reports, for sizes
 on both sides of each rule and for the settings that rule a path out."""
+import threading
+
+import numpy as np
 import pytest
 
 import analogsat_amd as A
@@ -43,3 +46,50 @@ def test_settings_that_rule_a_path_out():
     assert rk.Workgroups() >= 8
     assert configured("f64", 2000, 8500, family="tanh")[1].Workgroups() == 0
     assert configured("f64", 50, 213, family="tanh")[1].Workgroups() == 1
+
+
+def stepped(sat, rk):
+    old, new = sat.MakeState(), sat.MakeState()
+    old.CopyFrom(np.concatenate([np.random.default_rng(3).uniform(-1, 1, sat.Get_N()),
+                                 np.ones(sat.Get_M())]).astype(sat.dtype))
+    assert rk.Step(old, new, 12)
+    return old.CopyTo(), rk.stats().attempts
+
+
+def test_a_path_chosen_after_configure():
+    """The few-workgroup layout is made when an integrator can first use it: here
+    by the setting after Configure, by the family, and by two integrators of one
+    system from two threads."""
+    sat = A.HipSat("f32")
+    sat.SetProblem(A.fastsat(2000, 8500, 3, 2))
+    rk = A.HipRungeKutta()
+    rk.SetEpsilon(1e-6)
+    rk.SetOneWorkgroup(False)
+    rk.Configure(sat)
+    assert rk.Workgroups() == 0
+    want = stepped(sat, rk)
+    rk.Reset()
+    rk.SetOneWorkgroup(True)
+    got = stepped(sat, rk)
+    assert rk.Workgroups() >= 8
+    assert np.array_equal(got[0], want[0]) and got[1] == want[1]
+
+    sat = A.HipSat("f32")
+    sat.SetProblem(A.fastsat(2000, 8500, 3, 2))
+    seen = {}
+
+    def configure(i):
+        rk = A.HipRungeKutta()
+        rk.SetEpsilon(1e-6)
+        rk.Configure(sat)
+        seen[i] = rk
+
+    threads = [threading.Thread(target=configure, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for rk in seen.values():
+        got = stepped(sat, rk)
+        assert rk.Workgroups() >= 8
+        assert np.array_equal(got[0], want[0]) and got[1] == want[1]
