@@ -2630,7 +2630,8 @@ struct RK {
     double timer_ms = 0.0;
     long long timer_launches = 0;
     // small problems: GRAPH_ATTEMPTS attempts captured once and replayed; the
-    // key is the exact launch arguments the graph was captured with
+    // key is the exact launch arguments the graph was captured with, or without a
+    // graph those of the last Step that could have had one
     hipGraphExec_t gexec = nullptr;
     std::vector<unsigned char> gkey;
 
@@ -2779,22 +2780,35 @@ static StageArgs<T> rk_stage_args(RK* r, int parity)
 // Launch-bound problems (few literal slots) replay a captured graph of
 // GRAPH_ATTEMPTS attempts instead of launching 13 kernels per attempt, as
 // long as a round still needs that many; the rest are launched one by one.
-// Larger ones gain nothing (N = 20 011, M = 196 107: 143 and 144 us per attempt)
-// and would pay the capture in their first Step (0.3 ms).
-constexpr long long GRAPH_MAX_SLOTS = 1LL << 18;
-constexpr int GRAPH_ATTEMPTS = 8;
+// Up to GRAPH_FIRST_SLOTS from the first Step on.  From there to GRAPH_MAX_BYTES
+// of contributions a graph saves 2 to 4 us per attempt (without and with: FP32, N =
+// 40 000, M = 170 000 80.9 and 77.6; N = 70 000, M = 297 500 90.4 and 88.1; FP64, N =
+// 30 000, M = 127 500 79.2 and 75.7; 4-SAT, FP32, N = 20 000, M = 198 600 89.2 and
+// 87.1), less than the 0.15 to 0.25 ms of its capture in a short Step, so only a Step
+// that repeats the last one's arguments, or is of GRAPH_LONG steps, makes one.
+// Beyond, the kernels hide their launches (FP64, N = 70 000: 113.7 and 114.5).
+constexpr long long GRAPH_FIRST_SLOTS = 1LL << 18, GRAPH_MAX_BYTES = 1LL << 22;
+constexpr int GRAPH_ATTEMPTS = 8, GRAPH_LONG = 128;
 
+// makes the graph unless it is there; false where this Step of count goes without
 template <typename T>
-static void ensure_graph(RK* r, const StageArgs<T>& a)
+static bool ensure_graph(RK* r, const StageArgs<T>& a, int count)
 {
     Sys* s = r->sys;
     hipStream_t st = s->stream;
+    if (r->timer_kind >= 0 || s->nslots * s->esize > GRAPH_MAX_BYTES || count < GRAPH_ATTEMPTS) return false;
     // the key: the arguments and every launch size the attempts depend on
     std::vector<unsigned char> key(sizeof(a) + 4 * sizeof(int));
     memcpy(key.data(), &a, sizeof(a));
     const int dims[4] = {clause_grid(s), var_grid(s), s->var_lds, s->tiled ? 1 : 0};
     memcpy(key.data() + sizeof(a), dims, sizeof(dims));
-    if (r->gexec && r->gkey == key) return;
+    const bool repeated = r->gkey == key;
+    if (r->gexec && repeated) return true;
+    if (s->nslots > GRAPH_FIRST_SLOTS && !repeated && count < GRAPH_LONG) {
+        r->drop_graph();
+        r->gkey = std::move(key);
+        return false;
+    }
     r->drop_graph();
     var_lds_attrs<T>();
     hipGraph_t g = nullptr;
@@ -2811,6 +2825,7 @@ static void ensure_graph(RK* r, const StageArgs<T>& a)
     (void)hipGraphDestroy(g);
     HIP_CHECK(e);
     r->gkey = std::move(key);
+    return true;
 }
 
 template <typename T>
@@ -2830,8 +2845,7 @@ static int rk_step_impl(RK* r, State* olds, State* news, int count)
     long long remaining = count;
     const long long target = r->h_ctrl->steps + count;
     long long last_attempts = r->h_ctrl->attempts;
-    const bool graphed = r->timer_kind < 0 && s->nslots <= GRAPH_MAX_SLOTS && count >= GRAPH_ATTEMPTS;
-    if (graphed) ensure_graph<T>(r, a);
+    const bool graphed = ensure_graph<T>(r, a, count);
     while (remaining > 0) {
         const int tk = r->timer_kind;
         if (graphed) {
