@@ -450,12 +450,17 @@ __device__ __forceinline__ Control traj_control(double v, double eps, double* re
     __syncthreads();
     return *out;
 }
-// sum over the trajectory's threads, in every one of them
+// sum over the trajectory's threads, in every one of them; LDS written before is
+// seen after, as with traj_sync
 template <int TT>
 __device__ __forceinline__ int traj_sum(int v, int* sh)
 {
-    if constexpr (TT == 64) return wave_sum(v);
-    else return block_sum_all<TT>(v, sh);
+    if constexpr (TT == 64) {
+        traj_sync<TT>();
+        return wave_sum(v);
+    } else {
+        return block_sum_all<TT>(v, sh);
+    }
 }
 
 template <int TT, int CPT, int VPT, int KK>
