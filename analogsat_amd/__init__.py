@@ -200,7 +200,7 @@ def lib():
             "asat_rk_set_one_workgroup": ([vp, i], i),
             "asat_rk_uses_one_workgroup": ([vp, ctypes.POINTER(i)], i),
             "asat_rk_workgroups": ([vp, ctypes.POINTER(i)], i),
-            "asat_rk_set_grid_limits": ([vp, i, ctypes.c_longlong, i], i),
+            "asat_rk_set_grid_limits": ([vp, i, i, i], i),
             "asat_rk_solve": ([vp, vp, vp, i, ctypes.c_longlong, ctypes.c_double, i, ctypes.POINTER(SolveResult)], i),
             "asat_rk_reset": ([vp], i),
             "asat_rk_stats": ([vp, ctypes.POINTER(RkStats)], i),
@@ -646,7 +646,7 @@ class HipRungeKutta:
 
     def SetGridLimits(self, workgroups=0, attempts=0, launches=-1):
         """Test hook: limits of the 8 to 128 workgroup kernel (most workgroups,
-        attempts per launch, the launch whose first workgroup gives up)."""
+        attempts per launch, the launch whose first wait is given up)."""
         _check(lib().asat_rk_set_grid_limits(self._h, int(workgroups), int(attempts), int(launches)))
 
     def Workgroups(self):

@@ -60,7 +60,7 @@ constexpr int GRID_MAX = 128;            // workgroups
 constexpr int GRID_WAVES = GRID_BT / 64; // variable groups a workgroup can own
 constexpr int GRID_POLLS = 1 << 21;      // a second or two
 constexpr unsigned GRID_GIVE_UP = 1u << 31;    // in the arrival word
-constexpr long long GRID_ATTEMPT_CAP = 4096;   // attempts per launch
+constexpr int GRID_ATTEMPT_CAP = 4096;   // attempts per launch
 
 struct GridArgs {
     const uint32_t* code;    // per workgroup, clause and literal: term entry << 16 | rank << 1 | negated
@@ -75,12 +75,11 @@ struct GridArgs {
     double* err;             // [2][GRID_MAX] error maxima
     int* count;              // [2][GRID_MAX] violated clauses
     unsigned* barrier;       // arrivals, and GRID_GIVE_UP; cleared before the launch
-    int polls;               // of a wait before it is given up (< 0: the first workgroup gives up instead of arriving)
-    long long attempt_cap;   // attempts per launch
     long long target, max_steps;
     double max_time;
     int time_float, batch;
-    int ngroups, aoff, k;
+    int attempt_cap;         // attempts per launch
+    int ngroups, aoff;
     double knorm;
 };
 
@@ -343,29 +342,21 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
             }
             if constexpr (ERR || CNT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             const unsigned want = phase * (unsigned)G;
+            __hip_atomic_fetch_add(a.barrier, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             int polls = 0;
-            if (a.polls < 0 && w == 0) {
-                __hip_atomic_fetch_or(a.barrier, GRID_GIVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                sh.give_up = 1;
-            } else {
-                __hip_atomic_fetch_add(a.barrier, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            while (!sh.give_up) {
-                unsigned v = agent_load(a.barrier);
-                if (v & GRID_GIVE_UP) {
-                    sh.give_up = 1;
-                    break;
-                }
-                if (v >= want) break;
-                // marked only while an arrival is missing: nobody has passed
-                // this exchange, and nobody will
-                if (++polls > a.polls && a.polls >= 0 &&
+            unsigned v;
+            // (a marked word is past every count)
+            while ((v = agent_load(a.barrier)) < want) {
+                // marked only while an arrival is missing: nobody has passed this
+                // exchange, and nobody will
+                if (++polls > GRID_POLLS &&
                     __hip_atomic_compare_exchange_strong(a.barrier, &v, v | GRID_GIVE_UP, __ATOMIC_RELAXED,
                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                    sh.give_up = 1;
+                    v = GRID_GIVE_UP;
                     break;
                 }
             }
+            if (v & GRID_GIVE_UP) sh.give_up = 1;
         }
         __syncthreads();
         if (sh.give_up) return false;
@@ -395,7 +386,7 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
     using Yes = std::integral_constant<bool, true>;
     using No = std::integral_constant<bool, false>;
 
-    long long launched = 0;
+    int launched = 0;
     bool done = underflow || (a.solve ? ss.result >= 0 : steps >= a.target);
     bool alive = true;
     while (!done && alive) {

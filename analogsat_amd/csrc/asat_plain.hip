@@ -2618,8 +2618,7 @@ struct RK {
     bool grid_off = false;           // its workgroups did not all run, or it had no memory: not tried again for
                                      // this problem
     // test limits (asat_rk_set_grid_limits)
-    int grid_workgroups = 0, grid_launches = -1;
-    long long grid_attempts = 0;
+    int grid_workgroups = 0, grid_launches = -1, grid_attempts = 0;
     void* pair[2] = {nullptr, nullptr};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = -1.f;
@@ -3008,14 +3007,14 @@ static bool grid_args(RK* r, const SmallArgs& a, GridArgs& g)
     g.pub = p + 64 + 2 * GRID_MAX * (sizeof(double) + sizeof(int));
     g.target = a.target; g.max_steps = a.max_steps; g.max_time = a.max_time;
     g.time_float = a.time_float; g.batch = a.batch;
-    g.ngroups = s->grid_groups; g.aoff = s->aoff; g.k = s->k;
+    g.ngroups = s->grid_groups; g.aoff = s->aoff;
     g.knorm = a.knorm;
-    g.polls = GRID_POLLS;
     g.attempt_cap = r->grid_attempts > 0 ? r->grid_attempts : GRID_ATTEMPT_CAP;
     return true;
 }
 
-static void grid_launch(RK* r, GridArgs& g)
+// give_up: the workgroups find the arrival word marked
+static void grid_launch(RK* r, GridArgs& g, bool give_up)
 {
     Sys* s = r->sys;
     const bool solo = s->grid_wgs == 1;
@@ -3027,7 +3026,7 @@ static void grid_launch(RK* r, GridArgs& g)
         HIP_CHECK(hipLaunchKernel(f, dim3(1), dim3(GRID_BT), args, (size_t)s->grid_lds, s->stream));
         return;
     }
-    HIP_CHECK(hipMemsetAsync(g.barrier, 0, sizeof(unsigned), s->stream));
+    HIP_CHECK(hipMemsetD32Async((hipDeviceptr_t)g.barrier, give_up ? (int)GRID_GIVE_UP : 0, 1, s->stream));
     HIP_CHECK(hipLaunchCooperativeKernel(f, dim3(s->grid_wgs), dim3(GRID_BT), args, (unsigned)s->grid_lds, s->stream));
     HIP_CHECK(hipMemcpyAsync(r->h_arrived, g.barrier, sizeof(unsigned), hipMemcpyDeviceToHost, s->stream));
 }
@@ -3053,8 +3052,7 @@ static bool small_run(RK* r, const SmallArgs& a)
     HIP_CHECK(hipEventRecord(r->ev0, st));
     long long last = r->h_ctrl->attempts;
     for (int launch = 0;; launch++) {
-        if (r->grid_launches >= 0 && launch >= r->grid_launches) g.polls = -1;
-        if (grid) grid_launch(r, g);
+        if (grid) grid_launch(r, g, launch == r->grid_launches);
         else small_launch<T>(s, a, st);
         HIP_CHECK(hipMemcpyAsync(r->h_ctrl, r->d_ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, st));
         if (a.solve) HIP_CHECK(hipMemcpyAsync(r->h_solve, r->d_solve, sizeof(SmallSolve), hipMemcpyDeviceToHost, st));
@@ -3663,7 +3661,7 @@ int asat_rk_workgroups(const asat_rk_t* rk, int* workgroups)
     API_END
 }
 
-int asat_rk_set_grid_limits(asat_rk_t* rk, int workgroups, long long attempts, int launches)
+int asat_rk_set_grid_limits(asat_rk_t* rk, int workgroups, int attempts, int launches)
 {
     API_BEGIN
     CHECK_PTR(rk);

@@ -219,11 +219,11 @@ int asat_rk_workgroups(const asat_rk_t* rk, int* workgroups);
    workgroups: a problem that needs more takes the multi-kernel path, as on a
    device that does not hold them all at once (0: what the device says);
    attempts: after so many a launch pauses between steps (0: the default);
-   launches: in this launch of a Step or solve the first workgroup gives up, as
-   after a long wait for one that does not run; the problem then goes on by the
-   multi-kernel path (negative: in none).
+   launches: in this launch of a Step or solve (from 0) the workgroups give up their
+   first wait, as after a long one for a workgroup that does not run; the problem
+   then goes on by the multi-kernel path (negative: in none).
    Results do not depend on any of them. */
-int asat_rk_set_grid_limits(asat_rk_t* rk, int workgroups, long long attempts, int launches);
+int asat_rk_set_grid_limits(asat_rk_t* rk, int workgroups, int attempts, int launches);
 /* SatSolver::DoSolve's loop without a callback (AnalogSAT/solver/SatSolver.h:313-331):
    while (time < max_time && steps < max_steps) { Step(batch); count the
    violated clauses of old_state; stop on 0 }, ending with SAT_UNDERFLOW on
