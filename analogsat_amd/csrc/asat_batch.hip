@@ -1746,9 +1746,12 @@ static void get_state(Batch& B, int index, float* pub)
 {
     const Instance& I = B.inst[(size_t)index];
     const size_t len = (size_t)I.n + I.m;
-    B.readers++;
-    std::lock_guard<std::mutex> lock(B.win_lock);
-    B.readers--;
+    std::unique_lock<std::mutex> lock(B.win_lock, std::try_to_lock);
+    if (!lock.owns_lock()) {
+        B.readers++;
+        lock.lock();
+        B.readers--;
+    }
     HIP_CHECK(hipStreamSynchronize(B.stream));
     const bool in_order = B.last_state >= 0 && index == B.last_state + 1;
     B.last_state = index;
