@@ -42,9 +42,11 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <numeric>
+#include <system_error>
 #include <thread>
 #include <type_traits>
 #include <vector>
@@ -1292,17 +1294,25 @@ static void reg_codes(const Instance& I, const RegLayout& L, int kk, uint32_t* o
 {
     const uint32_t none = (uint32_t)L.ncontrib << 16;
     const uint32_t pad = none | (8u * (uint32_t)I.n), absent = none | (8u * (uint32_t)(I.n + 1));
-    for (int j = 0; j < I.m; j++)
-        for (int q = 0; q < kk; q++) {
-            uint32_t& o = out[(size_t)j * kk + q];
-            if (q >= I.k) { o = absent; continue; }
-            const uint32_t c = I.code[(size_t)j * I.k + q];
-            const int v = (int)(c >> 19) - 1;
-            if (v < 0) { o = pad; continue; }
-            const int r = L.rank[v], e = (int)(c & 0x3FFFFu) - I.rowptr[v];
-            const uint32_t at = (uint32_t)(L.group[2 * (r / 64)] + 64 * e + r % 64);
-            o = (at << 16) | (8u * (uint32_t)r) | (((c >> 18) & 1u) << 2);
+    // per variable: the contribution entry of position 0 of the instance's var-major
+    // order, of which each position is 64 entries further on, and 8 times its rank
+    struct Place { uint32_t entry, rank8; };
+    std::vector<Place> place((size_t)I.n);
+    for (int v = 0; v < I.n; v++) {
+        const int r = L.rank[v];
+        place[(size_t)v] = {(uint32_t)(L.group[2 * (r / 64)] + r % 64 - 64 * I.rowptr[v]), 8u * (uint32_t)r};
+    }
+    for (int j = 0; j < I.m; j++) {
+        const uint32_t* c = I.code.data() + (size_t)j * I.k;
+        uint32_t* o = out + (size_t)j * kk;
+        for (int q = 0; q < I.k; q++) {
+            const int v = (int)(c[q] >> 19) - 1;
+            o[q] = v < 0 ? pad
+                         : (place[(size_t)v].entry + 64 * (c[q] & 0x3FFFFu)) << 16 | place[(size_t)v].rank8 |
+                               ((c[q] >> 18) & 1u) << 2;
         }
+        for (int q = I.k; q < kk; q++) o[q] = absent;
+    }
     for (long long s = (long long)I.m * kk; s < rcode_len(I, kk); s++) out[s] = absent;
 }
 
@@ -1545,6 +1555,52 @@ static void build_instance(const int* lits, const int* lens, int nclauses, Insta
         I.code[s] = ((uint32_t)v << 19) | ((l < 0 ? 1u : 0u) << 18) | p;
     }
 }
+
+// f(i) for every i in [0, count), on up to 8 threads while each gets 60 000 of the
+// literal slots (about 0.2 ms; a thread costs about 50 us).  Instances are
+// independent; building the layouts of 1024 of N = 2000, M = 8500 takes 85 ms on one.
+template <typename F>
+static void each_instance(int count, long long slots, F f)
+{
+    const long long most = std::min<long long>(8, std::max(1u, std::thread::hardware_concurrency()));
+    const int nt = (int)std::max<long long>(1, std::min<long long>({most, (long long)count, 1 + slots / 60000}));
+    std::atomic<int> next{0};
+    std::mutex lock;
+    std::exception_ptr failed;
+    auto work = [&] {
+        try {
+            for (int i; (i = next++) < count;) f(i);
+        } catch (...) {
+            std::lock_guard<std::mutex> l(lock);
+            failed = std::current_exception();
+            next = count;
+        }
+    };
+    std::vector<std::thread> th;
+    th.reserve((size_t)nt);
+    try {
+        for (int t = 1; t < nt; t++) th.emplace_back(work);
+    } catch (const std::system_error&) {
+        // no more threads: those there are, and this one, do it
+    }
+    work();
+    for (std::thread& t : th) t.join();
+    if (failed) std::rethrow_exception(failed);
+}
+
+// host memory on its way to the device, not cleared first
+template <typename V>
+struct Staging {
+    std::unique_ptr<unsigned char[]> raw;
+    size_t count;
+    explicit Staging(size_t n) : raw(new unsigned char[std::max<size_t>(n, 1) * sizeof(V)]), count(n) {}
+    V* data() { return (V*)raw.get(); }
+    void upload(V*& d)
+    {
+        HIP_CHECK(hipMalloc((void**)&d, sizeof(V) * std::max<size_t>(count, 1)));
+        if (count) HIP_CHECK(hipMemcpy(d, raw.get(), sizeof(V) * count, hipMemcpyHostToDevice));
+    }
+};
 
 static size_t bucket_lds(const Bucket& b, bool lds)
 {
@@ -1804,9 +1860,15 @@ static void autotune(Batch& B)
         B.chunk_steps = std::min(32, std::max(2, 60000 / std::max(b.maxl, 1)));
         struct Cand { int bs, mode, cap; const RegVariant* rv; };
         std::vector<Cand> cand;
+        // register variants: the first that fits, and those of at most twice as many
+        // threads as clauses or variables (run of 200 steps with 256, 512 and
+        // 1024 threads, ms, N = 50, M = 213: 1000 trajectories 1.5, 4.5, 5.5, 64 of them
+        // 1.1, 1.4, 1.7; N = 100, M = 426: 500 1.6, 2.8, 3.5)
+        const int idle = 2 * std::max(b.maxm, b.maxn);
         if (B.force_lds == -1 || B.force_lds == 2)
             for (const RegVariant& r : REG_VARIANTS)
-                if ((!B.force_block || r.block() == B.force_block) && reg_fits(r, b, B.lds_limit))
+                if ((!B.force_block || r.block() == B.force_block) && reg_fits(r, b, B.lds_limit) &&
+                    (r.tt <= idle || cand.empty()))
                     cand.push_back({r.block(), 2, 0, &r});
         const bool reg_only = !cand.empty() && B.force_lds == -1;
         const long long contrib_bytes = 4 * round_up_ll(b.maxl, 64);
@@ -1857,13 +1919,6 @@ static void autotune(Batch& B)
     reset_state(B);
 }
 
-template <typename V>
-static void upload_vec(V*& d, const std::vector<V>& h)
-{
-    HIP_CHECK(hipMalloc((void**)&d, sizeof(V) * h.size()));
-    HIP_CHECK(hipMemcpy(d, h.data(), sizeof(V) * h.size(), hipMemcpyHostToDevice));
-}
-
 static void prepare(Batch& B, bool tune)
 {
     require(!B.inst.empty(), ASAT_ERR_INVALID_ARGUMENT, "no trajectories added");
@@ -1882,30 +1937,23 @@ static void prepare(Batch& B, bool tune)
             B.lds_limit = (size_t)v2;
     }
     std::vector<Desc> desc(T);
-    long long code_total = 0, row_total = 0, state_total = 0;
+    long long state_total = 0;
     B.state_off.assign(T, 0);
     for (int i = 0; i < T; i++) {
         const Instance& I = B.inst[i];
-        desc[i].code_off = code_total;
-        desc[i].row_off = row_total;
+        desc[i].code_off = desc[i].row_off = -1;
         desc[i].state_off = state_total;
         B.state_off[i] = state_total;
         desc[i].n = I.n; desc[i].m = I.m; desc[i].k = I.k; desc[i].nslots = I.nslots;
         desc[i].rcode_off = desc[i].rgroup_off = desc[i].rvmap_off = -1;
         desc[i].ccode_off = desc[i].cgroup_off = desc[i].crec_off = desc[i].cstart_off = -1;
         desc[i].knorm = (float)std::pow(2.0, -I.k);
-        code_total += (long long)I.code.size();
-        row_total += (long long)I.rowptr.size();
         state_total += round_up_ll((long long)I.n + I.m, 64);
     }
-    std::vector<uint32_t> code(code_total);
-    std::vector<int> rows(row_total);
     std::vector<float> x0((size_t)state_total, 0.f);
     B.state_total = state_total;
     for (int i = 0; i < T; i++) {
         const Instance& I = B.inst[i];
-        std::copy(I.code.begin(), I.code.end(), code.begin() + desc[i].code_off);
-        std::copy(I.rowptr.begin(), I.rowptr.end(), rows.begin() + desc[i].row_off);
         std::copy(I.pub0.begin(), I.pub0.end(), x0.begin() + desc[i].state_off);
     }
     // size buckets: trajectories sorted by work (slots + clauses), largest
@@ -1933,6 +1981,11 @@ static void prepare(Batch& B, bool tune)
         HIP_CHECK(hipMalloc((void**)&b.d_queue, sizeof(int)));
         HIP_CHECK(hipMemcpy(b.d_order, b.ids.data(), sizeof(int) * b.ids.size(), hipMemcpyHostToDevice));
     }
+    auto slots_of = [&](const Bucket& b) {
+        long long n = 0;
+        for (int id : b.ids) n += B.inst[id].nslots;
+        return n;
+    };
     // the register kernel's layout for the buckets that fit one of its
     // variants, the clause-chunked layout for the others
     {
@@ -1942,10 +1995,12 @@ static void prepare(Batch& B, bool tune)
             bool may = false;
             for (const RegVariant& r : REG_VARIANTS) may = may || reg_fits(r, b, B.lds_limit);
             if (!may || (B.force_lds != -1 && B.force_lds != 2)) { b.ncontrib = 1 << 30; continue; }
-            for (int id : b.ids) {
+            // (the ranking goes through variables, a tenth of the slots)
+            each_instance((int)b.ids.size(), slots_of(b) / 10, [&](int i) {
+                const int id = b.ids[(size_t)i];
                 reg_layout(B.inst[id], reg[(size_t)id]);
-                b.ncontrib = std::max(b.ncontrib, reg[(size_t)id].ncontrib);
-            }
+            });
+            for (int id : b.ids) b.ncontrib = std::max(b.ncontrib, reg[(size_t)id].ncontrib);
             if (!reg_variant(b, B.lds_limit)) continue;
             for (int id : b.ids) {
                 const RegLayout& L = reg[(size_t)id];
@@ -1957,65 +2012,102 @@ static void prepare(Batch& B, bool tune)
             }
         }
         if (rcode > 0) {
-            std::vector<uint32_t> hc((size_t)rcode);
-            std::vector<int> hg((size_t)rgroup), hv((size_t)rvmap);
+            Staging<uint32_t> hc((size_t)rcode);
+            Staging<int> hg((size_t)rgroup), hv((size_t)rvmap);
             for (auto& b : B.buckets)
-                for (int id : b.ids) {
-                    if (desc[id].rcode_off < 0) continue;
-                    const RegLayout& L = reg[(size_t)id];
+                each_instance((int)b.ids.size(), slots_of(b), [&](int i) {
+                    const int id = b.ids[(size_t)i];
+                    if (desc[id].rcode_off < 0) return;
+                    RegLayout& L = reg[(size_t)id];
                     reg_codes(B.inst[id], L, b.kk, hc.data() + desc[id].rcode_off);
-                    std::copy(L.group.begin(), L.group.end(), hg.begin() + desc[id].rgroup_off);
-                    std::copy(L.vmap.begin(), L.vmap.end(), hv.begin() + desc[id].rvmap_off);
-                }
-            upload_vec(B.d_rcode, hc);
-            upload_vec(B.d_rgroup, hg);
-            upload_vec(B.d_rvmap, hv);
+                    std::copy(L.group.begin(), L.group.end(), hg.data() + desc[id].rgroup_off);
+                    std::copy(L.vmap.begin(), L.vmap.end(), hv.data() + desc[id].rvmap_off);
+                });
+            hc.upload(B.d_rcode);
+            hg.upload(B.d_rgroup);
+            hv.upload(B.d_rvmap);
         }
     }
     {
-        std::vector<uint2> hcode;
-        std::vector<int2> hgroup;
-        std::vector<uint16_t> hperm;
-        std::vector<uint32_t> hrec;
-        std::vector<int> hstart;
+        std::vector<ChunkLayout> chunk((size_t)T);
+        long long ccode = 0, cgroup = 0, crec = 0, cstart = 0;
         for (auto& b : B.buckets) {
             const bool want = B.force_lds == 3 || (B.force_lds == -1 && !reg_variant(b, B.lds_limit));
             b.chunk_terms = chunk_terms_for(b, B.lds_limit);
             b.chunked = want && b.chunk_terms >= 4 * 64;
             if (!b.chunked) continue;
+            each_instance((int)b.ids.size(), slots_of(b), [&](int i) {
+                const Instance& I = B.inst[b.ids[(size_t)i]];
+                chunk_layout(I, chunk_max(I, b.chunk_terms, B.force_chunk), b.chunk_terms,
+                             chunk[(size_t)b.ids[(size_t)i]]);
+            });
             for (int id : b.ids) {
-                ChunkLayout L;
-                chunk_layout(B.inst[id], chunk_max(B.inst[id], b.chunk_terms, B.force_chunk), b.chunk_terms, L);
+                const ChunkLayout& L = chunk[(size_t)id];
                 Desc& d = desc[id];
-                d.ccode_off = (long long)hcode.size(); d.cgroup_off = (long long)hgroup.size();
-                d.crec_off = (long long)hrec.size(); d.cstart_off = (long long)hstart.size();
+                d.ccode_off = ccode; d.cgroup_off = cgroup; d.crec_off = crec; d.cstart_off = cstart;
                 d.nchunks = L.nchunks; d.chunk = L.cs;
-                hcode.insert(hcode.end(), L.code.begin(), L.code.end());
-                hgroup.insert(hgroup.end(), L.group.begin(), L.group.end());
-                hperm.insert(hperm.end(), L.perm.begin(), L.perm.end());
-                hrec.insert(hrec.end(), L.rec.begin(), L.rec.end());
-                hstart.insert(hstart.end(), L.start.begin(), L.start.end());
+                ccode += (long long)L.code.size(); cgroup += (long long)L.group.size();
+                crec += (long long)L.rec.size(); cstart += (long long)L.start.size();
             }
         }
-        if (!hcode.empty()) {
-            upload_vec(B.d_ccode, hcode);
-            upload_vec(B.d_cgroup, hgroup);
-            upload_vec(B.d_cperm, hperm);
-            upload_vec(B.d_crec, hrec);
-            upload_vec(B.d_cstart, hstart);
+        if (ccode > 0) {
+            Staging<uint2> hcode((size_t)ccode);
+            Staging<int2> hgroup((size_t)cgroup);
+            Staging<uint16_t> hperm((size_t)cgroup * 64);
+            Staging<uint32_t> hrec((size_t)crec);
+            Staging<int> hstart((size_t)cstart);
+            for (auto& b : B.buckets)
+                each_instance((int)b.ids.size(), slots_of(b), [&](int i) {
+                    const Desc& d = desc[(size_t)b.ids[(size_t)i]];
+                    if (d.ccode_off < 0) return;
+                    ChunkLayout& L = chunk[(size_t)b.ids[(size_t)i]];
+                    std::copy(L.code.begin(), L.code.end(), hcode.data() + d.ccode_off);
+                    std::copy(L.group.begin(), L.group.end(), hgroup.data() + d.cgroup_off);
+                    std::copy(L.perm.begin(), L.perm.end(), hperm.data() + d.cgroup_off * 64);
+                    std::copy(L.rec.begin(), L.rec.end(), hrec.data() + d.crec_off);
+                    std::copy(L.start.begin(), L.start.end(), hstart.data() + d.cstart_off);
+                });
+            hcode.upload(B.d_ccode);
+            hgroup.upload(B.d_cgroup);
+            hperm.upload(B.d_cperm);
+            hrec.upload(B.d_crec);
+            hstart.upload(B.d_cstart);
         }
     }
+    // k_batch's codes and rows, for the buckets that may run it
+    {
+        long long code = 0, rows = 0;
+        for (auto& b : B.buckets) {
+            const bool reg_ok = reg_variant(b, B.lds_limit, B.force_block) != nullptr;
+            if (B.force_lds != 0 && B.force_lds != 1 && (B.force_lds != -1 || reg_ok || (b.chunked && !b.lds_fits)))
+                continue;
+            for (int id : b.ids) {
+                desc[id].code_off = code;
+                desc[id].row_off = rows;
+                code += (long long)B.inst[id].code.size();
+                rows += (long long)B.inst[id].rowptr.size();
+            }
+        }
+        Staging<uint32_t> hcode((size_t)code);
+        Staging<int> hrows((size_t)rows);
+        for (auto& b : B.buckets)
+            each_instance(code > 0 ? (int)b.ids.size() : 0, slots_of(b), [&](int i) {
+                const int id = b.ids[(size_t)i];
+                if (desc[id].code_off < 0) return;
+                const Instance& I = B.inst[id];
+                std::copy(I.code.begin(), I.code.end(), hcode.data() + desc[id].code_off);
+                std::copy(I.rowptr.begin(), I.rowptr.end(), hrows.data() + desc[id].row_off);
+            });
+        hcode.upload(B.d_code);
+        hrows.upload(B.d_rowptr);
+    }
     HIP_CHECK(hipMalloc((void**)&B.d_desc, sizeof(Desc) * T));
-    HIP_CHECK(hipMalloc((void**)&B.d_code, sizeof(uint32_t) * std::max<long long>(code_total, 1)));
-    HIP_CHECK(hipMalloc((void**)&B.d_rowptr, sizeof(int) * std::max<long long>(row_total, 1)));
     HIP_CHECK(hipMalloc((void**)&B.d_xa, sizeof(float) * std::max<long long>(state_total, 1)));
     HIP_CHECK(hipMalloc((void**)&B.d_xb, sizeof(float) * std::max<long long>(state_total, 1)));
     HIP_CHECK(hipMalloc((void**)&B.d_x0, sizeof(float) * std::max<long long>(state_total, 1)));
     HIP_CHECK(hipMemcpy(B.d_x0, x0.data(), sizeof(float) * state_total, hipMemcpyHostToDevice));
     HIP_CHECK(hipMalloc((void**)&B.d_ctrl, sizeof(TrajCtrl) * T));
     HIP_CHECK(hipMemcpy(B.d_desc, desc.data(), sizeof(Desc) * T, hipMemcpyHostToDevice));
-    HIP_CHECK(hipMemcpy(B.d_code, code.data(), sizeof(uint32_t) * code_total, hipMemcpyHostToDevice));
-    HIP_CHECK(hipMemcpy(B.d_rowptr, rows.data(), sizeof(int) * row_total, hipMemcpyHostToDevice));
     B.h_ctrl0.assign(T, TrajCtrl());
     for (int i = 0; i < T; i++) {
         TrajCtrl& c = B.h_ctrl0[i];
