@@ -74,7 +74,8 @@ struct GridArgs {
     void* pub;               // [2][64 * ngroups] published spins
     double* err;             // [2][GRID_MAX] error maxima
     int* count;              // [2][GRID_MAX] violated clauses
-    unsigned* barrier;       // arrivals, and GRID_GIVE_UP; cleared before the launch
+    unsigned* barrier;       // arrivals of all launches so far, and GRID_GIVE_UP
+    unsigned phase;          // exchanges so far
     long long target, max_steps;
     double max_time;
     int time_float, batch;
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(GRID_BT) void k_grid(GridArgs a)
     if (a.solve) ss = *a.solve;
     __syncthreads();
 
-    unsigned phase = 0;
+    unsigned phase = a.phase;
     double ctl_errmax = 0.0, ctl_power = 0.0;     // what an exchange brought
     int ctl_count = 0;
     // Publish this thread's spin (waves that own a group), wait for every

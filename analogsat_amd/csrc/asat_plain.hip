@@ -1999,9 +1999,8 @@ static void build_small_lists(Sys* s, const HostProblem& P)
 //   N =  2000, M =  8500, FP32   22.5 / 20.6 / 22.6 / 28.1 / 33.4
 //   N =  5000, M = 21250, FP32   36.5 / 31.8 / 30.9 / 32.9 / 39.1
 //   N = 12000, M = 51120, FP64      - /    - /    - / 59.9 / 69.5
-// The path ends where the spins of all variables no longer fit in LDS or the
-// clauses in registers; up to there it is faster than 13 kernels per attempt
-// (N = 24000, M = 102000, FP32: 68 against 76 us; N = 14000, FP64: 63 against 67).
+// The layout ends where the spins of all variables no longer fit in LDS or the
+// clauses in registers; grid_gain says which calls take it.
 constexpr int GRID_CPT_F64 = 4, GRID_CPT_F32 = 8;
 constexpr long long GRID_LDS = 158 * 1024;     // beside the kernel's 0.3 KB of static LDS
 
@@ -2015,7 +2014,6 @@ static int grid_resident(const void* f, size_t lds)
     HIP_CHECK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
     HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     if (!f || !coop) return 0;
-    HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, GRID_BT, lds));
     return per_cu * ncu;
 }
@@ -2093,7 +2091,10 @@ static void build_grid(Sys* s, const std::vector<int>& lit)
     const long long lds = (long long)s->esize * (nranks + 2 + most_con + 1);
     if (most_con > 65535 || lds > GRID_LDS) return;
     const int kcpt = cpt <= 1 ? 1 : cpt <= 2 ? 2 : cpt <= 4 ? 4 : 8;
-    if (G > 1 && grid_resident(grid_kernel(s->prec, K, kcpt, false), (size_t)lds) < G) return;
+    const void* f = grid_kernel(s->prec, K, kcpt, G == 1);
+    require(f != nullptr, ASAT_ERR_HIP, "no few-workgroup kernel for this layout");
+    HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GRID_LDS));
+    if (G > 1 && grid_resident(f, (size_t)lds) < G) return;
     // term entry of every slot in its variable's workgroup: the variable's clauses
     // in input order, literals in clause order (the reference's accumulation order)
     std::vector<int> visit((size_t)m), fill((size_t)nranks), entry(slots);
@@ -2594,6 +2595,13 @@ static int sys_violations(Sys* s, const State* x)
 // ---------------------------------------------------------------------------
 // integrator
 // ---------------------------------------------------------------------------
+// The control block and, in a line of its own, the few-workgroup kernel's arrival
+// word, which one copy brings to the host.
+struct CtrlBlock {
+    Ctrl ctrl;
+    alignas(128) unsigned arrived;
+};
+
 struct RK {
     Sys* sys = nullptr;
     double eps = 1e-4;      // CudaRungeKutta() default (CudaRungeKutta.cu:175)
@@ -2607,14 +2615,13 @@ struct RK {
     int tmp_n = 0;            // tmp holds n+1 values of the problem at Configure
     double* partial = nullptr;
     int npartial = 0;
-    Ctrl* d_ctrl = nullptr;
+    Ctrl* d_ctrl = nullptr;   // of a CtrlBlock
     Ctrl* h_ctrl = nullptr;   // pinned mirror
     int small_mode = 1;              // 1: one-workgroup path where the problem fits, 0: never
     SmallSolve* d_solve = nullptr;   // device SatSolver loop state (one-workgroup path)
     SmallSolve* h_solve = nullptr;   // pinned mirror
     void* d_grid = nullptr;          // exchange buffers of the few-workgroup path
     size_t grid_bytes = 0;
-    unsigned* h_arrived = nullptr;   // pinned: its arrival word after a launch
     bool grid_off = false;           // its workgroups did not all run, or it had no memory: not tried again for
                                      // this problem
     // test limits (asat_rk_set_grid_limits)
@@ -2646,7 +2653,6 @@ struct RK {
         for (auto& p : k) dfree(p);
         dfree(tmp); dfree(partial); dfree(d_ctrl); dfree(d_solve); dfree(d_grid);
         grid_bytes = 0;
-        if (h_arrived) { (void)hipHostFree(h_arrived); h_arrived = nullptr; }
         if (h_ctrl) { (void)hipHostFree(h_ctrl); h_ctrl = nullptr; }
         if (h_solve) { (void)hipHostFree(h_solve); h_solve = nullptr; }
     }
@@ -2656,6 +2662,15 @@ struct RK {
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         for (hipEvent_t e : tev) (void)hipEventDestroy(e);
+    }
+    unsigned* d_arrived() const { return &((CtrlBlock*)d_ctrl)->arrived; }
+    unsigned& h_arrived() const { return ((CtrlBlock*)h_ctrl)->arrived; }
+    // no arrivals, for the next launch of the few-workgroup kernel
+    void clear_arrived(hipStream_t st)
+    {
+        if (h_arrived() == 0) return;
+        HIP_CHECK(hipMemsetD32Async((hipDeviceptr_t)d_arrived(), 0, 1, st));
+        h_arrived() = 0;
     }
     void require_configured() const
     {
@@ -2698,6 +2713,7 @@ static void rk_configure(RK* r, Sys* s)
         // same sizes (SatSolver configures before every Solve): keep the
         // buffers, clear them and reset the control block
         r->drop_graph();
+        if (r->gen != s->gen) r->clear_arrived(s->stream);
         r->sys = s;
         r->gen = s->gen;
         // the persistent paths keep everything on the CUs and read none of
@@ -2729,9 +2745,10 @@ static void rk_configure(RK* r, Sys* s)
     r->npartial = npartial;
     HIP_CHECK(hipMalloc((void**)&r->partial, sizeof(double) * r->npartial));
     HIP_CHECK(hipMemset(r->partial, 0, sizeof(double) * r->npartial));
-    HIP_CHECK(hipMalloc((void**)&r->d_ctrl, sizeof(Ctrl)));
-    HIP_CHECK(hipHostMalloc((void**)&r->h_ctrl, sizeof(Ctrl), hipHostMallocDefault));
-    memset(r->h_ctrl, 0, sizeof(Ctrl));
+    HIP_CHECK(hipMalloc((void**)&r->d_ctrl, sizeof(CtrlBlock)));
+    HIP_CHECK(hipMemset(r->d_ctrl, 0, sizeof(CtrlBlock)));
+    HIP_CHECK(hipHostMalloc((void**)&r->h_ctrl, sizeof(CtrlBlock), hipHostMallocDefault));
+    memset((void*)r->h_ctrl, 0, sizeof(CtrlBlock));
     HIP_CHECK(hipMalloc((void**)&r->d_solve, sizeof(SmallSolve)));
     HIP_CHECK(hipHostMalloc((void**)&r->h_solve, sizeof(SmallSolve), hipHostMallocDefault));
     memset(r->h_solve, 0, sizeof(SmallSolve));
@@ -2973,6 +2990,31 @@ static bool grid_path(RK* r)
     return s->grid_wgs > 0 && !(r->grid_workgroups > 0 && s->grid_wgs > r->grid_workgroups);
 }
 
+// What the 8 to 128 workgroups gain over the multi-kernel path in `steps` steps, us:
+// about 0.3 per attempt for every KB that the spins, which each of them reads six
+// times an attempt, stay below 124.  us per attempt, here and there: FP32, N = 12 000,
+// M = 51 000 44 and 67, 20 000, 85 000 62 and 71, 24 000, 102 000 68 and 72, 28 000,
+// 119 000 74.4 and 73.9, 32 000, 136 000 82 and 76 (50 000 clauses: 68.2 and 68.3);
+// FP64, 8000, 34 000 49 and 63, 12 000, 51 120 58 and 65, 15 000, 63 000 64 and 66,
+// 17 000, 40 000 61.1 and 61.0; 4-SAT, FP64, 8000, 79 000 68 and 84.
+static double grid_gain(const Sys* s, long long steps)
+{
+    return 0.3 * (double)steps * (124.0 - s->esize * 64.0 * s->grid_groups / 1024.0);
+}
+// A call costs 20 us more (a cooperative launch, the layout into registers and LDS):
+// a Step has to gain that (Step(1), FP32, N = 24 000 130 and 107 us, N = 2000 68 and
+// 100).  A solve saves about 60 us per batch for the Step's end and the count on
+// the host, so there a batch may lose them.
+constexpr double GRID_CALL_US = 20.0;
+static bool grid_step(RK* r, int count)
+{
+    return grid_path(r) && (r->sys->grid_wgs == 1 || grid_gain(r->sys, count) >= GRID_CALL_US);
+}
+static bool grid_solve(RK* r, int batch)
+{
+    return grid_path(r) && (r->sys->grid_wgs == 1 || grid_gain(r->sys, batch) >= -GRID_CALL_US);
+}
+
 // workgroups of the persistent kernel that runs the problem (0: the multi-kernel path)
 static int persistent_workgroups(RK* r)
 {
@@ -2985,7 +3027,7 @@ static bool grid_args(RK* r, const SmallArgs& a, GridArgs& g)
 {
     const Sys* s = r->sys;
     const size_t pub = (size_t)s->esize * 2 * 64 * s->grid_groups;
-    const size_t need = 64 + 2 * GRID_MAX * (sizeof(double) + sizeof(int)) + pub;
+    const size_t need = 2 * GRID_MAX * (sizeof(double) + sizeof(int)) + pub;
     if (r->grid_bytes < need) {
         dfree(r->d_grid);
         r->grid_bytes = 0;
@@ -2996,15 +3038,14 @@ static bool grid_args(RK* r, const SmallArgs& a, GridArgs& g)
         }
         r->grid_bytes = need;
     }
-    if (!r->h_arrived) HIP_CHECK(hipHostMalloc((void**)&r->h_arrived, sizeof(unsigned), hipHostMallocDefault));
     memset(&g, 0, sizeof(g));
     g.code = s->d_gcode; g.cpos = s->d_gcpos; g.wg = s->d_gwg; g.group = s->d_ggroup; g.vmap = s->d_gvmap;
     g.x = a.x; g.ctrl = a.ctrl; g.solve = a.solve;
     char* p = (char*)r->d_grid;
-    g.barrier = (unsigned*)p;
-    g.err = (double*)(p + 64);
-    g.count = (int*)(p + 64 + 2 * GRID_MAX * sizeof(double));
-    g.pub = p + 64 + 2 * GRID_MAX * (sizeof(double) + sizeof(int));
+    g.barrier = r->d_arrived();
+    g.err = (double*)p;
+    g.count = (int*)(p + 2 * GRID_MAX * sizeof(double));
+    g.pub = p + 2 * GRID_MAX * (sizeof(double) + sizeof(int));
     g.target = a.target; g.max_steps = a.max_steps; g.max_time = a.max_time;
     g.time_float = a.time_float; g.batch = a.batch;
     g.ngroups = s->grid_groups; g.aoff = s->aoff;
@@ -3019,30 +3060,30 @@ static void grid_launch(RK* r, GridArgs& g, bool give_up)
     Sys* s = r->sys;
     const bool solo = s->grid_wgs == 1;
     const void* f = grid_kernel(s->prec, s->k, s->grid_cpt, solo);
-    require(f != nullptr, ASAT_ERR_HIP, "no few-workgroup kernel for this layout");
-    HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)s->grid_lds));
     void* args[] = {&g};
     if (solo) {
         HIP_CHECK(hipLaunchKernel(f, dim3(1), dim3(GRID_BT), args, (size_t)s->grid_lds, s->stream));
         return;
     }
-    HIP_CHECK(hipMemsetD32Async((hipDeviceptr_t)g.barrier, give_up ? (int)GRID_GIVE_UP : 0, 1, s->stream));
+    // every launch counts on from the last one
+    if (r->h_arrived() >= GRID_GIVE_UP / 2) r->clear_arrived(s->stream);
+    g.phase = r->h_arrived() / (unsigned)s->grid_wgs;
+    if (give_up) HIP_CHECK(hipMemsetD32Async((hipDeviceptr_t)g.barrier, (int)GRID_GIVE_UP, 1, s->stream));
     HIP_CHECK(hipLaunchCooperativeKernel(f, dim3(s->grid_wgs), dim3(GRID_BT), args, (unsigned)s->grid_lds, s->stream));
-    HIP_CHECK(hipMemcpyAsync(r->h_arrived, g.barrier, sizeof(unsigned), hipMemcpyDeviceToHost, s->stream));
 }
 
-// Launches the persistent kernel of either path until it reports done: each
+// Launches a persistent kernel (grid: the few-workgroup one) until it reports done: each
 // launch runs at most SMALL_ATTEMPT_CAP (GRID_ATTEMPT_CAP) attempts and leaves its
 // state in the control block (and the solver block), so the next launch resumes
 // where it stopped.  False: the workgroups of a launch did not all run, which has
 // changed nothing, and no persistent kernel is left for the problem; the
 // control and solver blocks say how far the launches before it came.
 template <typename T>
-static bool small_run(RK* r, const SmallArgs& a)
+static bool small_run(RK* r, const SmallArgs& a, bool grid)
 {
     Sys* s = r->sys;
     hipStream_t st = s->stream;
-    bool grid = grid_path(r), left = true;
+    bool left = true;
     GridArgs g;
     if (grid && !grid_args(r, a, g)) {
         r->grid_off = true;
@@ -3054,10 +3095,11 @@ static bool small_run(RK* r, const SmallArgs& a)
     for (int launch = 0;; launch++) {
         if (grid) grid_launch(r, g, launch == r->grid_launches);
         else small_launch<T>(s, a, st);
-        HIP_CHECK(hipMemcpyAsync(r->h_ctrl, r->d_ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, st));
+        HIP_CHECK(hipMemcpyAsync(r->h_ctrl, r->d_ctrl, grid ? sizeof(CtrlBlock) : sizeof(Ctrl), hipMemcpyDeviceToHost, st));
         if (a.solve) HIP_CHECK(hipMemcpyAsync(r->h_solve, r->d_solve, sizeof(SmallSolve), hipMemcpyDeviceToHost, st));
         HIP_CHECK(hipStreamSynchronize(st));
-        if (grid && s->grid_wgs > 1 && (*r->h_arrived & GRID_GIVE_UP)) {
+        if (grid && (r->h_arrived() & GRID_GIVE_UP)) {
+            r->clear_arrived(st);
             r->grid_off = true;
             grid = false;
             left = small_path(r);
@@ -3090,11 +3132,12 @@ static int rk_step(RK* r, State* olds, State* news, int count)
     require(count >= 0, ASAT_ERR_INVALID_ARGUMENT, "negative step count");
     if (r->h_ctrl->underflow) return ASAT_UNDERFLOW;
     if (count == 0) return ASAT_OK;
-    if (small_path(r) || grid_path(r)) {
+    const bool grid = grid_step(r, count);
+    if (small_path(r) || grid) {
         // the state stays in olds; news is not touched
         SmallArgs a = small_args(r, olds->d);
         a.target = r->h_ctrl->steps + count;
-        if (r->prec == ASAT_F64 ? small_run<double>(r, a) : small_run<float>(r, a))
+        if (r->prec == ASAT_F64 ? small_run<double>(r, a, grid) : small_run<float>(r, a, grid))
             return r->h_ctrl->underflow ? ASAT_UNDERFLOW : ASAT_OK;
         count = (int)(a.target - r->h_ctrl->steps);
     }
@@ -3125,7 +3168,8 @@ static void rk_solve(RK* r, State* olds, State* news, int batch, long long max_s
     double time = 0.0;
     int lastv = 0, result = -1, todo = 0;     // todo: steps left of the batch
     bool due = false;                         // a batch has ended and its count is due
-    if ((small_path(r) || grid_path(r)) && !r->h_ctrl->underflow) {
+    const bool grid = grid_solve(r, batch);
+    if ((small_path(r) || grid) && !r->h_ctrl->underflow) {
         SmallSolve init;
         memset(&init, 0, sizeof(init));
         init.result = -1;
@@ -3137,7 +3181,7 @@ static void rk_solve(RK* r, State* olds, State* news, int batch, long long max_s
         a.max_steps = max_steps;
         a.max_time = max_time;
         a.time_float = time_float;
-        if (r->prec == ASAT_F64 ? small_run<double>(r, a) : small_run<float>(r, a)) {
+        if (r->prec == ASAT_F64 ? small_run<double>(r, a, grid) : small_run<float>(r, a, grid)) {
             out->result = r->h_solve->result;
             out->steps = r->h_solve->solver_steps;
             out->last_violations = r->h_solve->last_viol;

@@ -209,7 +209,8 @@ int asat_rk_step(asat_rk_t* rk, asat_state_t* old_state, asat_state_t* new_state
    FP32, run in one of 8 to 128 workgroups where the device holds that many at once.
    enable = 0 forces the multi-kernel path (13 launches per attempt).
    asat_rk_workgroups reports in how many workgroups of a persistent kernel Step
-   and asat_rk_solve run the configured problem (0: the multi-kernel path);
+   and asat_rk_solve run the configured problem (0: the multi-kernel path; Steps
+   too short to pay for the launch take that too, and the largest problems' Steps);
    asat_rk_uses_one_workgroup whether it fits the single-workgroup kernel and runs
    in one workgroup. */
 int asat_rk_set_one_workgroup(asat_rk_t* rk, int enable);

@@ -93,3 +93,36 @@ def test_a_path_chosen_after_configure():
         got = stepped(sat, rk)
         assert rk.Workgroups() >= 8
         assert np.array_equal(got[0], want[0]) and got[1] == want[1]
+
+
+@pytest.mark.parametrize("prec,n,m,k", [
+    ("f32", 32700, 120000, 3), ("f64", 17000, 40000, 3), ("f32", 20000, 60000, 3), ("f64", 8000, 79000, 4)])
+def test_short_steps_long_steps_and_solves(prec, n, m, k):
+    """Near the end of the few-workgroup path's sizes its calls go by their length:
+    short Steps by the multi-kernel path, long ones by either, solves of short
+    batches on the device.  A mixture of them equals the multi-kernel path alone."""
+    p = A.fastsat(n, m, k, 4)
+    out = []
+    for persistent in (True, False):
+        sat = A.HipSat(prec)
+        sat.SetProblem(p)
+        rk = A.HipRungeKutta()
+        rk.SetEpsilon(1e-6)
+        rk.Configure(sat)
+        rk.SetOneWorkgroup(persistent)
+        assert rk.Workgroups() >= 8 if persistent else rk.Workgroups() == 0
+        old, new = sat.MakeState(), sat.MakeState()
+        old.CopyFrom(np.concatenate([np.random.default_rng(3).uniform(-1, 1, sat.Get_N()),
+                                     np.ones(sat.Get_M())]).astype(sat.dtype))
+        got = []
+        for count in (1, 30, 2):
+            assert rk.Step(old, new, count)
+            r = rk.SolveBatches(old, new, 2, 5, 1e300)
+            assert r.on_device == int(persistent)
+            st = rk.stats()
+            got.append((r.result, r.steps, r.last_violations, st.time, st.hdid, st.hnext, st.attempts, st.rhscount,
+                        old.CopyTo()))
+        out.append(got)
+    for a, b in zip(*out):
+        assert a[:-1] == b[:-1]
+        assert np.array_equal(a[-1], b[-1])
