@@ -2390,11 +2390,19 @@ static void state_set_public(State* st, const void* pub)
 
 // N = 1e6, M = 4.2e6, FP32: 10.5 ms with the clause weights permuted on
 // the host through a second buffer, 1.6 ms now (a 21 MB copy into memory
-// the caller has not touched yet)
+// the caller has not touched yet).  Weights in clause order are copied as they lie:
+// through the block, N = 5000, M = 5000, 2 literals takes 27 us instead of 22.
 static void state_get_public(const State* st, void* pub)
 {
     state_check(st);
     Sys* s = st->sys;
+    if (s->perm.empty()) {
+        const size_t e = (size_t)s->esize;
+        HIP_CHECK(hipStreamSynchronize(s->stream));
+        HIP_CHECK(hipMemcpy(pub, (const char*)st->d + e, e * s->n, hipMemcpyDeviceToHost));
+        HIP_CHECK(hipMemcpy((char*)pub + e * s->n, (const char*)st->d + e * s->aoff, e * s->m, hipMemcpyDeviceToHost));
+        return;
+    }
     std::lock_guard<std::mutex> lock(s->public_lock);
     void* blk = public_block(s);
     const size_t len = (size_t)s->n + s->m;
