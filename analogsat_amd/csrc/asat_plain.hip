@@ -1938,7 +1938,8 @@ static void upload(V*& d, const std::vector<V>& h)
 // 256 (one workgroup per CU per round), at least 256 groups while groups
 // keep 128+ variables (4-SAT, N = 20 011, M = 196 107: 143 us per attempt with
 // FP64 and 115 with FP32, against 152 and 120 with 256+; sizes with 256 groups
-// either way are the same); halved until the largest region fits in LDS.  When no
+// either way are the same); halved until the largest region fits in LDS (counted
+// with two bytes more per entry, from when the pass kept offsets beside it).  When no
 // size fits (a variable with more occurrences than the LDS holds), the gather
 // var pass runs with ~400 KB regions.
 // LDS of the region var pass: the longest group's slot list, a place for entries
@@ -2159,7 +2160,7 @@ static void build_grid(Sys* s, const std::vector<int>& lit)
 
 // The layout, at the first integrator that can use it: a system that only serves
 // GetDerivatives, the tanh family or a bias term never pays for it (N = 2000,
-// M = 8500: 0.54 ms of SetProblem's 1.7).  Integrators of one system may ask from
+// M = 8500 0.5 ms, N = 24 000, M = 102 000 3 ms).  Integrators of one system may ask from
 // several threads.  Without memory for it the problem goes without.
 static void ensure_grid(Sys* s)
 {
@@ -2767,12 +2768,7 @@ static void rk_configure(RK* r, Sys* s)
     rk_reset(r);
 }
 
-// Stage arguments of the integrator.  With slot spins (tiled clause pass and
-// LDS var pass), contrib is first filled with the slot spins of the current
-// state x, which the caller may have changed since the last Step.  Inside
-// Step the var passes keep contrib holding the next clause pass's spins: a
-// rejected attempt's J = 1 clause pass is skipped, and its J = 1 var pass
-// (which reuses k1 and reads no contributions) writes stage 2's spins.
+// the tanh table of a state, where the passes use one
 template <typename T>
 static void fill_tanh(const StageArgs<T>& a, const T* x, hipStream_t st)
 {
@@ -2781,6 +2777,12 @@ static void fill_tanh(const StageArgs<T>& a, const T* x, hipStream_t st)
     HIP_CHECK(hipGetLastError());
 }
 
+// Stage arguments of the integrator.  With slot spins (tiled clause pass and
+// LDS var pass), contrib is first filled with the slot spins of the current
+// state x, which the caller may have changed since the last Step.  Inside
+// Step the var passes keep contrib holding the next clause pass's spins: a
+// rejected attempt's J = 1 clause pass is skipped, and its J = 1 var pass
+// (which reuses k1 and reads no contributions) writes stage 2's spins.
 template <typename T>
 static StageArgs<T> rk_stage_args(RK* r, int parity)
 {

@@ -231,10 +231,10 @@ int asat_rk_set_grid_limits(asat_rk_t* rk, int workgroups, int attempts, int lau
    step-size underflow.  `time` is the integrator's time, compared as a float
    when time_float != 0 (TFloat = float); the solver's step count starts at 0,
    the integrator's counters continue (SatSolver::Solve configures the
-   integrator first).  Problems whose whole integrator fits in one
-   workgroup's LDS (and use no bias term) run the loop inside one persistent
-   kernel with no host round trip per batch; others run it on the host over
-   asat_rk_step and asat_sys_violations.  Same results either way.  No
+   integrator first).  Problems that a persistent kernel takes (see
+   asat_rk_set_one_workgroup) run the loop inside it with no host round trip per
+   batch, but for the largest of them with long batches; others run it on the host
+   over asat_rk_step and asat_sys_violations.  Same results either way.  No
    reference counterpart as one call (the reference loops on the host). */
 typedef struct {
     int result;              /* SatResult code (AnalogSAT/solver/SatResult.h:24-32) */
