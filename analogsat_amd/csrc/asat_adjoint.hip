@@ -812,13 +812,15 @@ static void alloc_batch(Adj& A, int ntraj)
     HIP_CHECK(hipMalloc((void**)&A.ctl, sizeof(TCtl) * ntraj));
     HIP_CHECK(hipMalloc((void**)&A.hstep, sizeof(double) * ntraj));
     HIP_CHECK(hipMalloc((void**)&A.eparts, sizeof(double) * (size_t)ntraj * (nblk + nblkv)));
-    HIP_CHECK(hipMemset(A.seg, 0, sizeof(float) * V * (A.C + 1)));
-    HIP_CHECK(hipMemset(A.Y, 0, sizeof(float) * V * 6));
-    HIP_CHECK(hipMemset(A.kk, 0, sizeof(float) * V * 6));
-    HIP_CHECK(hipMemset(A.lam, 0, sizeof(double) * V));
+    // (on the kernels' stream: a plain hipMemset returns before it is done, on a
+    // stream that theirs does not wait for)
+    HIP_CHECK(hipMemsetAsync(A.seg, 0, sizeof(float) * V * (A.C + 1), A.stream));
+    HIP_CHECK(hipMemsetAsync(A.Y, 0, sizeof(float) * V * 6, A.stream));
+    HIP_CHECK(hipMemsetAsync(A.kk, 0, sizeof(float) * V * 6, A.stream));
+    HIP_CHECK(hipMemsetAsync(A.lam, 0, sizeof(double) * V, A.stream));
     // the last one: its presence says that all are there
     HIP_CHECK(hipMalloc((void**)&A.ckpt, sizeof(float) * V * A.ncheck));
-    HIP_CHECK(hipMemset(A.ckpt, 0, sizeof(float) * V * A.ncheck));
+    HIP_CHECK(hipMemsetAsync(A.ckpt, 0, sizeof(float) * V * A.ncheck, A.stream));
 }
 
 // start states, public rows on the host, into x; stage: ntraj (n + m) values on

@@ -1769,7 +1769,7 @@ static void configure_bucket(Batch& B, Bucket& b, int bs, int mode, int grid_cap
     b.d_scratch = nullptr;
     const size_t sbytes = sizeof(float) * std::max<size_t>((size_t)b.scratch_per_wg * b.grid, 1);
     HIP_CHECK(hipMalloc((void**)&b.d_scratch, sbytes));
-    HIP_CHECK(hipMemset(b.d_scratch, 0, sbytes));
+    HIP_CHECK(hipMemsetAsync(b.d_scratch, 0, sbytes, B.stream));
     const void* f = mode == 2   ? reg_kernel(*b.reg, b.kk)
                     : mode == 3 ? chunk_kernel(bs)
                     : mode == 1 ? kernel_of<1>(bs)

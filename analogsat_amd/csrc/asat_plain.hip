@@ -2289,7 +2289,7 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
             // one term per clause padded to whole tiles, plus a 16-byte unit
             const size_t np = mpad + 16;
             HIP_CHECK(hipMalloc(&s->d_pcontrib, (size_t)s->esize * np));
-            HIP_CHECK(hipMemset(s->d_pcontrib, 0, (size_t)s->esize * np));
+            HIP_CHECK(hipMemsetAsync(s->d_pcontrib, 0, (size_t)s->esize * np, s->stream));
         }
     } else {
         s->mq = 0;
@@ -2329,9 +2329,9 @@ static void sys_set_problem(Sys* s, const int* lits, const int* lens, int nclaus
     s->perm = std::move(P.perm);
     const size_t ncontrib = (size_t)P.gstart[P.ngroups] + REGION_ALIGN;
     HIP_CHECK(hipMalloc(&s->d_contrib, (size_t)s->esize * ncontrib));
-    HIP_CHECK(hipMemset(s->d_contrib, 0, (size_t)s->esize * ncontrib));
+    HIP_CHECK(hipMemsetAsync(s->d_contrib, 0, (size_t)s->esize * ncontrib, s->stream));
     HIP_CHECK(hipMalloc((void**)&s->d_apart, sizeof(double) * clause_grid(s)));
-    HIP_CHECK(hipMemset(s->d_apart, 0, sizeof(double) * clause_grid(s)));
+    HIP_CHECK(hipMemsetAsync(s->d_apart, 0, sizeof(double) * clause_grid(s), s->stream));
     // up to 512 clauses and variables asat_small.h is the faster one
     s->grid_due = tiled && (s->small_lds == 0 || std::max(P.m, P.n) > 512);
     s->ready = true;
@@ -2744,18 +2744,20 @@ static void rk_configure(RK* r, Sys* s)
     r->gen = s->gen;
     r->prec = s->prec;
     const size_t bytes = (size_t)s->esize * s->alloc;
+    // clears on the kernels' stream: a plain hipMemset returns before it is done, on a
+    // stream that theirs does not wait for
     for (auto& p : r->k) {
         HIP_CHECK(hipMalloc(&p, bytes));
-        HIP_CHECK(hipMemset(p, 0, bytes));
+        HIP_CHECK(hipMemsetAsync(p, 0, bytes, s->stream));
     }
     HIP_CHECK(hipMalloc(&r->tmp, (size_t)s->esize * (s->n + 1)));
     r->tmp_n = s->n;
-    HIP_CHECK(hipMemset(r->tmp, 0, (size_t)s->esize * (s->n + 1)));
+    HIP_CHECK(hipMemsetAsync(r->tmp, 0, (size_t)s->esize * (s->n + 1), s->stream));
     r->npartial = npartial;
     HIP_CHECK(hipMalloc((void**)&r->partial, sizeof(double) * r->npartial));
-    HIP_CHECK(hipMemset(r->partial, 0, sizeof(double) * r->npartial));
+    HIP_CHECK(hipMemsetAsync(r->partial, 0, sizeof(double) * r->npartial, s->stream));
     HIP_CHECK(hipMalloc((void**)&r->d_ctrl, sizeof(CtrlBlock)));
-    HIP_CHECK(hipMemset(r->d_ctrl, 0, sizeof(CtrlBlock)));
+    HIP_CHECK(hipMemsetAsync(r->d_ctrl, 0, sizeof(CtrlBlock), s->stream));
     HIP_CHECK(hipHostMalloc((void**)&r->h_ctrl, sizeof(CtrlBlock), hipHostMallocDefault));
     memset((void*)r->h_ctrl, 0, sizeof(CtrlBlock));
     HIP_CHECK(hipMalloc((void**)&r->d_solve, sizeof(SmallSolve)));
