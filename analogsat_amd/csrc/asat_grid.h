@@ -38,7 +38,7 @@
 // 4.7-5.1 against 4.6), so those keep asat_small.h.
 //
 // The layout is used where the device holds all its workgroups at once, and the
-// launch is cooperative. Where they wait for each other all the same (another
+// launch is cooperative where the runtime grants it. Where they wait for each other all the same (another
 // process keeps part of the CUs busy), a wait that lasts GRID_POLLS polls gives
 // up: it marks the arrival word unless the last arrival came in between, so
 // every workgroup gives up at the same exchange, and none stores anything. The

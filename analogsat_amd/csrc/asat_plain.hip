@@ -2005,18 +2005,17 @@ static void build_small_lists(Sys* s, const HostProblem& P)
 constexpr int GRID_CPT_F64 = 4, GRID_CPT_F32 = 8;
 constexpr long long GRID_LDS = 158 * 1024;     // beside the kernel's 0.3 KB of static LDS
 
-// Workgroups of the kernel that the device holds at once; 0 where it cannot
-// launch cooperatively.  A whole MI355X has 256 CUs and holds the largest layout
-// twice, a partition of it may have fewer than the layout has workgroups.
-static int grid_resident(const void* f, size_t lds)
+// Workgroups of 1024 threads that the device holds at once: one on each CU (the
+// kernels use more than half of the registers).  An MI355X has 256 CUs, a partition of it may have fewer than a
+// layout has workgroups.  (The runtime's occupancy query is no guide: with a second
+// ROCm's libraries loaded before the first GPU call, as PyTorch's are when imported in
+// between, it counts half the registers and finds room for none.)
+static int grid_resident()
 {
-    int dev = 0, coop = 0, ncu = 0, per_cu = 0;
+    int dev = 0, ncu = 0;
     HIP_CHECK(hipGetDevice(&dev));
-    HIP_CHECK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
     HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    if (!f || !coop) return 0;
-    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, GRID_BT, lds));
-    return per_cu * ncu;
+    return ncu;
 }
 
 // lit: m K literals in processing order, as SetProblem left them
@@ -2095,7 +2094,7 @@ static void build_grid(Sys* s, const std::vector<int>& lit)
     const void* f = grid_kernel(s->prec, K, kcpt, G == 1);
     require(f != nullptr, ASAT_ERR_HIP, "no few-workgroup kernel for this layout");
     HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GRID_LDS));
-    if (G > 1 && grid_resident(f, (size_t)lds) < G) return;
+    if (G > 1 && grid_resident() < G) return;
     // term entry of every slot in its variable's workgroup: the variable's clauses
     // in input order, literals in clause order (the reference's accumulation order)
     std::vector<int> visit((size_t)m), fill((size_t)nranks), entry(slots);
@@ -2631,6 +2630,7 @@ struct RK {
     SmallSolve* h_solve = nullptr;   // pinned mirror
     void* d_grid = nullptr;          // exchange buffers of the few-workgroup path
     size_t grid_bytes = 0;
+    bool grid_plain = false;         // launched without the runtime's cooperation, see grid_launch
     bool grid_off = false;           // its workgroups did not all run, or it had no memory: not tried again for
                                      // this problem
     // test limits (asat_rk_set_grid_limits)
@@ -3066,22 +3066,34 @@ static bool grid_args(RK* r, const SmallArgs& a, GridArgs& g)
     return true;
 }
 
-// give_up: the workgroups find the arrival word marked
-static void grid_launch(RK* r, GridArgs& g, bool give_up)
+// One launch of the few-workgroup kernel, cooperative where the runtime grants that:
+// it takes one such kernel of a process at a time, and launches of several threads
+// then never share the CUs out between them.  It grants it to one process on a GPU
+// (the next one's launches fail, with "the operation cannot be performed in the
+// present state"); there an ordinary launch does, of one thread at a time (alone,
+// held until the kernel has ended), and the bounded wait covers what other processes
+// run.  give_up: the workgroups find the arrival word marked.
+static std::mutex grid_alone;
+static void grid_launch(RK* r, GridArgs& g, bool give_up, std::unique_lock<std::mutex>& alone)
 {
     Sys* s = r->sys;
     const bool solo = s->grid_wgs == 1;
     const void* f = grid_kernel(s->prec, s->k, s->grid_cpt, solo);
+    const dim3 grid(s->grid_wgs), block(GRID_BT);
     void* args[] = {&g};
-    if (solo) {
-        HIP_CHECK(hipLaunchKernel(f, dim3(1), dim3(GRID_BT), args, (size_t)s->grid_lds, s->stream));
-        return;
+    if (!solo) {
+        // every launch counts on from the last one
+        if (r->h_arrived() >= GRID_GIVE_UP / 2) r->clear_arrived(s->stream);
+        g.phase = r->h_arrived() / (unsigned)s->grid_wgs;
+        if (give_up) HIP_CHECK(hipMemsetD32Async((hipDeviceptr_t)g.barrier, (int)GRID_GIVE_UP, 1, s->stream));
+        if (!r->grid_plain) {
+            if (hipLaunchCooperativeKernel(f, grid, block, args, (unsigned)s->grid_lds, s->stream) == hipSuccess) return;
+            (void)hipGetLastError();
+            r->grid_plain = true;
+        }
+        alone = std::unique_lock<std::mutex>(grid_alone);
     }
-    // every launch counts on from the last one
-    if (r->h_arrived() >= GRID_GIVE_UP / 2) r->clear_arrived(s->stream);
-    g.phase = r->h_arrived() / (unsigned)s->grid_wgs;
-    if (give_up) HIP_CHECK(hipMemsetD32Async((hipDeviceptr_t)g.barrier, (int)GRID_GIVE_UP, 1, s->stream));
-    HIP_CHECK(hipLaunchCooperativeKernel(f, dim3(s->grid_wgs), dim3(GRID_BT), args, (unsigned)s->grid_lds, s->stream));
+    HIP_CHECK(hipLaunchKernel(f, grid, block, args, (size_t)s->grid_lds, s->stream));
 }
 
 // Launches a persistent kernel (grid: the few-workgroup one) until it reports done: each
@@ -3105,11 +3117,13 @@ static bool small_run(RK* r, const SmallArgs& a, bool grid)
     HIP_CHECK(hipEventRecord(r->ev0, st));
     long long last = r->h_ctrl->attempts;
     for (int launch = 0;; launch++) {
-        if (grid) grid_launch(r, g, launch == r->grid_launches);
+        std::unique_lock<std::mutex> alone;
+        if (grid) grid_launch(r, g, launch == r->grid_launches, alone);
         else small_launch<T>(s, a, st);
         HIP_CHECK(hipMemcpyAsync(r->h_ctrl, r->d_ctrl, grid ? sizeof(CtrlBlock) : sizeof(Ctrl), hipMemcpyDeviceToHost, st));
         if (a.solve) HIP_CHECK(hipMemcpyAsync(r->h_solve, r->d_solve, sizeof(SmallSolve), hipMemcpyDeviceToHost, st));
         HIP_CHECK(hipStreamSynchronize(st));
+        if (alone.owns_lock()) alone.unlock();
         if (grid && (r->h_arrived() & GRID_GIVE_UP)) {
             r->clear_arrived(st);
             r->grid_off = true;

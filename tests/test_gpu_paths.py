@@ -1,5 +1,8 @@
 """Which integrator runs: the number of workgroups that the query reports, for sizes
 on both sides of each rule and for the settings that rule a path out."""
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -126,3 +129,46 @@ def test_short_steps_long_steps_and_solves(prec, n, m, k):
     for a, b in zip(*out):
         assert a[:-1] == b[:-1]
         assert np.array_equal(a[-1], b[-1])
+
+
+@pytest.mark.parametrize("first", ["import torch", "pass"])
+def test_second_process(first):
+    """A process beside this one, which holds the runtime's one cooperative queue
+    of the GPU; also with torch imported between loading the library and its first
+    GPU call, where the runtime's occupancy query finds no room for 1024 threads."""
+    sat, rk = configured("f32", 2000, 8500)
+    want = stepped(sat, rk)
+    code = '''
+import sys, threading
+sys.path.insert(0, %r)
+import numpy as np
+import analogsat_amd as A
+A.lib()
+%s
+out = {}
+def go(i, persistent):
+    sat = A.HipSat("f32")
+    sat.SetProblem(A.fastsat(2000, 8500, 3, 2))
+    rk = A.HipRungeKutta()
+    rk.Configure(sat)
+    rk.SetOneWorkgroup(persistent)
+    assert (rk.Workgroups() >= 8) == persistent, rk.Workgroups()
+    old, new = sat.MakeState(), sat.MakeState()
+    old.CopyFrom(np.concatenate([np.random.default_rng(3).uniform(-1, 1, sat.Get_N()), np.ones(sat.Get_M())]).astype("f4"))
+    assert rk.Step(old, new, 20)
+    r = rk.SolveBatches(old, new, 5, 20, 1e300)
+    assert r.on_device == int(persistent), r.on_device
+    out[i] = old.CopyTo()
+go(0, False)
+go(1, True)
+threads = [threading.Thread(target=go, args=(i, True)) for i in (2, 3)]
+for t in threads: t.start()
+for t in threads: t.join()
+assert all(np.array_equal(out[0], out[i]) for i in (1, 2, 3))
+print("same")
+''' % (os.path.dirname(os.path.dirname(os.path.abspath(A.__file__))), first)
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=90)
+    assert r.returncode == 0 and "same" in r.stdout, r.stdout + r.stderr
+    rk.Reset()
+    again = stepped(sat, rk)
+    assert np.array_equal(want[0], again[0]) and want[1] == again[1]
