@@ -167,7 +167,7 @@ for t in threads: t.join()
 assert all(np.array_equal(out[0], out[i]) for i in (1, 2, 3))
 print("same")
 ''' % (os.path.dirname(os.path.dirname(os.path.abspath(A.__file__))), first)
-    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=90)
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=180)
     assert r.returncode == 0 and "same" in r.stdout, r.stdout + r.stderr
     rk.Reset()
     again = stepped(sat, rk)
